@@ -193,7 +193,7 @@ int run_knn(mnrt_batch& b, const mnrt_batch_io& io, hipStream_t st) {
     G.out_count = io.d_out_count;
     return launch_knn_batch(G, b.d_knn, b.d_slot_begin, b.ns, io.d_sp_count, b.tun.knn_chunk, b.tun.parts,
                             b.d_tparts + 2 * kMaxParts, b.d_tparts + 3 * kMaxParts, b.d_work + kMaxParts,
-                            b.tun.knn_cap, b.tun.knn_waves, b.tun.knn_select, b.tun.knn_grid, st);
+                            b.tun.knn_cap, b.tun.knn_waves, b.tun.knn_grid, st);
 }
 
 // Accumulators of the adjoint phase for the current photon counts (synchronous; never
@@ -556,7 +556,6 @@ extern "C" int mnrt_batch_autotune(mnrt_batch* b, const mnrt_batch_io* io, uint3
     search(MNRT_PHASE_TRACE, &mnrt_batch_tuning::trace_grid, {2 * C, 4 * C, 8 * C, 16 * C, 32 * C});
     if (b->has_knn) {
         const uint32_t c0 = min_cap(b->k);
-        search(MNRT_PHASE_KNN, &mnrt_batch_tuning::knn_select, {0, 1, 2});
         search(MNRT_PHASE_KNN, &mnrt_batch_tuning::knn_cap, {c0, 2 * c0});
         search(MNRT_PHASE_KNN, &mnrt_batch_tuning::knn_waves, {1, 2, 4});
         search(MNRT_PHASE_KNN, &mnrt_batch_tuning::knn_chunk, {1, 4, 16, 64});

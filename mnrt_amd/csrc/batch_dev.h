@@ -118,7 +118,7 @@ struct ShadeBatchArgs {
 int launch_trace_batch(const TraceBatchArgs& B, int stack, uint32_t grid, uint32_t block, hipStream_t st);
 int launch_knn_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* slot_begin, uint32_t ns,
                      const uint32_t* count, uint32_t chunk, uint32_t num_parts, const uint32_t* part_begin,
-                     const uint32_t* part_end, uint32_t* work, uint32_t cap, uint32_t waves, uint32_t sel,
+                     const uint32_t* part_end, uint32_t* work, uint32_t cap, uint32_t waves,
                      uint32_t grid, hipStream_t st);
 int launch_knn_bwd_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* slot_begin, uint32_t ns,
                          const uint32_t* count, const uint32_t* photon_begin, uint32_t total_photons,

@@ -16,10 +16,10 @@
 //     whose photons can be taken: exact;
 //   * a leaf's photon records are contiguous, so its photons are tested one per lane
 //     with one coalesced 16-byte buffer load each (bounded at the leaf's end);
-//   * candidates (key = d2 bits << 32 | photon index, so integer order is (d2, index)
-//     order) are appended to a per-wave LDS buffer with ballot + mbcnt compaction; when
-//     k are known or the buffer would overflow, the k best are kept (radix selection of
-//     the k-th key, or a bitonic sort) and the pruning threshold tightens;
+//   * candidates (d2 bits << 32 | record position) are appended to a per-wave LDS buffer
+//     with ballot + mbcnt compaction; when k are known or the buffer would overflow, the
+//     candidates above a threshold are dropped (at least k stay) and the pruning limit
+//     tightens; the exact k best, ties by photon index, are selected once at the end;
 //   * the final set is sorted only when the caller asks for the neighbour lists; each
 //     lane fetches the records of its slots and the front-facing powers are summed per
 //     channel as exact 64-bit fixed-point integers (the reference adds floats in its
@@ -52,9 +52,8 @@ constexpr int kBufferWord3 = 0x00020000;
 
 enum : int { kModeRadii = 0, kModeRadiance = 1, kModeBackward = 2 };
 
-// Sorts keys[0..size) ascending (positions follow their keys), size a power of two.
-template <int CAP>
-__device__ __forceinline__ void wave_bitonic(uint64_t* keys, uint32_t* pos, uint32_t size, uint32_t lane) {
+// Sorts keys[0..size) ascending, size a power of two.
+__device__ __forceinline__ void wave_bitonic(uint64_t* keys, uint32_t size, uint32_t lane) {
     for (uint32_t k2 = 2; k2 <= size; k2 <<= 1) {
         for (uint32_t j = k2 >> 1; j > 0; j >>= 1) {
             for (uint32_t t = lane; t < (size >> 1); t += 64) {
@@ -65,9 +64,6 @@ __device__ __forceinline__ void wave_bitonic(uint64_t* keys, uint32_t* pos, uint
                 if ((a > b) == asc) {
                     keys[i] = b;
                     keys[l] = a;
-                    uint32_t pa = pos[i];
-                    pos[i] = pos[l];
-                    pos[l] = pa;
                 }
             }
             wave_sync();
@@ -118,86 +114,96 @@ __device__ __forceinline__ uint32_t pow2_at_least(uint32_t v) {
     return p;
 }
 
-// Selection of the k best candidates when the buffer fills up:
-//   kSelSort  : wave-wide bitonic sort of the buffer, keep the first k;
-//   kSelRadix : the k-th smallest key by a wave-wide binary search over its bits (count of
-//               keys below a probe: one ballot per key slot), then compaction of the keys
-//               up to it, unsorted; the final set is sorted once at the end.
-//   kSelWindow: intermediate selections keep any set of at least k and at most CAP - 64
-//               keys below a high-word threshold (a short binary search); the exact k
-//               best are selected once, at the end, as kSelRadix does.
-enum : int { kSelSort = 0, kSelRadix = 1, kSelWindow = 2 };
+// Candidates are d2 bits << 32 | record position.  The photon index, which breaks ties of
+// d2, is in the record and read only when a tie straddles the k-th place, so a candidate
+// costs one 8-byte LDS write.
 
-// k-th smallest (1-based) of the keys held R per lane (~0 for empty slots), wave-uniform;
-// the largest v with count(key < v) < k.
+// Masks of the k smallest (d2, photon index) among the candidates held R per lane (d2 bits h,
+// ~0 in empty slots; record positions pos), k < their number.  Bisection over the d2 bits,
+// one ballot per slot and probe, that ends at the first probe with exactly k candidates below
+// it: distances are mostly distinct, so that takes about log2 of the number of candidates
+// and not the 20 to 25 steps down to the k-th distance's last bit (with the 8-byte candidates,
+// 2.07M bounce-hit queries, k = 100, 1M photons: 5.12 -> 4.69 ms; 4067 queries, k = 50: 99 -> 92 us).  Returns the k-th d2's bits.
 template <int R>
-__device__ __forceinline__ uint64_t wave_kth_key(const uint64_t (&key)[R], uint32_t k) {
-    // high word (d2 bits) first, then the low word (photon index) among the ties.  Every
-    // key's high word lies in [hmin, hmax], so the answer shares their common leading
-    // bits and the search starts below the highest bit in which they differ.
+__device__ __forceinline__ uint32_t wave_select_k(const uint32_t (&h)[R], const uint32_t (&pos)[R], uint32_t k,
+                                                  const float4* __restrict__ recs, uint64_t (&keep)[R]) {
+    // every candidate's d2 bits lie in [hmin, hmax], so the answer shares their common leading
+    // bits and the search starts at the highest bit in which they differ
     uint32_t hmin = 0xFFFFFFFFu, hmax = 0u;
 #pragma unroll
     for (int t = 0; t < R; ++t) {
-        if (key[t] != ~0ull) {
-            hmin = min(hmin, (uint32_t)(key[t] >> 32));
-            hmax = max(hmax, (uint32_t)(key[t] >> 32));
-        }
+        hmin = min(hmin, h[t]);
+        hmax = max(hmax, h[t] != 0xFFFFFFFFu ? h[t] : 0u);
     }
     hmin = wave_min_u32(hmin);
     hmax = wave_max_u32(hmax);
     const uint32_t differ = hmin ^ hmax;
-    const int top = differ ? 31 - __clz(differ) : -1;
-    uint32_t hi = (top < 0) ? hmin : (top >= 31) ? 0u : (hmin & ~((2u << top) - 1u));
-    for (int b = top; b >= 0; --b) {
-        const uint32_t probe = hi | (1u << b);
-        uint32_t c = 0;
+    uint32_t hi = hmin;
+    if (differ != 0u) {
+        const int top = 31 - __clz(differ);
+        hi = hmin & ~((2u << top) - 1u);
+        for (int b = top; b >= 0; --b) {
+            const uint32_t probe = hi | (1u << b);
+            uint32_t c = 0;
 #pragma unroll
-        for (int t = 0; t < R; ++t) c += (uint32_t)__popcll(ballot((uint32_t)(key[t] >> 32) < probe));
-        if (c < k) hi = probe;
+            for (int t = 0; t < R; ++t) {
+                keep[t] = ballot(h[t] < probe);
+                c += (uint32_t)__popcll(keep[t]);
+            }
+            if (c == k) {
+                uint32_t m = 0;
+#pragma unroll
+                for (int t = 0; t < R; ++t) m = max(m, h[t] < probe ? h[t] : 0u);
+                return wave_max_u32(m);
+            }
+            if (c < k) hi = probe;
+        }
     }
+    // hi is the k-th d2 and more than one candidate has it
     uint32_t below = 0, tie = 0;
+    uint64_t eq[R];
 #pragma unroll
     for (int t = 0; t < R; ++t) {
-        const uint32_t h = (uint32_t)(key[t] >> 32);
-        below += (uint32_t)__popcll(ballot(h < hi));
-        tie += (uint32_t)__popcll(ballot(h == hi));
+        keep[t] = ballot(h[t] < hi);
+        eq[t] = ballot(h[t] == hi);
+        below += (uint32_t)__popcll(keep[t]);
+        tie += (uint32_t)__popcll(eq[t]);
     }
     const uint32_t need = k - below;  // 1 <= need <= tie
-    if (need == tie) {
-        // every tie is kept: the threshold is the largest tie
-        uint32_t lo = 0;
+    if (need < tie) {
+        uint32_t idx[R];  // photon indices of the ties; the `need` lowest are kept
 #pragma unroll
-        for (int t = 0; t < R; ++t) lo = max(lo, ((uint32_t)(key[t] >> 32) == hi) ? (uint32_t)key[t] : 0u);
-        return ((uint64_t)hi << 32) | wave_max_u32(lo);
+        for (int t = 0; t < R; ++t) {
+            idx[t] = 0xFFFFFFFFu;
+            if (__builtin_amdgcn_inverse_ballot_w64(eq[t])) idx[t] = __float_as_uint(recs[2ull * pos[t]].w);
+        }
+        uint32_t lo = 0;  // the need-th lowest index
+        for (int b = 31; b >= 0; --b) {
+            const uint32_t probe = lo | (1u << b);
+            uint32_t c = 0;
+#pragma unroll
+            for (int t = 0; t < R; ++t) c += (uint32_t)__popcll(eq[t] & ballot(idx[t] < probe));
+            if (c < need) lo = probe;
+        }
+#pragma unroll
+        for (int t = 0; t < R; ++t) eq[t] &= ballot(idx[t] <= lo);
     }
-    uint64_t eq[R];  // slots whose high word ties (separate ballots: a ballot of a && b costs two more)
 #pragma unroll
-    for (int t = 0; t < R; ++t) eq[t] = ballot((uint32_t)(key[t] >> 32) == hi);
-    uint32_t lo = 0;
-    for (int b = 31; b >= 0; --b) {
-        const uint32_t probe = lo | (1u << b);
-        uint32_t c = 0;
-#pragma unroll
-        for (int t = 0; t < R; ++t) c += (uint32_t)__popcll(eq[t] & ballot((uint32_t)key[t] < probe));
-        if (c < need) lo = probe;
-    }
-    return ((uint64_t)hi << 32) | lo;
+    for (int t = 0; t < R; ++t) keep[t] |= eq[t];
+    return hi;
 }
 
 // A pruning threshold on the high word (d2 bits) that keeps between k and hi_k of the cnt
-// keys held R per lane (~0 for empty slots): *upper = count(h <= T).  Binary search over
+// candidates' d2 bits h held R per lane (~0 for empty slots): *upper = count(h <= T).  Binary search over
 // the high word that stops as soon as the keys at or below the range top number at most
 // hi_k (far fewer steps than the exact k-th); *upper > hi_k means ties made it impossible.
 template <int R>
-__device__ __forceinline__ uint32_t wave_window_hi(const uint64_t (&key)[R], uint32_t k, uint32_t hi_k, uint32_t cnt,
+__device__ __forceinline__ uint32_t wave_window_hi(const uint32_t (&h)[R], uint32_t k, uint32_t hi_k, uint32_t cnt,
                                                    uint32_t* upper_out) {
     if (cnt <= hi_k) {
         uint32_t m = 0;
 #pragma unroll
-        for (int t = 0; t < R; ++t) {
-            const uint32_t h = (uint32_t)(key[t] >> 32);
-            m = max(m, h != 0xFFFFFFFFu ? h : 0u);
-        }
+        for (int t = 0; t < R; ++t) m = max(m, h[t] != 0xFFFFFFFFu ? h[t] : 0u);
         *upper_out = cnt;
         return wave_max_u32(m);
     }
@@ -209,7 +215,7 @@ __device__ __forceinline__ uint32_t wave_window_hi(const uint64_t (&key)[R], uin
         const uint32_t probe = prefix + (uint32_t)width;
         uint32_t c = 0;
 #pragma unroll
-        for (int t = 0; t < R; ++t) c += (uint32_t)__popcll(ballot((uint32_t)(key[t] >> 32) < probe));
+        for (int t = 0; t < R; ++t) c += (uint32_t)__popcll(ballot(h[t] < probe));
         if (c >= k) upper = c;
         else prefix = probe;
     }
@@ -266,10 +272,10 @@ __device__ __forceinline__ float warm_bound(const WarmHint& h, float qx, float q
     return b2 < r2max ? __uint_as_float(__float_as_uint(b2) + 1u) : r2max;
 }
 
-// One query by one wave; keys / kpos: CAP LDS entries, snode / soff: kKnnStack.
-template <int CAP, int kMode, int kSel = kSelSort, bool kPairs = false>
+// One query by one wave; cand: CAP LDS entries, snode / soff: kKnnStack.
+template <int CAP, int kMode>
 __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, uint32_t q, uint32_t lane,
-                                          uint64_t* keys, uint32_t* kpos, uint32_t* snode, float4* soff,
+                                          uint64_t* cand, uint32_t* snode, float4* soff,
                                           const PairSink* sink = nullptr, WarmHint* hint = nullptr) {
     const float4 qp4 = A.pos[q];
     const float qx = uniformf(qp4.x), qy = uniformf(qp4.y), qz = uniformf(qp4.z);
@@ -321,101 +327,71 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, u
     };
     auto set_rest = [&]() { rlane = lane == 0 ? oy2 + oz2 : (lane == 1 ? ox2 + oz2 : ox2 + oy2); };
 
-    // sorts the buffer and keeps the first `keep`
-    auto sort_keep = [&](uint32_t keep) {
-        uint32_t size = pow2_at_least(cnt);
-        for (uint32_t t = cnt + lane; t < size; t += 64) {
-            keys[t] = ~0ull;
-            kpos[t] = 0u;
+    // loads the candidates of R slots per lane
+    auto load_cands = [&](auto& h, auto& pos) {
+        constexpr int R = sizeof(h) / sizeof(h[0]);
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const uint32_t i = lane + 64u * t;
+            const uint64_t c = cand[i];
+            h[t] = i < cnt ? (uint32_t)(c >> 32) : 0xFFFFFFFFu;
+            pos[t] = (uint32_t)c;
+        }
+    };
+    // writes the candidates of the masks back, in order, from slot 0
+    auto store_cands = [&](const auto& h, const auto& pos, const auto& keep) {
+        constexpr int R = sizeof(h) / sizeof(h[0]);
+        wave_sync();
+        uint32_t base = 0;
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            if (__builtin_amdgcn_inverse_ballot_w64(keep[t]))
+                cand[mask_prefix_from(keep[t], base)] = ((uint64_t)h[t] << 32) | pos[t];
+            base += (uint32_t)__popcll(keep[t]);
         }
         wave_sync();
-        wave_bitonic<CAP>(keys, kpos, size, lane);
-        if (cnt > keep) cnt = keep;
-        if (cnt == k) {
-            full = true;
-            thr_d2 = __uint_as_float((uint32_t)(keys[k - 1] >> 32));
-            set_limits();
-        }
     };
     // keeps the k best, unsorted (cnt > k)
-    auto radix_keep_slots = [&](auto slots) {
+    auto exact_keep_slots = [&](auto slots) {
         constexpr int R = decltype(slots)::value;
-        uint64_t key[R];
-        uint32_t pos[R];
-#pragma unroll
-        for (int t = 0; t < R; ++t) {
-            const uint32_t i = lane + 64u * t;
-            key[t] = i < cnt ? keys[i] : ~0ull;
-            pos[t] = i < cnt ? kpos[i] : 0u;
-        }
-        const uint64_t kth = wave_kth_key<R>(key, k);
-        wave_sync();
-        uint32_t base = 0;
-#pragma unroll
-        for (int t = 0; t < R; ++t) {
-            const bool keepit = key[t] <= kth;
-            const uint64_t m = ballot(keepit);
-            if (keepit) {
-                const uint32_t slot = base + mask_prefix(m);
-                keys[slot] = key[t];
-                kpos[slot] = pos[t];
-            }
-            base += (uint32_t)__popcll(m);
-        }
-        wave_sync();
+        uint32_t h[R], pos[R];
+        uint64_t keep[R];
+        load_cands(h, pos);
+        thr_d2 = __uint_as_float(wave_select_k<R>(h, pos, k, Tr.recs, keep));
+        store_cands(h, pos, keep);
         cnt = k;
         full = true;
-        thr_d2 = __uint_as_float((uint32_t)(kth >> 32));
         set_limits();
     };
-    // keeps the k best, unsorted (cnt > k); searches only the ceil(cnt / 64) key slots per
-    // lane that hold candidates
-    auto radix_keep = [&]() {
+    // keeps the k best, unsorted (cnt > k); looks only at the ceil(cnt / 64) slots per lane that
+    // hold candidates
+    auto exact_keep = [&]() {
         constexpr int R = CAP / 64;
-        if (R > 2 && cnt <= 128u) radix_keep_slots(std::integral_constant<int, (R > 2 ? 2 : R)>{});
-        else if (R > 3 && cnt <= 192u) radix_keep_slots(std::integral_constant<int, (R > 3 ? 3 : R)>{});
-        else if (R > 4 && cnt <= 256u) radix_keep_slots(std::integral_constant<int, (R > 4 ? 4 : R)>{});
-        else radix_keep_slots(std::integral_constant<int, R>{});
+        if (R > 2 && cnt <= 128u) exact_keep_slots(std::integral_constant<int, (R > 2 ? 2 : R)>{});
+        else if (R > 3 && cnt <= 192u) exact_keep_slots(std::integral_constant<int, (R > 3 ? 3 : R)>{});
+        else if (R > 4 && cnt <= 256u) exact_keep_slots(std::integral_constant<int, (R > 4 ? 4 : R)>{});
+        else exact_keep_slots(std::integral_constant<int, R>{});
     };
-    // keeps at least k and at most CAP - 64 candidates under a high-word threshold
+    // when the buffer fills up: keeps at least k and at most CAP - 64 candidates under a
+    // threshold on d2 (the exact k best are selected once, at the end)
     auto window_keep = [&]() {
         constexpr int R = CAP / 64;
-        uint64_t key[R];
-        uint32_t pos[R];
-#pragma unroll
-        for (int t = 0; t < R; ++t) {
-            const uint32_t i = lane + 64u * t;
-            key[t] = i < cnt ? keys[i] : ~0ull;
-            pos[t] = i < cnt ? kpos[i] : 0u;
-        }
+        uint32_t h[R], pos[R];
+        uint64_t keep[R];
+        load_cands(h, pos);
         uint32_t upper = 0;
-        const uint32_t T = wave_window_hi<R>(key, k, (uint32_t)CAP - 64u, cnt, &upper);
+        const uint32_t T = wave_window_hi<R>(h, k, (uint32_t)CAP - 64u, cnt, &upper);
         if (upper > (uint32_t)CAP - 64u) {  // equal distances: only the exact selection fits
-            radix_keep();
+            exact_keep();
             return;
         }
-        wave_sync();
-        uint32_t base = 0;
 #pragma unroll
-        for (int t = 0; t < R; ++t) {
-            const uint64_t m = ballot((uint32_t)(key[t] >> 32) <= T) & ballot(key[t] != ~0ull);
-            if (__builtin_amdgcn_inverse_ballot_w64(m)) {
-                const uint32_t slot = base + mask_prefix(m);
-                keys[slot] = key[t];
-                kpos[slot] = pos[t];
-            }
-            base += (uint32_t)__popcll(m);
-        }
-        wave_sync();
+        for (int t = 0; t < R; ++t) keep[t] = ballot(h[t] <= T);
+        store_cands(h, pos, keep);
         cnt = upper;
         full = true;
         thr_d2 = __uint_as_float(T);
         set_limits();
-    };
-    auto select = [&](uint32_t keep) {
-        if (kSel == kSelWindow) window_keep();
-        else if (kSel == kSelRadix && cnt > keep) radix_keep();
-        else sort_keep(keep);
     };
 
     for (;;) {  // a second pass with r_max only if the warm-start bound held fewer than k
@@ -466,19 +442,18 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, u
                 uint32_t nm = (uint32_t)__popcll(m);
                 if (nm == 0) continue;
                 if (cnt + nm > (uint32_t)CAP) {
-                    select(k);
+                    window_keep();
                     m &= ballot(d2 < tlim);
                     nm = (uint32_t)__popcll(m);
                 }
                 if (__builtin_amdgcn_inverse_ballot_w64(m)) {
                     const uint32_t slot = mask_prefix_from(m, cnt);
-                    keys[slot] = ((uint64_t)__float_as_uint(d2) << 32) | (uint64_t)w[3];
-                    kpos[slot] = begin + base + lane;
+                    cand[slot] = ((uint64_t)__float_as_uint(d2) << 32) | (begin + base + lane);
                 }
                 cnt += nm;
                 wave_sync();
             }
-            if (!full && cnt >= k) select(k);
+            if (!full && cnt >= k) window_keep();
             bool found = false;
             while (sp > 0) {
                 --sp;
@@ -509,16 +484,15 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, u
         ox2 = oy2 = oz2 = 0.0f;
         rlane = 0.0f;
     }
-    if (kSel != kSelSort && cnt > k) radix_keep();
-    // the buffer now holds exactly the set; it is sorted only for callers of the lists
-    if (kSel == kSelSort || A.out_nbr) sort_keep(k);
+    if (cnt > k) exact_keep();
+    // the buffer now holds exactly the set, in no particular order
     const uint32_t found = cnt;  // min(#photons closer than r_max, k)
 
     float r2 = r2max;
     if (found >= k && k > 0) {
         // the k-th distance: the largest d2 of the set
         uint32_t hi = 0;
-        for (uint32_t i = lane; i < found; i += 64) hi = max(hi, (uint32_t)(keys[i] >> 32));
+        for (uint32_t i = lane; i < found; i += 64) hi = max(hi, (uint32_t)(cand[i] >> 32));
         r2 = __uint_as_float(wave_max_u32(hi));
     }
 
@@ -529,13 +503,25 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, u
         hint->r2 = (found >= k && k > 0) ? r2 : -1.0f;
     }
     if (A.out_count && lane == 0) A.out_count[q] = found;
-    if (A.out_nbr) {
+    // neighbour lists, for callers that ask for them: (d2, photon index) order (after the last
+    // read of the candidates' record positions)
+    auto write_lists = [&]() {
+        if (!A.out_nbr) return;
+        const uint32_t size = pow2_at_least(found);
+        for (uint32_t i = lane; i < size; i += 64) {
+            const uint64_t c = cand[i];
+            cand[i] = i < found ? ((c >> 32) << 32) | __float_as_uint(Tr.recs[2ull * (uint32_t)c].w) : ~0ull;
+        }
+        wave_sync();
+        wave_bitonic(cand, size, lane);
         for (uint32_t i = lane; i < k; i += 64)
-            A.out_nbr[(size_t)q * k + i] = (i < found) ? (uint32_t)(keys[i] & 0xFFFFFFFFull) : 0xFFFFFFFFu;
-    }
+            A.out_nbr[(size_t)q * k + i] = (i < found) ? (uint32_t)cand[i] : 0xFFFFFFFFu;
+        wave_sync();
+    };
     if (kMode == kModeRadii) {
         if (A.out_radius && lane == 0) A.out_radius[q] = (found >= k && k > 0) ? sqrtf(r2) : rq;
         if (A.out_r2 && lane == 0) A.out_r2[q] = r2;
+        write_lists();
         return;
     }
 
@@ -559,7 +545,7 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, u
             const uint32_t i = lane + 64u * (uint32_t)t;
             vx[t] = vy[t] = vz[t] = 0.0f;
             if (i < found) {
-                const float4 pw = Tr.recs[2ull * kpos[i] + 1];
+                const float4 pw = Tr.recs[2ull * (uint32_t)cand[i] + 1];
                 if (dot3(nq, oct_decode(__float_as_uint(pw.w))) < 0.0f) {
                     vx[t] = pw.x;
                     vy[t] = pw.y;
@@ -604,48 +590,33 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, u
                                             g.z * (((c4.w * kInvPi) * iz) * in4.z), 0.0f);
         // fixed-point adds are associative, so the per-photon sums do not depend on the
         // order in which queries arrive
-        const double fs = kPairs ? sink->fix_scale : A.fix_scale;
+        const double fs = sink->fix_scale;
         long long fx = __double2ll_rn((double)wx * fs);
         long long fy = __double2ll_rn((double)wy * fs);
         long long fz = __double2ll_rn((double)wz * fs);
-        if (kPairs) {
-            if (fx == 0 && fy == 0 && fz == 0) return;
-            if (lane == 0) {
-                sink->wtab[3 * sink->slot + 0] = fx;
-                sink->wtab[3 * sink->slot + 1] = fy;
-                sink->wtab[3 * sink->slot + 2] = fz;
-            }
-            uint32_t np = uniform(*sink->npairs);
-            for (uint32_t base = 0; base < found; base += 64) {
-                const uint32_t i = base + lane;
-                bool front = false;
-                uint64_t key = 0;
-                if (i < found) {
-                    const float4 pw = Tr.recs[2ull * kpos[i] + 1];
-                    front = dot3(nq, oct_decode(__float_as_uint(pw.w))) < 0.0f;
-                    key = (((keys[i] & 0xFFFFFFFFull) + sink->pbase) << 8) | sink->slot;
-                }
-                const uint64_t m = ballot(front);
-                if (front) sink->pairs[np + mask_prefix(m)] = key;
-                np += (uint32_t)__popcll(m);
-            }
-            wave_sync();
-            if (lane == 0) *sink->npairs = np;
-            wave_sync();
-            return;
+        if (fx == 0 && fy == 0 && fz == 0) return;
+        if (lane == 0) {
+            sink->wtab[3 * sink->slot + 0] = fx;
+            sink->wtab[3 * sink->slot + 1] = fy;
+            sink->wtab[3 * sink->slot + 2] = fz;
         }
-        if (fx != 0 || fy != 0 || fz != 0) {
-            for (uint32_t i = lane; i < found; i += 64) {
-                float4 pw = Tr.recs[2ull * kpos[i] + 1];
-                f3 pd = oct_decode(__float_as_uint(pw.w));
-                if (dot3(nq, pd) < 0.0f) {
-                    size_t p = (size_t)(keys[i] & 0xFFFFFFFFull);
-                    atomicAdd(&A.acc[3 * p + 0], (unsigned long long)fx);
-                    atomicAdd(&A.acc[3 * p + 1], (unsigned long long)fy);
-                    atomicAdd(&A.acc[3 * p + 2], (unsigned long long)fz);
-                }
+        uint32_t np = uniform(*sink->npairs);
+        for (uint32_t base = 0; base < found; base += 64) {
+            const uint32_t i = base + lane;
+            bool front = false;
+            uint64_t key = 0;
+            if (i < found) {
+                const float4* rec = Tr.recs + 2ull * (uint32_t)cand[i];
+                front = dot3(nq, oct_decode(__float_as_uint(rec[1].w))) < 0.0f;
+                key = (((uint64_t)__float_as_uint(rec[0].w) + sink->pbase) << 8) | sink->slot;
             }
+            const uint64_t m = ballot(front);
+            if (front) sink->pairs[np + mask_prefix(m)] = key;
+            np += (uint32_t)__popcll(m);
         }
+        wave_sync();
+        if (lane == 0) *sink->npairs = np;
+        wave_sync();
         return;
     }
     float rx = (((c4.w * c4.x) * kInvPi) * ix) * in4.x;
@@ -667,16 +638,16 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, u
             A.rad_out[q] = make_float4(rx, ry, rz, 0.0f);
         }
     }
+    write_lists();
 }
 
 // Consecutive queries per wave: each after the first starts from the previous one's
 // k-th distance (WarmHint); neighbouring pixels' hits share most of their neighbours.
 constexpr uint32_t kKnnChain = 8;
 
-template <int CAP, int kMode, int kSel>
+template <int CAP, int kMode>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_knn(KnnArgs A) {
-    __shared__ uint64_t s_key[kWavesPerBlock][CAP];
-    __shared__ uint32_t s_pos[kWavesPerBlock][CAP];
+    __shared__ uint64_t s_cand[kWavesPerBlock][CAP];
     __shared__ uint32_t s_snode[kWavesPerBlock][kKnnStack];
     __shared__ float4 s_soff[kWavesPerBlock][kKnnStack];
     const uint32_t wave = threadIdx.x >> 6;
@@ -688,8 +659,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     WarmHint hint{0.0f, 0.0f, 0.0f, -1.0f, A.order_far && !order_coherent(A.n, A.order_far)};
     for (uint32_t j = (uint32_t)j0; j < j1; ++j) {
         const uint32_t q = A.order ? ld_uniform(A.order, j) : j;
-        knn_query<CAP, kMode, kSel>(A, Tr, q, lane, s_key[wave], s_pos[wave], s_snode[wave], s_soff[wave], nullptr,
-                                    &hint);
+        knn_query<CAP, kMode>(A, Tr, q, lane, s_cand[wave], s_snode[wave], s_soff[wave], nullptr, &hint);
         wave_sync();
     }
 }
@@ -698,15 +668,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // counter (one counter per XCD share, as k_trace_batch), slot g belonging to the scene
 // whose slot range holds it.  Slots at or past a scene's count (count[s], device side:
 // the number of shading points the batched compaction wrote) are left untouched.
-template <int CAP, int kWaves, int kSel>
+template <int CAP, int kWaves>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_knn_batch(KnnArgs G, const KnnScene* __restrict__ scenes,
                                                            const uint32_t* __restrict__ slot_begin, uint32_t ns,
                                                            const uint32_t* __restrict__ count, uint32_t chunk,
                                                            uint32_t num_parts, const uint32_t* __restrict__ part_begin,
                                                            const uint32_t* __restrict__ part_end,
                                                            uint32_t* __restrict__ work) {
-    __shared__ uint64_t s_key[kWaves][CAP];
-    __shared__ uint32_t s_pos[kWaves][CAP];
+    __shared__ uint64_t s_cand[kWaves][CAP];
     __shared__ uint32_t s_snode[kWaves][kKnnStack];
     __shared__ float4 s_soff[kWaves][kKnnStack];
     const uint32_t wave = threadIdx.x >> 6;
@@ -744,8 +713,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(8, 
                     enter();
                 }
                 if (g - b >= m) continue;
-                knn_query<CAP, kModeRadiance, kSel>(G, Tr, g, lane, s_key[wave], s_pos[wave], s_snode[wave],
-                                                    s_soff[wave], nullptr, &hint);
+                knn_query<CAP, kModeRadiance>(G, Tr, g, lane, s_cand[wave], s_snode[wave], s_soff[wave], nullptr,
+                                              &hint);
                 wave_sync();
             }
         }
@@ -799,10 +768,9 @@ __device__ __forceinline__ void merge_pairs(uint64_t* pairs, uint32_t np, const 
     }
 }
 
-template <int CAP, int kSel>
+template <int CAP>
 __global__ __launch_bounds__(256) void k_knn_bwd_chunks(KnnArgs A, uint32_t chunk) {
-    __shared__ uint64_t s_key[kWavesPerBlock][CAP];
-    __shared__ uint32_t s_pos[kWavesPerBlock][CAP];
+    __shared__ uint64_t s_cand[kWavesPerBlock][CAP];
     __shared__ uint32_t s_snode[kWavesPerBlock][kKnnStack];
     __shared__ float4 s_soff[kWavesPerBlock][kKnnStack];
     __shared__ uint64_t s_pairs[kWavesPerBlock][kPairCap];
@@ -822,8 +790,7 @@ __global__ __launch_bounds__(256) void k_knn_bwd_chunks(KnnArgs A, uint32_t chun
     for (uint32_t j = (uint32_t)j0; j < j1; ++j) {
         const uint32_t q = A.order ? ld_uniform(A.order, j) : j;
         const PairSink sink{pairs, &s_np[wave], s_w[wave], j - (uint32_t)j0, 0u, A.fix_scale};
-        knn_query<CAP, kModeBackward, kSel, true>(A, Tr, q, lane, s_key[wave], s_pos[wave], s_snode[wave],
-                                                  s_soff[wave], &sink, &hint);
+        knn_query<CAP, kModeBackward>(A, Tr, q, lane, s_cand[wave], s_snode[wave], s_soff[wave], &sink, &hint);
         wave_sync();
     }
     merge_pairs(pairs, uniform(s_np[wave]), s_w[wave], A.acc, lane);
@@ -955,7 +922,7 @@ __global__ __launch_bounds__(64) void k_bwd_scale_batch(uint32_t ns, const uint3
 // kPairCap) from the work counters, as k_knn_batch does.  A pair carries the photon's index
 // in the concatenation of the scenes' photon arrays (scene offset + original index) and its
 // weight in the scene's own fixed-point unit, so one work item may span scenes.
-template <int CAP, int kSel>
+template <int CAP>
 __global__ __launch_bounds__(256) void k_knn_bwd_batch(KnnArgs G, const KnnScene* __restrict__ scenes,
                                                        const uint32_t* __restrict__ slot_begin, uint32_t ns,
                                                        const uint32_t* __restrict__ count,
@@ -964,8 +931,7 @@ __global__ __launch_bounds__(256) void k_knn_bwd_batch(KnnArgs G, const KnnScene
                                                        uint32_t num_parts, const uint32_t* __restrict__ part_begin,
                                                        const uint32_t* __restrict__ part_end,
                                                        uint32_t* __restrict__ work) {
-    __shared__ uint64_t s_key[kWavesPerBlock][CAP];
-    __shared__ uint32_t s_pos[kWavesPerBlock][CAP];
+    __shared__ uint64_t s_cand[kWavesPerBlock][CAP];
     __shared__ uint32_t s_snode[kWavesPerBlock][kKnnStack];
     __shared__ float4 s_soff[kWavesPerBlock][kKnnStack];
     __shared__ uint64_t s_pairs[kWavesPerBlock][kPairCap];
@@ -1012,8 +978,8 @@ __global__ __launch_bounds__(256) void k_knn_bwd_batch(KnnArgs G, const KnnScene
                 }
                 if (g - b >= m) continue;
                 const PairSink sink{pairs, &s_np[wave], s_w[wave], g - (uint32_t)g0, poff, fs};
-                knn_query<CAP, kModeBackward, kSel, true>(G, Tr, g, lane, s_key[wave], s_pos[wave], s_snode[wave],
-                                                          s_soff[wave], &sink, &hint);
+                knn_query<CAP, kModeBackward>(G, Tr, g, lane, s_cand[wave], s_snode[wave], s_soff[wave], &sink,
+                                              &hint);
                 wave_sync();
             }
             merge_pairs(pairs, uniform(s_np[wave]), s_w[wave], G.acc, lane);
@@ -1042,9 +1008,6 @@ __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long* __restrict
         p[i] = 0ull;
 }
 
-// Selection strategy of the single-tree launches.
-constexpr int kKnnSelDefault = kSelWindow;
-
 // Backward launches: queries in chunks of floor(kPairCap / k) per wave (at most 8).
 int launch_knn_bwd(const KnnArgs& A, hipStream_t st) {
     const uint32_t chunk = std::max<uint32_t>(1u, std::min<uint32_t>(8u, (uint32_t)kPairCap / A.k));
@@ -1052,11 +1015,11 @@ int launch_knn_bwd(const KnnArgs& A, hipStream_t st) {
     dim3 block(64 * kWavesPerBlock), grid((chunks + kWavesPerBlock - 1) / kWavesPerBlock);
     const uint32_t need = A.k + 64;
     if (need <= 128)
-        hipLaunchKernelGGL((k_knn_bwd_chunks<128, kKnnSelDefault>), grid, block, 0, st, A, chunk);
+        hipLaunchKernelGGL((k_knn_bwd_chunks<128>), grid, block, 0, st, A, chunk);
     else if (need <= 256)
-        hipLaunchKernelGGL((k_knn_bwd_chunks<256, kKnnSelDefault>), grid, block, 0, st, A, chunk);
+        hipLaunchKernelGGL((k_knn_bwd_chunks<256>), grid, block, 0, st, A, chunk);
     else
-        hipLaunchKernelGGL((k_knn_bwd_chunks<512, kKnnSelDefault>), grid, block, 0, st, A, chunk);
+        hipLaunchKernelGGL((k_knn_bwd_chunks<512>), grid, block, 0, st, A, chunk);
     MNRT_HIP_CHECK(hipGetLastError());
     return MNRT_OK;
 }
@@ -1067,45 +1030,34 @@ int launch_knn(const KnnArgs& A, hipStream_t st) {
     dim3 block(64 * kWavesPerBlock), grid((uint32_t)((A.n + per_block - 1) / per_block));
     uint32_t need = A.k + 64;
     if (need <= 128)
-        hipLaunchKernelGGL((k_knn<128, kMode, kKnnSelDefault>), grid, block, 0, st, A);
+        hipLaunchKernelGGL((k_knn<128, kMode>), grid, block, 0, st, A);
     else if (need <= 256)
-        hipLaunchKernelGGL((k_knn<256, kMode, kKnnSelDefault>), grid, block, 0, st, A);
+        hipLaunchKernelGGL((k_knn<256, kMode>), grid, block, 0, st, A);
     else
-        hipLaunchKernelGGL((k_knn<512, kMode, kKnnSelDefault>), grid, block, 0, st, A);
+        hipLaunchKernelGGL((k_knn<512, kMode>), grid, block, 0, st, A);
     MNRT_HIP_CHECK(hipGetLastError());
     return MNRT_OK;
 }
 
 int launch_knn_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* slot_begin, uint32_t ns,
                      const uint32_t* count, uint32_t chunk, uint32_t num_parts, const uint32_t* part_begin,
-                     const uint32_t* part_end, uint32_t* work, uint32_t cap, uint32_t waves, uint32_t sel,
+                     const uint32_t* part_end, uint32_t* work, uint32_t cap, uint32_t waves,
                      uint32_t grid, hipStream_t st) {
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, work, num_parts, 0u);
-#define MNRT_KB(C, W, S)                                                                                    \
-    hipLaunchKernelGGL((k_knn_batch<C, W, S>), dim3(grid), dim3(64 * W), 0, st, G, scenes, slot_begin, ns, \
+#define MNRT_KB(C, W)                                                                                    \
+    hipLaunchKernelGGL((k_knn_batch<C, W>), dim3(grid), dim3(64 * W), 0, st, G, scenes, slot_begin, ns, \
                        count, chunk, num_parts, part_begin, part_end, work)
-#define MNRT_KB_W(C, S)                   \
-    do {                                  \
-        if (waves == 1) MNRT_KB(C, 1, S); \
-        else if (waves == 2) MNRT_KB(C, 2, S); \
-        else MNRT_KB(C, 4, S);            \
+#define MNRT_KB_W(C)                   \
+    do {                               \
+        if (waves == 1) MNRT_KB(C, 1); \
+        else if (waves == 2) MNRT_KB(C, 2); \
+        else MNRT_KB(C, 4);            \
     } while (0)
     if (waves != 1 && waves != 2 && waves != 4) return MNRT_ERR_ARG;
-    if (cap == 128) {
-        if (sel == 2) MNRT_KB_W(128, kSelWindow);
-        else if (sel == 1) MNRT_KB_W(128, kSelRadix);
-        else MNRT_KB_W(128, kSelSort);
-    } else if (cap == 256) {
-        if (sel == 2) MNRT_KB_W(256, kSelWindow);
-        else if (sel == 1) MNRT_KB_W(256, kSelRadix);
-        else MNRT_KB_W(256, kSelSort);
-    } else if (cap == 512) {
-        if (sel == 2) MNRT_KB_W(512, kSelWindow);
-        else if (sel == 1) MNRT_KB_W(512, kSelRadix);
-        else MNRT_KB_W(512, kSelSort);
-    } else {
-        return MNRT_ERR_ARG;
-    }
+    if (cap == 128) MNRT_KB_W(128);
+    else if (cap == 256) MNRT_KB_W(256);
+    else if (cap == 512) MNRT_KB_W(512);
+    else return MNRT_ERR_ARG;
 #undef MNRT_KB_W
 #undef MNRT_KB
     MNRT_HIP_CHECK(hipGetLastError());
@@ -1134,7 +1086,7 @@ int launch_knn_bwd_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_
     const uint32_t chunk = std::max<uint32_t>(1u, std::min<uint32_t>(8u, (uint32_t)kPairCap / G.k));
     const uint32_t need = G.k + 64;
 #define MNRT_KBB(C) \
-    hipLaunchKernelGGL((k_knn_bwd_batch<C, kKnnSelDefault>), dim3(grid), dim3(64 * kWavesPerBlock), 0, st, G, scenes, \
+    hipLaunchKernelGGL((k_knn_bwd_batch<C>), dim3(grid), dim3(64 * kWavesPerBlock), 0, st, G, scenes, \
                        slot_begin, ns, count, photon_begin, scale, chunk, num_parts, part_begin, part_end, work)
     if (need <= 128) MNRT_KBB(128);
     else if (need <= 256) MNRT_KBB(256);
