@@ -103,8 +103,14 @@ typedef struct mnrt_tree {
     uint32_t owns_recs;  /* library allocated d_recs */
     uint32_t* d_qnodes;  /* query-time node words (NULL: d_nodes), see mnrt_tree_collapse */
     uint32_t qleaf_max;  /* subtrees with at most this many references are leaves in d_qnodes */
-    uint32_t owns_qnodes;
+    uint32_t owns_qnodes; /* MNRT_QNODES_* bits; 0 for node words a caller supplies */
 } mnrt_tree;
+
+/* owns_qnodes bits: the library allocated d_qnodes; a box hierarchy over the photon records
+ * precedes d_qnodes (mnrt_tree_attach_photon_records and the batched and recorded builds
+ * make it; kNN queries then read it instead of the node words). */
+#define MNRT_QNODES_OWNED 1u
+#define MNRT_QNODES_BOXES 2u
 
 const char* mnrt_status_string(int status);
 int mnrt_abi_version(void);

@@ -98,7 +98,7 @@ class DeviceTree:
         return c.value
 
     def _owns(self):
-        return self._batch is None and (self.t.owns_nodes or self.t.owns_recs or self.t.owns_qnodes)
+        return self._batch is None and (self.t.owns_nodes or self.t.owns_recs or self.t.owns_qnodes & N.QNODES_OWNED)
 
     def release(self):
         if self._owns():
@@ -139,7 +139,8 @@ class TreeBatch:
         return self.offsets.ctypes.data_as(ctypes.POINTER(N.u32))
 
     def release(self):
-        if self.num_scenes and (self.arr[0].owns_nodes or self.arr[0].owns_recs or self.arr[0].owns_qnodes):
+        if self.num_scenes and (self.arr[0].owns_nodes or self.arr[0].owns_recs
+                                or self.arr[0].owns_qnodes & N.QNODES_OWNED):
             _torch().cuda.synchronize()
             N.check(N.load().mnrt_tree_release(ctypes.byref(self.arr[0])), "mnrt_tree_release")
         self._keep = []

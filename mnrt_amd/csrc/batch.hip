@@ -22,6 +22,7 @@ struct mnrt_batch {
     uint32_t ns = 0;
     uint32_t k = 0;
     bool has_knn = false;
+    bool boxes = false;  // every photon tree has a box hierarchy (boxes.h)
     uint32_t total_slots = 0;
     uint32_t max_level = 0;
     uint32_t cus = 256;
@@ -193,7 +194,7 @@ int run_knn(mnrt_batch& b, const mnrt_batch_io& io, hipStream_t st) {
     G.out_count = io.d_out_count;
     return launch_knn_batch(G, b.d_knn, b.d_slot_begin, b.ns, io.d_sp_count, b.tun.knn_chunk, b.tun.parts,
                             b.d_tparts + 2 * kMaxParts, b.d_tparts + 3 * kMaxParts, b.d_work + kMaxParts,
-                            b.tun.knn_cap, b.tun.knn_waves, b.tun.knn_grid, st);
+                            b.tun.knn_cap, b.tun.knn_waves, b.tun.knn_grid, b.boxes, st);
 }
 
 // Accumulators of the adjoint phase for the current photon counts (synchronous; never
@@ -251,7 +252,7 @@ int run_knn_bwd(mnrt_batch& b, const mnrt_batch_io& io, hipStream_t st) {
     return launch_knn_bwd_batch(G, b.d_knn, b.d_slot_begin, b.ns, io.d_sp_count, b.d_poff, b.h_poff[b.ns],
                                 io.d_out_r2, io.d_out_count, b.d_wmax, b.d_scale, b.tun.parts,
                                 b.d_tparts + 2 * kMaxParts, b.d_tparts + 3 * kMaxParts, b.d_work + kMaxParts,
-                                b.tun.knn_grid, io.d_grad_pow4, st);
+                                b.tun.knn_grid, b.boxes, io.d_grad_pow4, st);
 }
 
 int run_phases(mnrt_batch& b, const mnrt_batch_io& io, uint32_t phases, hipStream_t st) {
@@ -301,6 +302,7 @@ int fill_scenes(mnrt_batch& b, const mnrt_tree* tri, const mnrt_tree* pm, const 
     const bool knn = b.has_knn;
     uint32_t max_level = 0;
     b.h_poff.assign(ns + 1, 0);
+    bool boxes = true;
     for (uint32_t s = 0; s < ns; ++s) {
         const mnrt_tree& t = tri[s];
         if (t.kind != MNRT_KIND_TRI || !t.d_nodes || !t.d_recs || t.num_nodes == 0) return MNRT_ERR_STATE;
@@ -323,6 +325,8 @@ int fill_scenes(mnrt_batch& b, const mnrt_tree* tri, const mnrt_tree* pm, const 
             KnnScene& kq = b.h_knn[s];
             kq.nodes = (const uint2*)(p.d_qnodes ? p.d_qnodes : p.d_nodes);
             kq.recs = (const float4*)p.d_recs;
+            kq.boxes = box_tree(p);
+            boxes = boxes && kq.boxes.p;
             if (r_max) {
                 if (!(r_max[s] > 0.0f)) return MNRT_ERR_ARG;
                 kq.r_max = r_max[s];
@@ -334,6 +338,8 @@ int fill_scenes(mnrt_batch& b, const mnrt_tree* tri, const mnrt_tree* pm, const 
             b.h_poff[s + 1] = b.h_poff[s] + p.num_elems;
         }
     }
+    if (knn && boxes != b.boxes) drop_graphs(b, MNRT_PHASE_KNN | MNRT_PHASE_KNN_BWD);  // another kernel
+    b.boxes = knn && boxes;
     b.max_level = max_level;
     return MNRT_OK;
 }

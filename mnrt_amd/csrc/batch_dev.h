@@ -7,6 +7,7 @@
 // into tiles of consecutive slots that never straddle two scenes.
 #pragma once
 
+#include "boxes.h"
 #include "mnrt_common.h"
 
 namespace mnrt {
@@ -55,6 +56,7 @@ struct TraceBatchArgs {
 struct KnnArgs {
     const uint2* nodes;
     const float4* recs;  // 2 float4 per reference
+    BoxTree boxes;
     uint32_t k;
     float r2max;
     float r_max;
@@ -80,6 +82,7 @@ struct KnnArgs {
     unsigned long long* acc;       // 3 fixed-point accumulators per photon (original index)
     double fix_scale;              // accumulator units per unit gradient (a power of two)
     float4* out_grad_clr;          // dLoss/d(diffuse colour) per query
+    uint32_t chain;                // consecutive queries per wave (plain launches, set there)
     const uint32_t* order;         // processing order of the queries (null: 0..n-1)
     const uint32_t* order_far;     // the order's far-pair count (order_coherent), or null
 };
@@ -87,6 +90,7 @@ struct KnnArgs {
 struct KnnScene {
     const uint2* nodes;  // query-time node words
     const float4* recs;
+    BoxTree boxes;
     float r2max, r_max;
     uint32_t slot_begin, slot_end;
 };
@@ -119,18 +123,34 @@ int launch_trace_batch(const TraceBatchArgs& B, int stack, uint32_t grid, uint32
 int launch_knn_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* slot_begin, uint32_t ns,
                      const uint32_t* count, uint32_t chunk, uint32_t num_parts, const uint32_t* part_begin,
                      const uint32_t* part_end, uint32_t* work, uint32_t cap, uint32_t waves,
-                     uint32_t grid, hipStream_t st);
+                     uint32_t grid, bool boxes, hipStream_t st);
 int launch_knn_bwd_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* slot_begin, uint32_t ns,
                          const uint32_t* count, const uint32_t* photon_begin, uint32_t total_photons,
                          const float* fwd_r2, const uint32_t* fwd_count, uint32_t* wmax, double* scale,
                          uint32_t num_parts, const uint32_t* part_begin, const uint32_t* part_end, uint32_t* work,
-                         uint32_t grid, float* grad_pow4, hipStream_t st);
+                         uint32_t grid, bool boxes, float* grad_pow4, hipStream_t st);
 int launch_shade_batch(const ShadeBatchArgs& A, uint32_t* flags, uint32_t* scan_tmp, hipStream_t st);
-int launch_records_batch(int kind, const uint32_t* refs, DN nrefs, const uint32_t* rbase, const uint32_t* ebase,
-                         uint32_t ns, const float4* a, const float4* b, const float4* c, float4* recs,
-                         const uint32_t* err, hipStream_t st);
-int launch_collapse_batch(const uint2* nodes, DN nnodes, const uint32_t* nbase, uint32_t ns, uint32_t max_refs,
-                          uint2* qnodes, const uint32_t* err, hipStream_t st);
+// Device tables of a batch of photon trees (ns + 1 entries each): first node, reference and
+// input element of every tree, its first level-0 slot and box_begin (boxes.h).
+struct PhotonTables {
+    uint32_t ns;  // 0: one tree, no tables
+    const uint32_t* nbase;
+    const uint32_t* rbase;
+    const uint32_t* ebase;
+    const uint32_t* slot_begin;
+    const uint32_t* box_begin;
+};
+// The last two on the host, from the trees' element counts.
+void photon_tables(const uint32_t* elems, uint32_t ns, uint32_t* slot_begin, uint32_t* box_begin);
+
+int launch_tri_records_batch(const uint32_t* refs, DN nrefs, const uint32_t* rbase, const uint32_t* ebase, uint32_t ns,
+                             const float4* v0, const float4* v1, const float4* v2, float4* recs, const uint32_t* err,
+                             hipStream_t st);
+int launch_photon_records_batch(const uint32_t* refs, const PhotonTables& tab, uint32_t slots, uint32_t max_elems,
+                                const float4* pos, const float4* pw, const float4* dir, float4* recs, float4* boxes,
+                                const uint32_t* err, hipStream_t st);
+int launch_collapse_batch(const uint2* nodes, DN nnodes, const uint32_t* nbase, uint32_t ns, const uint32_t* box_begin,
+                          uint32_t max_refs, uint2* qnodes, const uint32_t* err, hipStream_t st);
 
 }  // namespace mnrt
 

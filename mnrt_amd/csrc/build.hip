@@ -2140,6 +2140,7 @@ struct mnrt_build_graph {
     uint32_t ns = 0, ntot = 0;
     std::vector<uint32_t> h_base;      // ns + 1
     std::vector<uint32_t> h_plan;      // kind / index / offset per scene
+    std::vector<uint32_t> h_photon;    // slot_begin, box_begin (ns + 1 each, photon_tables)
     std::vector<float> h_qr, h_roots;  // per scene (roots: empty when not given)
     mnrt_build_params prm{};
     const float *v0 = nullptr, *v1 = nullptr, *v2 = nullptr, *pow4 = nullptr, *dir4 = nullptr;
@@ -2167,6 +2168,7 @@ struct GraphTab {
     uint32_t *base, *pkind, *pindex, *poff;
     float *qr, *given, *rootbox;
     uint32_t *snodes, *srefs, *nbase, *rbase, *sleaves, *smaxlvl;
+    uint32_t *slot_begin, *box_begin;  // photon_tables
 };
 
 GraphTab graph_tab(uint32_t* t, uint32_t S_) {
@@ -2184,6 +2186,8 @@ GraphTab graph_tab(uint32_t* t, uint32_t S_) {
     T.rbase = T.nbase + S_ + 1;
     T.sleaves = T.rbase + S_ + 1;
     T.smaxlvl = T.sleaves + S_;
+    T.slot_begin = T.smaxlvl + S_;
+    T.box_begin = T.slot_begin + S_ + 1;
     return T;
 }
 
@@ -2309,7 +2313,10 @@ int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
     uint32_t* nodes = cv.take<uint32_t>(2ull * C.nodes);
     uint32_t* refs = cv.take<uint32_t>(C.refs);
     float* recs = cv.take<float>((uint64_t)C.refs * (kind == MNRT_KIND_TRI ? 12u : 8u));
-    uint32_t* qnodes = kind == MNRT_KIND_POINT ? cv.take<uint32_t>(2ull * C.nodes) : nullptr;
+    // box hierarchies and query-time node words (box_block)
+    uint32_t* qnodes = kind == MNRT_KIND_POINT
+                           ? cv.take<uint32_t>(box_block(g.h_photon[2 * S_ + 1], S_, C.nodes) + 8u)
+                           : nullptr;
     if (!base) {
         g.dbytes = cv.size();
         return MNRT_OK;
@@ -2470,16 +2477,19 @@ int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
     // records and query-time node words
     const DN nrefs = dn(T.rbase + S_, C.refs), nnodes = dn(T.nbase + S_, C.nodes);
     if (kind == MNRT_KIND_TRI) {
-        int rc = launch_records_batch(kind, refs, nrefs, T.rbase, T.base, S_, (const float4*)g.v0, (const float4*)g.v1,
-                                      (const float4*)g.v2, (float4*)recs, counters + C_ERR, st);
+        int rc = launch_tri_records_batch(refs, nrefs, T.rbase, T.base, S_, (const float4*)g.v0, (const float4*)g.v1,
+                                          (const float4*)g.v2, (float4*)recs, counters + C_ERR, st);
         if (rc != MNRT_OK) return rc;
     } else if (g.pow4 && g.dir4) {
-        int rc = launch_records_batch(kind, refs, nrefs, T.rbase, T.base, S_, (const float4*)g.v0,
-                                      (const float4*)g.pow4, (const float4*)g.dir4, (float4*)recs, counters + C_ERR,
-                                      st);
+        uint32_t max_elems = 0;
+        for (uint32_t s = 0; s < S_; ++s) max_elems = std::max(max_elems, g.h_base[s + 1] - g.h_base[s]);
+        const PhotonTables tab{S_, T.nbase, T.rbase, T.base, T.slot_begin, T.box_begin};
+        int rc = launch_photon_records_batch(refs, tab, g.h_photon[S_], max_elems, (const float4*)g.v0,
+                                             (const float4*)g.pow4, (const float4*)g.dir4, (float4*)recs,
+                                             (float4*)qnodes, counters + C_ERR, st);
         if (rc == MNRT_OK)
-            rc = launch_collapse_batch((const uint2*)nodes, nnodes, T.nbase, S_, kQueryLeafRefs, (uint2*)qnodes,
-                                       counters + C_ERR, st);
+            rc = launch_collapse_batch((const uint2*)nodes, nnodes, T.nbase, S_, T.box_begin, kQueryLeafRefs,
+                                       (uint2*)qnodes, counters + C_ERR, st);
         if (rc != MNRT_OK) return rc;
     }
     MNRT_HIP_CHECK(hipGetLastError());
@@ -2621,6 +2631,13 @@ extern "C" int mnrt_build_graph_create(const mnrt_build_graph_desc* d, mnrt_tree
         if (na != bs.na0 || ne != bs.ne0 || nsmall != bs.nsmall0 || nse != bs.nse0) return fail(MNRT_ERR_STATE);
     }
 
+    g->h_photon.assign(2ull * (S_ + 1), 0u);
+    if (g->kind == MNRT_KIND_POINT) {
+        std::vector<uint32_t> elems(S_);
+        for (uint32_t s = 0; s < S_; ++s) elems[s] = g->h_base[s + 1] - g->h_base[s];
+        photon_tables(elems.data(), S_, g->h_photon.data(), g->h_photon.data() + S_ + 1);
+    }
+
     // 2. the fixed device block, and the per-scene tables in it
     int rc = graph_record(*g, nullptr, nullptr);
     if (rc != MNRT_OK) return fail(rc);
@@ -2637,7 +2654,8 @@ extern "C" int mnrt_build_graph_create(const mnrt_build_graph_desc* d, mnrt_tree
         for (size_t i = 0; i < g->h_roots.size(); ++i) fq[S_ + i] = g->h_roots[i];
         if (hipMemcpy(T.base, g->h_base.data(), 4ull * (S_ + 1), hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy(T.pkind, g->h_plan.data(), 12ull * S_, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(T.qr, fq.data(), 4ull * fq.size(), hipMemcpyHostToDevice) != hipSuccess)
+            hipMemcpy(T.qr, fq.data(), 4ull * fq.size(), hipMemcpyHostToDevice) != hipSuccess ||
+            hipMemcpy(T.slot_begin, g->h_photon.data(), 8ull * (S_ + 1), hipMemcpyHostToDevice) != hipSuccess)
             return fail(MNRT_ERR_HIP);
     }
 
@@ -2714,11 +2732,13 @@ extern "C" int mnrt_build_graph_status(mnrt_build_graph* g, mnrt_tree* out, uint
         t.d_refs = g->refs + hrb[s];
         t.d_recs = recs ? g->recs + (uint64_t)per * hrb[s] : nullptr;
         if (g->kind == MNRT_KIND_POINT && recs) {
-            t.d_qnodes = g->qnodes + 2ull * hnb[s];
+            const uint32_t* bb = g->h_photon.data() + S_ + 1;
+            t.d_qnodes = g->qnodes + box_block(bb[s], s, hnb[s]) + (bb[s + 1] - bb[s]);
             t.qleaf_max = kQueryLeafRefs;
+            t.owns_qnodes = MNRT_QNODES_BOXES;
         }
         // the arrays belong to the graph (mnrt_build_graph_destroy frees them)
-        t.owns_nodes = t.owns_recs = t.owns_qnodes = 0u;
+        t.owns_nodes = t.owns_recs = 0u;
     }
     return MNRT_OK;
 }

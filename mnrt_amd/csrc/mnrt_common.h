@@ -233,6 +233,12 @@ __device__ __forceinline__ float uniformf(float v) {
 // a 0/1 vector value and compares that against 0: two more vector instructions).
 __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
+// A wave-uniform mask with bit i (wave-uniform) cleared, in one scalar instruction.
+__device__ __forceinline__ uint64_t bit_clear(uint64_t m, uint32_t i) {
+    asm("s_bitset0_b64 %0, %1" : "+s"(m) : "s"(i));
+    return m;
+}
+
 // Lanes below this one whose predicate is set (exclusive prefix of a 64-bit ballot).
 __device__ __forceinline__ uint32_t mask_prefix(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));

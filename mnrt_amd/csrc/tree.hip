@@ -9,9 +9,11 @@
 #include <cstdint>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "batch_dev.h"
+#include "boxes.h"
 
 namespace mnrt {
 
@@ -27,19 +29,6 @@ __global__ __launch_bounds__(256) void k_tri_records(const uint32_t* __restrict_
     recs[3ull * r + 0] = make_float4(a.x, a.y, a.z, __uint_as_float(t));
     recs[3ull * r + 1] = make_float4(b.x - a.x, b.y - a.y, b.z - a.z, 0.0f);
     recs[3ull * r + 2] = make_float4(c.x - a.x, c.y - a.y, c.z - a.z, 0.0f);
-}
-
-__global__ __launch_bounds__(256) void k_photon_records(const uint32_t* __restrict__ refs, uint32_t num_refs,
-                                                        const float4* __restrict__ pos,
-                                                        const float4* __restrict__ pw,
-                                                        const float4* __restrict__ dir,
-                                                        float4* __restrict__ recs) {
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= num_refs) return;
-    uint32_t p = refs[r];
-    float4 x = pos[p], w = pw[p], d = dir[p];
-    recs[2ull * r + 0] = make_float4(x.x, x.y, x.z, __uint_as_float(p));
-    recs[2ull * r + 1] = make_float4(w.x, w.y, w.z, __uint_as_float(oct_encode(d.x, d.y, d.z)));
 }
 
 // Batched records: reference r of the shared array belongs to tree s (rbase), its element
@@ -62,35 +51,103 @@ __global__ __launch_bounds__(256) void k_tri_records_batch(const uint32_t* __res
     recs[3ull * r + 2] = make_float4(c.x - a.x, c.y - a.y, c.z - a.z, 0.0f);
 }
 
-__global__ __launch_bounds__(256) void k_photon_records_batch(const uint32_t* __restrict__ refs, DN dnum_refs,
-                                                              const uint32_t* __restrict__ rbase,
-                                                              const uint32_t* __restrict__ ebase, uint32_t ns,
-                                                              const float4* __restrict__ pos,
-                                                              const float4* __restrict__ pw,
-                                                              const float4* __restrict__ dir,
-                                                              float4* __restrict__ recs,
-                                                              const uint32_t* __restrict__ err) {
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= dnum_refs.get() || (err && *err != 0u)) return;
-    uint32_t p = refs[r];
-    uint32_t g = ebase[seg_of(rbase, ns, r)] + p;
-    float4 x = pos[g], w = pw[g], d = dir[g];
-    recs[2ull * r + 0] = make_float4(x.x, x.y, x.z, __uint_as_float(p));
-    recs[2ull * r + 1] = make_float4(w.x, w.y, w.z, __uint_as_float(oct_encode(d.x, d.y, d.z)));
+// Photon records of one tree or a batch, and the bounds of every group of 64 (boxes.h): a
+// wave per level-0 slot, which has the group's 64 positions in its lanes, so the bounds cost
+// no second pass over the records.
+struct PhotonRecArgs {
+    const uint32_t* refs;
+    const float4* pos;
+    const float4* pw;
+    const float4* dir;
+    float4* recs;
+    uint32_t nrefs, elems;  // one tree (tables null)
+    PhotonTables tab;       // a batch
+    uint32_t slots;         // level-0 slots of all trees
+    float4* boxes;          // hierarchies (one tree: its own; a batch: the shared array), or null
+    const uint32_t* err;
+};
+
+__global__ __launch_bounds__(256) void k_photon_records(PhotonRecArgs A) {
+    const uint32_t slot = uniform(blockIdx.x * 4u + (threadIdx.x >> 6)), lane = threadIdx.x & 63u;
+    if (slot >= A.slots || (A.err && *A.err != 0u)) return;
+    uint32_t g = slot, r0 = 0, nr = A.nrefs, e0 = 0;
+    uint64_t block = 0;
+    if (A.tab.ns) {
+        const uint32_t s = seg_of(A.tab.slot_begin, A.tab.ns, slot);
+        g = slot - A.tab.slot_begin[s];
+        r0 = A.tab.rbase[s];
+        nr = A.tab.rbase[s + 1] - r0;
+        e0 = A.tab.ebase[s];
+        block = box_block(A.tab.box_begin[s], s, A.tab.nbase[s]);
+    }
+    const uint32_t i = g * 64u + lane;
+    Box b = empty_box();
+    if (i < nr) {
+        const uint64_t r = (uint64_t)r0 + i;
+        const uint32_t p = A.refs[r], e = e0 + p;
+        const float4 x = A.pos[e], w = A.pw[e], d = A.dir[e];
+        A.recs[2 * r + 0] = make_float4(x.x, x.y, x.z, __uint_as_float(p));
+        A.recs[2 * r + 1] = make_float4(w.x, w.y, w.z, __uint_as_float(oct_encode(d.x, d.y, d.z)));
+        b.lo = b.hi = make_float4(x.x, x.y, x.z, 0.0f);
+    }
+    if (!A.boxes) return;
+    b = wave_box(b);
+    if (lane < 2u) A.boxes[block / 4u + 2ull * g + lane] = lane ? b.hi : b.lo;
+}
+
+// Levels 1 and 2 from level 0: workgroup s * per + x makes level-2 box x of tree s and the 64
+// level-1 boxes below it (16 waves, 4 boxes each), a tree's first workgroup also the padding of
+// its level 2.
+__global__ __launch_bounds__(1024) void k_boxes_up(float4* __restrict__ boxes, uint32_t elems, uint32_t per,
+                                                   PhotonTables T, const uint32_t* __restrict__ err) {
+    __shared__ float4 s_lo[64], s_hi[64];
+    if (err && *err != 0u) return;
+    const uint32_t s = blockIdx.x / per, x = blockIdx.x % per, wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const BoxGeom G = box_geom(T.ns ? T.ebase[s + 1] - T.ebase[s] : elems);
+    if (x >= G.g2) return;  // uniform per workgroup
+    float4* p = boxes + (T.ns ? box_block(T.box_begin[s], s, T.nbase[s]) / 4u : 0u);
+    for (uint32_t j = 4u * wave; j < 4u * wave + 4u; ++j) {
+        const uint32_t l1 = x * 64u + j;
+        Box b = empty_box();
+        if (l1 < G.g1) {
+            const float4* c = p + 2ull * (l1 * 64u + lane);
+            b = wave_box(Box{c[0], c[1]});
+        }
+        if (lane < 2u) p[2ull * G.s0 + 2ull * l1 + lane] = lane ? b.hi : b.lo;
+        if (lane == 0u) {
+            s_lo[j] = b.lo;
+            s_hi[j] = b.hi;
+        }
+    }
+    __syncthreads();
+    if (wave != 0u) return;
+    float4* top = p + 2ull * ((uint64_t)G.s0 + G.s1);
+    const Box b = wave_box(Box{s_lo[lane], s_hi[lane]});
+    if (lane < 2u) top[2ull * x + lane] = lane ? b.hi : b.lo;
+    if (x == 0u) {
+        const Box e = empty_box();
+        for (uint32_t i = G.g2 + lane; i < G.s2; i += 64u) {
+            top[2ull * i] = e.lo;
+            top[2ull * i + 1] = e.hi;
+        }
+    }
 }
 
 // One lane per node: the subtree's reference range runs from its leftmost leaf's first
 // reference to the end of its rightmost leaf.  nbase (ns + 1 entries, or null for one
-// tree) places the trees of a batch in the shared node array; err as for the records.
+// tree) places the trees of a batch in the shared node array, box_begin (or null) their query-time
+// nodes behind their box hierarchies (box_block); err as for the records.
 __global__ __launch_bounds__(256) void k_collapse(const uint2* __restrict__ nodes_all, DN dnum_nodes,
                                                   const uint32_t* __restrict__ nbase, uint32_t ns,
-                                                  uint32_t max_refs, uint2* __restrict__ qnodes_all,
-                                                  const uint32_t* __restrict__ err) {
+                                                  const uint32_t* __restrict__ box_begin, uint32_t max_refs,
+                                                  uint2* __restrict__ qnodes_all, const uint32_t* __restrict__ err) {
     uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= dnum_nodes.get() || (err && *err != 0u)) return;
-    const uint32_t b = nbase ? nbase[seg_of(nbase, ns, g)] : 0u;
+    const uint32_t s = nbase ? seg_of(nbase, ns, g) : 0u;
+    const uint32_t b = nbase ? nbase[s] : 0u;
     const uint2* nodes = nodes_all + b;
     uint2* qnodes = qnodes_all + b;
+    if (box_begin) qnodes = qnodes_all + (box_block(box_begin[s], s, b) + (box_begin[s + 1] - box_begin[s])) / 2u;
     const uint32_t i = g - b;
     uint2 nd = nodes[i];
     if (is_leaf(nd.y)) {
@@ -117,25 +174,43 @@ __global__ __launch_bounds__(256) void k_collapse(const uint2* __restrict__ node
         qnodes[i] = nd;
 }
 
-// Records (and, for photon trees, query-time node words) of the trees of a batch whose
-// sizes are device words (a recorded build): grids cover the capacities nrefs.v / nnodes.v.
-int launch_records_batch(int kind, const uint32_t* refs, DN nrefs, const uint32_t* rbase, const uint32_t* ebase,
-                         uint32_t ns, const float4* a, const float4* b, const float4* c, float4* recs,
-                         const uint32_t* err, hipStream_t st) {
-    const dim3 grid((std::max<uint32_t>(nrefs.v, 1u) + 255) / 256);
-    if (kind == MNRT_KIND_TRI)
-        hipLaunchKernelGGL(k_tri_records_batch, grid, dim3(256), 0, st, refs, nrefs, rbase, ebase, ns, a, b, c, recs,
-                           err);
-    else
-        hipLaunchKernelGGL(k_photon_records_batch, grid, dim3(256), 0, st, refs, nrefs, rbase, ebase, ns, a, b, c,
-                           recs, err);
+// Triangle records of the trees of a batch whose sizes are device words (a recorded build):
+// the grid covers the capacity nrefs.v.
+int launch_tri_records_batch(const uint32_t* refs, DN nrefs, const uint32_t* rbase, const uint32_t* ebase, uint32_t ns,
+                             const float4* v0, const float4* v1, const float4* v2, float4* recs, const uint32_t* err,
+                             hipStream_t st) {
+    hipLaunchKernelGGL(k_tri_records_batch, dim3((std::max<uint32_t>(nrefs.v, 1u) + 255) / 256), dim3(256), 0, st,
+                       refs, nrefs, rbase, ebase, ns, v0, v1, v2, recs, err);
     return hipGetLastError() == hipSuccess ? MNRT_OK : MNRT_ERR_HIP;
 }
 
-int launch_collapse_batch(const uint2* nodes, DN nnodes, const uint32_t* nbase, uint32_t ns, uint32_t max_refs,
-                          uint2* qnodes, const uint32_t* err, hipStream_t st) {
+void photon_tables(const uint32_t* elems, uint32_t ns, uint32_t* slot_begin, uint32_t* box_begin) {
+    slot_begin[0] = box_begin[0] = 0u;
+    for (uint32_t s = 0; s < ns; ++s) {
+        slot_begin[s + 1] = slot_begin[s] + box_geom(elems[s]).s0;
+        box_begin[s + 1] = box_begin[s] + (uint32_t)box_words(elems[s]);
+    }
+}
+
+static int launch_photon_records(const PhotonRecArgs& A, uint32_t ns, uint32_t max_elems, hipStream_t st) {
+    if (A.slots) hipLaunchKernelGGL(k_photon_records, dim3((A.slots + 3u) / 4u), dim3(256), 0, st, A);
+    const uint32_t g2 = box_geom(max_elems).g2;
+    if (A.boxes && g2)
+        hipLaunchKernelGGL(k_boxes_up, dim3(g2 * ns), dim3(1024), 0, st, A.boxes, A.elems, g2, A.tab, A.err);
+    return hipGetLastError() == hipSuccess ? MNRT_OK : MNRT_ERR_HIP;
+}
+
+int launch_photon_records_batch(const uint32_t* refs, const PhotonTables& tab, uint32_t slots, uint32_t max_elems,
+                                const float4* pos, const float4* pw, const float4* dir, float4* recs, float4* boxes,
+                                const uint32_t* err, hipStream_t st) {
+    PhotonRecArgs A{refs, pos, pw, dir, recs, 0u, 0u, tab, slots, boxes, err};
+    return launch_photon_records(A, tab.ns, max_elems, st);
+}
+
+int launch_collapse_batch(const uint2* nodes, DN nnodes, const uint32_t* nbase, uint32_t ns, const uint32_t* box_begin,
+                          uint32_t max_refs, uint2* qnodes, const uint32_t* err, hipStream_t st) {
     const dim3 grid((std::max<uint32_t>(nnodes.v, 1u) + 255) / 256);
-    hipLaunchKernelGGL(k_collapse, grid, dim3(256), 0, st, nodes, nnodes, nbase, ns, max_refs, qnodes, err);
+    hipLaunchKernelGGL(k_collapse, grid, dim3(256), 0, st, nodes, nnodes, nbase, ns, box_begin, max_refs, qnodes, err);
     return hipGetLastError() == hipSuccess ? MNRT_OK : MNRT_ERR_HIP;
 }
 
@@ -201,12 +276,11 @@ extern "C" int mnrt_tree_collapse(mnrt_tree* tree, uint32_t max_refs, void* stre
         void* p = nullptr;
         if (mnrt::pool_alloc(&p, (size_t)tree->num_nodes * 8, st) != hipSuccess) return MNRT_ERR_NOMEM;
         tree->d_qnodes = (uint32_t*)p;
-        tree->owns_qnodes = 1;
+        tree->owns_qnodes = MNRT_QNODES_OWNED;
     }
-    hipLaunchKernelGGL(mnrt::k_collapse, dim3((tree->num_nodes + 255) / 256), dim3(256), 0, st,
-                       (const uint2*)tree->d_nodes, mnrt::hn(tree->num_nodes), (const uint32_t*)nullptr, 1u, max_refs,
-                       (uint2*)tree->d_qnodes, (const uint32_t*)nullptr);
-    MNRT_HIP_CHECK(hipGetLastError());
+    int rc = mnrt::launch_collapse_batch((const uint2*)tree->d_nodes, mnrt::hn(tree->num_nodes), nullptr, 1u, nullptr,
+                                         max_refs, (uint2*)tree->d_qnodes, nullptr, st);
+    if (rc != MNRT_OK) return rc;
     tree->qleaf_max = max_refs;
     return MNRT_OK;
 }
@@ -219,6 +293,26 @@ static int ensure_recs(mnrt_tree* t, size_t floats_per_ref, hipStream_t st) {
     if (mnrt::pool_alloc(&p, bytes, st) != hipSuccess) return MNRT_ERR_NOMEM;
     t->d_recs = (float*)p;
     t->owns_recs = 1;
+    return MNRT_OK;
+}
+
+// Room for the box hierarchy and the query-time node words behind it (boxes.h).  Node words
+// that the caller supplied stay as they are, and so do trees with more references than
+// elements (no tree of the builders is one): queries then walk the node words.
+static int ensure_boxes(mnrt_tree* t, hipStream_t st) {
+    if ((t->owns_qnodes & MNRT_QNODES_BOXES) || (t->d_qnodes && !(t->owns_qnodes & MNRT_QNODES_OWNED)) ||
+        t->num_refs > t->num_elems)
+        return MNRT_OK;
+    const uint64_t bw = mnrt::box_words(t->num_elems);
+    if (bw > 0xFFFFFFFFull) return MNRT_OK;
+    void* p = nullptr;
+    if (mnrt::pool_alloc(&p, 4ull * (bw + 2ull * t->num_nodes), st) != hipSuccess) return MNRT_ERR_NOMEM;
+    if (t->d_qnodes && mnrt::pool_free(t->d_qnodes, st) != hipSuccess) {
+        (void)mnrt::pool_free(p, st);
+        return MNRT_ERR_HIP;
+    }
+    t->d_qnodes = (uint32_t*)p + bw;
+    t->owns_qnodes = MNRT_QNODES_OWNED | MNRT_QNODES_BOXES;
     return MNRT_OK;
 }
 
@@ -247,11 +341,17 @@ extern "C" int mnrt_tree_attach_photon_records(mnrt_tree* tree, const float* d_p
     int rc = ensure_recs(tree, 8, st);
     if (rc != MNRT_OK) return rc;
     if (tree->num_refs == 0) return MNRT_OK;
-    hipLaunchKernelGGL(mnrt::k_photon_records, dim3((tree->num_refs + 255) / 256), dim3(256), 0, st,
-                       tree->d_refs, tree->num_refs, (const float4*)d_pos4, (const float4*)d_pow4,
-                       (const float4*)d_dir4, (float4*)tree->d_recs);
-    MNRT_HIP_CHECK(hipGetLastError());
-    return mnrt_tree_collapse(tree, mnrt::kQueryLeafRefs, stream);
+    rc = ensure_boxes(tree, st);
+    if (rc != MNRT_OK) return rc;
+    mnrt::PhotonRecArgs A{tree->d_refs, (const float4*)d_pos4, (const float4*)d_pow4, (const float4*)d_dir4,
+                          (float4*)tree->d_recs, tree->num_refs, tree->num_elems, {}, 0u, nullptr, nullptr};
+    A.slots = (tree->num_refs + 63u) / 64u;
+    if (tree->owns_qnodes & MNRT_QNODES_BOXES) {
+        A.boxes = (float4*)(tree->d_qnodes - mnrt::box_words(tree->num_elems));
+        A.slots = mnrt::box_geom(tree->num_elems).s0;
+    }
+    rc = mnrt::launch_photon_records(A, 1u, tree->num_elems, st);
+    return rc == MNRT_OK ? mnrt_tree_collapse(tree, mnrt::kQueryLeafRefs, stream) : rc;
 }
 
 // ---- batches: trees[s] view shared arrays owned by trees[0] ----
@@ -259,13 +359,17 @@ extern "C" int mnrt_tree_attach_photon_records(mnrt_tree* tree, const float* d_p
 namespace {
 
 struct BatchTables {
-    std::vector<uint32_t> h;  // nbase (S+1), rbase (S+1), ebase (S+1)
-    uint32_t total_nodes = 0, total_refs = 0;
+    std::vector<uint32_t> h;  // nbase, rbase, ebase, slot_begin, box_begin (S + 1 each)
+    uint32_t total_nodes = 0, total_refs = 0, max_elems = 0;
+    bool boxes = true;
+    mnrt::PhotonTables on(const uint32_t* d, uint32_t ns) const {
+        return mnrt::PhotonTables{ns, d, d + (ns + 1), d + 2 * (ns + 1), d + 3 * (ns + 1), d + 4 * (ns + 1)};
+    }
 };
 
 int batch_tables(const mnrt_tree* t, uint32_t ns, const uint32_t* h_offsets, uint32_t kind, BatchTables& B) {
     if (!t || ns == 0 || !h_offsets || !t[0].d_nodes) return MNRT_ERR_ARG;
-    B.h.assign(3ull * (ns + 1), 0u);
+    B.h.assign(5ull * (ns + 1), 0u);
     uint32_t* nb = B.h.data();
     uint32_t* rb = nb + ns + 1;
     uint32_t* eb = rb + ns + 1;
@@ -279,10 +383,17 @@ int batch_tables(const mnrt_tree* t, uint32_t ns, const uint32_t* h_offsets, uin
         eb[s] = h_offsets[s];
         B.total_nodes += t[s].num_nodes;
         B.total_refs += t[s].num_refs;
+        B.max_elems = std::max(B.max_elems, t[s].num_elems);
     }
     nb[ns] = B.total_nodes;
     rb[ns] = B.total_refs;
     eb[ns] = h_offsets[ns];
+    std::vector<uint32_t> cover(ns);  // no tree of the builders has more references than elements
+    for (uint32_t s = 0; s < ns; ++s) {
+        cover[s] = std::max(t[s].num_elems, t[s].num_refs);
+        B.boxes = B.boxes && t[s].num_refs <= t[s].num_elems;
+    }
+    mnrt::photon_tables(cover.data(), ns, eb + ns + 1, eb + 2 * (ns + 1));
     return MNRT_OK;
 }
 
@@ -344,20 +455,28 @@ extern "C" int mnrt_tree_attach_photon_records_batch(mnrt_tree* trees, uint32_t 
         none = none && !trees[s].d_recs && !trees[s].d_qnodes;
     }
     if (!all && !none) return MNRT_ERR_STATE;
+    const uint32_t* bb = B.h.data() + 4 * (ns + 1);
+    // scene s's query-time node words in the shared array (boxes.h)
+    auto qnodes_at = [&](uint32_t s) { return mnrt::box_block(bb[s], s, B.h[s]) + (bb[s + 1] - bb[s]); };
+    uint32_t* d_tab = nullptr;
     if (all) {
         // records attached by an earlier call: rewritten in place (new photon powers, say);
         // the query-time nodes depend on the tree only and stay
-        for (uint32_t s = 0; s < ns; ++s)
+        uint32_t boxed = 0;
+        uint32_t* const q0 = trees[0].d_qnodes - bb[1];
+        for (uint32_t s = 0; s < ns; ++s) {
             if (trees[s].d_recs != trees[0].d_recs + 8ull * B.h[ns + 1 + s]) return MNRT_ERR_STATE;
-        uint32_t* d_tab = nullptr;
-        rc = upload(B, &d_tab, st);
-        if (rc == MNRT_OK && B.total_refs > 0) {
-            hipLaunchKernelGGL(mnrt::k_photon_records_batch, dim3((B.total_refs + 255) / 256), dim3(256), 0, st,
-                               trees[0].d_refs, mnrt::hn(B.total_refs), d_tab + ns + 1, d_tab + 2 * (ns + 1), ns,
-                               (const float4*)d_pos4, (const float4*)d_pow4, (const float4*)d_dir4,
-                               (float4*)trees[0].d_recs, (const uint32_t*)nullptr);
-            if (hipGetLastError() != hipSuccess) rc = MNRT_ERR_HIP;
+            if (!(trees[s].owns_qnodes & MNRT_QNODES_BOXES)) continue;
+            if (trees[s].d_qnodes != q0 + qnodes_at(s)) return MNRT_ERR_STATE;
+            ++boxed;
         }
+        if (boxed != 0 && boxed != ns) return MNRT_ERR_STATE;
+        rc = upload(B, &d_tab, st);
+        if (rc == MNRT_OK)
+            rc = mnrt::launch_photon_records_batch(trees[0].d_refs, B.on(d_tab, ns), B.h[3 * (ns + 1) + ns],
+                                                   B.max_elems, (const float4*)d_pos4, (const float4*)d_pow4,
+                                                   (const float4*)d_dir4, (float4*)trees[0].d_recs,
+                                                   boxed ? (float4*)q0 : nullptr, nullptr, st);
         if (d_tab) (void)mnrt::pool_free(d_tab, st);
         if (hipStreamSynchronize(st) != hipSuccess && rc == MNRT_OK) rc = MNRT_ERR_HIP;
         return rc;
@@ -365,22 +484,18 @@ extern "C" int mnrt_tree_attach_photon_records_batch(mnrt_tree* trees, uint32_t 
     float* recs = nullptr;
     uint32_t* qn = nullptr;
     if (mnrt::pool_alloc((void**)&recs, (size_t)B.total_refs * 32, st) != hipSuccess) return MNRT_ERR_NOMEM;
-    if (mnrt::pool_alloc((void**)&qn, (size_t)B.total_nodes * 8, st) != hipSuccess) {
+    if (mnrt::pool_alloc((void**)&qn, (qnodes_at(ns - 1) + 2ull * trees[ns - 1].num_nodes) * 4, st) != hipSuccess) {
         (void)mnrt::pool_free(recs, st);
         return MNRT_ERR_NOMEM;
     }
-    uint32_t* d_tab = nullptr;
     rc = upload(B, &d_tab, st);
-    if (rc == MNRT_OK && B.total_refs > 0)
-        hipLaunchKernelGGL(mnrt::k_photon_records_batch, dim3((B.total_refs + 255) / 256), dim3(256), 0, st,
-                           trees[0].d_refs, mnrt::hn(B.total_refs), d_tab + ns + 1, d_tab + 2 * (ns + 1), ns,
-                           (const float4*)d_pos4, (const float4*)d_pow4, (const float4*)d_dir4, (float4*)recs,
-                           (const uint32_t*)nullptr);
     if (rc == MNRT_OK)
-        hipLaunchKernelGGL(mnrt::k_collapse, dim3((B.total_nodes + 255) / 256), dim3(256), 0, st,
-                           (const uint2*)trees[0].d_nodes, mnrt::hn(B.total_nodes), (const uint32_t*)d_tab, ns,
-                           mnrt::kQueryLeafRefs, (uint2*)qn, (const uint32_t*)nullptr);
-    if (rc == MNRT_OK && hipGetLastError() != hipSuccess) rc = MNRT_ERR_HIP;
+        rc = mnrt::launch_photon_records_batch(trees[0].d_refs, B.on(d_tab, ns), B.h[3 * (ns + 1) + ns], B.max_elems,
+                                               (const float4*)d_pos4, (const float4*)d_pow4, (const float4*)d_dir4,
+                                               (float4*)recs, B.boxes ? (float4*)qn : nullptr, nullptr, st);
+    if (rc == MNRT_OK)
+        rc = mnrt::launch_collapse_batch((const uint2*)trees[0].d_nodes, mnrt::hn(B.total_nodes), d_tab, ns,
+                                         d_tab + 4 * (ns + 1), mnrt::kQueryLeafRefs, (uint2*)qn, nullptr, st);
     if (d_tab) (void)mnrt::pool_free(d_tab, st);
     if (hipStreamSynchronize(st) != hipSuccess && rc == MNRT_OK) rc = MNRT_ERR_HIP;
     if (rc != MNRT_OK) {
@@ -390,9 +505,10 @@ extern "C" int mnrt_tree_attach_photon_records_batch(mnrt_tree* trees, uint32_t 
     }
     for (uint32_t s = 0; s < num_scenes; ++s) {
         trees[s].d_recs = recs + 8ull * B.h[ns + 1 + s];
-        trees[s].d_qnodes = qn + 2ull * B.h[s];
+        trees[s].d_qnodes = qn + qnodes_at(s);
         trees[s].qleaf_max = mnrt::kQueryLeafRefs;
-        trees[s].owns_recs = trees[s].owns_qnodes = s == 0 ? 1u : 0u;
+        trees[s].owns_recs = s == 0 ? 1u : 0u;
+        trees[s].owns_qnodes = (B.boxes ? MNRT_QNODES_BOXES : 0u) | (s == 0 ? MNRT_QNODES_OWNED : 0u);
     }
     return MNRT_OK;
 }
@@ -407,10 +523,14 @@ extern "C" int mnrt_tree_release(mnrt_tree* tree) {
         if (tree->d_nodes && mnrt::pool_free(tree->d_nodes, nullptr) != hipSuccess) rc = MNRT_ERR_HIP;
         if (tree->d_refs && mnrt::pool_free(tree->d_refs, nullptr) != hipSuccess) rc = MNRT_ERR_HIP;
     }
-    if (tree->owns_qnodes && tree->d_qnodes && mnrt::pool_free(tree->d_qnodes, nullptr) != hipSuccess)
-        rc = MNRT_ERR_HIP;
-    if (tree->owns_qnodes) tree->d_qnodes = nullptr;
-    tree->owns_qnodes = 0;
+    if ((tree->owns_qnodes & MNRT_QNODES_OWNED) && tree->d_qnodes) {
+        const uint64_t bw = (tree->owns_qnodes & MNRT_QNODES_BOXES) ? mnrt::box_words(tree->num_elems) : 0u;
+        if (mnrt::pool_free(tree->d_qnodes - bw, nullptr) != hipSuccess) rc = MNRT_ERR_HIP;
+    }
+    if (tree->owns_qnodes & MNRT_QNODES_OWNED) {
+        tree->d_qnodes = nullptr;
+        tree->owns_qnodes = 0;
+    }
     if (tree->owns_recs) tree->d_recs = nullptr;
     if (tree->owns_nodes) {
         tree->d_nodes = nullptr;

@@ -18,6 +18,7 @@ KIND_TRI = 0
 KIND_POINT = 1
 MAX_LEVEL = 48
 KNN_MAX_K = 256
+QNODES_OWNED, QNODES_BOXES = 1, 2  # owns_qnodes bits
 
 u32 = ctypes.c_uint32
 f32 = ctypes.c_float
