@@ -164,7 +164,7 @@ int mnrt_tree_attach_photon_records_batch(mnrt_tree* trees, uint32_t num_scenes,
 /* Device-driven batched build recorded into a hipGraph (no reference counterpart: the
  * reference's level loop reads its counters on the host every level, KDTreeGPU.cpp:247-281).
  * mnrt_build_graph_create builds the batch once as mnrt_build_*_batch does, sizes fixed
- * buffers from that build (each quantity the level loop grows a buffer for, times
+ * buffers from that build (nodes, elements, small roots, copied leaf elements: times
  * 1 + margin), and records the whole build into a graph: every level (num_levels of the
  * first build + 2), the small-node stage, layout, emission, the records (photon trees
  * when d_power4 / d_dir4 are given) and, for photon trees, the query-time node words.
@@ -180,7 +180,7 @@ int mnrt_tree_attach_photon_records_batch(mnrt_tree* trees, uint32_t num_scenes,
  * invalid until a replay that fits; create a new graph for the new sizes).  Bits: 64 a
  * level outgrew the level buffers, 128 more levels than recorded, 256 the trees outgrew
  * the output arrays, 512 the large-node stage went more than 6 levels deeper than the
- * first build (the recorded layout's depth); 1..32 as the host-driven build's errors. */
+ * first build; 1..32 an inconsistency, as in a host-driven build. */
 typedef struct mnrt_build_graph mnrt_build_graph;
 typedef struct mnrt_build_graph_desc {
     int kind;                         /* MNRT_KIND_TRI or MNRT_KIND_POINT */

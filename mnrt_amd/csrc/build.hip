@@ -4,22 +4,21 @@
 //
 //   large-node stage (LargeNodeStage / ProcessLargeNodes, KDTreeGPU.cpp:247-782):
 //     per level, for all active nodes at once:
-//       chunk list + tight bounds   k_chunk_*, k_tight     (kdtree_chunklist.cu:73-184, kdtree.cu:310-445)
-//       empty-space cuts + median   k_plan                 (kdtree.cu:467-682, 1986-2033)
-//       element classification      k_classify             (kdtree.cu:752-824)
-//       stream compaction           scan of L/R flags      (CompactElementData, KDTreeGPU.cpp:664-782)
-//       small/large partition       k_child_plan/_write    (UpdateSmallList, KDTreeGPU.cpp:784-941)
-//       split clipping + scatter    k_scatter              (kdtree_tri.cu:190-489)
-//     The level loop keeps all per-element work on the device; the host reads five
-//     counters once per level (the reference synchronises about ten times per level).
+//       classification counts       k_count     (kdtree.cu:467-682, 752-824, 1986-2033)
+//       compaction offsets, children, small/large partition
+//                                   k_children  (CompactElementData / UpdateSmallList, KDTreeGPU.cpp:664-941)
+//       scatter + tight bounds      k_scatter   (kdtree_chunklist.cu:73-184, kdtree.cu:310-445)
+//       split clipping              k_clip      (kdtree_tri.cu:190-489)
+//     All counts stay on the device; the host waits for a run of levels at a time (the
+//     reference synchronises about ten times per level).
 //
 //   small-node stage (PreProcessSmallNodes / ProcessSmallNodes, KDTreeGPU.cpp:945-1154):
 //     one wave64 per small root builds the whole subtree in LDS: split candidates and
 //     their 64-bit element masks (kdtree.cu:1035-1251), exact SAH / VVH per node with a
 //     wave argmin over (cost, candidate index) (kdtree.cu:1288-1471), preorder emission.
 //
-//   layout: subtree sizes bottom-up, addresses top-down (KDTreeGPU::PreorderTraversal,
-//   KDTreeGPU.cpp:1156-1209), in one single-workgroup pass over the large-stage nodes.
+//   layout: subtree sizes climb from the leaves, addresses are sums over the ancestors
+//   (KDTreeGPU::PreorderTraversal, KDTreeGPU.cpp:1156-1209): two launches.
 //
 // Deterministic rules replace the reference's random and racy choices (elements in a
 // split plane go left for even index, right for odd; equal SAH costs resolve to the
@@ -37,35 +36,15 @@
 
 namespace mnrt {
 
-constexpr uint32_t kChunk = 256;
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 
-enum : uint32_t { BN_LEAF = 3, BN_SMALL = 4, BN_PENDING = 5, BN_DEAD = 6 };
-// counters[] slots written by device kernels
-enum : uint32_t {
-    C_NCHUNKS = 0,
-    C_NEWNODES,
-    C_NSMALL_NEW,
-    C_NNEXT,
-    C_ESMALL_NEW,
-    C_ENEXT,
-    C_MAXLEVEL,
-    C_LLCOUNT,
-    C_TOTAL_NODES,
-    C_TOTAL_REFS,
-    C_LEAVES,
-    C_NLEAFCOPY,
-    C_ERR,
-    C_SMALL_OVF,  // small roots whose subtree outgrew its staging area
-    C_COUNT
-};
-
+enum : uint32_t { BN_LEAF = 3, BN_SMALL = 4, BN_PENDING = 5 };
 // Build-node table: one entry per node of the large-stage tree (inner nodes, empty
-// and capped leaves, small roots), 8 uint32 columns of `cap` entries.  Build nodes
+// and capped leaves, small roots), 10 uint32 columns of `cap` entries.  Build nodes
 // 0..S-1 are the roots of the S scenes built together.
-constexpr int kBnCols = 8;
+constexpr int kBnCols = 10;
 struct BnView {
-    uint32_t* type;   // 0..2 inner split axis, BN_LEAF, BN_SMALL, BN_PENDING, BN_DEAD
+    uint32_t* type;   // 0..2 inner split axis, BN_LEAF, BN_SMALL, BN_PENDING
     uint32_t* split;  // split position bits (inner)
     uint32_t* left;
     uint32_t* right;
@@ -73,6 +52,8 @@ struct BnView {
     uint32_t* aux;  // small-root index (BN_SMALL) or first copied element (BN_LEAF)
     uint32_t* cnt;  // element count (BN_LEAF)
     uint32_t* scene;
+    uint32_t* parent;  // kNone for a root
+    uint32_t* flag;    // children whose subtree sizes are known (k_layout_sizes)
 };
 
 struct SmallView {  // small roots
@@ -82,23 +63,6 @@ struct SmallView {  // small roots
     uint32_t* bn;
     float4* lo;
     float4* hi;
-    uint32_t* scene;
-};
-
-struct ElemView {  // element arrays: original index, bounds, owning active node
-    uint32_t* idx;
-    float4* lo;
-    float4* hi;
-    uint32_t* node;
-};
-
-struct NodeView {  // active large nodes
-    float4* lo;
-    float4* hi;
-    uint32_t* first;
-    uint32_t* cnt;
-    uint32_t* level;
-    uint32_t* bn;
     uint32_t* scene;
 };
 
@@ -258,155 +222,269 @@ __device__ void clip_bounds(const Geometry& G, uint32_t idx, float4& lo, float4&
         f4set(hi, ax, canon(h));
     }
 }
-
 // ---------------------------------------------------------------------------------------
-// kernels
+// large-node stage
 // ---------------------------------------------------------------------------------------
-// Counts come as DN (host value or device word).  Per-item kernels stride over the grid,
-// so any grid is correct: the host-driven build launches one item per thread, the
-// recorded device-driven build launches grids sized from the first build's counts.
-#define MNRT_GRID_STRIDE(i, n) \
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += gridDim.x * blockDim.x)
+// Elements of an active node fill consecutive slots from a multiple of 64 on, so every wave of
+// 64 slots belongs to one node: its values are wave-uniform, and a stable partition needs a
+// prefix sum over waves (one packed word each), not over elements.  A level is four launches
+// (three for points):
+//   k_count     classifies every element, one packed (left, right) count per wave;
+//   k_children  per node: prefix of its waves' counts, the children's places and build nodes;
+//   k_scatter   classifies again, writes every element into its children and accumulates the
+//               tight bounds of the next level's nodes;
+//   k_clip      bounds of straddling triangles, from a queue.
+// Places are handed out by atomics, aggregated per workgroup, so nodes and small roots lie in an
+// arbitrary order (the tree does not depend on it: a node's elements keep theirs, and the final
+// addresses come from the layout).  All counts stay on the device: a launch reads the level's
+// (nodes, waves) from the level table, an empty level returns at once, and whatever would
+// outgrow a buffer sets kErrRoom instead, after which every later kernel returns.
+// Measured against one launch per step over chunk lists, element flags and three-pass scans (16
+// launches a level and a host synchronisation): 1.03M triangles 5.5 -> 3.2 ms, 1M photons 3.6 ->
+// 1.5 ms, 3001 triangles 1.28 -> 0.61 ms, 32 scenes' triangle and photon trees recorded 4.0 -> 2.0
+// ms.
 
-__global__ __launch_bounds__(256) void k_init_elems(Geometry G, uint32_t n, ElemView E) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t s = scene_of(G.base, G.num_scenes, i);
-    float4 a = G.v0[i];
-    float4 lo, hi;
-    if (G.kind == MNRT_KIND_TRI) {
-        float4 b = G.v1[i], c = G.v2[i];
-        lo = make_float4(canon(fminf(a.x, fminf(b.x, c.x))), canon(fminf(a.y, fminf(b.y, c.y))),
-                         canon(fminf(a.z, fminf(b.z, c.z))), 0.0f);
-        hi = make_float4(canon(fmaxf(a.x, fmaxf(b.x, c.x))), canon(fmaxf(a.y, fmaxf(b.y, c.y))),
-                         canon(fmaxf(a.z, fmaxf(b.z, c.z))), 0.0f);
-    } else {
-        lo = hi = make_float4(canon(a.x), canon(a.y), canon(a.z), 0.0f);
-    }
-    E.idx[i] = i - G.base[s];
-    E.lo[i] = lo;
-    E.hi[i] = hi;
-    E.node[i] = s;
+// Device words of a build: totals, then the level table.
+enum : uint32_t {
+    W_ERR = 0,
+    W_MAXLEVEL,    // deepest build node
+    W_SMALL_OVF,   // small roots whose subtree outgrew its staging area
+    W_NBN,         // build nodes
+    W_LL,          // elements of large-stage leaves
+    W_NSE = 6,     // small-root elements, small roots: one 64-bit word
+    W_NSMALL = 7,
+    W_LEVELS = 8,  // per level: waves, nodes (one 64-bit word), clip jobs, 0
+};
+constexpr uint32_t kLevels = MNRT_MAX_LEVEL + 2;  // every level's nodes are deeper than the last's
+constexpr uint32_t kWords = W_LEVELS + 4 * (kLevels + 1);
+
+constexpr uint32_t kErrRoom = 64u;          // a buffer was outgrown
+constexpr uint32_t kErrLevels = 128u;       // active nodes left after the last recorded level
+constexpr uint32_t kErrOutputRoom = 256u;   // the trees outgrew the output arrays
+constexpr uint32_t kErrLayoutDepth = 512u;  // a build node deeper than the recording covers
+
+struct BuildCaps {
+    uint32_t na;     // active nodes of a level
+    uint32_t nw;     // waves of a level (64 slots each)
+    uint32_t bn;     // build nodes
+    uint32_t small;  // small roots
+    uint32_t se;     // small-root elements
+    uint32_t ll;     // elements of large-stage leaves
+};
+
+// Active nodes of a level.  tb: tight bounds, 6 words per node, the minima of fenc(lo) and of
+// ~fenc(hi).
+struct NodeView {
+    float4* lo;
+    float4* hi;
+    uint32_t* first;
+    uint32_t* cnt;
+    uint32_t* level;
+    uint32_t* bn;
+    uint32_t* scene;
+    uint32_t* tb;
+};
+
+struct ElemView {  // element arrays: original index, bounds; wnode: active node of every wave
+    uint32_t* idx;
+    float4* lo;
+    float4* hi;
+    uint32_t* wnode;
+};
+
+// What k_children decided about a node.
+enum : uint32_t { CH_DEAD = 0, CH_SMALL, CH_LARGE, CH_LEAF };
+struct SplitView {
+    float4* lo;      // box after the empty-space cuts
+    float4* hi;
+    uint32_t* axis;
+    float* split;
+    uint4* child;    // 2 per node: CH_*, first destination (CH_LEAF: first copied element), next-level node
+};
+
+// Everything the level kernels work on.
+struct LevelArgs {
+    uint32_t* W;
+    uint32_t level;
+    BuildCaps cap;
+    float ratio;
+    uint32_t small_max;
+    NodeView A, An;
+    ElemView E, Nx, Sm;
+    uint32_t* wc;   // per wave: left count | right count << 16
+    uint2* woff;    // per wave: elements of its node before it, left and right
+    SplitView P;
+    SmallView S;
+    BnView B;
+    uint32_t* ll_idx;
+    uint2* q;       // clip jobs (two per slot at most): slot << 1 | side, destination
+};
+
+__device__ __forceinline__ uint32_t level_waves(const LevelArgs& L) {
+    return L.W[W_ERR] != 0u ? 0u : min(L.W[W_LEVELS + 4 * L.level], L.cap.nw);
+}
+__device__ __forceinline__ uint32_t level_nodes(const LevelArgs& L) {
+    return L.W[W_ERR] != 0u ? 0u : min(L.W[W_LEVELS + 4 * L.level + 1], L.cap.na);
 }
 
-// Chunks per node, and the node's tight-bound accumulators (3 per node, ordered-int
-// encoding) cleared for k_tight.
-__global__ __launch_bounds__(256) void k_chunk_counts(DN dn_, const uint32_t* __restrict__ cnt,
-                                                      uint32_t* __restrict__ cc, uint32_t* __restrict__ tlo,
-                                                      uint32_t* __restrict__ thi) {
-    const uint32_t n = dn_.get();
-    MNRT_GRID_STRIDE(p, n) {
-        cc[p] = (cnt[p] + kChunk - 1) / kChunk;
+// Empty-space cuts then the spatial median split (kernel_CanCutOffEmptySpace,
+// kernel_EmptySpaceCutting, kernel_SplitLargeNodes; kdtree.cu:467-682).  Sides are cut in
+// the reference's order (min x, y, z, then max x, y, z); each cut turns the node into an
+// inner node with an empty leaf and a tighter copy (on_cut).  The median splits the longest axis
+// of the cut box, ties to the lower axis.
+struct Plan {
+    float lo[3], hi[3];
+    uint32_t level;  // of the node that is split
+    uint32_t ncuts;
+    uint32_t axis;
+    float split;
+    bool leaf;  // level cap reached: the node is a leaf with its elements
+};
+
+template <typename F>
+__device__ __forceinline__ Plan plan_node(const NodeView& A, uint32_t p, float ratio, F&& on_cut) {
+    Plan R;
+    const float4 l4 = A.lo[p], h4 = A.hi[p];
+    R.lo[0] = l4.x; R.lo[1] = l4.y; R.lo[2] = l4.z;
+    R.hi[0] = h4.x; R.hi[1] = h4.y; R.hi[2] = h4.z;
+    R.level = A.level[p];
+    R.ncuts = 0;
 #pragma unroll
-        for (uint32_t a = 0; a < 3; ++a) {
-            tlo[3 * p + a] = 0xFFFFFFFFu;
-            thi[3 * p + a] = 0u;
-        }
+    for (int side = 0; side < 6; ++side) {
+        const int ax = side % 3;
+        const bool is_max = side >= 3;
+        if (R.level >= MNRT_MAX_LEVEL) continue;
+        const float tight = is_max ? fdec(~A.tb[6 * p + side]) : fdec(A.tb[6 * p + side]);
+        const float total = R.hi[ax] - R.lo[ax];
+        const float empty = is_max ? R.hi[ax] - tight : tight - R.lo[ax];
+        if (!(empty > total * ratio)) continue;
+        on_cut(ax, is_max, tight, R.level, R.ncuts);
+        ++R.ncuts;
+        ++R.level;
+        if (is_max) R.hi[ax] = tight;
+        else R.lo[ax] = tight;
     }
+    R.leaf = R.level >= MNRT_MAX_LEVEL;
+    const float ex = R.hi[0] - R.lo[0], ey = R.hi[1] - R.lo[1], ez = R.hi[2] - R.lo[2];
+    R.axis = 0;
+    float emax = ex, lo = R.lo[0], hi = R.hi[0];
+    if (ey > emax) { R.axis = 1; emax = ey; lo = R.lo[1]; hi = R.hi[1]; }
+    if (ez > emax) { R.axis = 2; lo = R.lo[2]; hi = R.hi[2]; }
+    R.split = lo + 0.5f * (hi - lo);
+    return R;
 }
 
-// Chunk -> node by binary search over the chunk offsets (kernel_GenerateChunks,
-// kdtree_chunklist.cu:110-134, runs one serial thread per node instead).
-__global__ __launch_bounds__(256) void k_chunk_fill(DN dn_, uint32_t max_chunks, const uint32_t* __restrict__ coff,
-                                                    const uint32_t* __restrict__ counters,
-                                                    const uint32_t* __restrict__ first,
-                                                    const uint32_t* __restrict__ cnt, uint32_t* __restrict__ ch_node,
-                                                    uint32_t* __restrict__ ch_first, uint32_t* __restrict__ ch_cnt) {
-    const uint32_t n = dn_.get();
-    const uint32_t nch = min(max_chunks, counters[C_NCHUNKS]);
-    MNRT_GRID_STRIDE(c, nch) {
-        uint32_t lo = 0, hi = n;  // last p with coff[p] <= c
-        while (hi - lo > 1) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (coff[mid] <= c) lo = mid;
-            else hi = mid;
-        }
-        uint32_t p = lo;
-        uint32_t local = c - coff[p];
-        ch_node[c] = p;
-        ch_first[c] = first[p] + local * kChunk;
-        ch_cnt[c] = min(kChunk, cnt[p] - local * kChunk);
-    }
+// Clears a build's words and sets its first level (na nodes in nw waves), small roots and build
+// nodes; the scenes' tight bounds start empty.
+__global__ __launch_bounds__(256) void k_build_init(uint32_t* __restrict__ W, uint32_t na, uint32_t nw, uint32_t nsmall,
+                                                    uint32_t nse, uint32_t nscenes, uint32_t* __restrict__ stb) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kWords)
+        W[i] = i == W_NBN ? nscenes : i == W_NSE ? nse : i == W_NSMALL ? nsmall : i == W_LEVELS ? nw
+               : i == W_LEVELS + 1 ? na : 0u;
+    for (uint32_t j = i; j < 6 * nscenes; j += gridDim.x * blockDim.x) stb[j] = 0xFFFFFFFFu;
 }
 
-// Tight node bounds: per-chunk wave/LDS min/max (kernel_GenChunkAABB + two segmented
-// reductions, kdtree.cu:310-445, KDTreeGPU.cpp:526-553).  A workgroup reduces
-// kTightChunks consecutive chunks and issues one atomic per component each time the
-// owning node changes (chunks are ordered by node, so a large node's many chunks cost
-// few atomics).  min/max are exact, so the order of the atomics does not matter.
-constexpr uint32_t kTightChunks = 8;
-
-__global__ __launch_bounds__(kChunk) void k_tight(uint32_t max_chunks, const uint32_t* __restrict__ counters,
-                                                  const uint32_t* __restrict__ ch_node,
-                                                  const uint32_t* __restrict__ ch_first,
-                                                  const uint32_t* __restrict__ ch_cnt, ElemView E, int kind,
-                                                  uint32_t* __restrict__ tlo, uint32_t* __restrict__ thi) {
-    __shared__ uint32_t s_red[6][kChunk / 64];
-    const uint32_t nch = min(max_chunks, counters[C_NCHUNKS]);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (uint32_t c0 = blockIdx.x * kTightChunks; c0 < nch; c0 += gridDim.x * kTightChunks) {  // uniform per block
-        const uint32_t c1 = min(c0 + kTightChunks, nch);
-        uint32_t cur = kNone;  // node of the running accumulation (thread 0)
-        uint32_t acc[6] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u, 0u};
-        for (uint32_t c = c0; c < c1; ++c) {
-            const uint32_t node = ch_node[c], first = ch_first[c], count = ch_cnt[c];
-            uint32_t v[6] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u, 0u};
-            if (threadIdx.x < count) {
-                float4 lo = E.lo[first + threadIdx.x];
-                float4 hi = (kind == MNRT_KIND_TRI) ? E.hi[first + threadIdx.x] : lo;
-                v[0] = fenc(lo.x);
-                v[1] = fenc(lo.y);
-                v[2] = fenc(lo.z);
-                v[3] = fenc(hi.x);
-                v[4] = fenc(hi.y);
-                v[5] = fenc(hi.z);
-            }
-#pragma unroll
-            for (int k = 0; k < 3; ++k) v[k] = wave_min_u32(v[k]);
-#pragma unroll
-            for (int k = 3; k < 6; ++k) v[k] = wave_max_u32(v[k]);
-            if (lane == 0)
-                for (int k = 0; k < 6; ++k) s_red[k][wave] = v[k];
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                for (uint32_t w = 1; w < kChunk / 64; ++w) {
-                    for (int k = 0; k < 3; ++k) v[k] = min(v[k], s_red[k][w]);
-                    for (int k = 3; k < 6; ++k) v[k] = max(v[k], s_red[k][w]);
-                }
-                if (node != cur && cur != kNone) {
-                    for (int k = 0; k < 3; ++k) atomicMin(&tlo[3 * cur + k], acc[k]);
-                    for (int k = 0; k < 3; ++k) atomicMax(&thi[3 * cur + k], acc[3 + k]);
-                    for (int k = 0; k < 3; ++k) acc[k] = 0xFFFFFFFFu;
-                    for (int k = 3; k < 6; ++k) acc[k] = 0u;
-                }
-                cur = node;
-                for (int k = 0; k < 3; ++k) acc[k] = min(acc[k], v[k]);
-                for (int k = 3; k < 6; ++k) acc[k] = max(acc[k], v[k]);
-            }
-            __syncthreads();  // s_red is rewritten by the next chunk
-        }
-        if (threadIdx.x == 0 && cur != kNone) {
-            for (int k = 0; k < 3; ++k) atomicMin(&tlo[3 * cur + k], acc[k]);
-            for (int k = 0; k < 3; ++k) atomicMax(&thi[3 * cur + k], acc[3 + k]);
-        }
-    }
-}
-
-// Per-scene placement decided on the host: an active (large) root or a small root, its
-// index in that list and its first element there.
+// Per-scene placement decided on the host: an active (large) root or a small root, its index in
+// that list and its first slot there.
 struct RootPlan {
-    const uint32_t* kind;   // 0 active, 1 small
+    const uint32_t* kind;  // 0 active, 1 small
     const uint32_t* index;
     const uint32_t* off;
 };
 
+__device__ __forceinline__ void tight_words(const float4& lo, const float4& hi, uint32_t (&v)[6]) {
+    v[0] = fenc(lo.x);
+    v[1] = fenc(lo.y);
+    v[2] = fenc(lo.z);
+    v[3] = ~fenc(hi.x);
+    v[4] = ~fenc(hi.y);
+    v[5] = ~fenc(hi.z);
+}
+
+// Adds the lanes' tight words to their targets tb[6 * to ..] (kNone: none), lanes that share a
+// target reduced first: one atomic per component and distinct target.  Whole wave.
+__device__ __forceinline__ void tight_by_key(uint32_t to, const uint32_t (&v)[6], uint32_t* __restrict__ tb,
+                                             uint32_t lane) {
+    for (uint64_t m = ballot(to != kNone); m != 0ull;) {
+        const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)to, (int)__builtin_ctzll(m));
+        const bool mine = to == t;
+        uint32_t best = ~0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 6; ++k) {
+            const uint32_t r = wave_min_u32(mine ? v[k] : ~0u);
+            if (lane == k) best = r;
+        }
+        if (lane < 6u) atomicMin(&tb[6u * t + lane], best);
+        m &= ~ballot(mine);
+    }
+}
+
+// Input elements: bounds, placed with their scene's root (elements of a small scene with the small
+// roots), and the scenes' tight bounds.  A workgroup takes kInitPer elements per thread, so a
+// scene's bounds cost one atomic per component and workgroup unless the workgroup spans scenes.
+constexpr uint32_t kInitBlock = 1024, kInitPer = 4;
+
+__global__ __launch_bounds__(kInitBlock) void k_init_elems(Geometry G, uint32_t n, RootPlan R, ElemView E, ElemView Sm,
+                                                           uint32_t* __restrict__ stb) {
+    __shared__ uint32_t s_min[kInitBlock / 64][6];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t b0 = blockIdx.x * (kInitBlock * kInitPer), b1 = min(b0 + kInitBlock * kInitPer, n);
+    const uint32_t s0 = scene_of(G.base, G.num_scenes, b0);
+    const bool one = b1 <= G.base[s0 + 1];  // the workgroup's elements are one scene's
+    uint32_t acc[6] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
+    for (uint32_t t = 0; t < kInitPer; ++t) {
+        const uint32_t i = b0 + t * kInitBlock + threadIdx.x;
+        uint32_t s = kNone;
+        uint32_t v[6] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
+        if (i < b1) {
+            s = one ? s0 : scene_of(G.base, G.num_scenes, i);
+            const float4 a = G.v0[i];
+            float4 lo, hi;
+            if (G.kind == MNRT_KIND_TRI) {
+                const float4 b = G.v1[i], c = G.v2[i];
+                lo = make_float4(canon(fminf(a.x, fminf(b.x, c.x))), canon(fminf(a.y, fminf(b.y, c.y))),
+                                 canon(fminf(a.z, fminf(b.z, c.z))), 0.0f);
+                hi = make_float4(canon(fmaxf(a.x, fmaxf(b.x, c.x))), canon(fmaxf(a.y, fmaxf(b.y, c.y))),
+                                 canon(fmaxf(a.z, fmaxf(b.z, c.z))), 0.0f);
+            } else {
+                lo = hi = make_float4(canon(a.x), canon(a.y), canon(a.z), 0.0f);
+            }
+            const uint32_t local = i - G.base[s], d = R.off[s] + local;
+            const bool small = R.kind[s] != 0u;
+            const ElemView& D = small ? Sm : E;
+            D.idx[d] = local;
+            D.lo[d] = lo;
+            if (G.kind == MNRT_KIND_TRI) D.hi[d] = hi;
+            if (!small && (d & 63u) == 0u) E.wnode[d >> 6] = R.index[s];
+            tight_words(lo, hi, v);
+        }
+        if (one) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) acc[k] = min(acc[k], v[k]);
+        } else {
+            tight_by_key(s, v, stb, lane);
+        }
+    }
+    if (!one) return;  // uniform per workgroup
+#pragma unroll
+    for (int k = 0; k < 6; ++k) acc[k] = wave_min_u32(acc[k]);
+    if (lane == 0)
+        for (int k = 0; k < 6; ++k) s_min[wave][k] = acc[k];
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        uint32_t m = ~0u;
+        for (uint32_t w = 0; w < kInitBlock / 64; ++w) m = min(m, s_min[w][threadIdx.x]);
+        atomicMin(&stb[6 * s0 + threadIdx.x], m);
+    }
+}
+
 // Root boxes (given, or the tight bounds of the scene's elements; (+max, -max) for an
 // empty scene) and the root entries of the active / small lists.
 __global__ __launch_bounds__(256) void k_roots_setup(uint32_t nscenes, const uint32_t* __restrict__ base,
-                                                     const uint32_t* __restrict__ tlo,
-                                                     const uint32_t* __restrict__ thi,
-                                                     const float* __restrict__ given, RootPlan R, NodeView A,
-                                                     SmallView S, BnView B, float* __restrict__ out_box) {
+                                                     const uint32_t* __restrict__ stb, const float* __restrict__ given,
+                                                     RootPlan R, NodeView A, SmallView S, BnView B,
+                                                     float* __restrict__ out_box) {
     uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nscenes) return;
     const uint32_t cnt = base[s + 1] - base[s];
@@ -418,11 +496,13 @@ __global__ __launch_bounds__(256) void k_roots_setup(uint32_t nscenes, const uin
         lo = make_float4(kInf, kInf, kInf, 0.0f);
         hi = make_float4(-kInf, -kInf, -kInf, 0.0f);
     } else {
-        lo = make_float4(fdec(tlo[3 * s]), fdec(tlo[3 * s + 1]), fdec(tlo[3 * s + 2]), 0.0f);
-        hi = make_float4(fdec(thi[3 * s]), fdec(thi[3 * s + 1]), fdec(thi[3 * s + 2]), 0.0f);
+        lo = make_float4(fdec(stb[6 * s]), fdec(stb[6 * s + 1]), fdec(stb[6 * s + 2]), 0.0f);
+        hi = make_float4(fdec(~stb[6 * s + 3]), fdec(~stb[6 * s + 4]), fdec(~stb[6 * s + 5]), 0.0f);
     }
     B.level[s] = 0;
     B.scene[s] = s;
+    B.parent[s] = kNone;
+    B.flag[s] = 0u;
     const uint32_t i = R.index[s];
     if (R.kind[s] == 0) {
         A.lo[i] = lo;
@@ -432,6 +512,7 @@ __global__ __launch_bounds__(256) void k_roots_setup(uint32_t nscenes, const uin
         A.level[i] = 0;
         A.bn[i] = s;
         A.scene[i] = s;
+        for (int k = 0; k < 6; ++k) A.tb[6 * i + k] = stb[6 * s + k];
         B.type[s] = BN_PENDING;
     } else {
         S.first[i] = R.off[s];
@@ -452,399 +533,361 @@ __global__ __launch_bounds__(256) void k_roots_setup(uint32_t nscenes, const uin
     out_box[6 * s + 5] = hi.z;
 }
 
-// Elements of large scenes go to the first level's arrays, those of small scenes to the
-// small-root buffer; each keeps its scene order.
-__global__ __launch_bounds__(256) void k_partition_elems(uint32_t n, ElemView In, int kind, RootPlan R, ElemView E,
-                                                         ElemView Sm) {
-    uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n) return;
-    const uint32_t s = In.node[g], local = In.idx[g];
-    const uint32_t d = R.off[s] + local;
-    float4 lo = In.lo[g];
-    if (R.kind[s] == 0) {
-        E.idx[d] = local;
-        E.lo[d] = lo;
-        if (kind == MNRT_KIND_TRI) E.hi[d] = In.hi[g];
-        E.node[d] = R.index[s];
-    } else {
-        Sm.idx[d] = local;
-        Sm.lo[d] = lo;
-        if (kind == MNRT_KIND_TRI) Sm.hi[d] = In.hi[g];
+// Left and right counts of every wave.  The wave makes its node's plan itself (about 100
+// instructions on values it shares, less than another launch and its latency).
+template <int kKind>
+__global__ __launch_bounds__(256) void k_count(LevelArgs L) {
+    const uint32_t nw = level_waves(L), lane = threadIdx.x & 63u;
+    for (uint32_t w = uniform(blockIdx.x * 4u + (threadIdx.x >> 6)); w < nw; w += gridDim.x * 4u) {
+        const uint32_t p = uniform(L.E.wnode[w]), e = 64u * w + lane;
+        const float4 lo = L.E.lo[e];  // (slots past the node's last element hold anything)
+        const float4 hi = (kKind == MNRT_KIND_TRI) ? L.E.hi[e] : lo;
+        const uint32_t idx = L.E.idx[e];
+        const Plan R = plan_node(L.A, p, L.ratio, [](int, bool, float, uint32_t, uint32_t) {});
+        bool l = false, r = false;
+        if (!R.leaf && e - L.A.first[p] < L.A.cnt[p]) classify(kKind, idx, lo, hi, R.axis, R.split, l, r);
+        const uint32_t c = (uint32_t)__popcll(ballot(l)) | (uint32_t)__popcll(ballot(r)) << 16;
+        if (lane == 0) L.wc[w] = c;
     }
 }
 
-struct PlanView {
-    uint32_t* newcnt;  // build nodes created per active node (count phase) / base (write phase)
-    uint32_t* axis;
-    float* split;
-    float4* lo;        // box after the empty-space cuts
-    float4* hi;
-    uint32_t* level;   // level of the node that is split (after cuts)
-    uint32_t* childL;  // build-node id of the left child (right = +1)
-    uint32_t* cur;     // build-node id of the node that is split or becomes a leaf
-    uint32_t* leaf;    // 1: level cap reached, the node is a leaf with its elements
-    uint32_t* noprog;  // 1: every element went to both children, the node is a leaf
+// Children of 16 nodes per workgroup step, one wave per node (512 of its waves' counts per
+// pass: the root of a million elements takes 32 passes, about 20 us, nodes below 32768
+// elements one).  The places of the 16 nodes' children come from one atomic per quantity.
+constexpr uint32_t kChildBlock = 1024, kChildNodes = kChildBlock / 64;
+
+struct ChildNeed {  // what a node asks for
+    uint32_t bn, na, nw, nsmall, nse, ll;
 };
 
-// Empty-space cuts then the spatial median split (kernel_CanCutOffEmptySpace,
-// kernel_EmptySpaceCutting, kernel_SplitLargeNodes; kdtree.cu:467-682).  Sides are cut in
-// the reference's order (min x, y, z, then max x, y, z); each cut turns the node into an
-// inner node with an empty leaf and a tighter copy.  The median splits the longest axis
-// of the cut box, ties to the lower axis.
-template <bool kWrite>
-__device__ __forceinline__ void plan_node(uint32_t p, const NodeView& A, const uint32_t* __restrict__ tlo,
-                                          const uint32_t* __restrict__ thi, float ratio, const PlanView& P,
-                                          const uint32_t* __restrict__ base, uint32_t bn_base, const BnView& B,
-                                          uint32_t* __restrict__ counters) {
-    float lo[3], hi[3], tl[3], th[3];
-    float4 l4 = A.lo[p], h4 = A.hi[p];
-    lo[0] = l4.x; lo[1] = l4.y; lo[2] = l4.z;
-    hi[0] = h4.x; hi[1] = h4.y; hi[2] = h4.z;
-    for (int k = 0; k < 3; ++k) {
-        tl[k] = fdec(tlo[3 * p + k]);
-        th[k] = fdec(thi[3 * p + k]);
-    }
-    uint32_t level = A.level[p];
-    uint32_t cur = A.bn[p];
-    uint32_t next_id = kWrite ? bn_base + base[p] : 0u;
-    uint32_t ncuts = 0;
-    for (int isMax = 0; isMax < 2; ++isMax) {
-        for (int ax = 0; ax < 3; ++ax) {
-            if (level >= MNRT_MAX_LEVEL) continue;
-            float total = hi[ax] - lo[ax];
-            float empty = isMax ? (hi[ax] - th[ax]) : (tl[ax] - lo[ax]);
-            if (!(empty > total * ratio)) continue;
-            float s = isMax ? th[ax] : tl[ax];
-            ++ncuts;
-            if (kWrite) {
-                uint32_t eleaf = next_id++, cont = next_id++;
-                B.type[cur] = (uint32_t)ax;
-                B.split[cur] = __float_as_uint(s);
-                B.left[cur] = isMax ? cont : eleaf;
-                B.right[cur] = isMax ? eleaf : cont;
-                B.type[eleaf] = BN_LEAF;
-                B.cnt[eleaf] = 0;
-                B.aux[eleaf] = 0;
-                B.level[eleaf] = level + 1;
-                B.scene[eleaf] = A.scene[p];
-                B.type[cont] = BN_PENDING;
-                B.level[cont] = level + 1;
-                B.scene[cont] = A.scene[p];
-                cur = cont;
+__global__ __launch_bounds__(kChildBlock) void k_children(LevelArgs L) {
+    __shared__ ChildNeed s_need[kChildNodes], s_base;
+    __shared__ uint32_t s_na;  // one read for the workgroup: others may set the error while it runs
+    if (threadIdx.x == 0) s_na = level_nodes(L);
+    __syncthreads();
+    const uint32_t na = uniform(s_na), lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
+    for (uint32_t p0 = blockIdx.x * kChildNodes; p0 < na; p0 += gridDim.x * kChildNodes) {  // uniform per workgroup
+        const uint32_t p = p0 + wave;
+        const bool live = p < na;
+        Plan R{};
+        uint32_t m = 0, n[2] = {0u, 0u};
+        ChildNeed need{};
+        uint32_t type[2] = {CH_DEAD, CH_DEAD};
+        if (live) {
+            R = plan_node(L.A, p, L.ratio, [](int, bool, float, uint32_t, uint32_t) {});
+            m = L.A.cnt[p];
+            const uint32_t w0 = L.A.first[p] >> 6, nwv = (m + 63u) >> 6;
+            for (uint32_t b = 0; b < nwv; b += 512u) {
+                uint32_t c[8], sum = 0;
+#pragma unroll
+                for (uint32_t t = 0; t < 8; ++t) {
+                    const uint32_t i = b + lane * 8u + t;
+                    c[t] = i < nwv ? L.wc[w0 + i] : 0u;
+                    sum += c[t];
+                }
+                // packed halves: at most 512 * 64 each
+                const uint32_t incl = wave_incl_scan(sum, lane);
+                uint32_t run = incl - sum;
+#pragma unroll
+                for (uint32_t t = 0; t < 8; ++t) {
+                    const uint32_t i = b + lane * 8u + t;
+                    if (i < nwv) L.woff[w0 + i] = make_uint2(n[0] + (run & 0xFFFFu), n[1] + (run >> 16));
+                    run += c[t];
+                }
+                const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+                n[0] += tot & 0xFFFFu;
+                n[1] += tot >> 16;
             }
-            if (isMax) hi[ax] = s;
-            else lo[ax] = s;
-            level += 1;
-        }
-    }
-    if (!kWrite) {
-        P.newcnt[p] = 2 * ncuts + (level >= MNRT_MAX_LEVEL ? 0u : 2u);
-        return;
-    }
-    atomicMax(&counters[C_MAXLEVEL], level);
-    P.cur[p] = cur;
-    P.level[p] = level;
-    P.lo[p] = make_float4(lo[0], lo[1], lo[2], 0.0f);
-    P.hi[p] = make_float4(hi[0], hi[1], hi[2], 0.0f);
-    P.noprog[p] = 0;
-    if (level >= MNRT_MAX_LEVEL) {
-        P.leaf[p] = 1;
-        P.axis[p] = 0;
-        P.split[p] = 0.0f;
-        P.childL[p] = kNone;
-        B.type[cur] = BN_LEAF;
-        return;
-    }
-    float ex = hi[0] - lo[0], ey = hi[1] - lo[1], ez = hi[2] - lo[2];
-    uint32_t axis = 0;
-    float emax = ex;
-    if (ey > emax) { axis = 1; emax = ey; }
-    if (ez > emax) axis = 2;
-    float s = lo[axis] + 0.5f * (hi[axis] - lo[axis]);
-    uint32_t L = next_id++, R = next_id++;
-    P.leaf[p] = 0;
-    P.axis[p] = axis;
-    P.split[p] = s;
-    P.childL[p] = L;
-    B.type[cur] = axis;
-    B.split[cur] = __float_as_uint(s);
-    B.left[cur] = L;
-    B.right[cur] = R;
-    B.level[L] = level + 1;
-    B.level[R] = level + 1;
-    B.type[L] = BN_PENDING;
-    B.type[R] = BN_PENDING;
-    B.scene[L] = A.scene[p];
-    B.scene[R] = A.scene[p];
-}
-
-template <bool kWrite>
-__global__ __launch_bounds__(256) void k_plan(DN dn_, NodeView A, const uint32_t* __restrict__ tlo,
-                                              const uint32_t* __restrict__ thi, float ratio, PlanView P,
-                                              const uint32_t* __restrict__ base, DN bn_base, BnView B,
-                                              uint32_t* __restrict__ counters) {
-    const uint32_t n = dn_.get(), b0 = bn_base.get();
-    MNRT_GRID_STRIDE(p, n) plan_node<kWrite>(p, A, tlo, thi, ratio, P, base, b0, B, counters);
-}
-
-// Flags per element: left child, right child and, for triangles, straddling the split on
-// the left / right side (fl[2 ne + e], fl[3 ne + e]); one scan over them gives each element
-// side its child rank and each straddling side its slot in the clip queue.
-__global__ __launch_bounds__(256) void k_classify(DN dne, ElemView E, int kind, PlanView P,
-                                                  uint32_t* __restrict__ fl) {
-    const uint32_t ne = dne.get();
-    MNRT_GRID_STRIDE(e, ne) {
-        uint32_t p = E.node[e];
-        bool L = false, R = false, straddle = false;
-        if (!P.leaf[p]) {
-            float4 lo = E.lo[e];
-            float4 hi = (kind == MNRT_KIND_TRI) ? E.hi[e] : lo;
-            const uint32_t axis = P.axis[p];
-            const float s = P.split[p];
-            classify(kind, E.idx[e], lo, hi, axis, s, L, R);
-            straddle = (kind == MNRT_KIND_TRI) && (f4c(lo, axis) < s && s < f4c(hi, axis));
-        }
-        fl[e] = L ? 1u : 0u;
-        fl[ne + e] = R ? 1u : 0u;
-        if (kind == MNRT_KIND_TRI) {
-            fl[2 * ne + e] = (straddle && L) ? 1u : 0u;
-            fl[3 * ne + e] = (straddle && R) ? 1u : 0u;
-        }
-    }
-}
-
-struct ChildView {
-    uint32_t* type;  // BN_SMALL, BN_PENDING (large), BN_DEAD
-    uint32_t* cnt;
-    uint32_t* fpos;  // flag-scan position of the child's first element
-    uint32_t* sflag;
-    uint32_t* lflag;
-    uint32_t* scnt;
-    uint32_t* lcnt;
-    uint32_t* sidx;  // scans of the four columns above
-    uint32_t* lidx;
-    uint32_t* soff;
-    uint32_t* loff;
-};
-
-// Child counts from the flag scan, the no-progress test, and the small/large split
-// (kernel_MarkSmallNodes, kdtree.cu:849-875: small iff count <= smallNodeMax).
-__global__ __launch_bounds__(256) void k_child_plan(DN dn_, DN dne, NodeView A, PlanView P,
-                                                    const uint32_t* __restrict__ pos, uint32_t small_max,
-                                                    ChildView Cv) {
-    const uint32_t n = dn_.get(), ne = dne.get();
-    MNRT_GRID_STRIDE(c, 2 * n) {
-        uint32_t side = c >= n ? 1u : 0u;
-        uint32_t p = c - side * n;
-        uint32_t type = BN_DEAD, cnt = 0, fpos = 0;
-        if (!P.leaf[p]) {
-            uint32_t f = A.first[p], m = A.cnt[p];
-            uint32_t nl = pos[f + m] - pos[f];
-            uint32_t nr = pos[ne + f + m] - pos[ne + f];
-            bool noprog = (nl == m && nr == m);
-            if (noprog) {
-                if (side == 0) P.noprog[p] = 1;
+            // no progress: every element went to both children
+            const bool leaf = R.leaf || (n[0] == m && n[1] == m);
+            need.bn = 2u * R.ncuts + (leaf ? 0u : 2u);
+            if (leaf) {
+                type[0] = CH_LEAF;
+                need.ll = m;
             } else {
-                fpos = pos[side * ne + f];
-                cnt = side ? nr : nl;
-                type = (cnt <= small_max) ? BN_SMALL : BN_PENDING;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    // small iff count <= smallNodeMax (kernel_MarkSmallNodes, kdtree.cu:849-875)
+                    type[s] = n[s] <= L.small_max ? CH_SMALL : CH_LARGE;
+                    if (type[s] == CH_SMALL) {
+                        need.nsmall += 1u;
+                        need.nse += n[s];
+                    } else {
+                        need.na += 1u;
+                        need.nw += (n[s] + 63u) >> 6;
+                    }
+                }
             }
         }
-        Cv.type[c] = type;
-        Cv.cnt[c] = cnt;
-        Cv.fpos[c] = fpos;
-        Cv.sflag[c] = type == BN_SMALL ? 1u : 0u;
-        Cv.lflag[c] = type == BN_PENDING ? 1u : 0u;
-        Cv.scnt[c] = type == BN_SMALL ? cnt : 0u;
-        Cv.lcnt[c] = type == BN_PENDING ? cnt : 0u;
-    }
-}
-
-__device__ __forceinline__ void child_write_one(uint32_t c, uint32_t n, const NodeView& A, const PlanView& P,
-                                                const ChildView& Cv, uint32_t small_base, uint32_t small_elem_base,
-                                                const SmallView& S, const NodeView& Nx, const BnView& B,
-                                                uint32_t* __restrict__ counters) {
-    uint32_t side = c >= n ? 1u : 0u;
-    uint32_t p = c - side * n;
-    if (P.leaf[p]) return;
-    if (P.noprog[p]) {
-        if (side == 0) {
-            B.type[P.cur[p]] = BN_LEAF;
-            B.type[P.childL[p]] = BN_DEAD;
-            B.type[P.childL[p] + 1] = BN_DEAD;
+        if (lane == 0) s_need[wave] = need;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            ChildNeed t{};
+            for (uint32_t i = 0; i < kChildNodes; ++i) {
+                const ChildNeed c = s_need[i];
+                s_need[i] = t;
+                t.bn += c.bn;
+                t.na += c.na;
+                t.nw += c.nw;
+                t.nsmall += c.nsmall;
+                t.nse += c.nse;
+                t.ll += c.ll;
+            }
+            unsigned long long* next = (unsigned long long*)&L.W[W_LEVELS + 4 * (L.level + 1)];
+            unsigned long long* small = (unsigned long long*)&L.W[W_NSE];
+            ChildNeed b{};
+            if (t.bn) b.bn = atomicAdd(&L.W[W_NBN], t.bn);
+            if (t.ll) b.ll = atomicAdd(&L.W[W_LL], t.ll);
+            if (t.na) {
+                const unsigned long long o = atomicAdd(next, (unsigned long long)t.na << 32 | t.nw);
+                b.nw = (uint32_t)o;
+                b.na = (uint32_t)(o >> 32);
+            }
+            if (t.nsmall) {
+                const unsigned long long o = atomicAdd(small, (unsigned long long)t.nsmall << 32 | t.nse);
+                b.nse = (uint32_t)o;
+                b.nsmall = (uint32_t)(o >> 32);
+            }
+            if ((uint64_t)b.bn + t.bn > L.cap.bn || (uint64_t)b.ll + t.ll > L.cap.ll ||
+                (uint64_t)b.na + t.na > L.cap.na || (uint64_t)b.nw + t.nw > L.cap.nw ||
+                (uint64_t)b.nsmall + t.nsmall > L.cap.small || (uint64_t)b.nse + t.nse > L.cap.se) {
+                atomicOr(&L.W[W_ERR], kErrRoom);
+                b.bn = kNone;  // nothing of these nodes is written
+            }
+            s_base = b;
         }
-        return;
-    }
-    uint32_t bn = P.childL[p] + side;
-    uint32_t level = P.level[p] + 1;
-    atomicMax(&counters[C_MAXLEVEL], level);
-    float4 lo = P.lo[p], hi = P.hi[p];
-    if (side == 0) f4set(hi, P.axis[p], P.split[p]);
-    else f4set(lo, P.axis[p], P.split[p]);
-    uint32_t type = Cv.type[c];
-    if (type == BN_SMALL) {
-        uint32_t s = small_base + Cv.sidx[c];
-        S.first[s] = small_elem_base + Cv.soff[c];
-        S.cnt[s] = Cv.cnt[c];
-        S.level[s] = level;
-        S.bn[s] = bn;
-        S.lo[s] = lo;
-        S.hi[s] = hi;
-        S.scene[s] = A.scene[p];
-        B.type[bn] = BN_SMALL;
-        B.aux[bn] = s;
-    } else {
-        uint32_t l = Cv.lidx[c];
-        Nx.lo[l] = lo;
-        Nx.hi[l] = hi;
-        Nx.first[l] = Cv.loff[c];
-        Nx.cnt[l] = Cv.cnt[c];
-        Nx.level[l] = level;
-        Nx.bn[l] = bn;
-        Nx.scene[l] = A.scene[p];
-        B.type[bn] = BN_PENDING;
-    }
-}
-
-// Elements of large-stage leaves (level cap, no progress) are copied out before the
-// level's element arrays are released.
-__device__ __forceinline__ void leaf_copy_one(uint32_t p, const NodeView& A, const PlanView& P, const ElemView& E,
-                                              uint32_t* __restrict__ ll_idx, uint32_t ll_cap, const BnView& B,
-                                              uint32_t* __restrict__ counters) {
-    if (!(P.leaf[p] || P.noprog[p])) return;
-    uint32_t m = A.cnt[p], f = A.first[p];
-    uint32_t start = atomicAdd(&counters[C_LLCOUNT], m);
-    if ((uint64_t)start + m > ll_cap) {
-        atomicOr(&counters[C_ERR], 32u);
-        return;
-    }
-    for (uint32_t i = 0; i < m; ++i) ll_idx[start + i] = E.idx[f + i];
-    uint32_t cur = P.cur[p];
-    B.aux[cur] = start;
-    B.cnt[cur] = m;
-}
-
-// The level's children (2 per node), and with the first n threads the copy of large-stage
-// leaves' elements.
-__global__ __launch_bounds__(256) void k_child_write(DN dn_, NodeView A, PlanView P, ChildView Cv, DN small_base,
-                                                     DN small_elem_base, SmallView S, NodeView Nx, BnView B,
-                                                     uint32_t* __restrict__ counters, ElemView E,
-                                                     uint32_t* __restrict__ ll_idx, uint32_t ll_cap) {
-    const uint32_t n = dn_.get(), sb = small_base.get(), seb = small_elem_base.get();
-    MNRT_GRID_STRIDE(c, 2 * n) {
-        child_write_one(c, n, A, P, Cv, sb, seb, S, Nx, B, counters);
-        if (c < n) leaf_copy_one(c, A, P, E, ll_idx, ll_cap, B, counters);
+        __syncthreads();
+        const ChildNeed base = s_base, own = s_need[wave];
+        __syncthreads();  // s_need is rewritten by the next step
+        if (!live || lane != 0u) continue;
+        const uint32_t none = base.bn == kNone ? 1u : 0u;
+        uint32_t id = base.bn + own.bn, cur = L.A.bn[p];
+        const uint32_t scene = L.A.scene[p];
+        if (none) {
+            L.P.child[2 * p] = L.P.child[2 * p + 1] = make_uint4(CH_DEAD, 0u, 0u, 0u);
+            continue;
+        }
+        auto node = [&](uint32_t i, uint32_t t, uint32_t level, uint32_t parent) {
+            L.B.type[i] = t;
+            L.B.level[i] = level;
+            L.B.scene[i] = scene;
+            L.B.parent[i] = parent;
+            L.B.flag[i] = 0u;
+        };
+        auto inner = [&](uint32_t i, uint32_t axis, float s, uint32_t l, uint32_t r) {
+            L.B.type[i] = axis;
+            L.B.split[i] = __float_as_uint(s);
+            L.B.left[i] = l;
+            L.B.right[i] = r;
+        };
+        (void)plan_node(L.A, p, L.ratio, [&](int ax, bool is_max, float s, uint32_t level, uint32_t) {
+            const uint32_t empty = id++, cont = id++;
+            inner(cur, (uint32_t)ax, s, is_max ? cont : empty, is_max ? empty : cont);
+            node(empty, BN_LEAF, level + 1, cur);
+            L.B.cnt[empty] = 0u;
+            L.B.aux[empty] = 0u;
+            node(cont, BN_PENDING, level + 1, cur);
+            cur = cont;
+        });
+        L.P.lo[p] = make_float4(R.lo[0], R.lo[1], R.lo[2], 0.0f);
+        L.P.hi[p] = make_float4(R.hi[0], R.hi[1], R.hi[2], 0.0f);
+        L.P.axis[p] = R.axis;
+        L.P.split[p] = R.split;
+        if (type[0] == CH_LEAF) {
+            const uint32_t at = base.ll + own.ll;
+            L.B.type[cur] = BN_LEAF;
+            L.B.cnt[cur] = m;
+            L.B.aux[cur] = at;
+            L.P.child[2 * p] = make_uint4(CH_LEAF, at, 0u, 0u);
+            L.P.child[2 * p + 1] = make_uint4(CH_DEAD, 0u, 0u, 0u);
+            continue;
+        }
+        inner(cur, R.axis, R.split, id, id + 1u);
+        uint32_t l = base.na + own.na, wv = base.nw + own.nw, s = base.nsmall + own.nsmall, se = base.nse + own.nse;
+#pragma unroll
+        for (uint32_t side = 0; side < 2; ++side) {
+            float4 lo = make_float4(R.lo[0], R.lo[1], R.lo[2], 0.0f), hi = make_float4(R.hi[0], R.hi[1], R.hi[2], 0.0f);
+            if (side == 0) f4set(hi, R.axis, R.split);
+            else f4set(lo, R.axis, R.split);
+            const uint32_t bn = id + side;
+            if (type[side] == CH_SMALL) {
+                L.S.first[s] = se;
+                L.S.cnt[s] = n[side];
+                L.S.level[s] = R.level + 1;
+                L.S.bn[s] = bn;
+                L.S.lo[s] = lo;
+                L.S.hi[s] = hi;
+                L.S.scene[s] = scene;
+                node(bn, BN_SMALL, R.level + 1, cur);
+                L.B.aux[bn] = s;
+                L.P.child[2 * p + side] = make_uint4(CH_SMALL, se, 0u, 0u);
+                ++s;
+                se += n[side];
+            } else {
+                L.An.lo[l] = lo;
+                L.An.hi[l] = hi;
+                L.An.first[l] = 64u * wv;
+                L.An.cnt[l] = n[side];
+                L.An.level[l] = R.level + 1;
+                L.An.bn[l] = bn;
+                L.An.scene[l] = scene;
+                for (int k = 0; k < 6; ++k) L.An.tb[6 * l + k] = 0xFFFFFFFFu;
+                node(bn, BN_PENDING, R.level + 1, cur);
+                L.P.child[2 * p + side] = make_uint4(CH_LARGE, 64u * wv, l, 0u);
+                ++l;
+                wv += (n[side] + 63u) >> 6;
+            }
+        }
     }
 }
 
 // Scatter each element into its children: small roots append to the small-element
-// buffer, large children to the next level's arrays.  A straddling triangle's bounds in a
-// child are its clip to the child box (kernel_PerformSplitClipping, kdtree_tri.cu:389-489),
-// which k_clip computes: each straddling element side has a slot in the clip queue from
-// the classification scan (pos[2 ne + side ne + e] - pos[2 ne]), where this writes the
-// side's job (e << 1 | side), or kNone when the side is not scattered, so that the clips
-// run 64 to a wave rather than one pass of a whole wave per straddler.
-__device__ __forceinline__ void scatter_one(uint32_t e, uint32_t n, uint32_t ne, const ElemView& E,
-                                            const Geometry& G, const NodeView& A, const PlanView& P,
-                                            const ChildView& Cv, const uint32_t* __restrict__ pos,
-                                            uint32_t small_elem_base, const ElemView& Sm, uint32_t sm_cap,
-                                            const ElemView& Nx, uint32_t nx_cap, uint32_t* __restrict__ counters,
-                                            uint32_t* __restrict__ clipq) {
-    const uint32_t p = E.node[e];
-    if (P.leaf[p]) return;  // no flags: k_classify skips leaves
-    const uint32_t idx = E.idx[e];
-    const float4 lo = E.lo[e];
-    const float4 hi = (G.kind == MNRT_KIND_TRI) ? E.hi[e] : lo;
-    const uint32_t axis = P.axis[p];
-    const float s = P.split[p];
-    bool L, R;
-    classify(G.kind, idx, lo, hi, axis, s, L, R);
-    const bool straddle = (G.kind == MNRT_KIND_TRI) && (f4c(lo, axis) < s && s < f4c(hi, axis));
-    const bool noprog = P.noprog[p] != 0u;  // its elements were copied out by k_child_write
-    for (uint32_t side = 0; side < 2; ++side) {
-        if (!(side ? R : L)) continue;
-        bool queued = false;
-        const uint32_t c = side * n + p;
-        const uint32_t type = noprog ? (uint32_t)BN_DEAD : Cv.type[c];
-        if (type != BN_DEAD) {
-            const uint32_t rank = pos[side * ne + e] - Cv.fpos[c];
-            if (type == BN_SMALL) {
-                const uint32_t d = small_elem_base + Cv.soff[c] + rank;
-                if (d >= sm_cap) {
-                    atomicOr(&counters[C_ERR], 1u);
-                } else {
-                    Sm.idx[d] = idx;
-                    if (!straddle) {
-                        Sm.lo[d] = lo;
-                        if (G.kind == MNRT_KIND_TRI) Sm.hi[d] = hi;
-                    }
-                    queued = straddle;
+// buffer, large children to the next level's arrays, whose tight bounds (kernel_GenChunkAABB and
+// two segmented reductions, kdtree.cu:310-445) are accumulated on the way: per wave, then per
+// run of waves of one node in the workgroup, one atomic per component and run.  A straddling
+// triangle's bounds in a child are its clip to the child box (kernel_PerformSplitClipping,
+// kdtree_tri.cu:389-489), which k_clip computes from the queue written here, 64 to a wave
+// rather than one pass of a whole wave per straddler.
+constexpr uint32_t kScatterBlock = 1024, kScatterWaves = kScatterBlock / 64;
+
+template <int kKind>
+__global__ __launch_bounds__(kScatterBlock) void k_scatter(LevelArgs L) {
+    __shared__ uint32_t s_tb[kScatterWaves][12];
+    __shared__ uint32_t s_node[kScatterWaves];
+    __shared__ uint32_t s_to[kScatterWaves][2];  // next-level nodes of the wave's children, or kNone
+    __shared__ uint32_t s_q[kScatterWaves + 1];
+    const uint32_t nw = level_waves(L), lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
+    for (uint32_t w0 = blockIdx.x * kScatterWaves; w0 < nw; w0 += gridDim.x * kScatterWaves) {  // uniform per workgroup
+        const uint32_t w = w0 + wave, e = 64u * w + lane;
+        uint32_t p = kNone, to[2] = {kNone, kNone};
+        uint32_t tb[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) tb[k] = ~0u;
+        uint64_t mq[2] = {0ull, 0ull};
+        uint32_t dst[2] = {0u, 0u};
+        if (w < nw) {
+            p = uniform(L.E.wnode[w]);
+            const uint4 c0 = L.P.child[2 * p], c1 = L.P.child[2 * p + 1];
+            const uint32_t type[2] = {uniform(c0.x), uniform(c1.x)}, at[2] = {uniform(c0.y), uniform(c1.y)};
+            const uint32_t local = e - L.A.first[p];
+            const bool in = local < L.A.cnt[p];
+            const uint32_t idx = in ? L.E.idx[e] : 0u;
+            if (type[0] == CH_LEAF) {
+                if (in) L.ll_idx[at[0] + local] = idx;
+            } else if (type[0] != CH_DEAD) {
+                bool go[2] = {false, false};
+                bool straddle = false;
+                float4 lo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), hi = lo;
+                if (in) {
+                    const uint32_t axis = L.P.axis[p];
+                    const float s = L.P.split[p];
+                    lo = L.E.lo[e];
+                    hi = (kKind == MNRT_KIND_TRI) ? L.E.hi[e] : lo;
+                    classify(kKind, idx, lo, hi, axis, s, go[0], go[1]);
+                    straddle = (kKind == MNRT_KIND_TRI) && (f4c(lo, axis) < s && s < f4c(hi, axis));
                 }
-            } else {
-                const uint32_t d = Cv.loff[c] + rank;
-                if (d >= nx_cap) {
-                    atomicOr(&counters[C_ERR], 2u);
-                } else {
-                    Nx.idx[d] = idx;
-                    Nx.node[d] = Cv.lidx[c];
-                    if (!straddle) {
-                        Nx.lo[d] = lo;
-                        if (G.kind == MNRT_KIND_TRI) Nx.hi[d] = hi;
+                const uint2 off = L.woff[w];
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    const uint64_t m = ballot(go[side]);
+                    dst[side] = at[side] + (side ? off.y : off.x) + mask_prefix(m);
+                    mq[side] = m & ballot(straddle);
+                    const bool large = type[side] == CH_LARGE;
+                    if (go[side]) {
+                        const ElemView& D = large ? L.Nx : L.Sm;
+                        D.idx[dst[side]] = idx;
+                        if (!straddle) {
+                            D.lo[dst[side]] = lo;
+                            if (kKind == MNRT_KIND_TRI) D.hi[dst[side]] = hi;
+                        }
+                        if (large && (dst[side] & 63u) == 0u) L.Nx.wnode[dst[side] >> 6] = side ? c1.z : c0.z;
                     }
-                    queued = straddle;
+                    if (large) {
+                        to[side] = uniform(side ? c1.z : c0.z);
+                        uint32_t v[6];
+                        tight_words(lo, hi, v);
+#pragma unroll
+                        for (int k = 0; k < 6; ++k)
+                            tb[6 * side + k] = wave_min_u32(go[side] && !straddle ? v[k] : ~0u);
+                    }
                 }
             }
         }
-        if (straddle) clipq[pos[2 * ne + side * ne + e] - pos[2 * ne]] = queued ? (e << 1 | side) : kNone;
+        const uint32_t nq = (uint32_t)(__popcll(mq[0]) + __popcll(mq[1]));
+        if (lane == 0) {
+            s_node[wave] = p;
+            s_to[wave][0] = to[0];
+            s_to[wave][1] = to[1];
+            if (kKind == MNRT_KIND_TRI) s_q[wave] = nq;
+        }
+#pragma unroll
+        for (int k = 0; k < 12; ++k)
+            if (lane == (uint32_t)k) s_tb[wave][k] = tb[k];
+        __syncthreads();
+        if (threadIdx.x < 12u * kScatterWaves) {
+            const uint32_t i = threadIdx.x / 12u, k = threadIdx.x % 12u, node = s_node[i], t = s_to[i][k / 6u];
+            if (t != kNone && (i == 0u || s_node[i - 1u] != node)) {
+                uint32_t v = s_tb[i][k];
+                for (uint32_t j = i + 1u; j < kScatterWaves && s_node[j] == node; ++j) v = min(v, s_tb[j][k]);
+                if (v != ~0u) atomicMin(&L.An.tb[6u * t + k % 6u], v);
+            }
+        }
+        if (kKind == MNRT_KIND_TRI && threadIdx.x == kScatterBlock - 1u) {
+            uint32_t tot = 0;
+            for (uint32_t i = 0; i < kScatterWaves; ++i) {
+                const uint32_t c = s_q[i];
+                s_q[i] = tot;
+                tot += c;
+            }
+            const uint32_t b = tot ? atomicAdd(&L.W[W_LEVELS + 4 * L.level + 2], tot) : 0u;
+            s_q[kScatterWaves] = b;
+        }
+        __syncthreads();
+        if (kKind == MNRT_KIND_TRI && nq) {
+            uint32_t b = s_q[kScatterWaves] + s_q[wave];
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                if ((mq[side] >> lane) & 1ull)
+                    L.q[b + mask_prefix(mq[side])] = make_uint2(e << 1 | (uint32_t)side, dst[side]);
+                b += (uint32_t)__popcll(mq[side]);
+            }
+        }
+        __syncthreads();  // the LDS words are rewritten by the next step
     }
 }
 
-__global__ __launch_bounds__(256) void k_scatter(DN dn_, DN dne, ElemView E, Geometry G, NodeView A, PlanView P,
-                                                 ChildView Cv, const uint32_t* __restrict__ pos, DN small_elem_base,
-                                                 ElemView Sm, uint32_t sm_cap, ElemView Nx, uint32_t nx_cap,
-                                                 uint32_t* __restrict__ counters, uint32_t* __restrict__ clipq) {
-    const uint32_t n = dn_.get(), ne = dne.get(), seb = small_elem_base.get();
-    MNRT_GRID_STRIDE(e, ne)
-    scatter_one(e, n, ne, E, G, A, P, Cv, pos, seb, Sm, sm_cap, Nx, nx_cap, counters, clipq);
-}
-
-// The clip queue of a triangle level (k_scatter): each job clips its triangle to the
-// child box and writes the bounds next to the index k_scatter placed.  A grid-stride
-// launch: the queue holds at most 2 ne jobs, usually a small part of that.
-__global__ __launch_bounds__(kClipBlock) void k_clip(DN dn_, DN dne, ElemView E, Geometry G, NodeView A, PlanView P,
-                                                     ChildView Cv, const uint32_t* __restrict__ pos,
-                                                     DN small_elem_base, ElemView Sm, ElemView Nx,
-                                                     const uint32_t* __restrict__ clipq) {
+// The clip queue of a triangle level: each job clips its triangle to the child box, writes the
+// bounds next to the index k_scatter placed and adds them to a large child's tight bounds (lanes
+// that share a child reduce first).
+__global__ __launch_bounds__(kClipBlock) void k_clip(LevelArgs L, Geometry G) {
     __shared__ float s_lists[2 * kClipVerts * 3 * kClipBlock];
     __attribute__((address_space(3))) float* col = (__attribute__((address_space(3))) float*)(s_lists + threadIdx.x);
-    const uint32_t n = dn_.get(), ne = dne.get(), seb = small_elem_base.get();
-    const uint32_t nq = pos[4 * ne] - pos[2 * ne];
-    MNRT_GRID_STRIDE(j, nq) {
-        const uint32_t w = clipq[j];
-        if (w == kNone) continue;
-        const uint32_t e = w >> 1, side = w & 1u, p = E.node[e], axis = P.axis[p];
-        const float s = P.split[p];
-        float4 lo = E.lo[e], hi = E.hi[e];
-        float4 bmin = P.lo[p], bmax = P.hi[p];
-        if (side == 0) f4set(bmax, axis, s);
-        else f4set(bmin, axis, s);
-        clip_bounds(G, G.base[A.scene[p]] + E.idx[e], lo, hi, bmin, bmax, col);
-        const uint32_t c = side * n + p, rank = pos[side * ne + e] - Cv.fpos[c];
-        if (Cv.type[c] == BN_SMALL) {
-            const uint32_t d = seb + Cv.soff[c] + rank;
-            Sm.lo[d] = lo;
-            Sm.hi[d] = hi;
-        } else {
-            const uint32_t d = Cv.loff[c] + rank;
-            Nx.lo[d] = lo;
-            Nx.hi[d] = hi;
+    if (L.W[W_ERR] != 0u) return;
+    const uint32_t nq = L.W[W_LEVELS + 4 * L.level + 2], lane = threadIdx.x;
+    for (uint32_t j0 = blockIdx.x * kClipBlock; j0 < nq; j0 += gridDim.x * kClipBlock) {
+        const uint32_t j = j0 + lane;
+        uint32_t to = kNone;
+        uint32_t v[6] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
+        if (j < nq) {
+            const uint2 job = L.q[j];
+            const uint32_t e = job.x >> 1, side = job.x & 1u, p = L.E.wnode[e >> 6], axis = L.P.axis[p];
+            const float s = L.P.split[p];
+            float4 lo = L.E.lo[e], hi = L.E.hi[e];
+            float4 bmin = L.P.lo[p], bmax = L.P.hi[p];
+            if (side == 0) f4set(bmax, axis, s);
+            else f4set(bmin, axis, s);
+            clip_bounds(G, G.base[L.A.scene[p]] + L.E.idx[e], lo, hi, bmin, bmax, col);
+            const uint4 c = L.P.child[2 * p + side];
+            const ElemView& D = c.x == CH_LARGE ? L.Nx : L.Sm;
+            D.lo[job.y] = lo;
+            D.hi[job.y] = hi;
+            if (c.x == CH_LARGE) {
+                to = c.z;
+                tight_words(lo, hi, v);
+            }
         }
+        tight_by_key(to, v, L.An.tb, lane);
     }
-}
-
-// Workgroups of k_clip (kClipBlock lanes) for a level of up to ne elements.
-inline dim3 clip_blocks(uint64_t ne) {
-    return dim3((uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((2 * ne + kClipBlock - 1) / kClipBlock, 4096)));
 }
 
 // ---- small-node stage: one wave64 per small root ----------------------------------------
@@ -873,6 +916,8 @@ struct SmallStackEnt {
 struct StageCap {
     uint32_t mul, add;
     __host__ __device__ uint32_t of(uint32_t n) const { return mul * n + add; }
+    // first slot of root r, whose elements start at `first` (both grow together over the roots)
+    __device__ uint32_t begin(uint32_t r, uint32_t first) const { return mul * first + add * r; }
 };
 
 enum : int { kSmallStage = 0, kSmallEmit = 1 };
@@ -881,7 +926,6 @@ struct SmallOut {
     uint32_t* nsize;  // stage: nodes per small subtree
     uint32_t* rsize;  // stage: references per small subtree
     uint32_t* mlvl;   // stage: deepest level in the small subtree
-    const uint32_t* st_off;  // stage: first slot of each small root's staging area
     uint2* st_nodes;         // stage: node words, subtree-local addresses
     uint32_t* st_refs;       // stage: references, subtree-local
     uint32_t* st_ovf;        // stage: 1 where the subtree did not fit; emit: only these
@@ -890,7 +934,7 @@ struct SmallOut {
     const uint32_t* bn_rbase;
     uint32_t* nodes;
     uint32_t* refs;
-    uint32_t* counters;
+    uint32_t* W;
     uint32_t max_nodes;
     uint32_t max_refs;
     const uint32_t* node_base;  // per scene: first node / reference of its tree
@@ -923,9 +967,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const uint32_t r = blockIdx.x * kSmallWaves + wave;
-    if (r >= dnsmall.get()) return;  // uniform per wave
+    if (r >= dnsmall.get() || O.W[W_ERR] != 0u) return;  // uniform per wave
     if (kMode == kSmallEmit && O.st_ovf && O.st_ovf[r] == 0u) return;
-    if (kMode == kSmallEmit && O.counters[C_ERR] != 0u) return;  // failed build: nothing is emitted
     SmallStackEnt* stack = s_stack[wave];
 
     const uint32_t first = S.first[r], n = S.cnt[r];
@@ -1022,7 +1065,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
         addr = O.bn_addr[bn];
         rbase = O.bn_rbase[bn];
     } else if (kMode == kSmallStage) {
-        const uint32_t off = O.st_off[r];
+        const uint32_t off = O.st_cap.begin(r, first);
         nodes = (uint32_t*)(O.st_nodes + off);
         refs = O.st_refs + off;
         lim_nodes = lim_refs = O.st_cap.of(n);
@@ -1047,7 +1090,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
         wave_sync();
         if (writing && (addr >= lim_nodes || rbase > lim_refs)) {
             if (kMode == kSmallEmit) {
-                if (lane == 0) atomicOr(&O.counters[C_ERR], 4u);
+                if (lane == 0) atomicOr(&O.W[W_ERR], 4u);
                 break;
             }
             writing = false;  // staging area full: counted on, emitted later
@@ -1123,7 +1166,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
         if (best == kNone || !(best_cost < (float)cnt)) {
             if (writing && rbase + cnt > lim_refs) {
                 if (kMode == kSmallEmit) {
-                    if (lane == 0) atomicOr(&O.counters[C_ERR], 8u);
+                    if (lane == 0) atomicOr(&O.W[W_ERR], 8u);
                     break;
                 }
                 writing = false;
@@ -1190,14 +1233,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
         O.rsize[r] = rbase;
         O.mlvl[r] = maxlvl;
         O.st_ovf[r] = writing ? 0u : 1u;
-        if (!writing) atomicAdd(&O.counters[C_SMALL_OVF], 1u);
+        if (!writing) atomicAdd(&O.W[W_SMALL_OVF], 1u);
     }
-}
-
-__global__ __launch_bounds__(256) void k_small_caps(DN dnsmall, const uint32_t* __restrict__ cnt, StageCap cap,
-                                                    uint32_t* __restrict__ caps) {
-    const uint32_t nsmall = dnsmall.get();
-    MNRT_GRID_STRIDE(r, nsmall) caps[r] = cap.of(cnt[r]);
 }
 
 StageCap stage_cap_setting() {
@@ -1215,19 +1252,19 @@ StageCap stage_cap_setting() {
 __global__ __launch_bounds__(64 * kSmallWaves) void k_small_place(DN dnsmall, SmallView S, SmallOut O) {
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t r = blockIdx.x * kSmallWaves + wave;
-    if (r >= dnsmall.get() || O.st_ovf[r] != 0u || O.counters[C_ERR] != 0u) return;
+    if (r >= dnsmall.get() || O.st_ovf[r] != 0u || O.W[W_ERR] != 0u) return;
     const uint32_t scene = S.scene[r];
     const uint32_t bn = S.bn[r];
     const uint32_t a0 = O.bn_addr[bn], r0 = O.bn_rbase[bn];
     const uint32_t nn = O.nsize[r], nr = O.rsize[r];
     const uint32_t lim_nodes = O.max_nodes - O.node_base[scene], lim_refs = O.max_refs - O.ref_base[scene];
     if (a0 + nn > lim_nodes || r0 + nr > lim_refs) {
-        if (lane == 0) atomicOr(&O.counters[C_ERR], 4u);
+        if (lane == 0) atomicOr(&O.W[W_ERR], 4u);
         return;
     }
     uint2* nodes = (uint2*)(O.nodes + 2ull * O.node_base[scene]) + a0;
     uint32_t* refs = O.refs + O.ref_base[scene] + r0;
-    const uint32_t off = O.st_off[r];
+    const uint32_t off = O.st_cap.begin(r, S.first[r]);
     for (uint32_t j = lane; j < nn; j += 64) {
         uint2 w = O.st_nodes[off + j];
         const uint32_t tag = w.y >> 30;
@@ -1237,155 +1274,154 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small_place(DN dnsmall, Sm
     for (uint32_t j = lane; j < nr; j += 64) refs[j] = O.st_refs[off + j];
 }
 
-// ---- layout: subtree sizes bottom-up, addresses top-down, one workgroup ------------------
+// ---- layout ---------------------------------------------------------------------------
+// (KDTreeGPU::PreorderTraversal launches two kernels per level over all nodes,
+// KDTreeGPU.cpp:1156-1209.)  Subtree sizes climb from the leaves in one launch, the second child
+// to arrive at a node going on; a node's address is the sum over its ancestors, so one more
+// launch places and emits every node at once.  58 launches, one per level and direction, took
+// 0.23 ms of the 1.03M-triangle build.
 
 struct LayoutView {
     uint32_t* size;   // nodes in the subtree
     uint32_t* rsize;  // references in the subtree
     uint32_t* depth;  // deepest level in the subtree
-    uint32_t* addr;
+    uint32_t* addr;   // small roots: subtree start
     uint32_t* rbase;
 };
 
-// Build nodes bucketed by level (the order inside a level does not matter).  Counts go
-// through a per-workgroup LDS histogram, so each workgroup adds to a level's global
-// counter once.
-// top: the deepest level the layout launches cover; a node below it sets err_bit in *err.
-__global__ __launch_bounds__(256) void k_level_hist(DN dnbn, BnView B, uint32_t* __restrict__ hist, uint32_t top,
-                                                    uint32_t* __restrict__ err, uint32_t err_bit) {
-    __shared__ uint32_t s_hist[64];
-    if (threadIdx.x < 64) s_hist[threadIdx.x] = 0u;
-    __syncthreads();
-    const uint32_t nbn = dnbn.get();
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nbn && B.type[i] < BN_PENDING) {
-        const uint32_t lvl = B.level[i] & 63u;
-        if (lvl > top) atomicOr(err, err_bit);
-        atomicAdd(&s_hist[lvl], 1u);
-    }
-    __syncthreads();
-    if (threadIdx.x < 64 && s_hist[threadIdx.x] != 0u) atomicAdd(&hist[threadIdx.x], s_hist[threadIdx.x]);
+// The climbing waves exchange sizes across dies within the launch: through atomics of device
+// scope only, each value stored and waited for before its node's arrival is counted.
+__device__ __forceinline__ void put_dev(uint32_t* p, uint32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t get_dev(const uint32_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(256) void k_level_scatter(DN dnbn, BnView B, uint32_t* __restrict__ cursor,
-                                                       uint32_t* __restrict__ list) {
-    __shared__ uint32_t s_cnt[64];
-    __shared__ uint32_t s_base[64];
-    if (threadIdx.x < 64) s_cnt[threadIdx.x] = 0u;
-    __syncthreads();
+// top: the deepest level the build may reach; a leaf below it sets kErrLayoutDepth.
+__global__ __launch_bounds__(256) void k_layout_sizes(DN dnbn, BnView B, LayoutView Lv, const uint32_t* __restrict__ s_nsize,
+                                                      const uint32_t* __restrict__ s_rsize,
+                                                      const uint32_t* __restrict__ s_mlvl, uint32_t top,
+                                                      uint32_t* __restrict__ W) {
+    if (W[W_ERR] != 0u) return;
     const uint32_t nbn = dnbn.get();
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = i < nbn && B.type[i] < BN_PENDING;
-    const uint32_t lvl = live ? (B.level[i] & 63u) : 0u;
-    const uint32_t local = live ? atomicAdd(&s_cnt[lvl], 1u) : 0u;
-    __syncthreads();
-    if (threadIdx.x < 64 && s_cnt[threadIdx.x] != 0u)
-        s_base[threadIdx.x] = atomicAdd(&cursor[threadIdx.x], s_cnt[threadIdx.x]);
-    __syncthreads();
-    if (live) list[s_base[lvl] + local] = i;
-}
-
-// Subtree sizes bottom-up, then preorder addresses top-down, one launch per level over the
-// level's bucket (KDTreeGPU::PreorderTraversal launches two kernels per level over all
-// nodes, KDTreeGPU.cpp:1156-1209; here only the level's nodes are touched).
-struct LayoutSrc {
-    const uint32_t* off;   // level bucket offsets (65)
-    const uint32_t* list;  // build nodes by level
-    const uint32_t* s_nsize;
-    const uint32_t* s_rsize;
-    const uint32_t* s_mlvl;
-};
-
-__global__ __launch_bounds__(256) void k_layout_up(uint32_t lvl, LayoutSrc Ls, BnView B, LayoutView Lv) {
-    const uint32_t end = Ls.off[lvl + 1];
-    for (uint32_t j = Ls.off[lvl] + blockIdx.x * blockDim.x + threadIdx.x; j < end; j += gridDim.x * blockDim.x) {
-        const uint32_t i = Ls.list[j];
-        const uint32_t t = B.type[i];
-        if (t <= 2) {
-            const uint32_t l = B.left[i], r = B.right[i];
-            Lv.size[i] = 1 + Lv.size[l] + Lv.size[r];
-            Lv.rsize[i] = Lv.rsize[l] + Lv.rsize[r];
-            Lv.depth[i] = max(Lv.depth[l], Lv.depth[r]);
-        } else if (t == BN_LEAF) {
-            Lv.size[i] = 1;
-            Lv.rsize[i] = B.cnt[i];
-            Lv.depth[i] = B.level[i];
-        } else if (t == BN_SMALL) {
-            const uint32_t x = B.aux[i];
-            Lv.size[i] = Ls.s_nsize[x];
-            Lv.rsize[i] = Ls.s_rsize[x];
-            Lv.depth[i] = Ls.s_mlvl[x];
+    uint32_t deepest = 0;
+    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nbn; j += gridDim.x * blockDim.x) {
+        const uint32_t t = B.type[j];
+        if (t != BN_LEAF && t != BN_SMALL) continue;
+        const uint32_t x = B.aux[j];
+        uint32_t i = j, size = 1u, rsize, depth = B.level[j];
+        deepest = max(deepest, depth);
+        if (t == BN_SMALL) {
+            size = s_nsize[x];
+            rsize = s_rsize[x];
+            depth = s_mlvl[x];
+        } else {
+            rsize = B.cnt[j];
+        }
+        for (;;) {
+            put_dev(&Lv.size[i], size);
+            put_dev(&Lv.rsize[i], rsize);
+            put_dev(&Lv.depth[i], depth);
+            const uint32_t p = B.parent[i];
+            if (p == kNone) break;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (__hip_atomic_fetch_add(&B.flag[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) break;
+            asm volatile("" ::: "memory");
+            const uint32_t l = B.left[p], o = l == i ? B.right[p] : l;
+            size += 1u + get_dev(&Lv.size[o]);
+            rsize += get_dev(&Lv.rsize[o]);
+            depth = max(depth, get_dev(&Lv.depth[o]));
+            i = p;
         }
     }
-}
-
-// Level lvl's nodes place their children; every scene's root (level 0) starts its own
-// tree at address 0.
-__global__ __launch_bounds__(256) void k_layout_down(uint32_t lvl, LayoutSrc Ls, BnView B, LayoutView Lv) {
-    const uint32_t end = Ls.off[lvl + 1];
-    for (uint32_t j = Ls.off[lvl] + blockIdx.x * blockDim.x + threadIdx.x; j < end; j += gridDim.x * blockDim.x) {
-        const uint32_t i = Ls.list[j];
-        if (lvl == 0) {
-            Lv.addr[i] = 0;
-            Lv.rbase[i] = 0;
-        }
-        if (B.type[i] > 2) continue;
-        const uint32_t l = B.left[i], r = B.right[i];
-        const uint32_t a = Lv.addr[i], rb = Lv.rbase[i];
-        Lv.addr[l] = a + 1;
-        Lv.rbase[l] = rb;
-        Lv.addr[r] = a + 1 + Lv.size[l];
-        Lv.rbase[r] = rb + Lv.rsize[l];
+    deepest = wave_max_u32(deepest);
+    if ((threadIdx.x & 63u) == 0u && deepest != 0u) {
+        atomicMax(&W[W_MAXLEVEL], deepest);
+        if (deepest > top) atomicOr(&W[W_ERR], kErrLayoutDepth);
     }
 }
 
-__global__ __launch_bounds__(256) void k_emit_large(DN dnbn, BnView B, LayoutView Lv, const uint32_t* __restrict__ ll_idx,
+// Per scene (root = build node s): nodes, references, leaves and max level, and the trees' places
+// in the shared arrays.  Every inner node has two children, so leaves = (nodes + 1) / 2.
+// max_nodes / max_refs: room of the output arrays.
+__global__ __launch_bounds__(1024) void k_scene_totals(uint32_t nscenes, LayoutView Lv, uint32_t* __restrict__ nodes,
+                                                       uint32_t* __restrict__ refs, uint32_t* __restrict__ nbase,
+                                                       uint32_t* __restrict__ rbase, uint32_t* __restrict__ leaves,
+                                                       uint32_t* __restrict__ maxlvl, uint32_t max_nodes,
+                                                       uint32_t max_refs, uint32_t* __restrict__ W) {
+    __shared__ uint64_t s_wave[16];
+    if (W[W_ERR] != 0u) return;  // (uniform: no thread of this launch has set it yet)
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    uint64_t n0 = 0, r0 = 0;
+    for (uint32_t b = 0; b < nscenes; b += 1024u) {
+        const uint32_t s = b + tid;
+        const uint32_t n = s < nscenes ? Lv.size[s] : 0u, r = s < nscenes ? Lv.rsize[s] : 0u;
+        const uint32_t ni = wave_incl_scan(n, lane), ri = wave_incl_scan(r, lane);
+        if (lane == 63u) s_wave[wave] = (uint64_t)ni << 32 | ri;
+        __syncthreads();
+        uint64_t nb = n0, rb = r0;
+        for (uint32_t i = 0; i < 16u; ++i) {
+            if (i < wave) {
+                nb += s_wave[i] >> 32;
+                rb += (uint32_t)s_wave[i];
+            }
+            n0 += s_wave[i] >> 32;
+            r0 += (uint32_t)s_wave[i];
+        }
+        if (s < nscenes) {
+            nodes[s] = n;
+            refs[s] = r;
+            nbase[s] = (uint32_t)(nb + ni - n);
+            rbase[s] = (uint32_t)(rb + ri - r);
+            leaves[s] = (n + 1u) / 2u;
+            maxlvl[s] = Lv.depth[s];
+        }
+        __syncthreads();  // s_wave is rewritten by the next step
+    }
+    if (tid == 0) {
+        nbase[nscenes] = (uint32_t)n0;
+        rbase[nscenes] = (uint32_t)r0;
+        if (n0 == 0u || n0 > max_nodes || r0 > max_refs) atomicOr(&W[W_ERR], kErrOutputRoom);
+    }
+}
+
+// Places every build node and writes the large stage's inner nodes and leaves.
+__global__ __launch_bounds__(256) void k_emit_large(DN dnbn, BnView B, LayoutView Lv,
+                                                    const uint32_t* __restrict__ ll_idx,
                                                     uint32_t* __restrict__ nodes_all, uint32_t* __restrict__ refs_all,
-                                                    uint32_t* __restrict__ counters, uint32_t max_nodes_all,
-                                                    uint32_t max_refs_all, const uint32_t* __restrict__ node_base,
+                                                    const uint32_t* __restrict__ W,
+                                                    const uint32_t* __restrict__ node_base,
                                                     const uint32_t* __restrict__ ref_base) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= dnbn.get() || counters[C_ERR] != 0u) return;  // failed build: nothing is emitted
-    uint32_t t = B.type[i];
-    if (t > BN_LEAF) return;
-    const uint32_t sc = B.scene[i];
-    uint32_t* nodes = nodes_all + 2ull * node_base[sc];
-    uint32_t* refs = refs_all + ref_base[sc];
-    const uint32_t max_nodes = max_nodes_all - node_base[sc], max_refs = max_refs_all - ref_base[sc];
-    if (t <= BN_LEAF && (Lv.addr[i] >= max_nodes || (t == BN_LEAF && Lv.rbase[i] + B.cnt[i] > max_refs) ||
-                         (t <= 2 && Lv.addr[B.right[i]] >= max_nodes))) {
-        atomicOr(&counters[C_ERR], 16u);
-        return;
+    if (W[W_ERR] != 0u) return;  // failed build: nothing is emitted
+    const uint32_t nbn = dnbn.get();
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nbn; i += gridDim.x * blockDim.x) {
+        const uint32_t t = B.type[i];
+        uint32_t a = 0, rb = 0;
+        for (uint32_t c = i, p = B.parent[i]; p != kNone; c = p, p = B.parent[p]) {
+            const uint32_t l = B.left[p];
+            a += 1u;
+            if (l != c) {
+                a += Lv.size[l];
+                rb += Lv.rsize[l];
+            }
+        }
+        if (t == BN_SMALL) {
+            Lv.addr[i] = a;
+            Lv.rbase[i] = rb;
+            continue;
+        }
+        const uint32_t sc = B.scene[i];
+        uint2* nodes = (uint2*)nodes_all + node_base[sc];
+        if (t == BN_LEAF) {
+            const uint32_t m = B.cnt[i], from = B.aux[i];
+            uint32_t* refs = refs_all + ref_base[sc];
+            nodes[a] = make_uint2(m, (MNRT_LEAF_TAG << 30) | rb);
+            for (uint32_t k = 0; k < m; ++k) refs[rb + k] = ll_idx[from + k];
+        } else {
+            nodes[a] = make_uint2(B.split[i], (t << 30) | (a + 1u + Lv.size[B.left[i]]));
+        }
     }
-    if (t <= 2) {
-        uint32_t a = Lv.addr[i];
-        nodes[2 * a] = B.split[i];
-        nodes[2 * a + 1] = (t << 30) | Lv.addr[B.right[i]];
-    } else if (t == BN_LEAF) {
-        uint32_t a = Lv.addr[i], rb = Lv.rbase[i], m = B.cnt[i];
-        nodes[2 * a] = m;
-        nodes[2 * a + 1] = (MNRT_LEAF_TAG << 30) | rb;
-        for (uint32_t k = 0; k < m; ++k) refs[rb + k] = ll_idx[B.aux[i] + k];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_scene_counts(uint32_t nscenes, const uint32_t* __restrict__ base,
-                                                      uint32_t* __restrict__ cnt) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < nscenes) cnt[s] = base[s + 1] - base[s];
-}
-
-// Per scene (root = build node s): nodes, references, leaves and max level.  Every inner
-// node has two children, so leaves = (nodes + 1) / 2.
-__global__ __launch_bounds__(256) void k_scene_sizes(uint32_t nscenes, LayoutView Lv, uint32_t* __restrict__ nodes,
-                                                     uint32_t* __restrict__ refs, uint32_t* __restrict__ leaves,
-                                                     uint32_t* __restrict__ maxlvl) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nscenes) return;
-    nodes[s] = Lv.size[s];
-    refs[s] = Lv.rsize[s];
-    leaves[s] = (Lv.size[s] + 1) / 2;
-    maxlvl[s] = Lv.depth[s];
 }
 
 }  // namespace mnrt
@@ -1420,10 +1456,10 @@ class Pool {
         // nothing may still use the workspace when the next build on this thread reuses it
         (void)hipStreamSynchronize(st_);
         for (void* p : ptrs_) (void)pool_free(p, st_);
-        if (arena_ && total_ > arena_->cap) {
+        if (arena_ && peak_ > arena_->cap) {
             (void)hipStreamSynchronize(st_);
             void* nb = nullptr;
-            const size_t ncap = total_ + total_ / 4 + (size_t(64) << 20);
+            const size_t ncap = peak_ + peak_ / 4 + (size_t(64) << 20);
             if (hipMalloc(&nb, ncap) == hipSuccess) {
                 if (arena_->base) (void)hipFree(arena_->base);
                 arena_->base = (char*)nb;
@@ -1432,9 +1468,10 @@ class Pool {
         }
     }
     template <typename T>
-    T* get(size_t count) {
+    T* get(uint64_t count) {
         const size_t bytes = (std::max<size_t>(count * sizeof(T), 16) + 255) & ~size_t(255);
         total_ += bytes;
+        peak_ = std::max(peak_, total_);
         if (arena_ && top_ + bytes <= arena_->cap) {
             void* p = arena_->base + top_;
             top_ += bytes;
@@ -1448,15 +1485,17 @@ class Pool {
         ptrs_.push_back(p);
         return (T*)p;
     }
-    // Returns a buffer early: pool buffers go back to the pool, workspace space stays
-    // carved until the build ends.
-    void release(void* p) {
-        if (!p) return;
-        auto it = std::find(ptrs_.begin(), ptrs_.end(), p);
-        if (it != ptrs_.end()) {
-            (void)pool_free(p, st_);
-            ptrs_.erase(it);
-        }
+    // Takes back every buffer handed out since mark() (work enqueued on the stream before may
+    // still use them: buffers handed out next are used on the same stream).
+    struct Mark {
+        size_t top, total, ptrs;
+    };
+    Mark mark() const { return Mark{top_, total_, ptrs_.size()}; }
+    void rewind(const Mark& m) {
+        for (size_t i = m.ptrs; i < ptrs_.size(); ++i) (void)pool_free(ptrs_[i], st_);
+        ptrs_.resize(m.ptrs);
+        top_ = m.top;
+        total_ = m.total;
     }
     bool ok = true;
 
@@ -1464,663 +1503,16 @@ class Pool {
     hipStream_t st_;
     Arena* arena_ = nullptr;
     size_t top_ = 0;
-    size_t total_ = 0;
+    size_t total_ = 0, peak_ = 0;
     std::vector<void*> ptrs_;
 };
-
-inline dim3 blocks_for(uint64_t n, uint32_t bs = 256) { return dim3((uint32_t)std::max<uint64_t>(1, (n + bs - 1) / bs)); }
-
-// Sizes a host-driven build met, from which a recorded device-driven build sizes its
-// fixed buffers: per level the active nodes / elements, and the largest value of each
-// quantity the level loop grows a buffer for (the same bounds the loop checks).
-struct BuildStats {
-    uint32_t na0 = 0, ne0 = 0, nsmall0 = 0, nse0 = 0;
-    std::vector<uint32_t> level_na, level_ne;
-    uint64_t max_2na = 0, max_ne = 0, max_bn = 0, max_small = 0, max_se = 0, max_ll = 0;
-    uint32_t nbn = 0, nsmall = 0, nse = 0, maxlvl = 0, total_nodes = 0, total_refs = 0;
-};
-
-// Builds the trees of S scenes together: one level loop over the active nodes of all
-// scenes, one small-node launch for all small roots, one layout / emission pass.  Each
-// scene's tree equals the tree a single-scene build of it gives (indices are
-// scene-local, all decisions are per node).
-//   h_base: S + 1 element offsets into the concatenated input.
-//   h_roots: 6 floats per scene (or null: tight bounds).  h_qr: VVH radius per scene
-//   (or null: params->max_query_radius).
-//   out[s] views into shared arrays; out[0] owns them (mnrt_tree_release(&out[0])
-//   frees every tree of the batch).
-int build_batch_impl(int kind, const float* d_v0, const float* d_v1, const float* d_v2, const uint32_t* h_base,
-                     uint32_t nscenes, const mnrt_build_params* prm, const float* h_roots, const float* h_qr,
-                     mnrt_tree* out, hipStream_t st, BuildStats* stats = nullptr) {
-    if (!out || !prm || !h_base || nscenes == 0) return MNRT_ERR_ARG;
-    const uint32_t ntot = h_base[nscenes];
-    for (uint32_t s = 0; s < nscenes; ++s)
-        if (h_base[s + 1] < h_base[s]) return MNRT_ERR_ARG;
-    if (ntot > 0 && !d_v0) return MNRT_ERR_ARG;
-    if (kind == MNRT_KIND_TRI && ntot > 0 && (!d_v1 || !d_v2)) return MNRT_ERR_ARG;
-    if (prm->small_node_max < 1 || prm->small_node_max > 64) return MNRT_ERR_ARG;
-    if (ntot > (MNRT_INDEX_MASK >> 2)) return MNRT_ERR_CAPACITY;
-    const uint32_t S_ = nscenes;
-    Pool pool(st);
-    uint32_t* counters = pool.get<uint32_t>(C_COUNT);
-    // per-scene device tables: base (S+1), plan kind/index/off (3S), qr (S), roots given (6S),
-    // root boxes out (6S), node/ref counts + bases (4S + 2), leaves / max level (2S)
-    uint32_t* d_tab = pool.get<uint32_t>(32ull * S_ + 64);
-    if (!pool.ok) return MNRT_ERR_NOMEM;
-    uint32_t* d_base = d_tab;
-    uint32_t* d_pkind = d_base + S_ + 1;
-    uint32_t* d_pindex = d_pkind + S_;
-    uint32_t* d_poff = d_pindex + S_;
-    float* d_qr = (float*)(d_poff + S_);
-    float* d_given = d_qr + S_;
-    float* d_rootbox = d_given + 6 * S_;
-    uint32_t* d_snodes = (uint32_t*)(d_rootbox + 6 * S_);
-    uint32_t* d_srefs = d_snodes + S_;
-    uint32_t* d_nbase = d_srefs + S_;      // S + 1 (total at [S])
-    uint32_t* d_rbase = d_nbase + S_ + 1;  // S + 1
-    uint32_t* d_sleaves = d_rbase + S_ + 1;
-    uint32_t* d_smaxlvl = d_sleaves + S_;
-
-    // host staging in pinned memory: counters, the per-scene tables
-    const size_t hwords = 64 + 32ull * S_;
-    uint32_t* h_pin = (uint32_t*)host_staging(0, hwords * 4);
-    if (!h_pin) return MNRT_ERR_NOMEM;
-    uint32_t* h_counters = h_pin;
-    uint32_t* h_tab = h_pin + 64;
-    // RootPlan on the host: large scenes become active roots, small ones small roots
-    uint32_t na = 0, nsmall = 0, ne = 0, nse = 0;
-    {
-        uint32_t* hb = h_tab;
-        uint32_t* hk = hb + S_ + 1;
-        uint32_t* hi = hk + S_;
-        uint32_t* ho = hi + S_;
-        float* hq = (float*)(ho + S_);
-        float* hg = hq + S_;
-        for (uint32_t s = 0; s <= S_; ++s) hb[s] = h_base[s];
-        for (uint32_t s = 0; s < S_; ++s) {
-            const uint32_t cnt = h_base[s + 1] - h_base[s];
-            if (cnt > prm->small_node_max) {
-                hk[s] = 0;
-                hi[s] = na++;
-                ho[s] = ne;
-                ne += cnt;
-            } else {
-                hk[s] = 1;
-                hi[s] = nsmall++;
-                ho[s] = nse;
-                nse += cnt;
-            }
-            hq[s] = h_qr ? h_qr[s] : prm->max_query_radius;
-            for (int k = 0; k < 6; ++k) hg[6 * s + k] = h_roots ? h_roots[6 * s + k] : 0.0f;
-        }
-        MNRT_HIP_CHECK(hipMemcpyAsync(d_tab, h_tab, (size_t)(S_ + 1 + 4 * S_ + 6 * S_) * 4, hipMemcpyHostToDevice, st));
-    }
-    MNRT_HIP_CHECK(hipMemsetAsync(counters, 0, C_COUNT * sizeof(uint32_t), st));
-    MNRT_HIP_CHECK(hipMemsetAsync(d_sleaves, 0, 2ull * S_ * 4, st));
-    Geometry G{kind, (const float4*)d_v0, d_v1 ? (const float4*)d_v1 : (const float4*)d_v0,
-               d_v2 ? (const float4*)d_v2 : (const float4*)d_v0, d_base, S_};
-    RootPlan RP{d_pkind, d_pindex, d_poff};
-
-    auto sync_counters = [&]() -> int {
-        MNRT_HIP_CHECK(hipMemcpyAsync(h_counters, counters, C_COUNT * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        MNRT_HIP_CHECK(hipStreamSynchronize(st));
-        return MNRT_OK;
-    };
-    auto alloc_elems = [&](uint32_t cap, bool with_node) {
-        ElemView V{};
-        V.idx = pool.get<uint32_t>(cap);
-        V.lo = pool.get<float4>(cap);
-        V.hi = kind == MNRT_KIND_TRI ? pool.get<float4>(cap) : V.lo;
-        V.node = with_node ? pool.get<uint32_t>(cap) : nullptr;
-        return V;
-    };
-    auto release_elems = [&](ElemView& V) {
-        pool.release(V.idx);
-        pool.release(V.lo);
-        if (kind == MNRT_KIND_TRI) pool.release(V.hi);
-        pool.release(V.node);
-        V = ElemView{};
-    };
-    auto alloc_nodes = [&](uint32_t cap) {
-        NodeView V{};
-        V.lo = pool.get<float4>(cap);
-        V.hi = pool.get<float4>(cap);
-        V.first = pool.get<uint32_t>(cap);
-        V.cnt = pool.get<uint32_t>(cap);
-        V.level = pool.get<uint32_t>(cap);
-        V.bn = pool.get<uint32_t>(cap);
-        V.scene = pool.get<uint32_t>(cap);
-        return V;
-    };
-    auto release_nodes = [&](NodeView& V) {
-        pool.release(V.lo);
-        pool.release(V.hi);
-        pool.release(V.first);
-        pool.release(V.cnt);
-        pool.release(V.level);
-        pool.release(V.bn);
-        pool.release(V.scene);
-        V = NodeView{};
-    };
-    auto alloc_small = [&](uint32_t cap) {
-        SmallView V{};
-        V.first = pool.get<uint32_t>(cap);
-        V.cnt = pool.get<uint32_t>(cap);
-        V.level = pool.get<uint32_t>(cap);
-        V.bn = pool.get<uint32_t>(cap);
-        V.lo = pool.get<float4>(cap);
-        V.hi = pool.get<float4>(cap);
-        V.scene = pool.get<uint32_t>(cap);
-        return V;
-    };
-
-    // ---- input elements, per-scene tight bounds, root placement ----
-    ElemView Ein = alloc_elems(std::max<uint32_t>(ntot, 1), true);
-    if (!pool.ok) return MNRT_ERR_NOMEM;
-    if (ntot > 0) hipLaunchKernelGGL(k_init_elems, blocks_for(ntot), dim3(256), 0, st, G, ntot, Ein);
-    uint32_t* tlo = nullptr;
-    uint32_t* thi = nullptr;
-    if (!h_roots && ntot > 0) {
-        // one node per scene over the concatenated elements
-        uint32_t max_chunks = ntot / kChunk + S_;
-        uint32_t* tb = pool.get<uint32_t>(3ull * max_chunks + 8ull * S_ + scan_scratch_words(S_) + 16);
-        if (!pool.ok) return MNRT_ERR_NOMEM;
-        uint32_t *chn = tb, *chf = chn + max_chunks, *chc = chf + max_chunks, *cc = chc + max_chunks;
-        uint32_t* cnts = cc + S_;
-        tlo = cnts + S_;
-        thi = tlo + 3 * S_;
-        uint32_t* sc = thi + 3 * S_;
-        hipLaunchKernelGGL(k_scene_counts, blocks_for(S_), dim3(256), 0, st, S_, d_base, cnts);
-        hipLaunchKernelGGL(k_chunk_counts, blocks_for(S_), dim3(256), 0, st, hn(S_), cnts, cc, tlo, thi);
-        MNRT_HIP_CHECK(scan_exclusive(cc, cc, S_, counters + C_NCHUNKS, sc, st));
-        hipLaunchKernelGGL(k_chunk_fill, blocks_for(max_chunks), dim3(256), 0, st, hn(S_), max_chunks, cc, counters,
-                           d_base, cnts, chn, chf, chc);
-        hipLaunchKernelGGL(k_tight, dim3((max_chunks + kTightChunks - 1) / kTightChunks), dim3(kChunk), 0, st,
-                           max_chunks, counters, chn, chf, chc, Ein,
-                           kind, tlo, thi);
-    }
-    // growable tables
-    uint32_t bn_cap = std::max<uint32_t>(1024, S_ + 8 * (ntot / std::max<uint32_t>(1, prm->small_node_max)) + 64);
-    uint32_t* bn_buf = pool.get<uint32_t>((size_t)kBnCols * bn_cap);
-    auto bn_view = [&](uint32_t* buf, uint32_t cap) {
-        return BnView{buf,           buf + cap,           buf + 2ull * cap, buf + 3ull * cap, buf + 4ull * cap,
-                      buf + 5ull * cap, buf + 6ull * cap, buf + 7ull * cap};
-    };
-    BnView B = bn_view(bn_buf, bn_cap);
-    uint32_t nbn = S_;
-    uint32_t s_cap = std::max<uint32_t>(256, nsmall + 4 * (ntot / std::max<uint32_t>(1, prm->small_node_max)) + 16);
-    SmallView SV = alloc_small(s_cap);
-    uint32_t se_cap = std::max<uint32_t>(1024, nse + ne + ne / 2);
-    ElemView Sm = alloc_elems(se_cap, false);
-    uint32_t a_cap = std::max<uint32_t>(na, 1);
-    NodeView A = alloc_nodes(a_cap);
-    uint32_t e_cap = std::max<uint32_t>(ne, 1);
-    ElemView E = alloc_elems(e_cap, true);
-    if (!pool.ok) return MNRT_ERR_NOMEM;
-    hipLaunchKernelGGL(k_roots_setup, blocks_for(S_), dim3(256), 0, st, S_, d_base, tlo, thi,
-                       h_roots ? (const float*)d_given : (const float*)nullptr, RP, A, SV, B, d_rootbox);
-    if (ntot > 0) hipLaunchKernelGGL(k_partition_elems, blocks_for(ntot), dim3(256), 0, st, ntot, Ein, kind, RP, E, Sm);
-    MNRT_HIP_CHECK(hipGetLastError());
-    release_elems(Ein);
-    if (ne == 0) {
-        release_elems(E);
-        e_cap = 0;
-    }
-
-    uint32_t ll_cap = 0;
-    uint32_t* ll_idx = nullptr;
-    uint32_t ll_count = 0;
-    uint32_t maxlvl = 0;
-
-    // ---- large-node stage ----
-    // Workspaces grow geometrically and are reused across levels; next-level arrays are
-    // sized by the upper bound (every element / node goes to at most two children), so
-    // the host waits on the device once per level, to read the level's counters.
-    uint32_t lv_na_cap = 0, lv_ne_cap = 0;
-    void* lv_buf = nullptr;
-    uint32_t *cc = nullptr, *chn = nullptr, *chf = nullptr, *chc = nullptr, *fl = nullptr, *pos = nullptr,
-             *cbuf = nullptr, *scr = nullptr;
-    PlanView P{};
-    ElemView Nx{};
-    uint32_t nx_cap = 0;
-    NodeView An{};
-    uint32_t an_cap = 0;
-    if (stats) {
-        *stats = BuildStats{};
-        stats->na0 = na;
-        stats->ne0 = ne;
-        stats->nsmall0 = nsmall;
-        stats->nse0 = nse;
-    }
-    while (na > 0) {
-        if (stats) {
-            BuildStats& b = *stats;
-            b.level_na.push_back(na);
-            b.level_ne.push_back(ne);
-            b.max_2na = std::max<uint64_t>(b.max_2na, 2ull * na);
-            b.max_ne = std::max<uint64_t>(b.max_ne, ne);
-            b.max_bn = std::max<uint64_t>(b.max_bn, nbn + 14ull * na);
-            b.max_small = std::max<uint64_t>(b.max_small, nsmall + 2ull * na);
-            b.max_se = std::max<uint64_t>(b.max_se, nse + 2ull * ne);
-            b.max_ll = std::max<uint64_t>(b.max_ll, (uint64_t)ll_count + ne);
-        }
-        if (nbn + 14ull * na > bn_cap) {
-            uint32_t ncap = std::max<uint32_t>(2 * bn_cap, nbn + 14 * na + 1024);
-            uint32_t* nb = pool.get<uint32_t>((size_t)kBnCols * ncap);
-            if (!pool.ok) return MNRT_ERR_NOMEM;
-            for (int col = 0; col < kBnCols; ++col)
-                MNRT_HIP_CHECK(hipMemcpyAsync(nb + (size_t)col * ncap, bn_buf + (size_t)col * bn_cap, (size_t)nbn * 4,
-                                              hipMemcpyDeviceToDevice, st));
-            pool.release(bn_buf);
-            bn_buf = nb;
-            bn_cap = ncap;
-            B = bn_view(bn_buf, bn_cap);
-        }
-        if (nsmall + 2ull * na > s_cap) {
-            uint32_t ncap = std::max<uint32_t>(2 * s_cap, nsmall + 2 * na + 256);
-            SmallView NS = alloc_small(ncap);
-            if (!pool.ok) return MNRT_ERR_NOMEM;
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.first, SV.first, (size_t)nsmall * 4, hipMemcpyDeviceToDevice, st));
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.cnt, SV.cnt, (size_t)nsmall * 4, hipMemcpyDeviceToDevice, st));
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.level, SV.level, (size_t)nsmall * 4, hipMemcpyDeviceToDevice, st));
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.bn, SV.bn, (size_t)nsmall * 4, hipMemcpyDeviceToDevice, st));
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.lo, SV.lo, (size_t)nsmall * 16, hipMemcpyDeviceToDevice, st));
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.hi, SV.hi, (size_t)nsmall * 16, hipMemcpyDeviceToDevice, st));
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.scene, SV.scene, (size_t)nsmall * 4, hipMemcpyDeviceToDevice, st));
-            pool.release(SV.first);
-            pool.release(SV.cnt);
-            pool.release(SV.level);
-            pool.release(SV.bn);
-            pool.release(SV.lo);
-            pool.release(SV.hi);
-            pool.release(SV.scene);
-            SV = NS;
-            s_cap = ncap;
-        }
-        if (ll_count + (uint64_t)ne > ll_cap) {
-            uint32_t ncap = std::max<uint32_t>(2 * ll_cap, ll_count + ne + 1024);
-            uint32_t* nl = pool.get<uint32_t>(ncap);
-            if (!pool.ok) return MNRT_ERR_NOMEM;
-            if (ll_count) MNRT_HIP_CHECK(hipMemcpyAsync(nl, ll_idx, (size_t)ll_count * 4, hipMemcpyDeviceToDevice, st));
-            pool.release(ll_idx);
-            ll_idx = nl;
-            ll_cap = ncap;
-        }
-        if ((uint64_t)nse + 2ull * ne > se_cap) {
-            uint32_t ncap = (uint32_t)std::max<uint64_t>(2ull * se_cap, (uint64_t)nse + 2ull * ne + 1024);
-            ElemView NS = alloc_elems(ncap, false);
-            if (!pool.ok) return MNRT_ERR_NOMEM;
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.idx, Sm.idx, (size_t)nse * 4, hipMemcpyDeviceToDevice, st));
-            MNRT_HIP_CHECK(hipMemcpyAsync(NS.lo, Sm.lo, (size_t)nse * 16, hipMemcpyDeviceToDevice, st));
-            if (kind == MNRT_KIND_TRI)
-                MNRT_HIP_CHECK(hipMemcpyAsync(NS.hi, Sm.hi, (size_t)nse * 16, hipMemcpyDeviceToDevice, st));
-            release_elems(Sm);
-            Sm = NS;
-            se_cap = ncap;
-        }
-        if (2ull * ne > nx_cap) {
-            release_elems(Nx);
-            nx_cap = (uint32_t)std::max<uint64_t>(2ull * ne, 1024);
-            Nx = alloc_elems(nx_cap, true);
-        }
-        if (2ull * na > an_cap) {
-            release_nodes(An);
-            an_cap = std::max<uint32_t>(2 * na, 256);
-            An = alloc_nodes(an_cap);
-        }
-        const uint32_t max_chunks = ne / kChunk + na;
-        if (na > lv_na_cap || ne > lv_ne_cap) {
-            pool.release(lv_buf);
-            lv_na_cap = std::max<uint32_t>(na, lv_na_cap + lv_na_cap / 2);
-            lv_ne_cap = std::max<uint32_t>(ne, lv_ne_cap + lv_ne_cap / 2);
-            const uint64_t A_ = lv_na_cap, E_ = lv_ne_cap, C_ = E_ / kChunk + A_;
-            auto r4 = [](uint64_t k) { return (k + 3) & ~3ull; };
-            // the columns handed out below, each rounded to 16 bytes
-            // element flags (left, right; triangles also straddle left / right) and their scan
-            const uint64_t flw = (kind == MNRT_KIND_TRI ? 4 : 2) * E_ + 1;
-            const uint64_t words = r4(A_) + 3 * r4(C_) + 2 * r4(3 * A_) + 9 * r4(A_) + 2 * r4(4 * A_) +
-                                   2 * r4(flw) + r4(22 * A_) +
-                                   std::max<uint64_t>(scan_scratch_words((uint32_t)flw),
-                                                      kScanSetMax * scan_scratch_words((uint32_t)(2 * A_))) +
-                                   16;
-            lv_buf = pool.get<uint32_t>(words);
-            if (!pool.ok) return MNRT_ERR_NOMEM;
-        }
-        {
-            uint32_t* w = (uint32_t*)lv_buf;
-            const uint64_t A_ = lv_na_cap, E_ = lv_ne_cap, C_ = E_ / kChunk + A_;
-            auto take = [&](uint64_t k) {
-                uint32_t* r = w;
-                w += (k + 3) & ~3ull;  // 16-byte alignment for float4 columns
-                return r;
-            };
-            cc = take(A_);
-            chn = take(C_);
-            chf = take(C_);
-            chc = take(C_);
-            tlo = take(3 * A_);
-            thi = take(3 * A_);
-            P.newcnt = take(A_);
-            P.axis = take(A_);
-            P.split = (float*)take(A_);
-            P.lo = (float4*)take(4 * A_);
-            P.hi = (float4*)take(4 * A_);
-            P.level = take(A_);
-            P.childL = take(A_);
-            P.cur = take(A_);
-            P.leaf = take(A_);
-            P.noprog = take(A_);
-            fl = take((kind == MNRT_KIND_TRI ? 4 : 2) * E_ + 1);  // after the scan: the clip queue
-            pos = take((kind == MNRT_KIND_TRI ? 4 : 2) * E_ + 1);
-            cbuf = take(22 * A_);
-            scr = w;
-        }
-        ChildView Cv{};
-        {
-            uint32_t m = 2 * na;
-            Cv.type = cbuf;
-            Cv.cnt = cbuf + m;
-            Cv.fpos = cbuf + 2 * m;
-            Cv.sflag = cbuf + 3 * m;
-            Cv.lflag = cbuf + 4 * m;
-            Cv.scnt = cbuf + 5 * m;
-            Cv.lcnt = cbuf + 6 * m;
-            Cv.sidx = cbuf + 7 * m;
-            Cv.lidx = cbuf + 8 * m;
-            Cv.soff = cbuf + 9 * m;
-            Cv.loff = cbuf + 10 * m;
-        }
-        hipLaunchKernelGGL(k_chunk_counts, blocks_for(na), dim3(256), 0, st, hn(na), A.cnt, cc, tlo, thi);
-        MNRT_HIP_CHECK(scan_exclusive(cc, cc, na, counters + C_NCHUNKS, scr, st));
-        hipLaunchKernelGGL(k_chunk_fill, blocks_for(max_chunks), dim3(256), 0, st, hn(na), max_chunks, cc, counters,
-                           A.first, A.cnt, chn, chf, chc);
-        hipLaunchKernelGGL(k_tight, dim3((max_chunks + kTightChunks - 1) / kTightChunks), dim3(kChunk), 0, st,
-                           max_chunks, counters, chn, chf, chc, E,
-                           kind, tlo, thi);
-        hipLaunchKernelGGL((k_plan<false>), blocks_for(na), dim3(256), 0, st, hn(na), A, tlo, thi,
-                           prm->empty_space_ratio, P, (const uint32_t*)nullptr, hn(0u), B, counters);
-        MNRT_HIP_CHECK(scan_exclusive(P.newcnt, P.newcnt, na, counters + C_NEWNODES, scr, st));
-        hipLaunchKernelGGL((k_plan<true>), blocks_for(na), dim3(256), 0, st, hn(na), A, tlo, thi,
-                           prm->empty_space_ratio, P, (const uint32_t*)P.newcnt, hn(nbn), B, counters);
-        hipLaunchKernelGGL(k_classify, blocks_for(ne), dim3(256), 0, st, hn(ne), E, kind, P, fl);
-        const uint32_t nfl = (kind == MNRT_KIND_TRI ? 4u : 2u) * ne;
-        MNRT_HIP_CHECK(scan_exclusive(fl, pos, nfl, pos + nfl, scr, st));
-        hipLaunchKernelGGL(k_child_plan, blocks_for(2ull * na), dim3(256), 0, st, hn(na), hn(ne), A, P, pos,
-                           prm->small_node_max, Cv);
-        {
-            ScanSet cs{{Cv.sflag, Cv.lflag, Cv.scnt, Cv.lcnt},
-                       {Cv.sidx, Cv.lidx, Cv.soff, Cv.loff},
-                       {},
-                       {counters + C_NSMALL_NEW, counters + C_NNEXT, counters + C_ESMALL_NEW, counters + C_ENEXT}};
-            MNRT_HIP_CHECK(scan_exclusive_set(cs, 4, 2 * na, scr, st));
-        }
-        hipLaunchKernelGGL(k_child_write, blocks_for(2ull * na), dim3(256), 0, st, hn(na), A, P, Cv, hn(nsmall),
-                           hn(nse), SV, An, B, counters, E, ll_idx, ll_cap);
-        hipLaunchKernelGGL(k_scatter, blocks_for(ne), dim3(256), 0, st, hn(na), hn(ne), E, G, A, P, Cv, pos, hn(nse),
-                           Sm, se_cap, Nx, nx_cap, counters, fl);
-        if (kind == MNRT_KIND_TRI)
-            hipLaunchKernelGGL(k_clip, clip_blocks(ne), dim3(kClipBlock), 0, st, hn(na), hn(ne), E, G, A, P, Cv,
-                               (const uint32_t*)pos, hn(nse), Sm, Nx, (const uint32_t*)fl);
-        MNRT_HIP_CHECK(hipGetLastError());
-        int rc = sync_counters();
-        if (rc != MNRT_OK) return rc;
-        if (h_counters[C_ERR] != 0) return MNRT_ERR_STATE;
-        const uint32_t n_next = h_counters[C_NNEXT], e_next = h_counters[C_ENEXT];
-        nbn += h_counters[C_NEWNODES];
-        nsmall += h_counters[C_NSMALL_NEW];
-        nse += h_counters[C_ESMALL_NEW];
-        ll_count = h_counters[C_LLCOUNT];
-        maxlvl = h_counters[C_MAXLEVEL];
-        std::swap(E, Nx);
-        std::swap(e_cap, nx_cap);
-        std::swap(A, An);
-        std::swap(a_cap, an_cap);
-        ne = e_next;
-        na = n_next;
-    }
-    release_elems(E);
-    release_elems(Nx);
-    pool.release(lv_buf);
-
-    // ---- small-node stage: subtree sizes, each subtree written to its staging area ----
-    uint32_t* s_nsize = pool.get<uint32_t>(std::max<uint32_t>(nsmall, 1));
-    uint32_t* s_rsize = pool.get<uint32_t>(std::max<uint32_t>(nsmall, 1));
-    uint32_t* s_mlvl = pool.get<uint32_t>(std::max<uint32_t>(nsmall, 1));
-    uint32_t* st_off = pool.get<uint32_t>(std::max<uint32_t>(nsmall, 1));
-    uint32_t* st_ovf = pool.get<uint32_t>(std::max<uint32_t>(nsmall, 1));
-    uint32_t* st_scr = pool.get<uint32_t>(scan_scratch_words(std::max<uint32_t>(nsmall, 1)));
-    const StageCap st_cap = stage_cap_setting();
-    const uint64_t st_total = (uint64_t)st_cap.mul * nse + (uint64_t)st_cap.add * nsmall;  // sum over the roots
-    if (st_total > 0xFFFFFFFFull) return MNRT_ERR_CAPACITY;
-    uint2* st_nodes = pool.get<uint2>(std::max<uint64_t>(st_total, 1));
-    uint32_t* st_refs = pool.get<uint32_t>(std::max<uint64_t>(st_total, 1));
-    if (!pool.ok) return MNRT_ERR_NOMEM;
-    SmallOut O{};
-    O.nsize = s_nsize;
-    O.rsize = s_rsize;
-    O.mlvl = s_mlvl;
-    O.st_off = st_off;
-    O.st_nodes = st_nodes;
-    O.st_refs = st_refs;
-    O.st_ovf = st_ovf;
-    O.st_cap = st_cap;
-    O.counters = counters;
-    const dim3 small_grid((nsmall + kSmallWaves - 1) / kSmallWaves), small_block(64 * kSmallWaves);
-    if (nsmall > 0) {
-        hipLaunchKernelGGL(k_small_caps, blocks_for(nsmall), dim3(256), 0, st, hn(nsmall), (const uint32_t*)SV.cnt,
-                           st_cap, st_off);
-        MNRT_HIP_CHECK(scan_exclusive(st_off, st_off, nsmall, nullptr, st_scr, st));
-        if (kind == MNRT_KIND_TRI)
-            hipLaunchKernelGGL((k_small<kSmallStage, MNRT_KIND_TRI>), small_grid, small_block, 0, st, hn(nsmall), SV,
-                               Sm, (const float*)d_qr, O);
-        else
-            hipLaunchKernelGGL((k_small<kSmallStage, MNRT_KIND_POINT>), small_grid, small_block, 0, st, hn(nsmall), SV,
-                               Sm, (const float*)d_qr, O);
-    }
-    // ---- layout ----
-    LayoutView Lv{};
-    Lv.size = pool.get<uint32_t>(nbn);
-    Lv.rsize = pool.get<uint32_t>(nbn);
-    Lv.depth = pool.get<uint32_t>(nbn);
-    Lv.addr = pool.get<uint32_t>(nbn);
-    Lv.rbase = pool.get<uint32_t>(nbn);
-    uint32_t* lvb = pool.get<uint32_t>(64 + 65 + 64 + nbn + scan_scratch_words(std::max<uint32_t>(64, S_ + 1)));
-    if (!pool.ok) return MNRT_ERR_NOMEM;
-    {
-        uint32_t* hist = lvb;
-        uint32_t* off = lvb + 64;
-        uint32_t* cursor = off + 65;
-        uint32_t* list = cursor + 64;
-        uint32_t* sc = list + nbn;
-        MNRT_HIP_CHECK(hipMemsetAsync(hist, 0, 64 * 4, st));
-        hipLaunchKernelGGL(k_level_hist, blocks_for(nbn), dim3(256), 0, st, hn(nbn), B, hist, 63u,
-                           (uint32_t*)nullptr, 0u);
-        MNRT_HIP_CHECK(scan_exclusive(hist, off, 64, off + 64, sc, st));
-        MNRT_HIP_CHECK(hipMemcpyAsync(cursor, off, 64 * 4, hipMemcpyDeviceToDevice, st));
-        hipLaunchKernelGGL(k_level_scatter, blocks_for(nbn), dim3(256), 0, st, hn(nbn), B, cursor, list);
-        LayoutSrc Ls{off, list, s_nsize, s_rsize, s_mlvl};
-        const uint32_t top = std::min<uint32_t>(maxlvl, 63);
-        const dim3 lgrid(std::min<uint32_t>(blocks_for(nbn).x, 512u));
-        for (int lvl = (int)top; lvl >= 0; --lvl)
-            hipLaunchKernelGGL(k_layout_up, lgrid, dim3(256), 0, st, (uint32_t)lvl, Ls, B, Lv);
-        for (uint32_t lvl = 0; lvl <= top; ++lvl)
-            hipLaunchKernelGGL(k_layout_down, lgrid, dim3(256), 0, st, lvl, Ls, B, Lv);
-        // per-scene sizes (root = build node s) and their offsets in the shared arrays
-        hipLaunchKernelGGL(k_scene_sizes, blocks_for(S_), dim3(256), 0, st, S_, Lv, d_snodes, d_srefs, d_sleaves,
-                           d_smaxlvl);
-        MNRT_HIP_CHECK(scan_exclusive(d_snodes, d_nbase, S_, d_nbase + S_, sc, st));
-        MNRT_HIP_CHECK(scan_exclusive(d_srefs, d_rbase, S_, d_rbase + S_, sc, st));
-        MNRT_HIP_CHECK(hipMemcpyAsync(h_counters + 40, d_nbase + S_, 4, hipMemcpyDeviceToHost, st));
-        MNRT_HIP_CHECK(hipMemcpyAsync(h_counters + 41, d_rbase + S_, 4, hipMemcpyDeviceToHost, st));
-        MNRT_HIP_CHECK(hipMemcpyAsync(h_counters + 42, counters + C_SMALL_OVF, 4, hipMemcpyDeviceToHost, st));
-        MNRT_HIP_CHECK(hipStreamSynchronize(st));
-    }
-    const uint32_t total_nodes = h_counters[40], total_refs = h_counters[41], small_ovf = h_counters[42];
-    if (total_nodes == 0 || total_nodes > MNRT_INDEX_MASK || total_refs > MNRT_INDEX_MASK) return MNRT_ERR_CAPACITY;
-    if (stats) {
-        stats->nbn = nbn;
-        stats->nsmall = nsmall;
-        stats->nse = nse;
-        stats->maxlvl = maxlvl;
-        stats->total_nodes = total_nodes;
-        stats->total_refs = total_refs;
-        stats->max_ll = std::max<uint64_t>(stats->max_ll, ll_count);
-    }
-
-    // ---- emission into the caller-visible trees ----
-    uint32_t* d_nodes = nullptr;
-    uint32_t* d_refs = nullptr;
-    if (pool_alloc((void**)&d_nodes, (size_t)total_nodes * 8, st) != hipSuccess) return MNRT_ERR_NOMEM;
-    if (pool_alloc((void**)&d_refs, (size_t)total_refs * 4, st) != hipSuccess) {
-        (void)pool_free(d_nodes, st);
-        return MNRT_ERR_NOMEM;
-    }
-    hipLaunchKernelGGL(k_emit_large, blocks_for(nbn), dim3(256), 0, st, hn(nbn), B, Lv, ll_idx, d_nodes, d_refs,
-                       counters, total_nodes, total_refs, d_nbase, d_rbase);
-    O.bn_addr = Lv.addr;
-    O.bn_rbase = Lv.rbase;
-    O.nodes = d_nodes;
-    O.refs = d_refs;
-    O.max_nodes = total_nodes;
-    O.max_refs = total_refs;
-    O.node_base = d_nbase;
-    O.ref_base = d_rbase;
-    if (nsmall > 0) {
-        hipLaunchKernelGGL(k_small_place, small_grid, small_block, 0, st, hn(nsmall), SV, O);
-        // subtrees that outgrew their staging area are built again at their final address
-        if (small_ovf > 0 && kind == MNRT_KIND_TRI)
-            hipLaunchKernelGGL((k_small<kSmallEmit, MNRT_KIND_TRI>), small_grid, small_block, 0, st, hn(nsmall), SV,
-                               Sm, (const float*)d_qr, O);
-        else if (small_ovf > 0)
-            hipLaunchKernelGGL((k_small<kSmallEmit, MNRT_KIND_POINT>), small_grid, small_block, 0, st, hn(nsmall), SV,
-                               Sm, (const float*)d_qr, O);
-    }
-    // per-scene results to the host: counts, bases, leaves, max level, root boxes
-    uint32_t* h_res = h_tab;
-    int rc = MNRT_OK;
-    if (hipMemcpyAsync(h_res, d_snodes, (size_t)(2 * S_ + 2 * (S_ + 1) + 2 * S_) * 4, hipMemcpyDeviceToHost, st) !=
-            hipSuccess ||
-        hipMemcpyAsync(h_res + 8 * S_ + 8, d_rootbox, (size_t)6 * S_ * 4, hipMemcpyDeviceToHost, st) != hipSuccess)
-        rc = MNRT_ERR_HIP;
-    if (rc == MNRT_OK) rc = sync_counters();
-    if (rc != MNRT_OK || hipGetLastError() != hipSuccess || h_counters[C_ERR] != 0) {
-        (void)pool_free(d_nodes, st);
-        (void)pool_free(d_refs, st);
-        return rc != MNRT_OK ? rc : (h_counters[C_ERR] != 0 ? MNRT_ERR_STATE : MNRT_ERR_HIP);
-    }
-    const uint32_t* hn = h_res;
-    const uint32_t* hr = hn + S_;
-    const uint32_t* hnb = hr + S_;
-    const uint32_t* hrb = hnb + S_ + 1;
-    const uint32_t* hl = hrb + S_ + 1;
-    const uint32_t* hm = hl + S_;
-    const float* hbox = (const float*)(h_res + 8 * S_ + 8);
-    for (uint32_t s = 0; s < S_; ++s) {
-        mnrt_tree& t = out[s];
-        std::memset(&t, 0, sizeof(t));
-        t.kind = (uint32_t)kind;
-        t.num_nodes = hn[s];
-        t.num_refs = hr[s];
-        t.num_elems = h_base[s + 1] - h_base[s];
-        t.num_leaves = hl[s];
-        t.max_level = hm[s];
-        for (int k = 0; k < 3; ++k) {
-            t.root_min[k] = hbox[6 * s + k];
-            t.root_max[k] = hbox[6 * s + 3 + k];
-        }
-        t.d_nodes = d_nodes + 2ull * hnb[s];
-        t.d_refs = d_refs + hrb[s];
-        t.owns_nodes = (s == 0) ? 1u : 0u;
-    }
-    return MNRT_OK;
-}
-
-
-// =========================================================================================
-// device-driven build, recorded once into a hipGraph
-// =========================================================================================
-// The same kernels as build_batch_impl, with every count a device word (DN) and every
-// buffer fixed: the level loop is unrolled to a recorded number of levels whose kernels
-// find the level's active nodes / elements in counters[G_NA], [G_NE]; k_graph_level_end
-// moves the loop on.  Capacities come from a host-driven build of the same scenes (its
-// BuildStats) with a margin; whatever would outgrow them sets an error bit instead.
-
-// State words of the recorded loop, after the counters.
-enum : uint32_t { G_NA = C_COUNT, G_NE, G_NBN, G_NSMALL, G_NSE, G_WORDS };
-
-// counters[C_ERR] bits of a recorded build (1, 2, 4, 8, 16, 32 as in the host-driven build):
-constexpr uint32_t kErrLevelRoom = 64u;    // a level's nodes / elements outgrew the fixed buffers
-constexpr uint32_t kErrLevels = 128u;      // active nodes left after the last recorded level
-constexpr uint32_t kErrOutputRoom = 256u;  // the trees outgrew the output arrays
-constexpr uint32_t kErrLayoutDepth = 512u; // a large-stage node deeper than the layout launches
-// Levels the recorded layout covers beyond the first build's deepest large-stage node.
-constexpr uint32_t kLayoutSpareLevels = 6u;
-
-struct GraphCaps {
-    uint32_t na;           // node arrays of a level (hold twice the active nodes: the next level)
-    uint32_t ne;           // element arrays of a level
-    uint32_t bn;           // build-node table
-    uint32_t small;        // small roots
-    uint32_t small_elems;  // small-root elements
-    uint32_t ll;           // elements of large-stage leaves
-    uint32_t nodes, refs;  // output arrays (all trees)
-};
-
-__global__ __launch_bounds__(64) void k_graph_init(uint32_t* __restrict__ c, uint32_t na, uint32_t ne,
-                                                   uint32_t nbn, uint32_t nsmall, uint32_t nse) {
-    for (uint32_t i = threadIdx.x; i < G_WORDS; i += blockDim.x)
-        c[i] = i == G_NA ? na : i == G_NE ? ne : i == G_NBN ? nbn : i == G_NSMALL ? nsmall : i == G_NSE ? nse : 0u;
-}
-
-// End of a recorded level: the running totals, and the next level's counts after the
-// checks the host-driven loop makes before growing its buffers.  On any error the loop
-// stops and the small stage takes no roots; emission, records and query-time nodes are
-// then skipped (they test counters[C_ERR]).
-__global__ __launch_bounds__(64) void k_graph_level_end(uint32_t* __restrict__ c, GraphCaps cap, uint32_t last) {
-    if (threadIdx.x != 0 || blockIdx.x != 0 || c[G_NA] == 0u) return;  // G_NA == 0: no level ran
-    const uint32_t nbn = c[G_NBN] + c[C_NEWNODES];
-    const uint32_t nsmall = c[G_NSMALL] + c[C_NSMALL_NEW];
-    const uint32_t nse = c[G_NSE] + c[C_ESMALL_NEW];
-    const uint32_t na = c[C_NNEXT], ne = c[C_ENEXT];
-    c[G_NBN] = nbn;
-    c[G_NSMALL] = nsmall;
-    c[G_NSE] = nse;
-    uint32_t err = c[C_ERR];
-    if (na > 0u) {
-        const bool fits = 2ull * na <= cap.na && ne <= cap.ne && nbn + 14ull * na <= cap.bn &&
-                          nsmall + 2ull * na <= cap.small && nse + 2ull * ne <= cap.small_elems &&
-                          (uint64_t)c[C_LLCOUNT] + ne <= cap.ll;
-        if (!fits) err |= kErrLevelRoom;
-        else if (last) err |= kErrLevels;
-    }
-    if (err != 0u) {
-        c[C_ERR] = err;
-        c[G_NA] = 0u;
-        c[G_NE] = 0u;
-        c[G_NSMALL] = 0u;
-        return;
-    }
-    c[G_NA] = na;
-    c[G_NE] = ne;
-}
-
-__global__ __launch_bounds__(64) void k_graph_copy(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
-                                                   uint32_t n) {
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
-}
-
-__global__ __launch_bounds__(64) void k_graph_check_totals(uint32_t* __restrict__ c, const uint32_t* __restrict__ nodes,
-                                                           const uint32_t* __restrict__ refs, GraphCaps cap) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && (*nodes == 0u || *nodes > cap.nodes || *refs > cap.refs))
-        c[C_ERR] |= kErrOutputRoom;
-}
 
 // Bump carving of one device block: a first pass (base null) measures, the second carves.
 class Carver {
    public:
     explicit Carver(char* base) : base_(base) {}
     template <typename T>
-    T* take(uint64_t count) {
+    T* get(uint64_t count) {
         const uint64_t bytes = (std::max<uint64_t>(count * sizeof(T), 16) + 255) & ~uint64_t(255);
         T* p = base_ ? (T*)(base_ + top_) : nullptr;
         top_ += bytes;
@@ -2133,46 +1525,200 @@ class Carver {
     uint64_t top_ = 0;
 };
 
-}  // namespace
+inline dim3 blocks_for(uint64_t n, uint32_t bs = 256) { return dim3((uint32_t)std::max<uint64_t>(1, (n + bs - 1) / bs)); }
+// Grid of a launch that strides: at most `most` workgroups.
+inline dim3 blocks_to(uint64_t n, uint32_t bs, uint32_t most) {
+    return dim3(std::min<uint32_t>(blocks_for(std::min<uint64_t>(n, 1ull << 40), bs).x, most));
+}
 
-struct mnrt_build_graph {
-    int kind = 0;
-    uint32_t ns = 0, ntot = 0;
-    std::vector<uint32_t> h_base;      // ns + 1
-    std::vector<uint32_t> h_plan;      // kind / index / offset per scene
-    std::vector<uint32_t> h_photon;    // slot_begin, box_begin (ns + 1 each, photon_tables)
-    std::vector<float> h_qr, h_roots;  // per scene (roots: empty when not given)
-    mnrt_build_params prm{};
-    const float *v0 = nullptr, *v1 = nullptr, *v2 = nullptr, *pow4 = nullptr, *dir4 = nullptr;
-    BuildStats stats;
-    GraphCaps cap{};
-    uint32_t levels = 0;
-    float margin = 0.25f;
-    char* dbuf = nullptr;
-    uint64_t dbytes = 0;
-    uint32_t* counters = nullptr;
-    uint32_t* d_tab = nullptr;
-    uint32_t* nodes = nullptr;
-    uint32_t* refs = nullptr;
-    float* recs = nullptr;
-    uint32_t* qnodes = nullptr;
-    hipStream_t cap_stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+// Placement of the scenes' roots: large scenes become active nodes, whose elements start at a
+// multiple of 64 slots, small ones small roots.
+struct RootCounts {
+    uint32_t na = 0, nw = 0, nsmall = 0, nse = 0, largest = 0;
+};
+RootCounts plan_roots(const uint32_t* h_base, uint32_t S_, uint32_t small_max, uint32_t* kind, uint32_t* index,
+                      uint32_t* off) {
+    RootCounts c;
+    for (uint32_t s = 0; s < S_; ++s) {
+        const uint32_t cnt = h_base[s + 1] - h_base[s];
+        c.largest = std::max(c.largest, cnt);
+        if (cnt > small_max) {
+            kind[s] = 0;
+            index[s] = c.na++;
+            off[s] = 64u * c.nw;
+            c.nw += (cnt + 63u) / 64u;
+        } else {
+            kind[s] = 1;
+            index[s] = c.nsmall++;
+            off[s] = c.nse;
+            c.nse += cnt;
+        }
+    }
+    return c;
+}
+
+// Buffers of the large-node stage.
+struct LevelBufs {
+    uint32_t* W;
+    uint32_t* stb;  // tight bounds per scene
+    NodeView N[2];
+    ElemView X[2], Sm;
+    SmallView S;
+    BnView B;
+    uint32_t* wc;
+    uint2* woff;
+    SplitView P;
+    uint32_t* ll_idx;
+    uint2* q;
 };
 
-namespace {
+template <typename A>
+ElemView take_elems(A& a, int kind, uint64_t slots, bool waves) {
+    ElemView V{};
+    V.idx = a.template get<uint32_t>(slots);
+    V.lo = a.template get<float4>(slots);
+    V.hi = kind == MNRT_KIND_TRI ? a.template get<float4>(slots) : V.lo;
+    V.wnode = waves ? a.template get<uint32_t>(slots / 64u) : nullptr;
+    return V;
+}
 
-// Per-scene device table of a recorded build, as build_batch_impl lays it out.
-struct GraphTab {
-    uint32_t *base, *pkind, *pindex, *poff;
+template <typename A>
+LevelBufs take_levels(A& a, int kind, uint32_t S_, const BuildCaps& C) {
+    LevelBufs b{};
+    b.W = a.template get<uint32_t>(kWords);
+    b.stb = a.template get<uint32_t>(6ull * S_);
+    for (NodeView& V : b.N) {
+        V.lo = a.template get<float4>(C.na);
+        V.hi = a.template get<float4>(C.na);
+        V.first = a.template get<uint32_t>(C.na);
+        V.cnt = a.template get<uint32_t>(C.na);
+        V.level = a.template get<uint32_t>(C.na);
+        V.bn = a.template get<uint32_t>(C.na);
+        V.scene = a.template get<uint32_t>(C.na);
+        V.tb = a.template get<uint32_t>(6ull * C.na);
+    }
+    const uint64_t slots = 64ull * C.nw;
+    for (ElemView& V : b.X) V = take_elems(a, kind, slots, true);
+    b.Sm = take_elems(a, kind, C.se, false);
+    b.S.first = a.template get<uint32_t>(C.small);
+    b.S.cnt = a.template get<uint32_t>(C.small);
+    b.S.level = a.template get<uint32_t>(C.small);
+    b.S.bn = a.template get<uint32_t>(C.small);
+    b.S.lo = a.template get<float4>(C.small);
+    b.S.hi = a.template get<float4>(C.small);
+    b.S.scene = a.template get<uint32_t>(C.small);
+    uint32_t* bn = a.template get<uint32_t>((uint64_t)kBnCols * C.bn);
+    auto col = [&](uint64_t k) { return bn ? bn + k * C.bn : nullptr; };
+    b.B = BnView{col(0), col(1), col(2), col(3), col(4), col(5), col(6), col(7), col(8), col(9)};
+    b.wc = a.template get<uint32_t>(C.nw);
+    b.woff = a.template get<uint2>(C.nw);
+    b.P.lo = a.template get<float4>(C.na);
+    b.P.hi = a.template get<float4>(C.na);
+    b.P.axis = a.template get<uint32_t>(C.na);
+    b.P.split = a.template get<float>(C.na);
+    b.P.child = a.template get<uint4>(2ull * C.na);
+    b.ll_idx = a.template get<uint32_t>(C.ll);
+    b.q = kind == MNRT_KIND_TRI ? a.template get<uint2>(2 * slots) : nullptr;
+    return b;
+}
+
+// Input elements, their tight bounds per scene and the root entries.
+void launch_roots(const LevelBufs& b, const Geometry& G, uint32_t ntot, const RootPlan& R, const RootCounts& c,
+                  const float* given, float* rootbox, hipStream_t st) {
+    const uint32_t S_ = G.num_scenes;
+    hipLaunchKernelGGL(k_build_init, blocks_to(std::max(kWords, 6u * S_), 256, 256), dim3(256), 0, st, b.W, c.na, c.nw,
+                       c.nsmall, c.nse, S_, b.stb);
+    if (ntot > 0)
+        hipLaunchKernelGGL(k_init_elems, blocks_for(ntot, kInitBlock * kInitPer), dim3(kInitBlock), 0, st, G, ntot, R,
+                           b.X[0], b.Sm, b.stb);
+    hipLaunchKernelGGL(k_roots_setup, blocks_for(S_), dim3(256), 0, st, S_, G.base, b.stb, given, R, b.N[0], b.S, b.B,
+                       rootbox);
+}
+
+// One level of the large-node stage, for about na nodes in nw waves (the grids' sizes only).
+void launch_level(const LevelBufs& b, const Geometry& G, const mnrt_build_params& prm, const BuildCaps& C,
+                  uint32_t level, uint64_t na, uint64_t nw, hipStream_t st) {
+    LevelArgs L{};
+    L.W = b.W;
+    L.level = level;
+    L.cap = C;
+    L.ratio = prm.empty_space_ratio;
+    L.small_max = prm.small_node_max;
+    L.A = b.N[level & 1u];
+    L.An = b.N[(level + 1u) & 1u];
+    L.E = b.X[level & 1u];
+    L.Nx = b.X[(level + 1u) & 1u];
+    L.Sm = b.Sm;
+    L.wc = b.wc;
+    L.woff = b.woff;
+    L.P = b.P;
+    L.S = b.S;
+    L.B = b.B;
+    L.ll_idx = b.ll_idx;
+    L.q = b.q;
+    const dim3 gc = blocks_to(nw, 4, 2048), gn = blocks_to(na, kChildNodes, 512), gs = blocks_to(nw, kScatterWaves, 512);
+    if (G.kind == MNRT_KIND_TRI) {
+        hipLaunchKernelGGL((k_count<MNRT_KIND_TRI>), gc, dim3(256), 0, st, L);
+        hipLaunchKernelGGL(k_children, gn, dim3(kChildBlock), 0, st, L);
+        hipLaunchKernelGGL((k_scatter<MNRT_KIND_TRI>), gs, dim3(kScatterBlock), 0, st, L);
+        hipLaunchKernelGGL(k_clip, blocks_to(nw, 1, 2048), dim3(kClipBlock), 0, st, L, G);
+    } else {
+        hipLaunchKernelGGL((k_count<MNRT_KIND_POINT>), gc, dim3(256), 0, st, L);
+        hipLaunchKernelGGL(k_children, gn, dim3(kChildBlock), 0, st, L);
+        hipLaunchKernelGGL((k_scatter<MNRT_KIND_POINT>), gs, dim3(kScatterBlock), 0, st, L);
+    }
+}
+
+// Buffers of the small-node stage and the layout.
+template <typename A>
+SmallOut take_small(A& a, uint32_t* W, const StageCap& cap, uint64_t nsmall, uint64_t nse) {
+    const uint64_t total = (uint64_t)cap.mul * nse + (uint64_t)cap.add * nsmall;  // sum over the roots
+    SmallOut O{};
+    O.nsize = a.template get<uint32_t>(nsmall);
+    O.rsize = a.template get<uint32_t>(nsmall);
+    O.mlvl = a.template get<uint32_t>(nsmall);
+    O.st_ovf = a.template get<uint32_t>(nsmall);
+    O.st_nodes = a.template get<uint2>(total);
+    O.st_refs = a.template get<uint32_t>(total);
+    O.st_cap = cap;
+    O.W = W;
+    return O;
+}
+
+template <typename A>
+LayoutView take_layout(A& a, uint64_t nbn) {
+    LayoutView v{};
+    v.size = a.template get<uint32_t>(nbn);
+    v.rsize = a.template get<uint32_t>(nbn);
+    v.depth = a.template get<uint32_t>(nbn);
+    v.addr = a.template get<uint32_t>(nbn);
+    v.rbase = a.template get<uint32_t>(nbn);
+    return v;
+}
+
+template <int kMode>
+void launch_small(int kind, DN nsmall, const SmallView& S, const ElemView& Sm, const float* qr, const SmallOut& O,
+                  hipStream_t st) {
+    const dim3 grid((nsmall.v + kSmallWaves - 1) / kSmallWaves), block(64 * kSmallWaves);
+    if (kind == MNRT_KIND_TRI)
+        hipLaunchKernelGGL((k_small<kMode, MNRT_KIND_TRI>), grid, block, 0, st, nsmall, S, Sm, qr, O);
+    else
+        hipLaunchKernelGGL((k_small<kMode, MNRT_KIND_POINT>), grid, block, 0, st, nsmall, S, Sm, qr, O);
+}
+
+// Per-scene device table: everything from rootbox to smaxlvl is one consecutive result block.
+struct SceneTab {
+    uint32_t *base, *pkind, *pindex, *poff;  // S + 1 element offsets, the roots' placement
     float *qr, *given, *rootbox;
-    uint32_t *snodes, *srefs, *nbase, *rbase, *sleaves, *smaxlvl;
-    uint32_t *slot_begin, *box_begin;  // photon_tables
+    uint32_t *snodes, *srefs, *nbase, *rbase, *sleaves, *smaxlvl;  // nbase, rbase: S + 1
+    uint32_t *slot_begin, *box_begin;  // photon_tables (recorded builds)
 };
+constexpr uint64_t scene_tab_words(uint64_t S_) { return 32ull * S_ + 64; }
+constexpr uint64_t scene_input_words(uint64_t S_) { return 11ull * S_ + 1; }    // base .. given
+constexpr uint64_t scene_result_words(uint64_t S_) { return 12ull * S_ + 2; }   // rootbox .. smaxlvl
 
-GraphTab graph_tab(uint32_t* t, uint32_t S_) {
-    GraphTab T;
+SceneTab scene_tab(uint32_t* t, uint32_t S_) {
+    SceneTab T;
     T.base = t;
     T.pkind = T.base + S_ + 1;
     T.pindex = T.pkind + S_;
@@ -2191,137 +1737,315 @@ GraphTab graph_tab(uint32_t* t, uint32_t S_) {
     return T;
 }
 
+// Tree s of a batch from the result block r; its arrays start at nodes / refs.
+void set_tree(mnrt_tree& t, int kind, uint32_t s, uint32_t S_, const uint32_t* r, const uint32_t* h_base,
+              uint32_t* nodes, uint32_t* refs) {
+    const float* box = (const float*)r + 6ull * s;
+    const uint32_t* n = r + 6ull * S_;
+    const uint32_t *nb = n + 2ull * S_, *rb = nb + S_ + 1, *lv = rb + S_ + 1;
+    std::memset(&t, 0, sizeof(t));
+    t.kind = (uint32_t)kind;
+    t.num_nodes = n[s];
+    t.num_refs = n[S_ + s];
+    t.num_elems = h_base[s + 1] - h_base[s];
+    t.num_leaves = lv[s];
+    t.max_level = lv[S_ + s];
+    for (int k = 0; k < 3; ++k) {
+        t.root_min[k] = box[k];
+        t.root_max[k] = box[3 + k];
+    }
+    t.d_nodes = nodes + 2ull * nb[s];
+    t.d_refs = refs + rb[s];
+}
+
+// Sizes a host-driven build met, from which a recorded device-driven build sizes its
+// fixed buffers.
+struct BuildStats {
+    RootCounts roots;
+    std::vector<uint32_t> level_na, level_nw;
+    uint32_t max_na = 0, max_nw = 0;
+    uint32_t nbn = 0, nsmall = 0, nse = 0, ll = 0, maxlvl = 0, total_nodes = 0, total_refs = 0;
+};
+
+// Buffer sizes a host-driven build starts with.  Points never straddle, so a level holds at
+// most the input and small_max + 1 elements per node; triangles are duplicated, and the rest is
+// what ordinary trees stay below.  A build that outgrows one of them is run again (grow_caps).
+BuildCaps first_caps(int kind, uint32_t S_, uint32_t ntot, uint32_t small_max, const RootCounts& c) {
+    const uint64_t ne = (kind == MNRT_KIND_TRI ? 2ull : 1ull) * ntot, lim = MNRT_INDEX_MASK;
+    const uint64_t per = ntot / small_max;
+    BuildCaps C{};
+    C.na = (uint32_t)std::min<uint64_t>(lim, ne / (small_max + 1) + c.na + 1);
+    C.nw = (uint32_t)std::min<uint64_t>(lim / 64, ne / 64 + C.na + c.nw);
+    C.bn = (uint32_t)std::min<uint64_t>(lim, S_ + 8 * per + 1024);
+    C.small = (uint32_t)std::min<uint64_t>(lim, c.nsmall + 4 * per + 256);
+    C.se = (uint32_t)std::min<uint64_t>(lim, ne + 1024);
+    C.ll = (uint32_t)std::min<uint64_t>(lim, ntot + 1024ull);
+    return C;
+}
+
+// The sizes that the words W of an outgrown build exceed, at least doubled.  An element of a
+// level or a small root ends in a leaf, a build node in the tree: beyond MNRT_INDEX_MASK of them
+// the tree itself has no room (false).
+bool grow_caps(BuildCaps& C, const uint32_t* W, uint32_t level) {
+    bool room = true, grown = false;
+    auto grow = [&](uint32_t& cap, uint64_t need, uint64_t lim) {
+        if (need <= cap) return;
+        grown = true;
+        if (cap >= lim) room = false;
+        cap = (uint32_t)std::min<uint64_t>(lim, std::max<uint64_t>(2ull * cap, need + need / 4));
+    };
+    const uint64_t lim = MNRT_INDEX_MASK;
+    for (uint32_t l = 0; l <= level; ++l) {
+        grow(C.nw, W[W_LEVELS + 4 * l], lim / 64);
+        grow(C.na, W[W_LEVELS + 4 * l + 1], lim);
+    }
+    grow(C.bn, W[W_NBN], lim);
+    grow(C.small, W[W_NSMALL], lim);
+    grow(C.se, W[W_NSE], lim);
+    grow(C.ll, W[W_LL], lim);
+    return room && grown;
+}
+
+// Builds the trees of S scenes together: one level loop over the active nodes of all
+// scenes, one small-node launch for all small roots, one layout / emission pass.  Each
+// scene's tree equals the tree a single-scene build of it gives (indices are
+// scene-local, all decisions are per node).
+//   h_base: S + 1 element offsets into the concatenated input.
+//   h_roots: 6 floats per scene (or null: tight bounds).  h_qr: VVH radius per scene
+//   (or null: params->max_query_radius).
+//   out[s] views into shared arrays; out[0] owns them (mnrt_tree_release(&out[0])
+//   frees every tree of the batch).
+// The host waits for the device after the levels (to see whether there are more, and to size the
+// small stage), after the layout (to allocate the trees) and at the end.
+int build_batch_impl(int kind, const float* d_v0, const float* d_v1, const float* d_v2, const uint32_t* h_base,
+                     uint32_t nscenes, const mnrt_build_params* prm, const float* h_roots, const float* h_qr,
+                     mnrt_tree* out, hipStream_t st, BuildStats* stats = nullptr) {
+    if (!out || !prm || !h_base || nscenes == 0) return MNRT_ERR_ARG;
+    const uint32_t ntot = h_base[nscenes];
+    for (uint32_t s = 0; s < nscenes; ++s)
+        if (h_base[s + 1] < h_base[s]) return MNRT_ERR_ARG;
+    if (ntot > 0 && !d_v0) return MNRT_ERR_ARG;
+    if (kind == MNRT_KIND_TRI && ntot > 0 && (!d_v1 || !d_v2)) return MNRT_ERR_ARG;
+    if (prm->small_node_max < 1 || prm->small_node_max > 64) return MNRT_ERR_ARG;
+    if (ntot > (MNRT_INDEX_MASK >> 2)) return MNRT_ERR_CAPACITY;
+    const uint32_t S_ = nscenes;
+    Pool pool(st);
+    uint32_t* d_tab = pool.get<uint32_t>(scene_tab_words(S_));
+    if (!pool.ok) return MNRT_ERR_NOMEM;
+    const SceneTab T = scene_tab(d_tab, S_);
+
+    // host staging in pinned memory: device words, the per-scene tables
+    const uint32_t hw = (kWords + 15u) & ~15u;
+    uint32_t* h_pin = (uint32_t*)host_staging(0, (hw + scene_tab_words(S_)) * 4);
+    if (!h_pin) return MNRT_ERR_NOMEM;
+    uint32_t* h_W = h_pin;
+    uint32_t* h_tab = h_pin + hw;
+    RootCounts c;
+    {
+        const SceneTab H = scene_tab(h_tab, S_);
+        for (uint32_t s = 0; s <= S_; ++s) H.base[s] = h_base[s];
+        c = plan_roots(h_base, S_, prm->small_node_max, H.pkind, H.pindex, H.poff);
+        for (uint32_t s = 0; s < S_; ++s) {
+            H.qr[s] = h_qr ? h_qr[s] : prm->max_query_radius;
+            for (int k = 0; k < 6; ++k) H.given[6 * s + k] = h_roots ? h_roots[6 * s + k] : 0.0f;
+        }
+        MNRT_HIP_CHECK(hipMemcpyAsync(d_tab, h_tab, scene_input_words(S_) * 4, hipMemcpyHostToDevice, st));
+    }
+    Geometry G{kind, (const float4*)d_v0, d_v1 ? (const float4*)d_v1 : (const float4*)d_v0,
+               d_v2 ? (const float4*)d_v2 : (const float4*)d_v0, T.base, S_};
+    const RootPlan RP{T.pkind, T.pindex, T.poff};
+
+    // ---- large-node stage ----
+    // Levels are enqueued ahead of the counts (a middle split halves a node's box, so about log2
+    // of the elements per small root, half as many again where they lie unevenly), then a few at
+    // a time until a level has no nodes.
+    uint32_t first_levels = 0;
+    if (c.na > 0) {
+        uint32_t lg = 1;
+        while ((c.largest >> lg) >= prm->small_node_max) ++lg;
+        first_levels = std::min<uint32_t>(lg + lg / 2 + 1, kLevels);
+    }
+    BuildCaps C = first_caps(kind, S_, ntot, prm->small_node_max, c);
+    LevelBufs b{};
+    uint32_t levels = 0;
+    const Pool::Mark mark = pool.mark();
+    for (;;) {
+        b = take_levels(pool, kind, S_, C);
+        if (!pool.ok) return MNRT_ERR_NOMEM;
+        launch_roots(b, G, ntot, RP, c, h_roots ? (const float*)T.given : (const float*)nullptr, T.rootbox, st);
+        levels = 0;
+        for (uint32_t until = first_levels;; until = std::min(levels + 4u, kLevels)) {
+            for (; levels < until; ++levels)
+                launch_level(b, G, *prm, C, levels, std::min<uint64_t>(C.na, (uint64_t)c.na << levels), C.nw, st);
+            MNRT_HIP_CHECK(hipGetLastError());
+            MNRT_HIP_CHECK(hipMemcpyAsync(h_W, b.W, kWords * 4, hipMemcpyDeviceToHost, st));
+            MNRT_HIP_CHECK(hipStreamSynchronize(st));
+            if (h_W[W_ERR] != 0u || h_W[W_LEVELS + 4 * levels + 1] == 0u) break;
+            if (levels == kLevels) return MNRT_ERR_STATE;
+        }
+        if (h_W[W_ERR] == 0u) break;
+        if (h_W[W_ERR] != kErrRoom) return MNRT_ERR_STATE;
+        if (!grow_caps(C, h_W, levels)) return MNRT_ERR_CAPACITY;
+        pool.rewind(mark);
+    }
+    const uint32_t nbn = h_W[W_NBN], nsmall = h_W[W_NSMALL], nse = h_W[W_NSE];
+    if (stats) {
+        *stats = BuildStats{};
+        stats->roots = c;
+        for (uint32_t l = 0; l < levels && h_W[W_LEVELS + 4 * l + 1] != 0u; ++l) {
+            stats->level_nw.push_back(h_W[W_LEVELS + 4 * l]);
+            stats->level_na.push_back(h_W[W_LEVELS + 4 * l + 1]);
+            stats->max_nw = std::max(stats->max_nw, stats->level_nw.back());
+            stats->max_na = std::max(stats->max_na, stats->level_na.back());
+        }
+        stats->nbn = nbn;
+        stats->nsmall = nsmall;
+        stats->nse = nse;
+        stats->ll = h_W[W_LL];
+    }
+
+    // ---- small-node stage: subtree sizes, each subtree written to its staging area ----
+    const StageCap st_cap = stage_cap_setting();
+    if ((uint64_t)st_cap.mul * nse + (uint64_t)st_cap.add * nsmall > 0xFFFFFFFFull) return MNRT_ERR_CAPACITY;
+    SmallOut O = take_small(pool, b.W, st_cap, nsmall, nse);
+    const LayoutView Lv = take_layout(pool, nbn);
+    if (!pool.ok) return MNRT_ERR_NOMEM;
+    if (nsmall > 0) launch_small<kSmallStage>(kind, hn(nsmall), b.S, b.Sm, T.qr, O, st);
+    // ---- layout ----
+    const dim3 lgrid = blocks_for(nbn);
+    hipLaunchKernelGGL(k_layout_sizes, lgrid, dim3(256), 0, st, hn(nbn), b.B, Lv, (const uint32_t*)O.nsize,
+                       (const uint32_t*)O.rsize, (const uint32_t*)O.mlvl, (uint32_t)MNRT_MAX_LEVEL, b.W);
+    hipLaunchKernelGGL(k_scene_totals, dim3(1), dim3(1024), 0, st, S_, Lv, T.snodes, T.srefs, T.nbase, T.rbase,
+                       T.sleaves, T.smaxlvl, (uint32_t)MNRT_INDEX_MASK, (uint32_t)MNRT_INDEX_MASK, b.W);
+    MNRT_HIP_CHECK(hipGetLastError());
+    uint32_t* h_res = h_tab;
+    MNRT_HIP_CHECK(hipMemcpyAsync(h_res, T.rootbox, scene_result_words(S_) * 4, hipMemcpyDeviceToHost, st));
+    MNRT_HIP_CHECK(hipMemcpyAsync(h_W, b.W, W_LEVELS * 4, hipMemcpyDeviceToHost, st));
+    MNRT_HIP_CHECK(hipStreamSynchronize(st));
+    if (h_W[W_ERR] != 0u) return h_W[W_ERR] == kErrOutputRoom ? MNRT_ERR_CAPACITY : MNRT_ERR_STATE;
+    const uint32_t total_nodes = h_res[9ull * S_], total_refs = h_res[10ull * S_ + 1];
+    if (stats) {
+        stats->maxlvl = h_W[W_MAXLEVEL];
+        stats->total_nodes = total_nodes;
+        stats->total_refs = total_refs;
+    }
+
+    // ---- emission into the caller-visible trees ----
+    uint32_t* d_nodes = nullptr;
+    uint32_t* d_refs = nullptr;
+    if (pool_alloc((void**)&d_nodes, (size_t)total_nodes * 8, st) != hipSuccess) return MNRT_ERR_NOMEM;
+    if (pool_alloc((void**)&d_refs, (size_t)total_refs * 4, st) != hipSuccess) {
+        (void)pool_free(d_nodes, st);
+        return MNRT_ERR_NOMEM;
+    }
+    hipLaunchKernelGGL(k_emit_large, lgrid, dim3(256), 0, st, hn(nbn), b.B, Lv, (const uint32_t*)b.ll_idx, d_nodes,
+                       d_refs, (const uint32_t*)b.W, (const uint32_t*)T.nbase, (const uint32_t*)T.rbase);
+    O.bn_addr = Lv.addr;
+    O.bn_rbase = Lv.rbase;
+    O.nodes = d_nodes;
+    O.refs = d_refs;
+    O.max_nodes = total_nodes;
+    O.max_refs = total_refs;
+    O.node_base = T.nbase;
+    O.ref_base = T.rbase;
+    if (nsmall > 0) {
+        hipLaunchKernelGGL(k_small_place, dim3((nsmall + kSmallWaves - 1) / kSmallWaves), dim3(64 * kSmallWaves), 0, st,
+                           hn(nsmall), b.S, O);
+        // subtrees that outgrew their staging area are built again at their final address
+        if (h_W[W_SMALL_OVF] > 0) launch_small<kSmallEmit>(kind, hn(nsmall), b.S, b.Sm, T.qr, O, st);
+    }
+    int rc = MNRT_OK;
+    if (hipMemcpyAsync(h_W, b.W, W_LEVELS * 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess || hipGetLastError() != hipSuccess)
+        rc = MNRT_ERR_HIP;
+    else if (h_W[W_ERR] != 0u)
+        rc = MNRT_ERR_STATE;
+    if (rc != MNRT_OK) {
+        (void)pool_free(d_nodes, st);
+        (void)pool_free(d_refs, st);
+        return rc;
+    }
+    for (uint32_t s = 0; s < S_; ++s) {
+        set_tree(out[s], kind, s, S_, h_res, h_base, d_nodes, d_refs);
+        out[s].owns_nodes = (s == 0) ? 1u : 0u;
+    }
+    return MNRT_OK;
+}
+
+// =========================================================================================
+// device-driven build, recorded once into a hipGraph
+// =========================================================================================
+// The same kernels as build_batch_impl, with every buffer fixed and the level loop unrolled to
+// a recorded number of levels.  Capacities come from a host-driven build of the same scenes (its
+// BuildStats) with a margin; whatever would outgrow them sets an error bit instead.
+
+// Levels a recorded build covers beyond the first build's deepest large-stage node.
+constexpr uint32_t kLayoutSpareLevels = 6u;
+
+// Active nodes left after the last recorded level.
+__global__ __launch_bounds__(64) void k_levels_done(uint32_t* __restrict__ W, uint32_t level) {
+    if (threadIdx.x == 0 && blockIdx.x == 0 && W[W_ERR] == 0u && W[W_LEVELS + 4 * level + 1] != 0u) W[W_ERR] = kErrLevels;
+}
+
+}  // namespace
+
+struct mnrt_build_graph {
+    int kind = 0;
+    uint32_t ns = 0, ntot = 0;
+    std::vector<uint32_t> h_base;      // ns + 1
+    std::vector<uint32_t> h_plan;      // kind / index / offset per scene
+    std::vector<uint32_t> h_photon;    // slot_begin, box_begin (ns + 1 each, photon_tables)
+    std::vector<float> h_qr, h_roots;  // per scene (roots: empty when not given)
+    mnrt_build_params prm{};
+    const float *v0 = nullptr, *v1 = nullptr, *v2 = nullptr, *pow4 = nullptr, *dir4 = nullptr;
+    BuildStats stats;
+    BuildCaps cap{};
+    uint32_t cap_nodes = 0, cap_refs = 0;  // output arrays (all trees)
+    uint32_t levels = 0;
+    float margin = 0.25f;
+    char* dbuf = nullptr;
+    uint64_t dbytes = 0;
+    uint32_t* W = nullptr;
+    uint32_t* d_tab = nullptr;
+    uint32_t* nodes = nullptr;
+    uint32_t* refs = nullptr;
+    float* recs = nullptr;
+    uint32_t* qnodes = nullptr;
+    hipStream_t cap_stream = nullptr;
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+};
+
+namespace {
+
 // Carves g's device block (base null: measures it) and, when st is given, enqueues the
 // whole build on st (which is capturing).  Every launch is a kernel: the sequence has no
 // memset, copy or allocation nodes.
 int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
     const uint32_t S_ = g.ns, ntot = g.ntot;
     const int kind = g.kind;
-    const GraphCaps C = g.cap;
-    const uint32_t NA = C.na, NE = C.ne, CH = NE / kChunk + NA;
+    const BuildCaps C = g.cap;
     Carver cv(base);
-    uint32_t* counters = cv.take<uint32_t>(G_WORDS);
-    uint32_t* tab = cv.take<uint32_t>(32ull * S_ + 64);
-    const GraphTab T = graph_tab(tab, S_);
-    auto elems = [&](uint64_t cap, bool with_node) {
-        ElemView V{};
-        V.idx = cv.take<uint32_t>(cap);
-        V.lo = cv.take<float4>(cap);
-        V.hi = kind == MNRT_KIND_TRI ? cv.take<float4>(cap) : V.lo;
-        V.node = with_node ? cv.take<uint32_t>(cap) : nullptr;
-        return V;
-    };
-    auto nodesv = [&](uint64_t cap) {
-        NodeView V{};
-        V.lo = cv.take<float4>(cap);
-        V.hi = cv.take<float4>(cap);
-        V.first = cv.take<uint32_t>(cap);
-        V.cnt = cv.take<uint32_t>(cap);
-        V.level = cv.take<uint32_t>(cap);
-        V.bn = cv.take<uint32_t>(cap);
-        V.scene = cv.take<uint32_t>(cap);
-        return V;
-    };
-    ElemView Ein = elems(std::max<uint32_t>(ntot, 1), true);
-    const uint32_t ch0 = ntot / kChunk + S_;
-    uint32_t* tb = cv.take<uint32_t>(3ull * ch0 + 8ull * S_ + scan_scratch_words(S_) + 16);
-    uint32_t* bnb = cv.take<uint32_t>((uint64_t)kBnCols * C.bn);
-    const BnView B{bnb,
-                   bnb + C.bn,
-                   bnb + 2ull * C.bn,
-                   bnb + 3ull * C.bn,
-                   bnb + 4ull * C.bn,
-                   bnb + 5ull * C.bn,
-                   bnb + 6ull * C.bn,
-                   bnb + 7ull * C.bn};
-    SmallView SV{};
-    SV.first = cv.take<uint32_t>(C.small);
-    SV.cnt = cv.take<uint32_t>(C.small);
-    SV.level = cv.take<uint32_t>(C.small);
-    SV.bn = cv.take<uint32_t>(C.small);
-    SV.lo = cv.take<float4>(C.small);
-    SV.hi = cv.take<float4>(C.small);
-    SV.scene = cv.take<uint32_t>(C.small);
-    const ElemView Sm = elems(C.small_elems, false);
-    const NodeView Nv[2] = {nodesv(NA), nodesv(NA)};
-    const ElemView Xv[2] = {elems(NE, true), elems(NE, true)};
-    uint32_t* ll_idx = cv.take<uint32_t>(C.ll);
-    // level buffers (fixed strides: NA nodes, NE elements)
-    uint32_t* cc = cv.take<uint32_t>(NA);
-    uint32_t* chn = cv.take<uint32_t>(CH);
-    uint32_t* chf = cv.take<uint32_t>(CH);
-    uint32_t* chc = cv.take<uint32_t>(CH);
-    uint32_t* tlo = cv.take<uint32_t>(3ull * NA);
-    uint32_t* thi = cv.take<uint32_t>(3ull * NA);
-    PlanView P{};
-    P.newcnt = cv.take<uint32_t>(NA);
-    P.axis = cv.take<uint32_t>(NA);
-    P.split = cv.take<float>(NA);
-    P.lo = cv.take<float4>(NA);
-    P.hi = cv.take<float4>(NA);
-    P.level = cv.take<uint32_t>(NA);
-    P.childL = cv.take<uint32_t>(NA);
-    P.cur = cv.take<uint32_t>(NA);
-    P.leaf = cv.take<uint32_t>(NA);
-    P.noprog = cv.take<uint32_t>(NA);
-    const uint64_t FLW = (kind == MNRT_KIND_TRI ? 4ull : 2ull) * NE;  // element flags (+ straddle flags)
-    uint32_t* fl = cv.take<uint32_t>(FLW + 1);  // after the scan: the clip queue
-    uint32_t* pos = cv.take<uint32_t>(FLW + 1);
-    uint32_t* cbuf = cv.take<uint32_t>(22ull * NA);
-    ChildView Cv{};
-    {
-        const uint64_t m = 2ull * NA;
-        Cv.type = cbuf;
-        Cv.cnt = cbuf + m;
-        Cv.fpos = cbuf + 2 * m;
-        Cv.sflag = cbuf + 3 * m;
-        Cv.lflag = cbuf + 4 * m;
-        Cv.scnt = cbuf + 5 * m;
-        Cv.lcnt = cbuf + 6 * m;
-        Cv.sidx = cbuf + 7 * m;
-        Cv.lidx = cbuf + 8 * m;
-        Cv.soff = cbuf + 9 * m;
-        Cv.loff = cbuf + 10 * m;
-    }
-    uint32_t* scr = cv.take<uint32_t>(std::max<uint64_t>({(uint64_t)dscan_tiles(NA), (uint64_t)dscan_tiles((uint32_t)FLW),
-                                                           4ull * dscan_tiles(2 * NA), (uint64_t)dscan_tiles(C.small)}) +
-                                      16);
-    // small stage
+    uint32_t* tab = cv.get<uint32_t>(scene_tab_words(S_));
+    const SceneTab T = scene_tab(tab, S_);
+    const LevelBufs b = take_levels(cv, kind, S_, C);
     const StageCap st_cap = stage_cap_setting();
-    const uint64_t st_total = (uint64_t)st_cap.mul * C.small_elems + (uint64_t)st_cap.add * C.small;
-    if (st_total > 0xFFFFFFFFull) return MNRT_ERR_CAPACITY;
-    SmallOut O{};
-    O.nsize = cv.take<uint32_t>(C.small);
-    O.rsize = cv.take<uint32_t>(C.small);
-    O.mlvl = cv.take<uint32_t>(C.small);
-    uint32_t* st_off = cv.take<uint32_t>(C.small);
-    O.st_off = st_off;
-    O.st_ovf = cv.take<uint32_t>(C.small);
-    O.st_nodes = cv.take<uint2>(st_total);
-    O.st_refs = cv.take<uint32_t>(st_total);
-    O.st_cap = st_cap;
-    O.counters = counters;
-    // layout
-    LayoutView Lv{};
-    Lv.size = cv.take<uint32_t>(C.bn);
-    Lv.rsize = cv.take<uint32_t>(C.bn);
-    Lv.depth = cv.take<uint32_t>(C.bn);
-    Lv.addr = cv.take<uint32_t>(C.bn);
-    Lv.rbase = cv.take<uint32_t>(C.bn);
-    uint32_t* lvb = cv.take<uint32_t>(64 + 65 + 64 + (uint64_t)C.bn + scan_scratch_words(std::max<uint32_t>(64, S_ + 1)));
+    if ((uint64_t)st_cap.mul * C.se + (uint64_t)st_cap.add * C.small > 0xFFFFFFFFull) return MNRT_ERR_CAPACITY;
+    SmallOut O = take_small(cv, b.W, st_cap, C.small, C.se);
+    const LayoutView Lv = take_layout(cv, C.bn);
     // outputs
-    uint32_t* nodes = cv.take<uint32_t>(2ull * C.nodes);
-    uint32_t* refs = cv.take<uint32_t>(C.refs);
-    float* recs = cv.take<float>((uint64_t)C.refs * (kind == MNRT_KIND_TRI ? 12u : 8u));
+    uint32_t* nodes = cv.get<uint32_t>(2ull * g.cap_nodes);
+    uint32_t* refs = cv.get<uint32_t>(g.cap_refs);
+    float* recs = cv.get<float>((uint64_t)g.cap_refs * (kind == MNRT_KIND_TRI ? 12u : 8u));
     // box hierarchies and query-time node words (box_block)
     uint32_t* qnodes = kind == MNRT_KIND_POINT
-                           ? cv.take<uint32_t>(box_block(g.h_photon[2 * S_ + 1], S_, C.nodes) + 8u)
+                           ? cv.get<uint32_t>(box_block(g.h_photon[2 * S_ + 1], S_, g.cap_nodes) + 8u)
                            : nullptr;
     if (!base) {
         g.dbytes = cv.size();
         return MNRT_OK;
     }
-    g.counters = counters;
+    g.W = b.W;
     g.d_tab = tab;
     g.nodes = nodes;
     g.refs = refs;
@@ -2335,150 +2059,49 @@ int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
     auto planned = [&](uint64_t x, uint64_t slack, uint64_t cap) {
         return std::min<uint64_t>(cap, (uint64_t)((double)x * grow) + slack);
     };
-    hipLaunchKernelGGL(k_graph_init, dim3(1), dim3(64), 0, st, counters, bs.na0, bs.ne0, S_, bs.nsmall0, bs.nse0);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, T.sleaves, 2 * S_, 0u);
     Geometry G{kind, (const float4*)g.v0, g.v1 ? (const float4*)g.v1 : (const float4*)g.v0,
                g.v2 ? (const float4*)g.v2 : (const float4*)g.v0, T.base, S_};
-    RootPlan RP{T.pkind, T.pindex, T.poff};
-    if (ntot > 0) hipLaunchKernelGGL(k_init_elems, blocks_for(ntot), dim3(256), 0, st, G, ntot, Ein);
-    uint32_t* rtlo = nullptr;
-    uint32_t* rthi = nullptr;
-    if (g.h_roots.empty() && ntot > 0) {
-        uint32_t *rchn = tb, *rchf = rchn + ch0, *rchc = rchf + ch0, *rcc = rchc + ch0;
-        uint32_t* cnts = rcc + S_;
-        rtlo = cnts + S_;
-        rthi = rtlo + 3 * S_;
-        uint32_t* sc = rthi + 3 * S_;
-        hipLaunchKernelGGL(k_scene_counts, blocks_for(S_), dim3(256), 0, st, S_, T.base, cnts);
-        hipLaunchKernelGGL(k_chunk_counts, blocks_for(S_), dim3(256), 0, st, hn(S_), cnts, rcc, rtlo, rthi);
-        MNRT_HIP_CHECK(scan_exclusive(rcc, rcc, S_, counters + C_NCHUNKS, sc, st));
-        hipLaunchKernelGGL(k_chunk_fill, blocks_for(ch0), dim3(256), 0, st, hn(S_), ch0, rcc, counters, T.base, cnts,
-                           rchn, rchf, rchc);
-        hipLaunchKernelGGL(k_tight, dim3((ch0 + kTightChunks - 1) / kTightChunks), dim3(kChunk), 0, st, ch0, counters,
-                           rchn, rchf, rchc, Ein, kind, rtlo, rthi);
-    }
-    hipLaunchKernelGGL(k_roots_setup, blocks_for(S_), dim3(256), 0, st, S_, T.base, rtlo, rthi,
-                       g.h_roots.empty() ? (const float*)nullptr : (const float*)T.given, RP, Nv[0], SV, B, T.rootbox);
-    if (ntot > 0)
-        hipLaunchKernelGGL(k_partition_elems, blocks_for(ntot), dim3(256), 0, st, ntot, Ein, kind, RP, Xv[0], Sm);
+    launch_roots(b, G, ntot, RootPlan{T.pkind, T.pindex, T.poff}, bs.roots,
+                 g.h_roots.empty() ? (const float*)nullptr : (const float*)T.given, T.rootbox, st);
     MNRT_HIP_CHECK(hipGetLastError());
-
-    // large-node stage: g.levels recorded levels
-    const DN na = dn(counters + G_NA, NA), ne = dn(counters + G_NE, NE);
-    const DN na2 = dn(counters + G_NA, 2 * NA, 1), ne2 = dn(counters + G_NE, 2 * NE, 1);
-    const DN nbn = dn(counters + G_NBN, C.bn), nsm = dn(counters + G_NSMALL, C.small);
-    const DN nse = dn(counters + G_NSE, C.small_elems);
     for (uint32_t l = 0; l < g.levels; ++l) {
-        const NodeView& A = Nv[l & 1u];
-        const NodeView& An = Nv[(l + 1) & 1u];
-        const ElemView& E = Xv[l & 1u];
-        const ElemView& Nx = Xv[(l + 1) & 1u];
         const size_t pl = std::min<size_t>(l, bs.level_na.size() - 1);
-        const uint64_t pna = planned(bs.level_na[pl], 256, NA), pne = planned(bs.level_ne[pl], 4096, NE);
-        const dim3 gna = blocks_for(pna), gna2 = blocks_for(2 * pna), gne = blocks_for(pne);
-        const dim3 gch((uint32_t)std::max<uint64_t>(1, (pne / kChunk + pna + kTightChunks - 1) / kTightChunks));
-        hipLaunchKernelGGL(k_chunk_counts, gna, dim3(256), 0, st, na, A.cnt, cc, tlo, thi);
-        MNRT_HIP_CHECK(dscan1(cc, cc, na, counters + C_NCHUNKS, false, scr, st));
-        hipLaunchKernelGGL(k_chunk_fill, blocks_for(pne / kChunk + pna), dim3(256), 0, st, na, CH, cc, counters,
-                           A.first, A.cnt, chn, chf, chc);
-        hipLaunchKernelGGL(k_tight, gch, dim3(kChunk), 0, st, CH, counters, chn, chf, chc, E, kind, tlo, thi);
-        hipLaunchKernelGGL((k_plan<false>), gna, dim3(256), 0, st, na, A, tlo, thi, g.prm.empty_space_ratio, P,
-                           (const uint32_t*)nullptr, hn(0u), B, counters);
-        MNRT_HIP_CHECK(dscan1(P.newcnt, P.newcnt, na, counters + C_NEWNODES, false, scr, st));
-        hipLaunchKernelGGL((k_plan<true>), gna, dim3(256), 0, st, na, A, tlo, thi, g.prm.empty_space_ratio, P,
-                           (const uint32_t*)P.newcnt, nbn, B, counters);
-        hipLaunchKernelGGL(k_classify, gne, dim3(256), 0, st, ne, E, kind, P, fl);
-        MNRT_HIP_CHECK(dscan1(fl, pos, kind == MNRT_KIND_TRI ? dn(counters + G_NE, 4 * NE, 2) : ne2, nullptr, true,
-                              scr, st));
-        hipLaunchKernelGGL(k_child_plan, gna2, dim3(256), 0, st, na, ne, A, P, pos, g.prm.small_node_max, Cv);
-        {
-            DScanSet cs{};
-            const uint32_t* ins[4] = {Cv.sflag, Cv.lflag, Cv.scnt, Cv.lcnt};
-            uint32_t* outs[4] = {Cv.sidx, Cv.lidx, Cv.soff, Cv.loff};
-            uint32_t* tots[4] = {counters + C_NSMALL_NEW, counters + C_NNEXT, counters + C_ESMALL_NEW,
-                                 counters + C_ENEXT};
-            for (int y = 0; y < 4; ++y) {
-                cs.in[y] = ins[y];
-                cs.out[y] = outs[y];
-                cs.total[y] = tots[y];
-            }
-            MNRT_HIP_CHECK(dscan(cs, 4, na2, scr, st));
-        }
-        hipLaunchKernelGGL(k_child_write, gna2, dim3(256), 0, st, na, A, P, Cv, nsm, nse, SV, An, B, counters, E,
-                           ll_idx, C.ll);
-        hipLaunchKernelGGL(k_scatter, gne, dim3(256), 0, st, na, ne, E, G, A, P, Cv, pos, nse, Sm, C.small_elems, Nx,
-                           NE, counters, fl);
-        if (kind == MNRT_KIND_TRI)
-            hipLaunchKernelGGL(k_clip, clip_blocks(pne), dim3(kClipBlock), 0, st, na, ne, E, G, A, P, Cv, (const uint32_t*)pos,
-                               nse, Sm, Nx, (const uint32_t*)fl);
-        hipLaunchKernelGGL(k_graph_level_end, dim3(1), dim3(64), 0, st, counters, C, l + 1 == g.levels ? 1u : 0u);
+        launch_level(b, G, g.prm, C, l, planned(bs.level_na[pl], 256, C.na), planned(bs.level_nw[pl], 64, C.nw), st);
         MNRT_HIP_CHECK(hipGetLastError());
     }
+    hipLaunchKernelGGL(k_levels_done, dim3(1), dim3(64), 0, st, b.W, g.levels);
 
     // small-node stage
-    const dim3 small_grid((C.small + kSmallWaves - 1) / kSmallWaves), small_block(64 * kSmallWaves);
-    hipLaunchKernelGGL(k_small_caps, blocks_for(C.small), dim3(256), 0, st, nsm, (const uint32_t*)SV.cnt, st_cap,
-                       st_off);
-    MNRT_HIP_CHECK(dscan1(st_off, st_off, nsm, nullptr, false, scr, st));
-    if (kind == MNRT_KIND_TRI)
-        hipLaunchKernelGGL((k_small<kSmallStage, MNRT_KIND_TRI>), small_grid, small_block, 0, st, nsm, SV, Sm,
-                           (const float*)T.qr, O);
-    else
-        hipLaunchKernelGGL((k_small<kSmallStage, MNRT_KIND_POINT>), small_grid, small_block, 0, st, nsm, SV, Sm,
-                           (const float*)T.qr, O);
+    const DN nbn = dn(b.W + W_NBN, C.bn), nsm = dn(b.W + W_NSMALL, C.small);
+    launch_small<kSmallStage>(kind, nsm, b.S, b.Sm, T.qr, O, st);
     // layout
-    {
-        uint32_t* hist = lvb;
-        uint32_t* off = lvb + 64;
-        uint32_t* cursor = off + 65;
-        uint32_t* list = cursor + 64;
-        uint32_t* sc = list + C.bn;
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, hist, 64u, 0u);
-        // the layout launches cover the first build's depth and a few levels more; a deeper
-        // replay sets kErrLayoutDepth here, before the layout, so nothing is emitted
-        const uint32_t top = std::min<uint32_t>({bs.maxlvl + kLayoutSpareLevels, (uint32_t)MNRT_MAX_LEVEL, 63u});
-        hipLaunchKernelGGL(k_level_hist, blocks_for(C.bn), dim3(256), 0, st, nbn, B, hist, top, counters + C_ERR,
-                           kErrLayoutDepth);
-        MNRT_HIP_CHECK(scan_exclusive(hist, off, 64, off + 64, sc, st));
-        hipLaunchKernelGGL(k_graph_copy, dim3(1), dim3(64), 0, st, cursor, (const uint32_t*)off, 64u);
-        hipLaunchKernelGGL(k_level_scatter, blocks_for(C.bn), dim3(256), 0, st, nbn, B, cursor, list);
-        LayoutSrc Ls{off, list, O.nsize, O.rsize, O.mlvl};
-        const dim3 lgrid(std::min<uint32_t>(blocks_for(C.bn).x, 512u));
-        for (int lvl = (int)top; lvl >= 0; --lvl)
-            hipLaunchKernelGGL(k_layout_up, lgrid, dim3(256), 0, st, (uint32_t)lvl, Ls, B, Lv);
-        for (uint32_t lvl = 0; lvl <= top; ++lvl)
-            hipLaunchKernelGGL(k_layout_down, lgrid, dim3(256), 0, st, lvl, Ls, B, Lv);
-        hipLaunchKernelGGL(k_scene_sizes, blocks_for(S_), dim3(256), 0, st, S_, Lv, T.snodes, T.srefs, T.sleaves,
-                           T.smaxlvl);
-        MNRT_HIP_CHECK(scan_exclusive(T.snodes, T.nbase, S_, T.nbase + S_, sc, st));
-        MNRT_HIP_CHECK(scan_exclusive(T.srefs, T.rbase, S_, T.rbase + S_, sc, st));
-        hipLaunchKernelGGL(k_graph_check_totals, dim3(1), dim3(64), 0, st, counters, (const uint32_t*)(T.nbase + S_),
-                           (const uint32_t*)(T.rbase + S_), C);
-    }
-    // emission (each kernel returns at once when counters[C_ERR] is set)
-    hipLaunchKernelGGL(k_emit_large, blocks_for(C.bn), dim3(256), 0, st, nbn, B, Lv, (const uint32_t*)ll_idx, nodes,
-                       refs, counters, C.nodes, C.refs, (const uint32_t*)T.nbase, (const uint32_t*)T.rbase);
+    // a replay deeper than the first build's depth and a few levels more sets kErrLayoutDepth
+    const uint32_t top = std::min<uint32_t>(bs.maxlvl + kLayoutSpareLevels, MNRT_MAX_LEVEL);
+    const dim3 lgrid = blocks_for(planned(bs.nbn, 256, C.bn));
+    hipLaunchKernelGGL(k_layout_sizes, lgrid, dim3(256), 0, st, nbn, b.B, Lv, (const uint32_t*)O.nsize,
+                       (const uint32_t*)O.rsize, (const uint32_t*)O.mlvl, top, b.W);
+    hipLaunchKernelGGL(k_scene_totals, dim3(1), dim3(1024), 0, st, S_, Lv, T.snodes, T.srefs, T.nbase, T.rbase,
+                       T.sleaves, T.smaxlvl, g.cap_nodes, g.cap_refs, b.W);
+    // emission (each kernel returns at once when W[W_ERR] is set)
+    hipLaunchKernelGGL(k_emit_large, lgrid, dim3(256), 0, st, nbn, b.B, Lv, (const uint32_t*)b.ll_idx, nodes, refs,
+                       (const uint32_t*)b.W, (const uint32_t*)T.nbase, (const uint32_t*)T.rbase);
     O.bn_addr = Lv.addr;
     O.bn_rbase = Lv.rbase;
     O.nodes = nodes;
     O.refs = refs;
-    O.max_nodes = C.nodes;
-    O.max_refs = C.refs;
+    O.max_nodes = g.cap_nodes;
+    O.max_refs = g.cap_refs;
     O.node_base = T.nbase;
     O.ref_base = T.rbase;
-    hipLaunchKernelGGL(k_small_place, small_grid, small_block, 0, st, nsm, SV, O);
+    hipLaunchKernelGGL(k_small_place, dim3((C.small + kSmallWaves - 1) / kSmallWaves), dim3(64 * kSmallWaves), 0, st,
+                       nsm, b.S, O);
     // subtrees that outgrew their staging area, built again at their final address
-    if (kind == MNRT_KIND_TRI)
-        hipLaunchKernelGGL((k_small<kSmallEmit, MNRT_KIND_TRI>), small_grid, small_block, 0, st, nsm, SV, Sm,
-                           (const float*)T.qr, O);
-    else
-        hipLaunchKernelGGL((k_small<kSmallEmit, MNRT_KIND_POINT>), small_grid, small_block, 0, st, nsm, SV, Sm,
-                           (const float*)T.qr, O);
+    launch_small<kSmallEmit>(kind, nsm, b.S, b.Sm, T.qr, O, st);
     // records and query-time node words
-    const DN nrefs = dn(T.rbase + S_, C.refs), nnodes = dn(T.nbase + S_, C.nodes);
+    const DN nrefs = dn(T.rbase + S_, g.cap_refs), nnodes = dn(T.nbase + S_, g.cap_nodes);
     if (kind == MNRT_KIND_TRI) {
         int rc = launch_tri_records_batch(refs, nrefs, T.rbase, T.base, S_, (const float4*)g.v0, (const float4*)g.v1,
-                                          (const float4*)g.v2, (float4*)recs, counters + C_ERR, st);
+                                          (const float4*)g.v2, (float4*)recs, b.W + W_ERR, st);
         if (rc != MNRT_OK) return rc;
     } else if (g.pow4 && g.dir4) {
         uint32_t max_elems = 0;
@@ -2486,10 +2109,10 @@ int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
         const PhotonTables tab{S_, T.nbase, T.rbase, T.base, T.slot_begin, T.box_begin};
         int rc = launch_photon_records_batch(refs, tab, g.h_photon[S_], max_elems, (const float4*)g.v0,
                                              (const float4*)g.pow4, (const float4*)g.dir4, (float4*)recs,
-                                             (float4*)qnodes, counters + C_ERR, st);
+                                             (float4*)qnodes, b.W + W_ERR, st);
         if (rc == MNRT_OK)
             rc = launch_collapse_batch((const uint2*)nodes, nnodes, T.nbase, S_, T.box_begin, kQueryLeafRefs,
-                                       (uint2*)qnodes, counters + C_ERR, st);
+                                       (uint2*)qnodes, b.W + W_ERR, st);
         if (rc != MNRT_OK) return rc;
     }
     MNRT_HIP_CHECK(hipGetLastError());
@@ -2599,37 +2222,23 @@ extern "C" int mnrt_build_graph_create(const mnrt_build_graph_desc* d, mnrt_tree
     auto cap = [&](uint64_t x, uint64_t slack) -> uint32_t {
         return (uint32_t)std::min<uint64_t>(MNRT_INDEX_MASK, (uint64_t)((double)x * grow) + slack);
     };
-    GraphCaps& C = g->cap;
-    C.na = cap(std::max<uint64_t>(bs.max_2na, 2ull * bs.na0), 64);
-    C.ne = cap(std::max<uint64_t>(bs.max_ne, bs.ne0), 1024);
-    C.bn = cap(std::max<uint64_t>({bs.max_bn, (uint64_t)bs.nbn, (uint64_t)S_}), 1024);
-    C.small = cap(std::max<uint64_t>({bs.max_small, (uint64_t)bs.nsmall, (uint64_t)bs.nsmall0}), 256);
-    C.small_elems = cap(std::max<uint64_t>({bs.max_se, (uint64_t)bs.nse, (uint64_t)bs.nse0}), 1024);
-    C.ll = cap(bs.max_ll, 1024);
-    C.nodes = cap(bs.total_nodes, 1024);
-    C.refs = cap(bs.total_refs, 1024);
+    // room for a replay that needs, at any level, the children of the widest level on top of the
+    // first build's totals
+    BuildCaps& C = g->cap;
+    C.na = cap(bs.max_na, 64);
+    C.nw = cap(bs.max_nw, 16ull + C.na);
+    C.bn = cap(bs.nbn + 14ull * bs.max_na, 1024);
+    C.small = cap(bs.nsmall + 2ull * bs.max_na, 256);
+    C.se = cap(bs.nse + 128ull * bs.max_nw, 1024);
+    C.ll = cap(bs.ll + 64ull * bs.max_nw, 1024);
+    C.nw = std::min<uint32_t>(C.nw, MNRT_INDEX_MASK / 64u);
+    g->cap_nodes = cap(bs.total_nodes, 1024);
+    g->cap_refs = cap(bs.total_refs, 1024);
     g->levels = bs.level_na.empty() ? 0u
                                     : std::min<uint32_t>((uint32_t)bs.level_na.size() + 2u, MNRT_MAX_LEVEL + 1u);
-    // the root plan, as build_batch_impl makes it
     g->h_plan.assign(3ull * S_, 0u);
-    {
-        uint32_t na = 0, nsmall = 0, ne = 0, nse = 0;
-        for (uint32_t s = 0; s < S_; ++s) {
-            const uint32_t cnt = g->h_base[s + 1] - g->h_base[s];
-            if (cnt > g->prm.small_node_max) {
-                g->h_plan[s] = 0;
-                g->h_plan[S_ + s] = na++;
-                g->h_plan[2 * S_ + s] = ne;
-                ne += cnt;
-            } else {
-                g->h_plan[s] = 1;
-                g->h_plan[S_ + s] = nsmall++;
-                g->h_plan[2 * S_ + s] = nse;
-                nse += cnt;
-            }
-        }
-        if (na != bs.na0 || ne != bs.ne0 || nsmall != bs.nsmall0 || nse != bs.nse0) return fail(MNRT_ERR_STATE);
-    }
+    (void)plan_roots(g->h_base.data(), S_, g->prm.small_node_max, g->h_plan.data(), g->h_plan.data() + S_,
+                     g->h_plan.data() + 2ull * S_);
 
     g->h_photon.assign(2ull * (S_ + 1), 0u);
     if (g->kind == MNRT_KIND_POINT) {
@@ -2648,7 +2257,7 @@ extern "C" int mnrt_build_graph_create(const mnrt_build_graph_desc* d, mnrt_tree
     rc = graph_record(*g, g->dbuf, nullptr);
     if (rc != MNRT_OK) return fail(rc);
     {
-        const GraphTab T = graph_tab(g->d_tab, S_);
+        const SceneTab T = scene_tab(g->d_tab, S_);
         std::vector<float> fq(S_ + 6ull * S_, 0.0f);
         for (uint32_t s = 0; s < S_; ++s) fq[s] = g->h_qr[s];
         for (size_t i = 0; i < g->h_roots.size(); ++i) fq[S_ + i] = g->h_roots[i];
@@ -2697,39 +2306,22 @@ extern "C" int mnrt_build_graph_status(mnrt_build_graph* g, mnrt_tree* out, uint
     if (!g || !g->dbuf || !h_flags) return MNRT_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
     const uint32_t S_ = g->ns;
-    const GraphTab T = graph_tab(g->d_tab, S_);
-    std::vector<uint32_t> c(G_WORDS), tab(8ull * S_ + 2);
-    std::vector<float> box(6ull * S_);
+    const SceneTab T = scene_tab(g->d_tab, S_);
+    uint32_t err = 0;
+    std::vector<uint32_t> res(scene_result_words(S_));
     MNRT_HIP_CHECK(hipStreamSynchronize(st));
-    MNRT_HIP_CHECK(hipMemcpy(c.data(), g->counters, 4ull * G_WORDS, hipMemcpyDeviceToHost));
-    // snodes, srefs, nbase (S+1), rbase (S+1), sleaves, smaxlvl are consecutive
-    MNRT_HIP_CHECK(hipMemcpy(tab.data(), T.snodes, 4ull * (6ull * S_ + 2), hipMemcpyDeviceToHost));
-    MNRT_HIP_CHECK(hipMemcpy(box.data(), T.rootbox, 4ull * 6 * S_, hipMemcpyDeviceToHost));
-    *h_flags = c[C_ERR];
-    if (c[C_ERR] != 0u || !out) return MNRT_OK;
-    const uint32_t* hn_ = tab.data();
-    const uint32_t* hr = hn_ + S_;
-    const uint32_t* hnb = hr + S_;
+    MNRT_HIP_CHECK(hipMemcpy(&err, g->W + W_ERR, 4, hipMemcpyDeviceToHost));
+    MNRT_HIP_CHECK(hipMemcpy(res.data(), T.rootbox, 4ull * res.size(), hipMemcpyDeviceToHost));
+    *h_flags = err;
+    if (err != 0u || !out) return MNRT_OK;
+    const uint32_t* hnb = res.data() + 8ull * S_;
     const uint32_t* hrb = hnb + S_ + 1;
-    const uint32_t* hl = hrb + S_ + 1;
-    const uint32_t* hm = hl + S_;
     const uint32_t per = g->kind == MNRT_KIND_TRI ? 12u : 8u;
     const bool recs = g->kind == MNRT_KIND_TRI || (g->pow4 && g->dir4);
     for (uint32_t s = 0; s < S_; ++s) {
         mnrt_tree& t = out[s];
-        std::memset(&t, 0, sizeof(t));
-        t.kind = (uint32_t)g->kind;
-        t.num_nodes = hn_[s];
-        t.num_refs = hr[s];
-        t.num_elems = g->h_base[s + 1] - g->h_base[s];
-        t.num_leaves = hl[s];
-        t.max_level = hm[s];
-        for (int k = 0; k < 3; ++k) {
-            t.root_min[k] = box[6 * s + k];
-            t.root_max[k] = box[6 * s + 3 + k];
-        }
-        t.d_nodes = g->nodes + 2ull * hnb[s];
-        t.d_refs = g->refs + hrb[s];
+        // the arrays belong to the graph (mnrt_build_graph_destroy frees them)
+        set_tree(t, g->kind, s, S_, res.data(), g->h_base.data(), g->nodes, g->refs);
         t.d_recs = recs ? g->recs + (uint64_t)per * hrb[s] : nullptr;
         if (g->kind == MNRT_KIND_POINT && recs) {
             const uint32_t* bb = g->h_photon.data() + S_ + 1;
@@ -2737,8 +2329,6 @@ extern "C" int mnrt_build_graph_status(mnrt_build_graph* g, mnrt_tree* out, uint
             t.qleaf_max = kQueryLeafRefs;
             t.owns_qnodes = MNRT_QNODES_BOXES;
         }
-        // the arrays belong to the graph (mnrt_build_graph_destroy frees them)
-        t.owns_nodes = t.owns_recs = 0u;
     }
     return MNRT_OK;
 }

@@ -1,5 +1,5 @@
-// scan.h — device-wide exclusive prefix sum of uint32 arrays (wave64 + LDS), used by
-// the kd-tree build for stream compaction.  Replaces the CUDPP scans the reference calls
+// scan.h — device-wide exclusive prefix sum of uint32 arrays (wave64 + LDS), used for stream
+// compaction, query ordering and the public scans.  Replaces the CUDPP scans the reference calls
 // through MNCudaPrimitives::Scan (MNCudaPrimitives.cpp:160).
 #pragma once
 
@@ -76,64 +76,7 @@ __global__ void k_scan_word(uint32_t* __restrict__ dst, const uint32_t* __restri
     if (threadIdx.x == 0 && blockIdx.x == 0) *dst = src ? *src : 0u;
 }
 
-// Up to kScanSetMax independent scans of n elements each, run by the same launches
-// (blockIdx.y picks the scan).
-constexpr int kScanSetMax = 4;
-struct ScanSet {
-    const uint32_t* in[kScanSetMax];
-    uint32_t* out[kScanSetMax];
-    uint32_t* sums[kScanSetMax];
-    uint32_t* total[kScanSetMax];  // may be null
-};
-
-__global__ __launch_bounds__(kScanBlock) void k_scan_tiles_set(ScanSet S, uint32_t n) {
-    const uint32_t y = blockIdx.y;
-    __shared__ uint32_t s_wave[kScanBlock / 64];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const size_t base = (size_t)blockIdx.x * kScanTile + (size_t)tid * kScanPerThread;
-    const uint32_t* in = S.in[y];
-    uint32_t* out = S.out[y];
-    uint32_t v[kScanPerThread];
-    uint32_t local = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kScanPerThread; ++j) {
-        size_t i = base + j;
-        v[j] = (i < n) ? in[i] : 0u;
-        local += v[j];
-    }
-    uint32_t incl = wave_incl_scan(local, lane);
-    if (lane == 63) s_wave[wave] = incl;
-    __syncthreads();
-    uint32_t wave_off = 0;
-    for (uint32_t w = 0; w < wave; ++w) wave_off += s_wave[w];
-    uint32_t run = wave_off + incl - local;
-#pragma unroll
-    for (uint32_t j = 0; j < kScanPerThread; ++j) {
-        size_t i = base + j;
-        if (i < n) out[i] = run;
-        run += v[j];
-    }
-    if (tid == kScanBlock - 1) {
-        S.sums[y][blockIdx.x] = wave_off + incl;
-        if (S.total[y] && gridDim.x == 1) *S.total[y] = wave_off + incl;
-    }
-}
-
-__global__ __launch_bounds__(kScanBlock) void k_scan_add_set(ScanSet S, uint32_t n, ScanSet offs) {
-    const uint32_t y = blockIdx.y;
-    const size_t base = (size_t)blockIdx.x * kScanTile;
-    const uint32_t add = offs.out[y][blockIdx.x];
-    if (S.total[y] && blockIdx.x == 0 && threadIdx.x == 0)
-        *S.total[y] = offs.out[y][gridDim.x - 1] + S.sums[y][gridDim.x - 1];
-    uint32_t* out = S.out[y];
-    for (uint32_t j = threadIdx.x; j < kScanTile; j += kScanBlock) {
-        size_t i = base + j;
-        if (i < n) out[i] += add;
-    }
-}
-
-// Scans of more than one tile and at most kScanBig elements (the build's per-node scans)
-// run in one workgroup: each thread takes a contiguous run of at most kScanBigPer elements,
+// Scans of more than one tile and at most kScanBig elements run in one workgroup: each thread takes a contiguous run of at most kScanBigPer elements,
 // the run totals are scanned per wave and the wave totals through LDS, so such a scan is one
 // launch instead of three.  in and out may alias (a thread reads each element of its run
 // before writing it, and the runs are disjoint).
@@ -168,12 +111,6 @@ __device__ __forceinline__ uint32_t block_scan_runs(const uint32_t* in, uint32_t
 __global__ __launch_bounds__(kScanBigBlock) void k_scan_big(const uint32_t* in, uint32_t n, uint32_t* out,
                                                             uint32_t* __restrict__ total) {
     block_scan_runs(in, n, out, total);
-}
-
-// blockIdx.x picks the scan of the set
-__global__ __launch_bounds__(kScanBigBlock) void k_scan_big_set(ScanSet S, uint32_t n) {
-    const uint32_t y = blockIdx.x;
-    block_scan_runs(S.in[y], n, S.out[y], S.total[y]);
 }
 
 // Scratch words needed by scan_exclusive for n elements.
@@ -212,46 +149,13 @@ inline hipError_t scan_exclusive(const uint32_t* in, uint32_t* out, uint32_t n, 
     return hipGetLastError();
 }
 
-// m (<= kScanSetMax) independent exclusive scans of n elements: out[y][i] = sum(in[y][0..i)),
-// *total[y] (may be null) = the sum.  scratch: m * scan_scratch_words(n) device words.
-inline hipError_t scan_exclusive_set(const ScanSet& S0, int m, uint32_t n, uint32_t* scratch, hipStream_t st) {
-    if (m <= 0 || m > kScanSetMax) return hipErrorInvalidValue;
-    if (n == 0) {
-        for (int y = 0; y < m; ++y)
-            if (S0.total[y]) hipLaunchKernelGGL(k_scan_word, dim3(1), dim3(1), 0, st, S0.total[y], (const uint32_t*)nullptr);
-        return hipGetLastError();
-    }
-    if (n > kScanTile && n <= kScanBig) {
-        hipLaunchKernelGGL(k_scan_big_set, dim3(m), dim3(kScanBigBlock), 0, st, S0, n);
-        return hipGetLastError();
-    }
-    const uint32_t blocks = (n + kScanTile - 1) / kScanTile;
-    const size_t per = scan_scratch_words(n);
-    ScanSet S = S0, O{};
-    for (int y = 0; y < m; ++y) {
-        uint32_t* sc = scratch + (size_t)y * per;
-        S.sums[y] = sc;
-        O.in[y] = sc;
-        O.out[y] = sc + blocks + 1;
-        O.total[y] = nullptr;
-    }
-    hipLaunchKernelGGL(k_scan_tiles_set, dim3(blocks, m), dim3(kScanBlock), 0, st, S, n);
-    if (blocks == 1) return hipGetLastError();
-    // tile sums: one scan each, through the single-scan path (it has its own scratch)
-    for (int y = 0; y < m; ++y) {
-        hipError_t e = scan_exclusive(O.in[y], O.out[y], blocks, nullptr, scratch + (size_t)y * per + 2 * blocks + 2, st);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(k_scan_add_set, dim3(blocks, m), dim3(kScanBlock), 0, st, S, n, O);
-    return hipGetLastError();
-}
-
 // ---- scans of a device count: n = DN::get(), read by every kernel of the scan, so the
 // launches below can be recorded once and replayed on other sizes (up to the capacity n.v).
 // A capacity of at most kScanBig is scanned by one workgroup per scan (one launch);
 // larger ones reduce each 2048-element tile to its total (tiles_cap words per scan), then
 // scan each tile from the sum of the totals before it (two launches; blocks stride over the
 // tiles and carry that sum from one of their tiles to the next).
+constexpr int kScanSetMax = 4;
 struct DScanSet {
     const uint32_t* in[kScanSetMax];
     uint32_t* out[kScanSetMax];
@@ -373,17 +277,6 @@ inline hipError_t dscan(const DScanSet& S0, int m, DN n, uint32_t* scratch, hipS
     hipLaunchKernelGGL(k_dscan_reduce, dim3(grid, m), dim3(kScanBlock), 0, st, S, n);
     hipLaunchKernelGGL(k_dscan_scan, dim3(grid, m), dim3(kScanBlock), 0, st, S, n);
     return hipGetLastError();
-}
-
-// One device-count scan (see dscan).
-inline hipError_t dscan1(const uint32_t* in, uint32_t* out, DN n, uint32_t* total, bool end_total,
-                         uint32_t* scratch, hipStream_t st) {
-    DScanSet S{};
-    S.in[0] = in;
-    S.out[0] = out;
-    S.total[0] = total;
-    S.end_total = end_total ? 1u : 0u;
-    return dscan(S, 1, n, scratch, st);
 }
 
 }  // namespace
