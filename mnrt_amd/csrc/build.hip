@@ -39,32 +39,39 @@ namespace mnrt {
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 
 enum : uint32_t { BN_LEAF = 3, BN_SMALL = 4, BN_PENDING = 5 };
-// Build-node table: one entry per node of the large-stage tree (inner nodes, empty
-// and capped leaves, small roots), 10 uint32 columns of `cap` entries.  Build nodes
-// 0..S-1 are the roots of the S scenes built together.
-constexpr int kBnCols = 10;
-struct BnView {
-    uint32_t* type;   // 0..2 inner split axis, BN_LEAF, BN_SMALL, BN_PENDING
-    uint32_t* split;  // split position bits (inner)
-    uint32_t* left;
-    uint32_t* right;
-    uint32_t* level;
-    uint32_t* aux;  // small-root index (BN_SMALL) or first copied element (BN_LEAF)
-    uint32_t* cnt;  // element count (BN_LEAF)
-    uint32_t* scene;
-    uint32_t* parent;  // kNone for a root
-    uint32_t* flag;    // children whose subtree sizes are known (k_layout_sizes)
+// Build nodes: one 64-byte record (a cache line) per node of the large-stage tree (inner nodes,
+// empty and capped leaves, small roots), written and read as quads.  Build nodes 0..S-1 are the
+// roots of the S scenes built together.
+struct alignas(64) BnRec {
+    uint32_t type;   // 0..2 inner split axis, BN_LEAF, BN_SMALL, BN_PENDING
+    uint32_t split;  // split position bits (inner)
+    uint32_t left, right;
+    uint32_t level;
+    uint32_t aux;  // small-root index (BN_SMALL) or first copied element (BN_LEAF)
+    uint32_t cnt;  // element count (BN_LEAF)
+    uint32_t scene;
+    uint32_t parent;  // kNone for a root; kCutParent | node below an empty-space cut
+    uint32_t pad;
+    uint32_t size, rsize;  // nodes and references in the subtree
+    unsigned long long acc;  // what the children that have arrived brought (k_layout_sizes)
+    uint32_t addr, rbase;  // small roots: subtree start in the scene's tree
 };
+static_assert(sizeof(BnRec) == 64, "one line");
+constexpr uint32_t kCutParent = 0x80000000u;
 
-struct SmallView {  // small roots
-    uint32_t* first;
-    uint32_t* cnt;
-    uint32_t* level;
-    uint32_t* bn;
-    float4* lo;
-    float4* hi;
-    uint32_t* scene;
+struct alignas(16) SmallRec {  // small roots
+    uint32_t first, cnt, level, bn;
+    float lo[3];
+    uint32_t scene;
+    float hi[3];
+    uint32_t pad;
 };
+static_assert(sizeof(SmallRec) == 48, "three quads");
+
+// Writes quad q of a record.
+__device__ __forceinline__ void put4(void* rec, uint32_t q, uint32_t x, uint32_t y, uint32_t z, uint32_t w) {
+    ((uint4*)rec)[q] = make_uint4(x, y, z, w);
+}
 
 // Concatenated input of S scenes: element e of scene s is entry base[s] + e; element
 // indices inside a build are scene-local, as a single-scene build would number them.
@@ -126,6 +133,11 @@ __device__ __forceinline__ void classify(int kind, uint32_t idx, const float4& l
     }
 }
 
+// Triangles that go to both children (and are clipped there).
+__device__ __forceinline__ bool straddles(int kind, const float4& lo, const float4& hi, uint32_t axis, float s) {
+    return kind == MNRT_KIND_TRI && f4c(lo, axis) < s && s < f4c(hi, axis);
+}
+
 // ---- split clipping (dev_ClipSegment / dev_ClipTriToBounds, kdtree_tri.cu:190-316) ----
 
 // Vertex lists of the clipping in LDS (a per-lane array indexed by the running vertex
@@ -137,17 +149,15 @@ constexpr int kClipVerts = 12;  // a triangle clipped by six planes has at most 
 
 struct ClipLists {
     __attribute__((address_space(3))) float* col;  // this lane's column
-    int n[2];
-    __device__ __forceinline__ float get(int l, int v, int c) const {
-        return col[((l * kClipVerts + v) * 3 + c) * kClipBlock];
-    }
-    __device__ __forceinline__ f3 vert(int l, int v) const { return mk3(get(l, v, 0), get(l, v, 1), get(l, v, 2)); }
-    __device__ __forceinline__ void push(int l, f3 p) {
-        const int v = n[l]++;
+    int list, n;                                   // current list, its vertices
+    __device__ __forceinline__ int at(int l, int v, int c) const { return ((l * kClipVerts + v) * 3 + c) * kClipBlock; }
+    __device__ __forceinline__ float get(int v, int c) const { return col[at(list, v, c)]; }
+    __device__ __forceinline__ f3 vert(int v) const { return mk3(get(v, 0), get(v, 1), get(v, 2)); }
+    __device__ __forceinline__ void put(int l, int v, f3 p) {
         if (v >= kClipVerts) return;  // (cannot happen: at most 9 vertices)
-        col[((l * kClipVerts + v) * 3 + 0) * kClipBlock] = p.x;
-        col[((l * kClipVerts + v) * 3 + 1) * kClipBlock] = p.y;
-        col[((l * kClipVerts + v) * 3 + 2) * kClipBlock] = p.z;
+        col[at(l, v, 0)] = p.x;
+        col[at(l, v, 1)] = p.y;
+        col[at(l, v, 2)] = p.z;
     }
 };
 
@@ -158,24 +168,38 @@ __device__ __forceinline__ void f3set(f3& v, int a, float x) {
     else v.z = x;
 }
 
-// Sutherland-Hodgman step: list `in` clipped by the plane x[axis] = val, keeping the side
-// where (x[axis] - val) * sense >= 0, into list `out`.
-__device__ void clip_segments(ClipLists& L, int in, int axis, float val, float sense, int out) {
-    L.n[out] = 0;
-    const int n = min(L.n[in], kClipVerts);
+// Sutherland-Hodgman step: the list clipped by the plane x[axis] = val, keeping the side
+// where (x[axis] - val) * sense >= 0, into the lane's other list.  A list that lies on that side
+// stays as it is: most planes cut few of a wave's triangles, and a step without a cut costs its
+// test only (k_clip in the 1.03M-triangle build, 26 levels: 527 -> 412 us, with the vertex loads a
+// step ahead and the node's words in the job).
+template <int axis>
+__device__ __forceinline__ void clip_segments(ClipLists& L, float val, float sense) {
+    const int n = min(L.n, kClipVerts);
+    bool out = false;
+    for (int i = 0; i < n; ++i) out |= !((L.get(i, axis) - val) * sense >= 0.0f);
+    if (!out) return;
+    const f3 first = L.vert(0);
+    f3 a = first, next = L.vert(min(1, n - 1));
+    bool ins = (f3c(a, axis) - val) * sense >= 0.0f;
+    const int to = L.list ^ 1;
+    int m = 0;
     for (int i = 0; i < n; ++i) {
-        f3 a = L.vert(in, i);
-        f3 b = L.vert(in, (i + 1 == n) ? 0 : i + 1);
-        bool ins = (f3c(a, axis) - val) * sense >= 0.0f;
-        bool ine = (f3c(b, axis) - val) * sense >= 0.0f;
+        const f3 b = (i + 1 == n) ? first : next;
+        next = L.vert(min(i + 2, n - 1));
+        const bool ine = (f3c(b, axis) - val) * sense >= 0.0f;
         if (ins != ine) {
             float t = (val - f3c(a, axis)) / (f3c(b, axis) - f3c(a, axis));
             f3 h = mk3(a.x + t * (b.x - a.x), a.y + t * (b.y - a.y), a.z + t * (b.z - a.z));
             f3set(h, axis, val);
-            L.push(out, h);
+            L.put(to, m++, h);
         }
-        if (ine) L.push(out, b);
+        if (ine) L.put(to, m++, b);
+        a = b;
+        ins = ine;
     }
+    L.list = to;
+    L.n = m;
 }
 
 // Clipped bounds of a straddling triangle inside a child box, padded outward by 2^-20 of
@@ -185,17 +209,25 @@ __device__ void clip_bounds(const Geometry& G, uint32_t idx, float4& lo, float4&
                             const float4& bmax, __attribute__((address_space(3))) float* col) {
     ClipLists L;
     L.col = col;
-    L.n[0] = L.n[1] = 0;
-    L.push(0, xyz(G.v0[idx]));
-    L.push(0, xyz(G.v1[idx]));
-    L.push(0, xyz(G.v2[idx]));
-    for (int ax = 0; ax < 3; ++ax) {
-        if (f4c(lo, ax) != f4c(hi, ax)) {
-            clip_segments(L, 0, ax, f4c(bmin, ax), 1.0f, 1);
-            clip_segments(L, 1, ax, f4c(bmax, ax), -1.0f, 0);
-        }
+    L.list = 0;
+    L.n = 3;
+    const float4 v0 = G.v0[idx], v1 = G.v1[idx], v2 = G.v2[idx];
+    L.put(0, 0, xyz(v0));
+    L.put(0, 1, xyz(v1));
+    L.put(0, 2, xyz(v2));
+    if (lo.x != hi.x) {
+        clip_segments<0>(L, bmin.x, 1.0f);
+        clip_segments<0>(L, bmax.x, -1.0f);
     }
-    const int na = min(L.n[0], kClipVerts);
+    if (lo.y != hi.y) {
+        clip_segments<1>(L, bmin.y, 1.0f);
+        clip_segments<1>(L, bmax.y, -1.0f);
+    }
+    if (lo.z != hi.z) {
+        clip_segments<2>(L, bmin.z, 1.0f);
+        clip_segments<2>(L, bmax.z, -1.0f);
+    }
+    const int na = min(L.n, kClipVerts);
     for (int ax = 0; ax < 3; ++ax) {
         float l, h;
         float bl = f4c(bmin, ax), bh = f4c(bmax, ax);
@@ -206,8 +238,8 @@ __device__ void clip_bounds(const Geometry& G, uint32_t idx, float4& lo, float4&
             l = kInf;
             h = -kInf;
             for (int i = 0; i < na; ++i) {
-                l = fminf(L.get(0, i, ax), l);
-                h = fmaxf(L.get(0, i, ax), h);
+                l = fminf(L.get(i, ax), l);
+                h = fmaxf(L.get(i, ax), h);
             }
             float m = fmaxf(fmaxf(fabsf(l), fabsf(h)), fmaxf(fabsf(bl), fabsf(bh)));
             float pad = m * (1.0f / 1048576.0f);
@@ -227,12 +259,13 @@ __device__ void clip_bounds(const Geometry& G, uint32_t idx, float4& lo, float4&
 // ---------------------------------------------------------------------------------------
 // Elements of an active node fill consecutive slots from a multiple of 64 on, so every wave of
 // 64 slots belongs to one node: its values are wave-uniform, and a stable partition needs a
-// prefix sum over waves (one packed word each), not over elements.  A level is four launches
+// prefix sum over waves (one packed word each), not over elements.  The element record is its
+// lower bound with the index in .w and, for triangles, the upper bound.  A level is four launches
 // (three for points):
-//   k_count     classifies every element, one packed (left, right) count per wave;
-//   k_children  per node: prefix of its waves' counts, the children's places and build nodes;
-//   k_scatter   classifies again, writes every element into its children and accumulates the
-//               tight bounds of the next level's nodes;
+//   k_count     classifies every element, one packed count per wave, summed per chunk of 64 waves;
+//   k_children  per node: prefix of its chunks' sums, the children's places and build nodes;
+//   k_scatter   classifies again, writes every element into its children (a wave sums the counts
+//               of its chunk before it) and accumulates the next level's tight bounds;
 //   k_clip      bounds of straddling triangles, from a queue.
 // Places are handed out by atomics, aggregated per workgroup, so nodes and small roots lie in an
 // arbitrary order (the tree does not depend on it: a node's elements keep theirs, and the final
@@ -240,8 +273,8 @@ __device__ void clip_bounds(const Geometry& G, uint32_t idx, float4& lo, float4&
 // (nodes, waves) from the level table, an empty level returns at once, and whatever would
 // outgrow a buffer sets kErrRoom instead, after which every later kernel returns.
 // Measured against one launch per step over chunk lists, element flags and three-pass scans (16
-// launches a level and a host synchronisation): 1.03M triangles 5.5 -> 3.2 ms, 1M photons 3.6 ->
-// 1.5 ms, 3001 triangles 1.28 -> 0.61 ms, 32 scenes' triangle and photon trees recorded 4.0 -> 2.0
+// launches a level and a host synchronisation): 1.03M triangles 5.6 -> 2.6 ms, 1M photons 3.5 ->
+// 1.3 ms, 3001 triangles 1.34 -> 0.53 ms, 32 scenes' triangle and photon trees recorded 4.0 -> 1.75
 // ms.
 
 // Device words of a build: totals, then the level table.
@@ -249,11 +282,11 @@ enum : uint32_t {
     W_ERR = 0,
     W_MAXLEVEL,    // deepest build node
     W_SMALL_OVF,   // small roots whose subtree outgrew its staging area
-    W_NBN,         // build nodes
-    W_LL,          // elements of large-stage leaves
+    W_NBN = 4,     // build nodes, elements of large-stage leaves: one 64-bit word
+    W_LL = 5,
     W_NSE = 6,     // small-root elements, small roots: one 64-bit word
     W_NSMALL = 7,
-    W_LEVELS = 8,  // per level: waves, nodes (one 64-bit word), clip jobs, 0
+    W_LEVELS = 8,  // per level: waves, nodes (one 64-bit word), clip jobs, 0 (another)
 };
 constexpr uint32_t kLevels = MNRT_MAX_LEVEL + 2;  // every level's nodes are deeper than the last's
 constexpr uint32_t kWords = W_LEVELS + 4 * (kLevels + 1);
@@ -272,35 +305,39 @@ struct BuildCaps {
     uint32_t ll;     // elements of large-stage leaves
 };
 
-// Active nodes of a level.  tb: tight bounds, 6 words per node, the minima of fenc(lo) and of
-// ~fenc(hi).
-struct NodeView {
-    float4* lo;
-    float4* hi;
-    uint32_t* first;
-    uint32_t* cnt;
-    uint32_t* level;
-    uint32_t* bn;
-    uint32_t* scene;
-    uint32_t* tb;
+// An active node: 18 of 32 words, which a wave loads at once, a word per lane.  tb: tight bounds,
+// the minima of fenc(lo) and of ~fenc(hi).
+struct alignas(128) NodeRec {
+    float lo[3], hi[3];
+    uint32_t first, cnt, level, bn, scene;
+    uint32_t base;  // of the scene's elements in the input
+    uint32_t tb[6];
+    uint32_t pad[14];
 };
+static_assert(sizeof(NodeRec) == 128, "one line");
+enum : uint32_t { ND_LO = 0, ND_HI = 3, ND_FIRST = 6, ND_CNT, ND_LEVEL, ND_BN, ND_SCENE, ND_BASE, ND_TB = 12, ND_WORDS = 18 };
 
-struct ElemView {  // element arrays: original index, bounds; wnode: active node of every wave
-    uint32_t* idx;
+// Element arrays: lower bound and original index (.w), upper bound; wnode: active node of every
+// wave.
+struct ElemView {
     float4* lo;
     float4* hi;
     uint32_t* wnode;
 };
 
-// What k_children decided about a node.
+// What k_children decided about a node: child 0 and 1 as CH_*, first destination (CH_LEAF: first
+// copied element) and next-level node, and the box after the empty-space cuts.
 enum : uint32_t { CH_DEAD = 0, CH_SMALL, CH_LARGE, CH_LEAF };
-struct SplitView {
-    float4* lo;      // box after the empty-space cuts
-    float4* hi;
-    uint32_t* axis;
-    float* split;
-    uint4* child;    // 2 per node: CH_*, first destination (CH_LEAF: first copied element), next-level node
+struct alignas(64) SplitRec {
+    uint32_t axis;
+    float split;
+    uint32_t type[2], at[2], to[2];
+    float lo[3];
+    uint32_t base;  // of the scene's elements in the input
+    float hi[3];
+    uint32_t job;  // first clip job
 };
+static_assert(sizeof(SplitRec) == 64, "one line");
 
 // Everything the level kernels work on.
 struct LevelArgs {
@@ -309,16 +346,27 @@ struct LevelArgs {
     BuildCaps cap;
     float ratio;
     uint32_t small_max;
-    NodeView A, An;
+    NodeRec *A, *An;
     ElemView E, Nx, Sm;
-    uint32_t* wc;   // per wave: left count | right count << 16
-    uint2* woff;    // per wave: elements of its node before it, left and right
-    SplitView P;
-    SmallView S;
-    BnView B;
+    uint32_t* wc;  // per wave: left, right and straddling counts, a byte each
+    unsigned long long *cs, *csn;  // sums per chunk (chunk_of) of this level and the next
+    uint4* coff;   // per chunk: elements of its node before it, left and right; its first clip job
+    SplitRec* P;
+    SmallRec* S;
+    BnRec* B;
     uint32_t* ll_idx;
-    uint2* q;       // clip jobs (two per slot at most): slot << 1 | side, destination
+    uint4* q;      // clip jobs, one per straddling element: slot, destinations left and right, node
 };
+
+// Chunks: 64 consecutive waves of a node, counted from its first.  Nodes and their waves are handed
+// out together, so a later node's waves come later, and chunk w0 / 64 + p on belong to node p alone.
+__host__ __device__ inline uint64_t chunks_for(uint64_t nw, uint64_t na) { return nw / 64u + na + 1u; }
+__device__ __forceinline__ uint32_t chunk_of(uint32_t p, uint32_t w0, uint32_t w) { return (w0 >> 6) + p + ((w - w0) >> 6); }
+// A chunk's sums: left, right and straddling counts (at most 4096 each).
+constexpr uint32_t kSumBits = 21u;
+__device__ __forceinline__ uint32_t sum_part(unsigned long long v, uint32_t k) {
+    return (uint32_t)(v >> (kSumBits * k)) & ((1u << kSumBits) - 1u);
+}
 
 __device__ __forceinline__ uint32_t level_waves(const LevelArgs& L) {
     return L.W[W_ERR] != 0u ? 0u : min(L.W[W_LEVELS + 4 * L.level], L.cap.nw);
@@ -330,39 +378,49 @@ __device__ __forceinline__ uint32_t level_nodes(const LevelArgs& L) {
 // Empty-space cuts then the spatial median split (kernel_CanCutOffEmptySpace,
 // kernel_EmptySpaceCutting, kernel_SplitLargeNodes; kdtree.cu:467-682).  Sides are cut in
 // the reference's order (min x, y, z, then max x, y, z); each cut turns the node into an
-// inner node with an empty leaf and a tighter copy (on_cut).  The median splits the longest axis
+// inner node with an empty leaf and a tighter copy.  The median splits the longest axis
 // of the cut box, ties to the lower axis.
 struct Plan {
-    float lo[3], hi[3];
+    float lo[3], hi[3];  // the box after the cuts
+    float tight[6];
+    uint32_t cuts;   // sides that are cut, one bit each
     uint32_t level;  // of the node that is split
-    uint32_t ncuts;
     uint32_t axis;
     float split;
     bool leaf;  // level cap reached: the node is a leaf with its elements
 };
 
-template <typename F>
-__device__ __forceinline__ Plan plan_node(const NodeView& A, uint32_t p, float ratio, F&& on_cut) {
+// w: this lane's word of the node record.  Whole wave; the result is uniform.
+__device__ __forceinline__ uint32_t rec_word(uint32_t w, uint32_t i) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)w, (int)i);
+}
+__device__ __forceinline__ uint32_t load_rec(const NodeRec* A, uint32_t p, uint32_t lane) {
+    return ((const uint32_t*)(A + p))[min(lane, (uint32_t)ND_WORDS - 1u)];
+}
+
+__device__ __forceinline__ Plan plan_node(uint32_t w, float ratio) {
     Plan R;
-    const float4 l4 = A.lo[p], h4 = A.hi[p];
-    R.lo[0] = l4.x; R.lo[1] = l4.y; R.lo[2] = l4.z;
-    R.hi[0] = h4.x; R.hi[1] = h4.y; R.hi[2] = h4.z;
-    R.level = A.level[p];
-    R.ncuts = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        R.lo[k] = __uint_as_float(rec_word(w, ND_LO + k));
+        R.hi[k] = __uint_as_float(rec_word(w, ND_HI + k));
+    }
+    R.level = rec_word(w, ND_LEVEL);
+    R.cuts = 0;
 #pragma unroll
     for (int side = 0; side < 6; ++side) {
         const int ax = side % 3;
         const bool is_max = side >= 3;
+        const uint32_t t = rec_word(w, ND_TB + side);
+        R.tight[side] = fdec(is_max ? ~t : t);
         if (R.level >= MNRT_MAX_LEVEL) continue;
-        const float tight = is_max ? fdec(~A.tb[6 * p + side]) : fdec(A.tb[6 * p + side]);
         const float total = R.hi[ax] - R.lo[ax];
-        const float empty = is_max ? R.hi[ax] - tight : tight - R.lo[ax];
+        const float empty = is_max ? R.hi[ax] - R.tight[side] : R.tight[side] - R.lo[ax];
         if (!(empty > total * ratio)) continue;
-        on_cut(ax, is_max, tight, R.level, R.ncuts);
-        ++R.ncuts;
+        R.cuts |= 1u << side;
         ++R.level;
-        if (is_max) R.hi[ax] = tight;
-        else R.lo[ax] = tight;
+        if (is_max) R.hi[ax] = R.tight[side];
+        else R.lo[ax] = R.tight[side];
     }
     R.leaf = R.level >= MNRT_MAX_LEVEL;
     const float ex = R.hi[0] - R.lo[0], ey = R.hi[1] - R.lo[1], ez = R.hi[2] - R.lo[2];
@@ -371,18 +429,26 @@ __device__ __forceinline__ Plan plan_node(const NodeView& A, uint32_t p, float r
     if (ey > emax) { R.axis = 1; emax = ey; lo = R.lo[1]; hi = R.hi[1]; }
     if (ez > emax) { R.axis = 2; lo = R.lo[2]; hi = R.hi[2]; }
     R.split = lo + 0.5f * (hi - lo);
+    R.axis = uniform(R.axis);
+    R.cuts = uniform(R.cuts);
+    R.level = uniform(R.level);
     return R;
 }
 
 // Clears a build's words and sets its first level (na nodes in nw waves), small roots and build
-// nodes; the scenes' tight bounds start empty.
+// nodes; the scenes' tight bounds start empty, their deepest levels and the first level's chunk sums
+// at 0.
 __global__ __launch_bounds__(256) void k_build_init(uint32_t* __restrict__ W, uint32_t na, uint32_t nw, uint32_t nsmall,
-                                                    uint32_t nse, uint32_t nscenes, uint32_t* __restrict__ stb) {
+                                                    uint32_t nse, uint32_t nscenes, uint32_t* __restrict__ stb,
+                                                    uint32_t* __restrict__ maxlvl,
+                                                    unsigned long long* __restrict__ cs) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < kWords)
         W[i] = i == W_NBN ? nscenes : i == W_NSE ? nse : i == W_NSMALL ? nsmall : i == W_LEVELS ? nw
                : i == W_LEVELS + 1 ? na : 0u;
     for (uint32_t j = i; j < 6 * nscenes; j += gridDim.x * blockDim.x) stb[j] = 0xFFFFFFFFu;
+    for (uint32_t j = i; j < nscenes; j += gridDim.x * blockDim.x) maxlvl[j] = 0u;
+    for (uint32_t j = i; j < chunks_for(nw, na); j += gridDim.x * blockDim.x) cs[j] = 0ull;
 }
 
 // Per-scene placement decided on the host: an active (large) root or a small root, its index in
@@ -402,10 +468,10 @@ __device__ __forceinline__ void tight_words(const float4& lo, const float4& hi, 
     v[5] = ~fenc(hi.z);
 }
 
-// Adds the lanes' tight words to their targets tb[6 * to ..] (kNone: none), lanes that share a
-// target reduced first: one atomic per component and distinct target.  Whole wave.
+// Adds the lanes' tight words to their targets tb[stride * to ..] (kNone: none), lanes that share
+// a target reduced first: one atomic per component and distinct target.  Whole wave.
 __device__ __forceinline__ void tight_by_key(uint32_t to, const uint32_t (&v)[6], uint32_t* __restrict__ tb,
-                                             uint32_t lane) {
+                                             uint32_t stride, uint32_t lane) {
     for (uint64_t m = ballot(to != kNone); m != 0ull;) {
         const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)to, (int)__builtin_ctzll(m));
         const bool mine = to == t;
@@ -415,7 +481,7 @@ __device__ __forceinline__ void tight_by_key(uint32_t to, const uint32_t (&v)[6]
             const uint32_t r = wave_min_u32(mine ? v[k] : ~0u);
             if (lane == k) best = r;
         }
-        if (lane < 6u) atomicMin(&tb[6u * t + lane], best);
+        if (lane < 6u) atomicMin(&tb[(size_t)stride * t + lane], best);
         m &= ~ballot(mine);
     }
 }
@@ -453,8 +519,7 @@ __global__ __launch_bounds__(kInitBlock) void k_init_elems(Geometry G, uint32_t 
             const uint32_t local = i - G.base[s], d = R.off[s] + local;
             const bool small = R.kind[s] != 0u;
             const ElemView& D = small ? Sm : E;
-            D.idx[d] = local;
-            D.lo[d] = lo;
+            D.lo[d] = make_float4(lo.x, lo.y, lo.z, __uint_as_float(local));
             if (G.kind == MNRT_KIND_TRI) D.hi[d] = hi;
             if (!small && (d & 63u) == 0u) E.wnode[d >> 6] = R.index[s];
             tight_words(lo, hi, v);
@@ -463,7 +528,7 @@ __global__ __launch_bounds__(kInitBlock) void k_init_elems(Geometry G, uint32_t 
 #pragma unroll
             for (int k = 0; k < 6; ++k) acc[k] = min(acc[k], v[k]);
         } else {
-            tight_by_key(s, v, stb, lane);
+            tight_by_key(s, v, stb, 6u, lane);
         }
     }
     if (!one) return;  // uniform per workgroup
@@ -483,7 +548,7 @@ __global__ __launch_bounds__(kInitBlock) void k_init_elems(Geometry G, uint32_t 
 // empty scene) and the root entries of the active / small lists.
 __global__ __launch_bounds__(256) void k_roots_setup(uint32_t nscenes, const uint32_t* __restrict__ base,
                                                      const uint32_t* __restrict__ stb, const float* __restrict__ given,
-                                                     RootPlan R, NodeView A, SmallView S, BnView B,
+                                                     RootPlan R, NodeRec* A, SmallRec* S, BnRec* B,
                                                      float* __restrict__ out_box) {
     uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nscenes) return;
@@ -499,31 +564,27 @@ __global__ __launch_bounds__(256) void k_roots_setup(uint32_t nscenes, const uin
         lo = make_float4(fdec(stb[6 * s]), fdec(stb[6 * s + 1]), fdec(stb[6 * s + 2]), 0.0f);
         hi = make_float4(fdec(~stb[6 * s + 3]), fdec(~stb[6 * s + 4]), fdec(~stb[6 * s + 5]), 0.0f);
     }
-    B.level[s] = 0;
-    B.scene[s] = s;
-    B.parent[s] = kNone;
-    B.flag[s] = 0u;
     const uint32_t i = R.index[s];
-    if (R.kind[s] == 0) {
-        A.lo[i] = lo;
-        A.hi[i] = hi;
-        A.first[i] = R.off[s];
-        A.cnt[i] = cnt;
-        A.level[i] = 0;
-        A.bn[i] = s;
-        A.scene[i] = s;
-        for (int k = 0; k < 6; ++k) A.tb[6 * i + k] = stb[6 * s + k];
-        B.type[s] = BN_PENDING;
+    const bool small = R.kind[s] != 0u;
+    put4(&B[s], 0, small ? BN_SMALL : BN_PENDING, 0u, 0u, 0u);
+    put4(&B[s], 1, 0u, i, 0u, s);
+    put4(&B[s], 2, kNone, 0u, 0u, 0u);
+    put4(&B[s], 3, 0u, 0u, 0u, 0u);
+    if (!small) {
+        NodeRec& a = A[i];
+        a.lo[0] = lo.x; a.lo[1] = lo.y; a.lo[2] = lo.z;
+        a.hi[0] = hi.x; a.hi[1] = hi.y; a.hi[2] = hi.z;
+        a.first = R.off[s];
+        a.cnt = cnt;
+        a.level = 0;
+        a.bn = s;
+        a.scene = s;
+        a.base = base[s];
+        for (int k = 0; k < 6; ++k) a.tb[k] = stb[6 * s + k];
     } else {
-        S.first[i] = R.off[s];
-        S.cnt[i] = cnt;
-        S.level[i] = 0;
-        S.bn[i] = s;
-        S.lo[i] = lo;
-        S.hi[i] = hi;
-        S.scene[i] = s;
-        B.type[s] = BN_SMALL;
-        B.aux[s] = i;
+        put4(&S[i], 0, R.off[s], cnt, 0u, s);
+        put4(&S[i], 1, __float_as_uint(lo.x), __float_as_uint(lo.y), __float_as_uint(lo.z), s);
+        put4(&S[i], 2, __float_as_uint(hi.x), __float_as_uint(hi.y), __float_as_uint(hi.z), 0u);
     }
     out_box[6 * s + 0] = lo.x;
     out_box[6 * s + 1] = lo.y;
@@ -533,35 +594,63 @@ __global__ __launch_bounds__(256) void k_roots_setup(uint32_t nscenes, const uin
     out_box[6 * s + 5] = hi.z;
 }
 
-// Left and right counts of every wave.  The wave makes its node's plan itself (about 100
-// instructions on values it shares, less than another launch and its latency).
+// Left, right and straddling counts of every wave, and their sums per chunk.  Bound by reading the elements (33 MB a
+// level at 1.03M triangles: 10-12 us).  The wave makes its node's plan itself: about 100 instructions on
+// values it shares, less than another launch and its latency.
+constexpr uint32_t kCountBlock = 1024, kCountWaves = kCountBlock / 64;
+
 template <int kKind>
-__global__ __launch_bounds__(256) void k_count(LevelArgs L) {
-    const uint32_t nw = level_waves(L), lane = threadIdx.x & 63u;
-    for (uint32_t w = uniform(blockIdx.x * 4u + (threadIdx.x >> 6)); w < nw; w += gridDim.x * 4u) {
-        const uint32_t p = uniform(L.E.wnode[w]), e = 64u * w + lane;
-        const float4 lo = L.E.lo[e];  // (slots past the node's last element hold anything)
-        const float4 hi = (kKind == MNRT_KIND_TRI) ? L.E.hi[e] : lo;
-        const uint32_t idx = L.E.idx[e];
-        const Plan R = plan_node(L.A, p, L.ratio, [](int, bool, float, uint32_t, uint32_t) {});
-        bool l = false, r = false;
-        if (!R.leaf && e - L.A.first[p] < L.A.cnt[p]) classify(kKind, idx, lo, hi, R.axis, R.split, l, r);
-        const uint32_t c = (uint32_t)__popcll(ballot(l)) | (uint32_t)__popcll(ballot(r)) << 16;
-        if (lane == 0) L.wc[w] = c;
+__global__ __launch_bounds__(kCountBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_count(LevelArgs L) {
+    // two sets, used in turn: one barrier a step
+    __shared__ unsigned long long s_sum[2][kCountWaves];
+    __shared__ uint32_t s_chunk[2][kCountWaves];
+    const uint32_t nw = level_waves(L), lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
+    uint32_t set = 0;
+    for (uint32_t w0 = blockIdx.x * kCountWaves; w0 < nw; w0 += gridDim.x * kCountWaves) {  // uniform per workgroup
+        const uint32_t w = w0 + wave;
+        uint32_t c = 0, chunk = kNone;
+        if (w < nw) {
+            const uint32_t p = uniform(L.E.wnode[w]), e = 64u * w + lane;
+            const float4 lo = L.E.lo[e];  // (slots past the node's last element hold anything)
+            const float4 hi = (kKind == MNRT_KIND_TRI) ? L.E.hi[e] : lo;
+            const uint32_t nd = load_rec(L.A, p, lane);
+            const Plan R = plan_node(nd, L.ratio);
+            bool l = false, r = false, both = false;
+            if (!R.leaf && e - rec_word(nd, ND_FIRST) < rec_word(nd, ND_CNT)) {
+                classify(kKind, __float_as_uint(lo.w), lo, hi, R.axis, R.split, l, r);
+                both = straddles(kKind, lo, hi, R.axis, R.split);
+            }
+            c = (uint32_t)__popcll(ballot(l)) | (uint32_t)__popcll(ballot(r)) << 8 | (uint32_t)__popcll(ballot(both)) << 16;
+            chunk = chunk_of(p, rec_word(nd, ND_FIRST) >> 6, w);
+            if (lane == 0) L.wc[w] = c;
+        }
+        if (lane == 0) {
+            s_chunk[set][wave] = chunk;
+            s_sum[set][wave] = (unsigned long long)(c & 0xFFu) | (unsigned long long)(c >> 8 & 0xFFu) << kSumBits |
+                               (unsigned long long)(c >> 16) << (2u * kSumBits);
+        }
+        __syncthreads();
+        if (threadIdx.x < kCountWaves) {  // one atomic per run of waves of one chunk
+            const uint32_t i = threadIdx.x, ch = s_chunk[set][i];
+            if (ch != kNone && (i == 0u || s_chunk[set][i - 1u] != ch)) {
+                unsigned long long v = s_sum[set][i];
+                for (uint32_t j = i + 1u; j < kCountWaves && s_chunk[set][j] == ch; ++j) v += s_sum[set][j];
+                atomicAdd(&L.cs[ch], v);
+            }
+        }
+        set ^= 1u;
     }
 }
 
-// Children of 16 nodes per workgroup step, one wave per node (512 of its waves' counts per
-// pass: the root of a million elements takes 32 passes, about 20 us, nodes below 32768
-// elements one).  The places of the 16 nodes' children come from one atomic per quantity.
+// Children of 16 nodes per workgroup step, one wave per node.  Bound by latency: the node's
+// record, its chunk sums, one atomic for the places of the 16 nodes' children (a lane per 64-bit
+// total) and the records, written by a lane each, every record a line or part of one.  With
+// column arrays, a field per store, a serial sum over the 16 nodes and one lane writing, and each
+// node's sum over all its waves (16 k for the root), the 26 levels of 1.03M triangles took 493 us
+// (35 at the root, 14 between); now 248 (6.5 and 9).
 constexpr uint32_t kChildBlock = 1024, kChildNodes = kChildBlock / 64;
-
-struct ChildNeed {  // what a node asks for
-    uint32_t bn, na, nw, nsmall, nse, ll;
-};
-
-__global__ __launch_bounds__(kChildBlock) void k_children(LevelArgs L) {
-    __shared__ ChildNeed s_need[kChildNodes], s_base;
+__global__ __launch_bounds__(kChildBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_children(LevelArgs L) {
+    __shared__ uint32_t s_need[kChildNodes][8], s_base[kChildNodes][8];
     __shared__ uint32_t s_na;  // one read for the workgroup: others may set the error while it runs
     if (threadIdx.x == 0) s_na = level_nodes(L);
     __syncthreads();
@@ -570,172 +659,159 @@ __global__ __launch_bounds__(kChildBlock) void k_children(LevelArgs L) {
         const uint32_t p = p0 + wave;
         const bool live = p < na;
         Plan R{};
-        uint32_t m = 0, n[2] = {0u, 0u};
-        ChildNeed need{};
+        uint32_t nd = 0, n[2] = {0u, 0u}, nq = 0;
         uint32_t type[2] = {CH_DEAD, CH_DEAD};
+        bool leaf = false;
+        uint32_t m = 0;
+        // what the node asks for, lane by lane: build nodes, leaf elements, small elements and
+        // roots, next-level waves and nodes, clip jobs, 0
+        uint32_t need = 0;
         if (live) {
-            R = plan_node(L.A, p, L.ratio, [](int, bool, float, uint32_t, uint32_t) {});
-            m = L.A.cnt[p];
-            const uint32_t w0 = L.A.first[p] >> 6, nwv = (m + 63u) >> 6;
-            for (uint32_t b = 0; b < nwv; b += 512u) {
-                uint32_t c[8], sum = 0;
+            nd = load_rec(L.A, p, lane);
+            m = rec_word(nd, ND_CNT);
+            // the chunks' offsets
+            const uint32_t c0 = chunk_of(p, rec_word(nd, ND_FIRST) >> 6, rec_word(nd, ND_FIRST) >> 6), nc = (m + 4095u) >> 12;
+            unsigned long long c = lane < nc ? L.cs[c0 + lane] : 0ull;
+            for (uint32_t b = 0; b < nc; b += 64u) {
+                const uint32_t i = b + lane;
+                const uint32_t v[3] = {sum_part(c, 0), sum_part(c, 1), sum_part(c, 2)};
+                if (i + 64u < nc) c = L.cs[c0 + i + 64u];
+                else c = 0ull;
+                uint32_t incl[3];
 #pragma unroll
-                for (uint32_t t = 0; t < 8; ++t) {
-                    const uint32_t i = b + lane * 8u + t;
-                    c[t] = i < nwv ? L.wc[w0 + i] : 0u;
-                    sum += c[t];
-                }
-                // packed halves: at most 512 * 64 each
-                const uint32_t incl = wave_incl_scan(sum, lane);
-                uint32_t run = incl - sum;
-#pragma unroll
-                for (uint32_t t = 0; t < 8; ++t) {
-                    const uint32_t i = b + lane * 8u + t;
-                    if (i < nwv) L.woff[w0 + i] = make_uint2(n[0] + (run & 0xFFFFu), n[1] + (run >> 16));
-                    run += c[t];
-                }
-                const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-                n[0] += tot & 0xFFFFu;
-                n[1] += tot >> 16;
+                for (uint32_t k = 0; k < 3; ++k) incl[k] = wave_scan_u32(v[k]);
+                if (i < nc)
+                    L.coff[c0 + i] = make_uint4(n[0] + incl[0] - v[0], n[1] + incl[1] - v[1], nq + incl[2] - v[2], 0u);
+                n[0] += rec_word(incl[0], 63u);
+                n[1] += rec_word(incl[1], 63u);
+                nq += rec_word(incl[2], 63u);
             }
+            R = plan_node(nd, L.ratio);
             // no progress: every element went to both children
-            const bool leaf = R.leaf || (n[0] == m && n[1] == m);
-            need.bn = 2u * R.ncuts + (leaf ? 0u : 2u);
+            leaf = R.leaf || (n[0] == m && n[1] == m);
+            uint32_t v[7] = {2u * (uint32_t)__popc(R.cuts) + (leaf ? 0u : 2u), 0u, 0u, 0u, 0u, 0u, leaf ? 0u : nq};
             if (leaf) {
                 type[0] = CH_LEAF;
-                need.ll = m;
+                v[1] = m;
             } else {
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
                     // small iff count <= smallNodeMax (kernel_MarkSmallNodes, kdtree.cu:849-875)
                     type[s] = n[s] <= L.small_max ? CH_SMALL : CH_LARGE;
                     if (type[s] == CH_SMALL) {
-                        need.nsmall += 1u;
-                        need.nse += n[s];
+                        v[2] += n[s];
+                        v[3] += 1u;
                     } else {
-                        need.na += 1u;
-                        need.nw += (n[s] + 63u) >> 6;
+                        v[4] += (n[s] + 63u) >> 6;
+                        v[5] += 1u;
                     }
                 }
             }
-        }
-        if (lane == 0) s_need[wave] = need;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            ChildNeed t{};
-            for (uint32_t i = 0; i < kChildNodes; ++i) {
-                const ChildNeed c = s_need[i];
-                s_need[i] = t;
-                t.bn += c.bn;
-                t.na += c.na;
-                t.nw += c.nw;
-                t.nsmall += c.nsmall;
-                t.nse += c.nse;
-                t.ll += c.ll;
-            }
-            unsigned long long* next = (unsigned long long*)&L.W[W_LEVELS + 4 * (L.level + 1)];
-            unsigned long long* small = (unsigned long long*)&L.W[W_NSE];
-            ChildNeed b{};
-            if (t.bn) b.bn = atomicAdd(&L.W[W_NBN], t.bn);
-            if (t.ll) b.ll = atomicAdd(&L.W[W_LL], t.ll);
-            if (t.na) {
-                const unsigned long long o = atomicAdd(next, (unsigned long long)t.na << 32 | t.nw);
-                b.nw = (uint32_t)o;
-                b.na = (uint32_t)(o >> 32);
-            }
-            if (t.nsmall) {
-                const unsigned long long o = atomicAdd(small, (unsigned long long)t.nsmall << 32 | t.nse);
-                b.nse = (uint32_t)o;
-                b.nsmall = (uint32_t)(o >> 32);
-            }
-            if ((uint64_t)b.bn + t.bn > L.cap.bn || (uint64_t)b.ll + t.ll > L.cap.ll ||
-                (uint64_t)b.na + t.na > L.cap.na || (uint64_t)b.nw + t.nw > L.cap.nw ||
-                (uint64_t)b.nsmall + t.nsmall > L.cap.small || (uint64_t)b.nse + t.nse > L.cap.se) {
-                atomicOr(&L.W[W_ERR], kErrRoom);
-                b.bn = kNone;  // nothing of these nodes is written
-            }
-            s_base = b;
-        }
-        __syncthreads();
-        const ChildNeed base = s_base, own = s_need[wave];
-        __syncthreads();  // s_need is rewritten by the next step
-        if (!live || lane != 0u) continue;
-        const uint32_t none = base.bn == kNone ? 1u : 0u;
-        uint32_t id = base.bn + own.bn, cur = L.A.bn[p];
-        const uint32_t scene = L.A.scene[p];
-        if (none) {
-            L.P.child[2 * p] = L.P.child[2 * p + 1] = make_uint4(CH_DEAD, 0u, 0u, 0u);
-            continue;
-        }
-        auto node = [&](uint32_t i, uint32_t t, uint32_t level, uint32_t parent) {
-            L.B.type[i] = t;
-            L.B.level[i] = level;
-            L.B.scene[i] = scene;
-            L.B.parent[i] = parent;
-            L.B.flag[i] = 0u;
-        };
-        auto inner = [&](uint32_t i, uint32_t axis, float s, uint32_t l, uint32_t r) {
-            L.B.type[i] = axis;
-            L.B.split[i] = __float_as_uint(s);
-            L.B.left[i] = l;
-            L.B.right[i] = r;
-        };
-        (void)plan_node(L.A, p, L.ratio, [&](int ax, bool is_max, float s, uint32_t level, uint32_t) {
-            const uint32_t empty = id++, cont = id++;
-            inner(cur, (uint32_t)ax, s, is_max ? cont : empty, is_max ? empty : cont);
-            node(empty, BN_LEAF, level + 1, cur);
-            L.B.cnt[empty] = 0u;
-            L.B.aux[empty] = 0u;
-            node(cont, BN_PENDING, level + 1, cur);
-            cur = cont;
-        });
-        L.P.lo[p] = make_float4(R.lo[0], R.lo[1], R.lo[2], 0.0f);
-        L.P.hi[p] = make_float4(R.hi[0], R.hi[1], R.hi[2], 0.0f);
-        L.P.axis[p] = R.axis;
-        L.P.split[p] = R.split;
-        if (type[0] == CH_LEAF) {
-            const uint32_t at = base.ll + own.ll;
-            L.B.type[cur] = BN_LEAF;
-            L.B.cnt[cur] = m;
-            L.B.aux[cur] = at;
-            L.P.child[2 * p] = make_uint4(CH_LEAF, at, 0u, 0u);
-            L.P.child[2 * p + 1] = make_uint4(CH_DEAD, 0u, 0u, 0u);
-            continue;
-        }
-        inner(cur, R.axis, R.split, id, id + 1u);
-        uint32_t l = base.na + own.na, wv = base.nw + own.nw, s = base.nsmall + own.nsmall, se = base.nse + own.nse;
 #pragma unroll
-        for (uint32_t side = 0; side < 2; ++side) {
-            float4 lo = make_float4(R.lo[0], R.lo[1], R.lo[2], 0.0f), hi = make_float4(R.hi[0], R.hi[1], R.hi[2], 0.0f);
-            if (side == 0) f4set(hi, R.axis, R.split);
-            else f4set(lo, R.axis, R.split);
-            const uint32_t bn = id + side;
-            if (type[side] == CH_SMALL) {
-                L.S.first[s] = se;
-                L.S.cnt[s] = n[side];
-                L.S.level[s] = R.level + 1;
-                L.S.bn[s] = bn;
-                L.S.lo[s] = lo;
-                L.S.hi[s] = hi;
-                L.S.scene[s] = scene;
-                node(bn, BN_SMALL, R.level + 1, cur);
-                L.B.aux[bn] = s;
-                L.P.child[2 * p + side] = make_uint4(CH_SMALL, se, 0u, 0u);
-                ++s;
-                se += n[side];
+            for (uint32_t k = 0; k < 7; ++k)
+                if (lane == k) need = v[k];
+        }
+        if (lane < 8u) s_need[wave][lane] = need;
+        __syncthreads();
+        if (wave == 0) {
+            // lane 16 k + i: 64-bit total k (build nodes | leaf elements, small elements | small
+            // roots, next waves | next nodes, clip jobs) of node i
+            const uint32_t i = lane & 15u, k = lane >> 4;
+            const uint32_t a = s_need[i][2u * k], b = s_need[i][2u * k + 1u];
+            const uint32_t ia = row_scan_u32(a), ib = row_scan_u32(b);
+            unsigned long long at = 0;
+            if (i == 15u) {
+                const uint32_t word = k == 0u ? W_NBN : k == 1u ? W_NSE
+                                      : k == 2u ? W_LEVELS + 4u * (L.level + 1u) : W_LEVELS + 4u * L.level + 2u;
+                if ((ia | ib) != 0u) at = atomicAdd((unsigned long long*)&L.W[word], (unsigned long long)ib << 32 | ia);
+                const uint32_t ca = k == 0u ? L.cap.bn : k == 1u ? L.cap.se : L.cap.nw;
+                const uint32_t cb = k == 0u ? L.cap.ll : k == 1u ? L.cap.small : L.cap.na;
+                if (k < 3u && ((at & 0xFFFFFFFFull) + ia > ca || (at >> 32) + ib > cb)) {
+                    atomicOr(&L.W[W_ERR], kErrRoom);
+                    at = ~0ull;
+                }
+            }
+            const uint32_t lo = row_last((uint32_t)at), hi = row_last((uint32_t)(at >> 32));
+            const bool none = ballot(lo == kNone && hi == kNone) != 0ull;  // nothing of these nodes is written
+            s_base[i][2u * k] = none ? kNone : lo + ia - a;
+            s_base[i][2u * k + 1u] = none ? kNone : hi + ib - b;
+        }
+        __syncthreads();
+        const uint32_t base = s_base[wave][min(lane, 7u)];  // (rewritten after the next step's barrier)
+        if (!live || rec_word(base, 0u) == kNone) continue;
+        const uint32_t scene = rec_word(nd, ND_SCENE), bn0 = rec_word(nd, ND_BN);
+        const uint32_t id0 = rec_word(base, 0u), ncuts = (uint32_t)__popc(R.cuts), level0 = rec_word(nd, ND_LEVEL);
+        const uint32_t cur = ncuts ? id0 + 2u * ncuts - 1u : bn0, id = id0 + 2u * ncuts;
+        const uint32_t tw = __shfl(nd, ND_TB + min(lane, 5u), 64);
+        // lanes 0..5: the cuts
+        if (lane < 6u && (R.cuts >> lane & 1u)) {
+            const uint32_t k = (uint32_t)__popc(R.cuts & ((1u << lane) - 1u)), above = k ? id0 + 2u * k - 1u : bn0;
+            const uint32_t empty = id0 + 2u * k, cont = empty + 1u, lv = level0 + k + 1u;
+            const bool is_max = lane >= 3u;
+            put4(&L.B[above], 0, is_max ? lane - 3u : lane, __float_as_uint(fdec(is_max ? ~tw : tw)),
+                 is_max ? cont : empty, is_max ? empty : cont);
+            put4(&L.B[empty], 0, BN_LEAF, 0u, 0u, 0u);
+            put4(&L.B[empty], 1, lv, 0u, 0u, scene);
+            put4(&L.B[empty], 2, above | kCutParent, 0u, 1u, 0u);
+            put4(&L.B[cont], 1, lv, 0u, 0u, scene);
+            put4(&L.B[cont], 2, above | kCutParent, 0u, 0u, 0u);
+            put4(&L.B[cont], 3, 0u, 0u, 0u, 0u);
+        }
+        const uint32_t bx[3] = {__float_as_uint(R.lo[0]), __float_as_uint(R.lo[1]), __float_as_uint(R.lo[2])};
+        const uint32_t bh[3] = {__float_as_uint(R.hi[0]), __float_as_uint(R.hi[1]), __float_as_uint(R.hi[2])};
+        if (leaf) {
+            if (lane == 0) {
+                const uint32_t at = rec_word(base, 1u);
+                put4(&L.B[cur], 0, BN_LEAF, 0u, 0u, 0u);
+                L.B[cur].aux = at;
+                L.B[cur].cnt = m;
+                put4(&L.P[p], 0, 0u, 0u, CH_LEAF, CH_DEAD);
+                put4(&L.P[p], 1, at, 0u, 0u, 0u);
+            }
+            continue;
+        }
+        const uint32_t spl = __float_as_uint(R.split);
+        auto clear_sums = [&](uint32_t to, uint32_t at, uint32_t cnt) {
+            for (uint32_t i = lane; i < (cnt + 4095u) >> 12; i += 64u) L.csn[(at >> 12) + to + i] = 0ull;
+        };
+        const uint32_t se = rec_word(base, 2u), sr = rec_word(base, 3u), nw0 = rec_word(base, 4u), nx = rec_word(base, 5u);
+        const bool small0 = type[0] == CH_SMALL, small1 = type[1] == CH_SMALL;
+        // places of the two children: the left one's first
+        const uint32_t at0 = small0 ? se : 64u * nw0, at1 = small1 ? se + (small0 ? n[0] : 0u)
+                                                                   : 64u * (nw0 + (small0 ? 0u : (n[0] + 63u) >> 6));
+        const uint32_t to0 = small0 ? sr : nx, to1 = small1 ? sr + (small0 ? 1u : 0u) : nx + (small0 ? 0u : 1u);
+        if (!small0) clear_sums(to0, at0, n[0]);
+        if (!small1) clear_sums(to1, at1, n[1]);
+        if (lane == 2u) {
+            put4(&L.P[p], 0, R.axis, spl, type[0], type[1]);
+            put4(&L.P[p], 1, at0, at1, to0, to1);
+            put4(&L.P[p], 2, bx[0], bx[1], bx[2], rec_word(nd, ND_BASE));
+            put4(&L.P[p], 3, bh[0], bh[1], bh[2], rec_word(base, 6u));
+            put4(&L.B[cur], 0, R.axis, spl, id, id + 1u);
+        } else if (lane < 2u) {
+            const bool right = lane == 1u, sm = right ? small1 : small0;
+            const uint32_t at = right ? at1 : at0, to = right ? to1 : to0, cnt = right ? n[1] : n[0];
+            const uint32_t bn = id + lane;
+            uint32_t x[3], y[3];
+#pragma unroll
+            for (uint32_t k = 0; k < 3; ++k) {
+                x[k] = right && R.axis == k ? spl : bx[k];
+                y[k] = !right && R.axis == k ? spl : bh[k];
+            }
+            put4(&L.B[bn], 0, sm ? BN_SMALL : BN_PENDING, 0u, 0u, 0u);
+            put4(&L.B[bn], 1, R.level + 1u, to, 0u, scene);
+            put4(&L.B[bn], 2, cur, 0u, 0u, 0u);
+            put4(&L.B[bn], 3, 0u, 0u, 0u, 0u);
+            if (sm) {
+                put4(&L.S[to], 0, at, cnt, R.level + 1u, bn);
+                put4(&L.S[to], 1, x[0], x[1], x[2], scene);
+                put4(&L.S[to], 2, y[0], y[1], y[2], 0u);
             } else {
-                L.An.lo[l] = lo;
-                L.An.hi[l] = hi;
-                L.An.first[l] = 64u * wv;
-                L.An.cnt[l] = n[side];
-                L.An.level[l] = R.level + 1;
-                L.An.bn[l] = bn;
-                L.An.scene[l] = scene;
-                for (int k = 0; k < 6; ++k) L.An.tb[6 * l + k] = 0xFFFFFFFFu;
-                node(bn, BN_PENDING, R.level + 1, cur);
-                L.P.child[2 * p + side] = make_uint4(CH_LARGE, 64u * wv, l, 0u);
-                ++l;
-                wv += (n[side] + 63u) >> 6;
+                put4(&L.An[to], 0, x[0], x[1], x[2], y[0]);
+                put4(&L.An[to], 1, y[1], y[2], at, cnt);
+                put4(&L.An[to], 2, R.level + 1u, bn, scene, rec_word(nd, ND_BASE));
+                put4(&L.An[to], 3, ~0u, ~0u, ~0u, ~0u);
+                put4(&L.An[to], 4, ~0u, ~0u, 0u, 0u);
             }
         }
     }
@@ -747,146 +823,132 @@ __global__ __launch_bounds__(kChildBlock) void k_children(LevelArgs L) {
 // run of waves of one node in the workgroup, one atomic per component and run.  A straddling
 // triangle's bounds in a child are its clip to the child box (kernel_PerformSplitClipping,
 // kdtree_tri.cu:389-489), which k_clip computes from the queue written here, 64 to a wave
-// rather than one pass of a whole wave per straddler.
+// rather than one pass of a whole wave per straddler.  Bound by memory (66 MB a level at 1.03M
+// triangles: 20 us, 3.3 TB/s; 28 with one 1024-thread workgroup on a CU instead of two) and, below
+// about 10^5 elements, by latency (7 us).
 constexpr uint32_t kScatterBlock = 1024, kScatterWaves = kScatterBlock / 64;
 
 template <int kKind>
-__global__ __launch_bounds__(kScatterBlock) void k_scatter(LevelArgs L) {
-    __shared__ uint32_t s_tb[kScatterWaves][12];
-    __shared__ uint32_t s_node[kScatterWaves];
-    __shared__ uint32_t s_to[kScatterWaves][2];  // next-level nodes of the wave's children, or kNone
-    __shared__ uint32_t s_q[kScatterWaves + 1];
+__global__ __launch_bounds__(kScatterBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_scatter(LevelArgs L) {
+    // two sets, used in turn: one barrier a step
+    __shared__ uint32_t s_tb[2][kScatterWaves][12];
+    __shared__ uint32_t s_node[2][kScatterWaves];
+    __shared__ uint32_t s_to[2][kScatterWaves][2];  // next-level nodes of the wave's children, or kNone
     const uint32_t nw = level_waves(L), lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
+    uint32_t set = 0;
     for (uint32_t w0 = blockIdx.x * kScatterWaves; w0 < nw; w0 += gridDim.x * kScatterWaves) {  // uniform per workgroup
         const uint32_t w = w0 + wave, e = 64u * w + lane;
-        uint32_t p = kNone, to[2] = {kNone, kNone};
-        uint32_t tb[12];
-#pragma unroll
-        for (int k = 0; k < 12; ++k) tb[k] = ~0u;
-        uint64_t mq[2] = {0ull, 0ull};
-        uint32_t dst[2] = {0u, 0u};
+        uint32_t p = kNone, to[2] = {kNone, kNone}, mine = ~0u;  // mine: lane k < 12, tight word k
         if (w < nw) {
             p = uniform(L.E.wnode[w]);
-            const uint4 c0 = L.P.child[2 * p], c1 = L.P.child[2 * p + 1];
-            const uint32_t type[2] = {uniform(c0.x), uniform(c1.x)}, at[2] = {uniform(c0.y), uniform(c1.y)};
-            const uint32_t local = e - L.A.first[p];
-            const bool in = local < L.A.cnt[p];
-            const uint32_t idx = in ? L.E.idx[e] : 0u;
-            if (type[0] == CH_LEAF) {
-                if (in) L.ll_idx[at[0] + local] = idx;
-            } else if (type[0] != CH_DEAD) {
-                bool go[2] = {false, false};
-                bool straddle = false;
-                float4 lo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), hi = lo;
+            const float4 lo = L.E.lo[e];  // (slots past the node's last element hold anything)
+            const float4 hi = (kKind == MNRT_KIND_TRI) ? L.E.hi[e] : lo;
+            const uint32_t sp = ((const uint32_t*)(L.P + p))[lane & 15u];
+            const uint32_t fc = ((const uint32_t*)(L.A + p))[ND_FIRST + (lane & 1u)];
+            const uint32_t idx = __float_as_uint(lo.w), local = e - rec_word(fc, 0u);
+            const bool in = local < rec_word(fc, 1u);
+            const uint32_t type0 = rec_word(sp, 2u), type1 = rec_word(sp, 3u);
+            if (type0 == CH_LEAF) {
+                if (in) L.ll_idx[rec_word(sp, 4u) + local] = idx;
+            } else if (type0 != CH_DEAD) {
+                const uint32_t axis = rec_word(sp, 0u);
+                const float s = __uint_as_float(rec_word(sp, 1u));
+                bool go[2] = {false, false}, both = false;
                 if (in) {
-                    const uint32_t axis = L.P.axis[p];
-                    const float s = L.P.split[p];
-                    lo = L.E.lo[e];
-                    hi = (kKind == MNRT_KIND_TRI) ? L.E.hi[e] : lo;
                     classify(kKind, idx, lo, hi, axis, s, go[0], go[1]);
-                    straddle = (kKind == MNRT_KIND_TRI) && (f4c(lo, axis) < s && s < f4c(hi, axis));
+                    both = straddles(kKind, lo, hi, axis, s);
                 }
-                const uint2 off = L.woff[w];
+                // the waves of the chunk before this one
+                const uint32_t wf = rec_word(fc, 0u) >> 6, ch = chunk_of(p, wf, w), wl = wf + ((w - wf) & ~63u) + lane;
+                const uint32_t cw = wl < w ? L.wc[wl] : 0u;
+                uint4 off = L.coff[ch];
+                const uint32_t before = wave_sum_u32((cw & 0xFFu) | (cw & 0xFF00u) << 8);
+                off.x += before & 0xFFFFu;
+                off.y += before >> 16;
+                if (kKind == MNRT_KIND_TRI) off.z += wave_sum_u32(cw >> 16);
+                uint32_t v[6], dst[2];
+                tight_words(lo, hi, v);
 #pragma unroll
                 for (int side = 0; side < 2; ++side) {
-                    const uint64_t m = ballot(go[side]);
-                    dst[side] = at[side] + (side ? off.y : off.x) + mask_prefix(m);
-                    mq[side] = m & ballot(straddle);
-                    const bool large = type[side] == CH_LARGE;
+                    const bool large = (side ? type1 : type0) == CH_LARGE;
+                    const uint32_t child = rec_word(sp, 6u + side);
+                    dst[side] = rec_word(sp, 4u + side) + (side ? off.y : off.x) + mask_prefix(ballot(go[side]));
+                    const ElemView& D = large ? L.Nx : L.Sm;
+                    if (go[side] && !both) {  // (a straddler's record comes with its clip)
+                        D.lo[dst[side]] = lo;
+                        if (kKind == MNRT_KIND_TRI) D.hi[dst[side]] = hi;
+                    }
                     if (go[side]) {
-                        const ElemView& D = large ? L.Nx : L.Sm;
-                        D.idx[dst[side]] = idx;
-                        if (!straddle) {
-                            D.lo[dst[side]] = lo;
-                            if (kKind == MNRT_KIND_TRI) D.hi[dst[side]] = hi;
-                        }
-                        if (large && (dst[side] & 63u) == 0u) L.Nx.wnode[dst[side] >> 6] = side ? c1.z : c0.z;
+                        if (large && (dst[side] & 63u) == 0u) L.Nx.wnode[dst[side] >> 6] = child;
                     }
                     if (large) {
-                        to[side] = uniform(side ? c1.z : c0.z);
-                        uint32_t v[6];
-                        tight_words(lo, hi, v);
+                        to[side] = child;
 #pragma unroll
-                        for (int k = 0; k < 6; ++k)
-                            tb[6 * side + k] = wave_min_u32(go[side] && !straddle ? v[k] : ~0u);
+                        for (uint32_t k = 0; k < 6; ++k) {
+                            const uint32_t t = wave_min_u32(go[side] && !both ? v[k] : ~0u);
+                            if (lane == 6u * side + k) mine = t;
+                        }
                     }
+                }
+                if (kKind == MNRT_KIND_TRI) {
+                    const uint64_t mq = ballot(both);
+                    if (both) L.q[rec_word(sp, 15u) + off.z + mask_prefix(mq)] = make_uint4(e, dst[0], dst[1], p);
                 }
             }
         }
-        const uint32_t nq = (uint32_t)(__popcll(mq[0]) + __popcll(mq[1]));
         if (lane == 0) {
-            s_node[wave] = p;
-            s_to[wave][0] = to[0];
-            s_to[wave][1] = to[1];
-            if (kKind == MNRT_KIND_TRI) s_q[wave] = nq;
+            s_node[set][wave] = p;
+            s_to[set][wave][0] = to[0];
+            s_to[set][wave][1] = to[1];
         }
-#pragma unroll
-        for (int k = 0; k < 12; ++k)
-            if (lane == (uint32_t)k) s_tb[wave][k] = tb[k];
+        if (lane < 12u) s_tb[set][wave][lane] = mine;
         __syncthreads();
         if (threadIdx.x < 12u * kScatterWaves) {
-            const uint32_t i = threadIdx.x / 12u, k = threadIdx.x % 12u, node = s_node[i], t = s_to[i][k / 6u];
-            if (t != kNone && (i == 0u || s_node[i - 1u] != node)) {
-                uint32_t v = s_tb[i][k];
-                for (uint32_t j = i + 1u; j < kScatterWaves && s_node[j] == node; ++j) v = min(v, s_tb[j][k]);
-                if (v != ~0u) atomicMin(&L.An.tb[6u * t + k % 6u], v);
+            const uint32_t i = threadIdx.x / 12u, k = threadIdx.x % 12u, node = s_node[set][i], t = s_to[set][i][k / 6u];
+            if (t != kNone && (i == 0u || s_node[set][i - 1u] != node)) {
+                uint32_t v = s_tb[set][i][k];
+                for (uint32_t j = i + 1u; j < kScatterWaves && s_node[set][j] == node; ++j) v = min(v, s_tb[set][j][k]);
+                if (v != ~0u) atomicMin(&L.An[t].tb[k % 6u], v);
             }
         }
-        if (kKind == MNRT_KIND_TRI && threadIdx.x == kScatterBlock - 1u) {
-            uint32_t tot = 0;
-            for (uint32_t i = 0; i < kScatterWaves; ++i) {
-                const uint32_t c = s_q[i];
-                s_q[i] = tot;
-                tot += c;
-            }
-            const uint32_t b = tot ? atomicAdd(&L.W[W_LEVELS + 4 * L.level + 2], tot) : 0u;
-            s_q[kScatterWaves] = b;
-        }
-        __syncthreads();
-        if (kKind == MNRT_KIND_TRI && nq) {
-            uint32_t b = s_q[kScatterWaves] + s_q[wave];
-#pragma unroll
-            for (int side = 0; side < 2; ++side) {
-                if ((mq[side] >> lane) & 1ull)
-                    L.q[b + mask_prefix(mq[side])] = make_uint2(e << 1 | (uint32_t)side, dst[side]);
-                b += (uint32_t)__popcll(mq[side]);
-            }
-        }
-        __syncthreads();  // the LDS words are rewritten by the next step
+        set ^= 1u;
     }
 }
 
-// The clip queue of a triangle level: each job clips its triangle to the child box, writes the
-// bounds next to the index k_scatter placed and adds them to a large child's tight bounds (lanes
+// The clip queue of a triangle level: two lanes per job clip its triangle to the child boxes, write
+// the record at the place k_scatter found and add them to a large child's tight bounds (lanes
 // that share a child reduce first).
 __global__ __launch_bounds__(kClipBlock) void k_clip(LevelArgs L, Geometry G) {
     __shared__ float s_lists[2 * kClipVerts * 3 * kClipBlock];
     __attribute__((address_space(3))) float* col = (__attribute__((address_space(3))) float*)(s_lists + threadIdx.x);
     if (L.W[W_ERR] != 0u) return;
-    const uint32_t nq = L.W[W_LEVELS + 4 * L.level + 2], lane = threadIdx.x;
+    const uint32_t nq = 2u * L.W[W_LEVELS + 4 * L.level + 2], lane = threadIdx.x;
     for (uint32_t j0 = blockIdx.x * kClipBlock; j0 < nq; j0 += gridDim.x * kClipBlock) {
         const uint32_t j = j0 + lane;
         uint32_t to = kNone;
         uint32_t v[6] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
         if (j < nq) {
-            const uint2 job = L.q[j];
-            const uint32_t e = job.x >> 1, side = job.x & 1u, p = L.E.wnode[e >> 6], axis = L.P.axis[p];
-            const float s = L.P.split[p];
+            const uint4 job = L.q[j >> 1];
+            const uint32_t e = job.x, side = j & 1u;
+            const uint4* P = (const uint4*)&L.P[job.w];
+            const uint4 p0 = P[0], p1 = P[1], p2 = P[2], p3 = P[3];
+            const uint32_t axis = p0.x, type = side ? p0.w : p0.z;
             float4 lo = L.E.lo[e], hi = L.E.hi[e];
-            float4 bmin = L.P.lo[p], bmax = L.P.hi[p];
-            if (side == 0) f4set(bmax, axis, s);
-            else f4set(bmin, axis, s);
-            clip_bounds(G, G.base[L.A.scene[p]] + L.E.idx[e], lo, hi, bmin, bmax, col);
-            const uint4 c = L.P.child[2 * p + side];
-            const ElemView& D = c.x == CH_LARGE ? L.Nx : L.Sm;
-            D.lo[job.y] = lo;
-            D.hi[job.y] = hi;
-            if (c.x == CH_LARGE) {
-                to = c.z;
+            float4 bmin = make_float4(__uint_as_float(p2.x), __uint_as_float(p2.y), __uint_as_float(p2.z), 0.0f);
+            float4 bmax = make_float4(__uint_as_float(p3.x), __uint_as_float(p3.y), __uint_as_float(p3.z), 0.0f);
+            if (side == 0) f4set(bmax, axis, __uint_as_float(p0.y));
+            else f4set(bmin, axis, __uint_as_float(p0.y));
+            clip_bounds(G, p2.w + __float_as_uint(lo.w), lo, hi, bmin, bmax, col);
+            const ElemView& D = type == CH_LARGE ? L.Nx : L.Sm;
+            const uint32_t d = side ? job.z : job.y;
+            D.lo[d] = lo;
+            D.hi[d] = hi;
+            if (type == CH_LARGE) {
+                to = side ? p1.w : p1.z;
                 tight_words(lo, hi, v);
             }
         }
-        tight_by_key(to, v, L.An.tb, lane);
+        tight_by_key(to, v, (uint32_t*)L.An + ND_TB, sizeof(NodeRec) / 4u, lane);
     }
 }
 
@@ -930,8 +992,7 @@ struct SmallOut {
     uint32_t* st_refs;       // stage: references, subtree-local
     uint32_t* st_ovf;        // stage: 1 where the subtree did not fit; emit: only these
     StageCap st_cap;
-    const uint32_t* bn_addr;  // emit: subtree start address / reference base
-    const uint32_t* bn_rbase;
+    const BnRec* bn;  // emit: subtree start address / reference base
     uint32_t* nodes;
     uint32_t* refs;
     uint32_t* W;
@@ -958,7 +1019,8 @@ __device__ __forceinline__ uint32_t write_lane(uint32_t v, int lane, uint32_t ol
 // elements have no upper bounds and 3n candidates (triangles: 6n), which halves the mask
 // arrays and lets more waves share a CU.
 template <int kMode, int kKind>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallView S, ElemView Sm,
+__global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, const SmallRec* __restrict__ S,
+                                                            ElemView Sm,
                                                             const float* __restrict__ scene_qr, SmallOut O) {
     constexpr int kind = kKind;
     // candidate slots of an element: (isMax, axis), slot = isMax * 3 + axis
@@ -971,7 +1033,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
     if (kMode == kSmallEmit && O.st_ovf && O.st_ovf[r] == 0u) return;
     SmallStackEnt* stack = s_stack[wave];
 
-    const uint32_t first = S.first[r], n = S.cnt[r];
+    const SmallRec root = S[r];
+    const uint32_t first = root.first, n = root.cnt;
     // lane j holds element j (n <= 64)
     const bool valid = lane < n;
     float4 mlo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), mhi = mlo;
@@ -979,7 +1042,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
     if (valid) {
         mlo = Sm.lo[first + lane];
         mhi = (kKind == MNRT_KIND_TRI) ? Sm.hi[first + lane] : mlo;
-        midx = Sm.idx[first + lane];
+        midx = __float_as_uint(mlo.w);
     }
     const bool mleft = plane_goes_left(midx);
     // Candidates axis-major, minimums then maximums (kernel_CreateSplitCandidates,
@@ -1049,7 +1112,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
     }
 
     uint32_t addr = 0, rbase = 0, maxlvl = 0;
-    const uint32_t scene = S.scene[r];
+    const uint32_t scene = root.scene;
     // emit: scene-local addresses into the scene's tree; stage: subtree-local addresses
     // into the staging area
     uint32_t* nodes = nullptr;
@@ -1061,9 +1124,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
         refs = O.refs + O.ref_base[scene];
         lim_nodes = O.max_nodes - O.node_base[scene];
         lim_refs = O.max_refs - O.ref_base[scene];
-        uint32_t bn = S.bn[r];
-        addr = O.bn_addr[bn];
-        rbase = O.bn_rbase[bn];
+        addr = O.bn[root.bn].addr;
+        rbase = O.bn[root.bn].rbase;
     } else if (kMode == kSmallStage) {
         const uint32_t off = O.st_cap.begin(r, first);
         nodes = (uint32_t*)(O.st_nodes + off);
@@ -1074,10 +1136,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, SmallVie
     if (lane == 0) {
         SmallStackEnt e;
         e.mask = (n == 64) ? ~0ull : ((1ull << n) - 1ull);
-        float4 lo = S.lo[r], hi = S.hi[r];
-        e.lo[0] = lo.x; e.lo[1] = lo.y; e.lo[2] = lo.z;
-        e.hi[0] = hi.x; e.hi[1] = hi.y; e.hi[2] = hi.z;
-        e.lvl_ax = S.level[r];
+        for (int k = 0; k < 3; ++k) {
+            e.lo[k] = root.lo[k];
+            e.hi[k] = root.hi[k];
+        }
+        e.lvl_ax = root.level;
         e.patch = kNone;
         stack[0] = e;
     }
@@ -1249,13 +1312,13 @@ StageCap stage_cap_setting() {
 // Moves staged small subtrees to their final addresses (one wave per small root):
 // inner words get the subtree's first address added to the right-child index, leaf words
 // its first reference added to the reference offset.
-__global__ __launch_bounds__(64 * kSmallWaves) void k_small_place(DN dnsmall, SmallView S, SmallOut O) {
+__global__ __launch_bounds__(64 * kSmallWaves) void k_small_place(DN dnsmall, const SmallRec* __restrict__ S, SmallOut O) {
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t r = blockIdx.x * kSmallWaves + wave;
     if (r >= dnsmall.get() || O.st_ovf[r] != 0u || O.W[W_ERR] != 0u) return;
-    const uint32_t scene = S.scene[r];
-    const uint32_t bn = S.bn[r];
-    const uint32_t a0 = O.bn_addr[bn], r0 = O.bn_rbase[bn];
+    const uint32_t scene = S[r].scene;
+    const BnRec& bn = O.bn[S[r].bn];
+    const uint32_t a0 = bn.addr, r0 = bn.rbase;
     const uint32_t nn = O.nsize[r], nr = O.rsize[r];
     const uint32_t lim_nodes = O.max_nodes - O.node_base[scene], lim_refs = O.max_refs - O.ref_base[scene];
     if (a0 + nn > lim_nodes || r0 + nr > lim_refs) {
@@ -1264,7 +1327,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small_place(DN dnsmall, Sm
     }
     uint2* nodes = (uint2*)(O.nodes + 2ull * O.node_base[scene]) + a0;
     uint32_t* refs = O.refs + O.ref_base[scene] + r0;
-    const uint32_t off = O.st_cap.begin(r, S.first[r]);
+    const uint32_t off = O.st_cap.begin(r, S[r].first);
     for (uint32_t j = lane; j < nn; j += 64) {
         uint2 w = O.st_nodes[off + j];
         const uint32_t tag = w.y >> 30;
@@ -1276,108 +1339,123 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small_place(DN dnsmall, Sm
 
 // ---- layout ---------------------------------------------------------------------------
 // (KDTreeGPU::PreorderTraversal launches two kernels per level over all nodes,
-// KDTreeGPU.cpp:1156-1209.)  Subtree sizes climb from the leaves in one launch, the second child
-// to arrive at a node going on; a node's address is the sum over its ancestors, so one more
-// launch places and emits every node at once.  58 launches, one per level and direction, took
-// 0.23 ms of the 1.03M-triangle build.
-
-struct LayoutView {
-    uint32_t* size;   // nodes in the subtree
-    uint32_t* rsize;  // references in the subtree
-    uint32_t* depth;  // deepest level in the subtree
-    uint32_t* addr;   // small roots: subtree start
-    uint32_t* rbase;
-};
-
-// The climbing waves exchange sizes across dies within the launch: through atomics of device
-// scope only, each value stored and waited for before its node's arrival is counted.
-__device__ __forceinline__ void put_dev(uint32_t* p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t get_dev(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+// KDTreeGPU.cpp:1156-1209.)  Subtree sizes climb from the leaves in one launch: a child brings
+// its sizes to its parent by one atomic, whose old value tells the second child to arrive what the
+// first brought, and that one goes on.  Below an empty-space cut the sibling is an empty leaf, so
+// the climb passes without an exchange.  A node's address is the sum over its ancestors, so one
+// more launch places and emits every node at once.  58 launches, one per level and direction, took
+// 234 us of the 1.03M-triangle build, these two 73 us.
+constexpr uint32_t kAccBits = 31u;  // acc: references, nodes, arrivals (31 + 31 + 2 bits)
 
 // top: the deepest level the build may reach; a leaf below it sets kErrLayoutDepth.
-__global__ __launch_bounds__(256) void k_layout_sizes(DN dnbn, BnView B, LayoutView Lv, const uint32_t* __restrict__ s_nsize,
+__global__ __launch_bounds__(256) void k_layout_sizes(DN dnbn, BnRec* __restrict__ B,
+                                                      const uint32_t* __restrict__ s_nsize,
                                                       const uint32_t* __restrict__ s_rsize,
                                                       const uint32_t* __restrict__ s_mlvl, uint32_t top,
-                                                      uint32_t* __restrict__ W) {
-    if (W[W_ERR] != 0u) return;
-    const uint32_t nbn = dnbn.get();
-    uint32_t deepest = 0;
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nbn; j += gridDim.x * blockDim.x) {
-        const uint32_t t = B.type[j];
-        if (t != BN_LEAF && t != BN_SMALL) continue;
-        const uint32_t x = B.aux[j];
-        uint32_t i = j, size = 1u, rsize, depth = B.level[j];
-        deepest = max(deepest, depth);
-        if (t == BN_SMALL) {
-            size = s_nsize[x];
-            rsize = s_rsize[x];
-            depth = s_mlvl[x];
-        } else {
-            rsize = B.cnt[j];
+                                                      uint32_t* __restrict__ maxlvl, uint32_t* __restrict__ W) {
+    if (W[W_ERR] != 0u) return;  // (per wave: another's error only ends the climb early)
+    const uint32_t nbn = dnbn.get(), lane = threadIdx.x & 63u;
+    for (uint32_t j0 = blockIdx.x * blockDim.x; j0 < nbn; j0 += gridDim.x * blockDim.x) {  // uniform per wave
+        const uint32_t j = j0 + threadIdx.x;
+        uint32_t scene = kNone, depth = 0, deepest = 0;
+        if (j < nbn) {
+            const uint4 q0 = ((const uint4*)&B[j])[0], q1 = ((const uint4*)&B[j])[1];
+            uint32_t parent = B[j].parent;
+            const uint32_t t = q0.x, x = q1.y;
+            // (an empty leaf of a cut has its size already and is no deeper than its sibling)
+            const bool cut_leaf = t == BN_LEAF && q1.z == 0u && parent != kNone && (parent & kCutParent);
+            if ((t == BN_LEAF || t == BN_SMALL) && !cut_leaf) {
+                uint32_t i = j, size = 1u, rsize = q1.z;
+                scene = q1.w;
+                deepest = depth = q1.x;
+                if (t == BN_SMALL) {
+                    size = s_nsize[x];
+                    rsize = s_rsize[x];
+                    depth = s_mlvl[x];
+                }
+                for (;;) {
+                    if (size > MNRT_INDEX_MASK || rsize > MNRT_INDEX_MASK) {
+                        atomicOr(&W[W_ERR], kErrOutputRoom);
+                        break;
+                    }
+                    *(uint2*)&B[i].size = make_uint2(size, rsize);
+                    if (parent == kNone) break;
+                    const uint32_t p = parent & ~kCutParent;
+                    const bool cut = (parent & kCutParent) != 0u;
+                    parent = B[p].parent;
+                    i = p;
+                    if (cut) {
+                        size += 2u;
+                        continue;
+                    }
+                    const unsigned long long old =
+                        atomicAdd(&B[p].acc, 1ull << 62 | (unsigned long long)size << kAccBits | rsize);
+                    if ((old >> 62) == 0ull) break;
+                    size += 1u + ((uint32_t)(old >> kAccBits) & 0x7FFFFFFFu);
+                    rsize += (uint32_t)old & 0x7FFFFFFFu;
+                }
+            }
         }
-        for (;;) {
-            put_dev(&Lv.size[i], size);
-            put_dev(&Lv.rsize[i], rsize);
-            put_dev(&Lv.depth[i], depth);
-            const uint32_t p = B.parent[i];
-            if (p == kNone) break;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            if (__hip_atomic_fetch_add(&B.flag[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) break;
-            asm volatile("" ::: "memory");
-            const uint32_t l = B.left[p], o = l == i ? B.right[p] : l;
-            size += 1u + get_dev(&Lv.size[o]);
-            rsize += get_dev(&Lv.rsize[o]);
-            depth = max(depth, get_dev(&Lv.depth[o]));
-            i = p;
+        deepest = wave_max_u32(deepest);
+        if (lane == 0u && deepest != 0u) {
+            atomicMax(&W[W_MAXLEVEL], deepest);
+            if (deepest > top) atomicOr(&W[W_ERR], kErrLayoutDepth);
         }
-    }
-    deepest = wave_max_u32(deepest);
-    if ((threadIdx.x & 63u) == 0u && deepest != 0u) {
-        atomicMax(&W[W_MAXLEVEL], deepest);
-        if (deepest > top) atomicOr(&W[W_ERR], kErrLayoutDepth);
+        for (uint64_t m = ballot(scene != kNone); m != 0ull;) {
+            const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)scene, (int)__builtin_ctzll(m));
+            const uint32_t d = wave_max_u32(scene == s ? depth : 0u);
+            if (lane == 0u) atomicMax(&maxlvl[s], d);
+            m &= ~ballot(scene == s);
+        }
     }
 }
 
-// Per scene (root = build node s): nodes, references, leaves and max level, and the trees' places
+// Per scene (root = build node s): nodes, references and leaves, and the trees' places
 // in the shared arrays.  Every inner node has two children, so leaves = (nodes + 1) / 2.
 // max_nodes / max_refs: room of the output arrays.
-__global__ __launch_bounds__(1024) void k_scene_totals(uint32_t nscenes, LayoutView Lv, uint32_t* __restrict__ nodes,
-                                                       uint32_t* __restrict__ refs, uint32_t* __restrict__ nbase,
-                                                       uint32_t* __restrict__ rbase, uint32_t* __restrict__ leaves,
-                                                       uint32_t* __restrict__ maxlvl, uint32_t max_nodes,
+__global__ __launch_bounds__(1024) void k_scene_totals(uint32_t nscenes, const BnRec* __restrict__ B,
+                                                       uint32_t* __restrict__ nodes, uint32_t* __restrict__ refs,
+                                                       uint32_t* __restrict__ nbase, uint32_t* __restrict__ rbase,
+                                                       uint32_t* __restrict__ leaves, uint32_t max_nodes,
                                                        uint32_t max_refs, uint32_t* __restrict__ W) {
-    __shared__ uint64_t s_wave[16];
-    if (W[W_ERR] != 0u) return;  // (uniform: no thread of this launch has set it yet)
+    __shared__ uint64_t s_wave[16], s_rwave[16];
+    if (W[W_ERR] != 0u) return;  // (uniform: this launch sets it after its last barrier only)
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     uint64_t n0 = 0, r0 = 0;
     for (uint32_t b = 0; b < nscenes; b += 1024u) {
         const uint32_t s = b + tid;
-        const uint32_t n = s < nscenes ? Lv.size[s] : 0u, r = s < nscenes ? Lv.rsize[s] : 0u;
-        const uint32_t ni = wave_incl_scan(n, lane), ri = wave_incl_scan(r, lane);
-        if (lane == 63u) s_wave[wave] = (uint64_t)ni << 32 | ri;
+        const uint32_t n = s < nscenes ? B[s].size : 0u, r = s < nscenes ? B[s].rsize : 0u;
+        uint64_t incl = n, rincl = r;  // (64 sizes of at most 2^30 - 1 pass 32 bits)
+#pragma unroll
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint64_t a = __shfl_up((unsigned long long)incl, o, 64), c = __shfl_up((unsigned long long)rincl, o, 64);
+            if (lane >= o) {
+                incl += a;
+                rincl += c;
+            }
+        }
+        if (lane == 63u) {
+            s_wave[wave] = incl;
+            s_rwave[wave] = rincl;
+        }
         __syncthreads();
         uint64_t nb = n0, rb = r0;
         for (uint32_t i = 0; i < 16u; ++i) {
             if (i < wave) {
-                nb += s_wave[i] >> 32;
-                rb += (uint32_t)s_wave[i];
+                nb += s_wave[i];
+                rb += s_rwave[i];
             }
-            n0 += s_wave[i] >> 32;
-            r0 += (uint32_t)s_wave[i];
+            n0 += s_wave[i];
+            r0 += s_rwave[i];
         }
         if (s < nscenes) {
             nodes[s] = n;
             refs[s] = r;
-            nbase[s] = (uint32_t)(nb + ni - n);
-            rbase[s] = (uint32_t)(rb + ri - r);
+            nbase[s] = (uint32_t)(nb + incl - n);
+            rbase[s] = (uint32_t)(rb + rincl - r);
             leaves[s] = (n + 1u) / 2u;
-            maxlvl[s] = Lv.depth[s];
         }
-        __syncthreads();  // s_wave is rewritten by the next step
+        __syncthreads();  // the LDS words are rewritten by the next step
     }
     if (tid == 0) {
         nbase[nscenes] = (uint32_t)n0;
@@ -1387,7 +1465,7 @@ __global__ __launch_bounds__(1024) void k_scene_totals(uint32_t nscenes, LayoutV
 }
 
 // Places every build node and writes the large stage's inner nodes and leaves.
-__global__ __launch_bounds__(256) void k_emit_large(DN dnbn, BnView B, LayoutView Lv,
+__global__ __launch_bounds__(256) void k_emit_large(DN dnbn, BnRec* __restrict__ B,
                                                     const uint32_t* __restrict__ ll_idx,
                                                     uint32_t* __restrict__ nodes_all, uint32_t* __restrict__ refs_all,
                                                     const uint32_t* __restrict__ W,
@@ -1396,30 +1474,33 @@ __global__ __launch_bounds__(256) void k_emit_large(DN dnbn, BnView B, LayoutVie
     if (W[W_ERR] != 0u) return;  // failed build: nothing is emitted
     const uint32_t nbn = dnbn.get();
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nbn; i += gridDim.x * blockDim.x) {
-        const uint32_t t = B.type[i];
+        const uint4 q0 = ((const uint4*)&B[i])[0], q1 = ((const uint4*)&B[i])[1];
+        const uint32_t t = q0.x, sc = q1.w;
         uint32_t a = 0, rb = 0;
-        for (uint32_t c = i, p = B.parent[i]; p != kNone; c = p, p = B.parent[p]) {
-            const uint32_t l = B.left[p];
+        for (uint32_t c = i, up = B[i].parent; up != kNone;) {
+            const uint32_t p = up & ~kCutParent, l = B[p].left;
+            const uint32_t above = B[p].parent;
             a += 1u;
             if (l != c) {
-                a += Lv.size[l];
-                rb += Lv.rsize[l];
+                const uint2 z = *(const uint2*)&B[l].size;
+                a += z.x;
+                rb += z.y;
             }
+            c = p;
+            up = above;
         }
         if (t == BN_SMALL) {
-            Lv.addr[i] = a;
-            Lv.rbase[i] = rb;
+            *(uint2*)&B[i].addr = make_uint2(a, rb);
             continue;
         }
-        const uint32_t sc = B.scene[i];
         uint2* nodes = (uint2*)nodes_all + node_base[sc];
         if (t == BN_LEAF) {
-            const uint32_t m = B.cnt[i], from = B.aux[i];
+            const uint32_t m = q1.z, from = q1.y;
             uint32_t* refs = refs_all + ref_base[sc];
             nodes[a] = make_uint2(m, (MNRT_LEAF_TAG << 30) | rb);
             for (uint32_t k = 0; k < m; ++k) refs[rb + k] = ll_idx[from + k];
         } else {
-            nodes[a] = make_uint2(B.split[i], (t << 30) | (a + 1u + Lv.size[B.left[i]]));
+            nodes[a] = make_uint2(q0.y, (t << 30) | (a + 1u + B[q0.z].size));
         }
     }
 }
@@ -1561,21 +1642,21 @@ RootCounts plan_roots(const uint32_t* h_base, uint32_t S_, uint32_t small_max, u
 struct LevelBufs {
     uint32_t* W;
     uint32_t* stb;  // tight bounds per scene
-    NodeView N[2];
+    NodeRec* N[2];
     ElemView X[2], Sm;
-    SmallView S;
-    BnView B;
+    SmallRec* S;
+    BnRec* B;
     uint32_t* wc;
-    uint2* woff;
-    SplitView P;
+    unsigned long long* cs[2];
+    uint4* coff;
+    SplitRec* P;
     uint32_t* ll_idx;
-    uint2* q;
+    uint4* q;
 };
 
 template <typename A>
 ElemView take_elems(A& a, int kind, uint64_t slots, bool waves) {
     ElemView V{};
-    V.idx = a.template get<uint32_t>(slots);
     V.lo = a.template get<float4>(slots);
     V.hi = kind == MNRT_KIND_TRI ? a.template get<float4>(slots) : V.lo;
     V.wnode = waves ? a.template get<uint32_t>(slots / 64u) : nullptr;
@@ -1587,47 +1668,27 @@ LevelBufs take_levels(A& a, int kind, uint32_t S_, const BuildCaps& C) {
     LevelBufs b{};
     b.W = a.template get<uint32_t>(kWords);
     b.stb = a.template get<uint32_t>(6ull * S_);
-    for (NodeView& V : b.N) {
-        V.lo = a.template get<float4>(C.na);
-        V.hi = a.template get<float4>(C.na);
-        V.first = a.template get<uint32_t>(C.na);
-        V.cnt = a.template get<uint32_t>(C.na);
-        V.level = a.template get<uint32_t>(C.na);
-        V.bn = a.template get<uint32_t>(C.na);
-        V.scene = a.template get<uint32_t>(C.na);
-        V.tb = a.template get<uint32_t>(6ull * C.na);
-    }
+    for (NodeRec*& n : b.N) n = a.template get<NodeRec>(C.na);
     const uint64_t slots = 64ull * C.nw;
     for (ElemView& V : b.X) V = take_elems(a, kind, slots, true);
     b.Sm = take_elems(a, kind, C.se, false);
-    b.S.first = a.template get<uint32_t>(C.small);
-    b.S.cnt = a.template get<uint32_t>(C.small);
-    b.S.level = a.template get<uint32_t>(C.small);
-    b.S.bn = a.template get<uint32_t>(C.small);
-    b.S.lo = a.template get<float4>(C.small);
-    b.S.hi = a.template get<float4>(C.small);
-    b.S.scene = a.template get<uint32_t>(C.small);
-    uint32_t* bn = a.template get<uint32_t>((uint64_t)kBnCols * C.bn);
-    auto col = [&](uint64_t k) { return bn ? bn + k * C.bn : nullptr; };
-    b.B = BnView{col(0), col(1), col(2), col(3), col(4), col(5), col(6), col(7), col(8), col(9)};
+    b.S = a.template get<SmallRec>(C.small);
+    b.B = a.template get<BnRec>(C.bn);
     b.wc = a.template get<uint32_t>(C.nw);
-    b.woff = a.template get<uint2>(C.nw);
-    b.P.lo = a.template get<float4>(C.na);
-    b.P.hi = a.template get<float4>(C.na);
-    b.P.axis = a.template get<uint32_t>(C.na);
-    b.P.split = a.template get<float>(C.na);
-    b.P.child = a.template get<uint4>(2ull * C.na);
+    for (unsigned long long*& v : b.cs) v = a.template get<unsigned long long>(chunks_for(C.nw, C.na));
+    b.coff = a.template get<uint4>(chunks_for(C.nw, C.na));
+    b.P = a.template get<SplitRec>(C.na);
     b.ll_idx = a.template get<uint32_t>(C.ll);
-    b.q = kind == MNRT_KIND_TRI ? a.template get<uint2>(2 * slots) : nullptr;
+    b.q = kind == MNRT_KIND_TRI ? a.template get<uint4>(slots) : nullptr;
     return b;
 }
 
 // Input elements, their tight bounds per scene and the root entries.
 void launch_roots(const LevelBufs& b, const Geometry& G, uint32_t ntot, const RootPlan& R, const RootCounts& c,
-                  const float* given, float* rootbox, hipStream_t st) {
+                  const float* given, float* rootbox, uint32_t* maxlvl, hipStream_t st) {
     const uint32_t S_ = G.num_scenes;
-    hipLaunchKernelGGL(k_build_init, blocks_to(std::max(kWords, 6u * S_), 256, 256), dim3(256), 0, st, b.W, c.na, c.nw,
-                       c.nsmall, c.nse, S_, b.stb);
+    hipLaunchKernelGGL(k_build_init, blocks_to(std::max<uint64_t>({kWords, 6ull * S_, chunks_for(c.nw, c.na)}), 256, 256), dim3(256), 0, st, b.W, c.na, c.nw,
+                       c.nsmall, c.nse, S_, b.stb, maxlvl, b.cs[0]);
     if (ntot > 0)
         hipLaunchKernelGGL(k_init_elems, blocks_for(ntot, kInitBlock * kInitPer), dim3(kInitBlock), 0, st, G, ntot, R,
                            b.X[0], b.Sm, b.stb);
@@ -1650,26 +1711,28 @@ void launch_level(const LevelBufs& b, const Geometry& G, const mnrt_build_params
     L.Nx = b.X[(level + 1u) & 1u];
     L.Sm = b.Sm;
     L.wc = b.wc;
-    L.woff = b.woff;
+    L.cs = b.cs[level & 1u];
+    L.csn = b.cs[(level + 1u) & 1u];
+    L.coff = b.coff;
     L.P = b.P;
     L.S = b.S;
     L.B = b.B;
     L.ll_idx = b.ll_idx;
     L.q = b.q;
-    const dim3 gc = blocks_to(nw, 4, 2048), gn = blocks_to(na, kChildNodes, 512), gs = blocks_to(nw, kScatterWaves, 512);
+    const dim3 gc = blocks_to(nw, kCountWaves, 512), gn = blocks_to(na, kChildNodes, 512), gs = blocks_to(nw, kScatterWaves, 512);
     if (G.kind == MNRT_KIND_TRI) {
-        hipLaunchKernelGGL((k_count<MNRT_KIND_TRI>), gc, dim3(256), 0, st, L);
+        hipLaunchKernelGGL((k_count<MNRT_KIND_TRI>), gc, dim3(kCountBlock), 0, st, L);
         hipLaunchKernelGGL(k_children, gn, dim3(kChildBlock), 0, st, L);
         hipLaunchKernelGGL((k_scatter<MNRT_KIND_TRI>), gs, dim3(kScatterBlock), 0, st, L);
         hipLaunchKernelGGL(k_clip, blocks_to(nw, 1, 2048), dim3(kClipBlock), 0, st, L, G);
     } else {
-        hipLaunchKernelGGL((k_count<MNRT_KIND_POINT>), gc, dim3(256), 0, st, L);
+        hipLaunchKernelGGL((k_count<MNRT_KIND_POINT>), gc, dim3(kCountBlock), 0, st, L);
         hipLaunchKernelGGL(k_children, gn, dim3(kChildBlock), 0, st, L);
         hipLaunchKernelGGL((k_scatter<MNRT_KIND_POINT>), gs, dim3(kScatterBlock), 0, st, L);
     }
 }
 
-// Buffers of the small-node stage and the layout.
+// Buffers of the small-node stage.
 template <typename A>
 SmallOut take_small(A& a, uint32_t* W, const StageCap& cap, uint64_t nsmall, uint64_t nse) {
     const uint64_t total = (uint64_t)cap.mul * nse + (uint64_t)cap.add * nsmall;  // sum over the roots
@@ -1685,19 +1748,8 @@ SmallOut take_small(A& a, uint32_t* W, const StageCap& cap, uint64_t nsmall, uin
     return O;
 }
 
-template <typename A>
-LayoutView take_layout(A& a, uint64_t nbn) {
-    LayoutView v{};
-    v.size = a.template get<uint32_t>(nbn);
-    v.rsize = a.template get<uint32_t>(nbn);
-    v.depth = a.template get<uint32_t>(nbn);
-    v.addr = a.template get<uint32_t>(nbn);
-    v.rbase = a.template get<uint32_t>(nbn);
-    return v;
-}
-
 template <int kMode>
-void launch_small(int kind, DN nsmall, const SmallView& S, const ElemView& Sm, const float* qr, const SmallOut& O,
+void launch_small(int kind, DN nsmall, const SmallRec* S, const ElemView& Sm, const float* qr, const SmallOut& O,
                   hipStream_t st) {
     const dim3 grid((nsmall.v + kSmallWaves - 1) / kSmallWaves), block(64 * kSmallWaves);
     if (kind == MNRT_KIND_TRI)
@@ -1872,7 +1924,7 @@ int build_batch_impl(int kind, const float* d_v0, const float* d_v1, const float
     for (;;) {
         b = take_levels(pool, kind, S_, C);
         if (!pool.ok) return MNRT_ERR_NOMEM;
-        launch_roots(b, G, ntot, RP, c, h_roots ? (const float*)T.given : (const float*)nullptr, T.rootbox, st);
+        launch_roots(b, G, ntot, RP, c, h_roots ? (const float*)T.given : (const float*)nullptr, T.rootbox, T.smaxlvl, st);
         levels = 0;
         for (uint32_t until = first_levels;; until = std::min(levels + 4u, kLevels)) {
             for (; levels < until; ++levels)
@@ -1908,15 +1960,14 @@ int build_batch_impl(int kind, const float* d_v0, const float* d_v1, const float
     const StageCap st_cap = stage_cap_setting();
     if ((uint64_t)st_cap.mul * nse + (uint64_t)st_cap.add * nsmall > 0xFFFFFFFFull) return MNRT_ERR_CAPACITY;
     SmallOut O = take_small(pool, b.W, st_cap, nsmall, nse);
-    const LayoutView Lv = take_layout(pool, nbn);
     if (!pool.ok) return MNRT_ERR_NOMEM;
     if (nsmall > 0) launch_small<kSmallStage>(kind, hn(nsmall), b.S, b.Sm, T.qr, O, st);
     // ---- layout ----
     const dim3 lgrid = blocks_for(nbn);
-    hipLaunchKernelGGL(k_layout_sizes, lgrid, dim3(256), 0, st, hn(nbn), b.B, Lv, (const uint32_t*)O.nsize,
-                       (const uint32_t*)O.rsize, (const uint32_t*)O.mlvl, (uint32_t)MNRT_MAX_LEVEL, b.W);
-    hipLaunchKernelGGL(k_scene_totals, dim3(1), dim3(1024), 0, st, S_, Lv, T.snodes, T.srefs, T.nbase, T.rbase,
-                       T.sleaves, T.smaxlvl, (uint32_t)MNRT_INDEX_MASK, (uint32_t)MNRT_INDEX_MASK, b.W);
+    hipLaunchKernelGGL(k_layout_sizes, lgrid, dim3(256), 0, st, hn(nbn), b.B, (const uint32_t*)O.nsize,
+                       (const uint32_t*)O.rsize, (const uint32_t*)O.mlvl, (uint32_t)MNRT_MAX_LEVEL, T.smaxlvl, b.W);
+    hipLaunchKernelGGL(k_scene_totals, dim3(1), dim3(1024), 0, st, S_, (const BnRec*)b.B, T.snodes, T.srefs, T.nbase,
+                       T.rbase, T.sleaves, (uint32_t)MNRT_INDEX_MASK, (uint32_t)MNRT_INDEX_MASK, b.W);
     MNRT_HIP_CHECK(hipGetLastError());
     uint32_t* h_res = h_tab;
     MNRT_HIP_CHECK(hipMemcpyAsync(h_res, T.rootbox, scene_result_words(S_) * 4, hipMemcpyDeviceToHost, st));
@@ -1938,10 +1989,9 @@ int build_batch_impl(int kind, const float* d_v0, const float* d_v1, const float
         (void)pool_free(d_nodes, st);
         return MNRT_ERR_NOMEM;
     }
-    hipLaunchKernelGGL(k_emit_large, lgrid, dim3(256), 0, st, hn(nbn), b.B, Lv, (const uint32_t*)b.ll_idx, d_nodes,
+    hipLaunchKernelGGL(k_emit_large, lgrid, dim3(256), 0, st, hn(nbn), b.B, (const uint32_t*)b.ll_idx, d_nodes,
                        d_refs, (const uint32_t*)b.W, (const uint32_t*)T.nbase, (const uint32_t*)T.rbase);
-    O.bn_addr = Lv.addr;
-    O.bn_rbase = Lv.rbase;
+    O.bn = b.B;
     O.nodes = d_nodes;
     O.refs = d_refs;
     O.max_nodes = total_nodes;
@@ -2032,7 +2082,6 @@ int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
     const StageCap st_cap = stage_cap_setting();
     if ((uint64_t)st_cap.mul * C.se + (uint64_t)st_cap.add * C.small > 0xFFFFFFFFull) return MNRT_ERR_CAPACITY;
     SmallOut O = take_small(cv, b.W, st_cap, C.small, C.se);
-    const LayoutView Lv = take_layout(cv, C.bn);
     // outputs
     uint32_t* nodes = cv.get<uint32_t>(2ull * g.cap_nodes);
     uint32_t* refs = cv.get<uint32_t>(g.cap_refs);
@@ -2062,7 +2111,7 @@ int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
     Geometry G{kind, (const float4*)g.v0, g.v1 ? (const float4*)g.v1 : (const float4*)g.v0,
                g.v2 ? (const float4*)g.v2 : (const float4*)g.v0, T.base, S_};
     launch_roots(b, G, ntot, RootPlan{T.pkind, T.pindex, T.poff}, bs.roots,
-                 g.h_roots.empty() ? (const float*)nullptr : (const float*)T.given, T.rootbox, st);
+                 g.h_roots.empty() ? (const float*)nullptr : (const float*)T.given, T.rootbox, T.smaxlvl, st);
     MNRT_HIP_CHECK(hipGetLastError());
     for (uint32_t l = 0; l < g.levels; ++l) {
         const size_t pl = std::min<size_t>(l, bs.level_na.size() - 1);
@@ -2078,15 +2127,14 @@ int graph_record(mnrt_build_graph& g, char* base, hipStream_t st) {
     // a replay deeper than the first build's depth and a few levels more sets kErrLayoutDepth
     const uint32_t top = std::min<uint32_t>(bs.maxlvl + kLayoutSpareLevels, MNRT_MAX_LEVEL);
     const dim3 lgrid = blocks_for(planned(bs.nbn, 256, C.bn));
-    hipLaunchKernelGGL(k_layout_sizes, lgrid, dim3(256), 0, st, nbn, b.B, Lv, (const uint32_t*)O.nsize,
-                       (const uint32_t*)O.rsize, (const uint32_t*)O.mlvl, top, b.W);
-    hipLaunchKernelGGL(k_scene_totals, dim3(1), dim3(1024), 0, st, S_, Lv, T.snodes, T.srefs, T.nbase, T.rbase,
-                       T.sleaves, T.smaxlvl, g.cap_nodes, g.cap_refs, b.W);
+    hipLaunchKernelGGL(k_layout_sizes, lgrid, dim3(256), 0, st, nbn, b.B, (const uint32_t*)O.nsize,
+                       (const uint32_t*)O.rsize, (const uint32_t*)O.mlvl, top, T.smaxlvl, b.W);
+    hipLaunchKernelGGL(k_scene_totals, dim3(1), dim3(1024), 0, st, S_, (const BnRec*)b.B, T.snodes, T.srefs, T.nbase,
+                       T.rbase, T.sleaves, g.cap_nodes, g.cap_refs, b.W);
     // emission (each kernel returns at once when W[W_ERR] is set)
-    hipLaunchKernelGGL(k_emit_large, lgrid, dim3(256), 0, st, nbn, b.B, Lv, (const uint32_t*)b.ll_idx, nodes, refs,
+    hipLaunchKernelGGL(k_emit_large, lgrid, dim3(256), 0, st, nbn, b.B, (const uint32_t*)b.ll_idx, nodes, refs,
                        (const uint32_t*)b.W, (const uint32_t*)T.nbase, (const uint32_t*)T.rbase);
-    O.bn_addr = Lv.addr;
-    O.bn_rbase = Lv.rbase;
+    O.bn = b.B;
     O.nodes = nodes;
     O.refs = refs;
     O.max_nodes = g.cap_nodes;

@@ -175,6 +175,27 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
     return (row_lane(v, 0) + row_lane(v, 1)) + (row_lane(v, 2) + row_lane(v, 3));
 }
 
+// Inclusive prefix sums: within rows of 16 lanes (each lane adds the lanes 1, 2, 4, 8 before it
+// in its row), then over the wave (the last lane of a row goes to the next row, lane 31 to the
+// upper half).
+__device__ __forceinline__ uint32_t row_scan_u32(uint32_t v) {
+    v += dpp_mov<0x111>(v);
+    v += dpp_mov<0x112>(v);
+    v += dpp_mov<0x114>(v);
+    v += dpp_mov<0x118>(v);
+    return v;
+}
+
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+    v = row_scan_u32(v);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
+// The last lane's value of each row, in all its lanes.
+__device__ __forceinline__ uint32_t row_last(uint32_t v) { return __shfl(v, (int)(threadIdx.x & 63u) | 15, 64); }
+
 template <int kCtrl>
 __device__ __forceinline__ long long dpp_mov64(long long v) {
     const uint32_t lo = dpp_mov<kCtrl>((uint32_t)(unsigned long long)v);
