@@ -410,7 +410,9 @@ extern "C" int mnrt_batch_create(const mnrt_batch_desc* d, mnrt_batch** out) {
     if (rc == MNRT_OK) {
         mnrt_batch_tuning& t = b->tun;
         t.trace_block = 256;
-        t.trace_tile = 1024;
+        // a wave's share of a tile is one set of rays until the tiles fill the chip (131072 rays of 32
+        // scenes are 512 workgroups, not 128), then a run that refills
+        t.trace_tile = b->total_slots >= (1u << 20) ? 1024 : 256;
         t.trace_grid = 8 * b->cus;
         t.trace_stack = smallest_stack(b->max_level);
         t.knn_waves = 4;

@@ -193,6 +193,15 @@ __device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
     return v;
 }
 
+__device__ __forceinline__ uint32_t wave_max_scan_u32(uint32_t v) {
+    v = max(v, dpp_mov<0x111>(v));
+    v = max(v, dpp_mov<0x112>(v));
+    v = max(v, dpp_mov<0x114>(v));
+    v = max(v, dpp_mov<0x118>(v));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+}
+
 // The last lane's value of each row, in all its lanes.
 __device__ __forceinline__ uint32_t row_last(uint32_t v) { return __shfl(v, (int)(threadIdx.x & 63u) | 15, 64); }
 

@@ -49,40 +49,49 @@ struct PhotonArgs {
     uint32_t* path_tris;  // 4 per slot: triangles scattered from before this photon
 };
 
-__global__ __launch_bounds__(256) void k_photon_paths(PhotonArgs A) {
-    extern __shared__ uint32_t s_stack[];
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.num_paths) return;
-    const uint32_t path = A.path_begin + i;
-    const uint32_t slots = A.max_bounces + 1;
-    const size_t base = (size_t)i * slots;
-    for (uint32_t b = 0; b < slots; ++b) A.valid[base + b] = 0u;
+// Paths of a run; a lane's next ray is its path's next bounce, or the next path.
+struct PathSource {
+    uint32_t next, end;
+    RayDeal deal;
+    const PhotonArgs& A;
+    uint32_t path, light, bounce;
+    float pr, pg, pb;
+    uint32_t tris[4];
 
-    const uint32_t light = path % A.num_lights;
-    float4 c = A.lights[4 * light + 0], eu = A.lights[4 * light + 1], ev = A.lights[4 * light + 2];
-    float4 lp = A.lights[4 * light + 3];
-    float u = rnd01(A.seed, path, 0xFFFFu, 0), v = rnd01(A.seed, path, 0xFFFFu, 1);
-    f3 o = mk3(c.x + u * eu.x + v * ev.x, c.y + u * eu.y + v * ev.y, c.z + u * eu.z + v * ev.z);
-    f3 ln = unit_normal(xyz(eu), xyz(ev));
-    f3 d = cosine_dir(ln, A.seed, path, 0xFFFEu);
-    float nl = (float)A.num_lights;
-    float pr = lp.x * nl, pg = lp.y * nl, pb = lp.z * nl;
-    uint32_t tris[4] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
-
-    for (uint32_t b = 0; b < slots; ++b) {
-        Hit h = trace_ray<kTraceStack, kTraceLds>(A.nodes, A.recs, A.root, o, d, A.eps, s_stack + threadIdx.x,
-                                                  blockDim.x);
-        if (h.tri < 0) break;
+    __device__ __forceinline__ bool start(uint32_t i, f3& o, f3& d, float&) {
+        const uint64_t at = deal.ray(i);
+        if (at >= deal.n) return false;
+        i = path = (uint32_t)at;
+        const uint32_t p = A.path_begin + i, slots = A.max_bounces + 1;
+        for (uint32_t b = 0; b < slots; ++b) A.valid[(size_t)i * slots + b] = 0u;
+        light = p % A.num_lights;
+        float4 c = A.lights[4 * light + 0], eu = A.lights[4 * light + 1], ev = A.lights[4 * light + 2];
+        float4 lp = A.lights[4 * light + 3];
+        float u = rnd01(A.seed, p, 0xFFFFu, 0), v = rnd01(A.seed, p, 0xFFFFu, 1);
+        o = mk3(c.x + u * eu.x + v * ev.x, c.y + u * eu.y + v * ev.y, c.z + u * eu.z + v * ev.z);
+        f3 ln = unit_normal(xyz(eu), xyz(ev));
+        d = cosine_dir(ln, A.seed, p, 0xFFFEu);
+        float nl = (float)A.num_lights;
+        pr = lp.x * nl;
+        pg = lp.y * nl;
+        pb = lp.z * nl;
+        for (int k = 0; k < 4; ++k) tris[k] = 0xFFFFFFFFu;
+        bounce = 0;
+        return true;
+    }
+    __device__ __forceinline__ bool finish(f3& o, f3& d, float, const Hit& h) {
+        const uint32_t b = bounce, p = A.path_begin + path, slots = A.max_bounces + 1;
+        if (h.tri < 0) return false;
         float4 alb = A.albedo[h.tri];
-        if (!(alb.x > 0.0f || alb.y > 0.0f || alb.z > 0.0f)) break;
+        if (!(alb.x > 0.0f || alb.y > 0.0f || alb.z > 0.0f)) return false;
         f3 x = mk3(o.x + d.x * h.t, o.y + d.y * h.t, o.z + d.z * h.t);
         if (b > 3) {
-            if (!(rnd01(A.seed, path, b, 100) <= 0.5f)) break;
+            if (!(rnd01(A.seed, p, b, 100) <= 0.5f)) return false;
             pr = pr * 2.0f;
             pg = pg * 2.0f;
             pb = pb * 2.0f;
         }
-        size_t s = base + b;
+        size_t s = (size_t)path * slots + b;
         A.valid[s] = 1u;
         A.pos[s] = make_float4(x.x, x.y, x.z, 0.0f);
         A.pw[s] = make_float4(pr, pg, pb, 0.0f);
@@ -90,17 +99,28 @@ __global__ __launch_bounds__(256) void k_photon_paths(PhotonArgs A) {
         if (A.meta) A.meta[s] = light | (b << 8);
         if (A.path_tris)
             for (int k = 0; k < 4; ++k) A.path_tris[4 * s + k] = tris[k];
-        if (b + 1 >= slots) break;
+        if (b + 1 >= slots) return false;
         float4 a0 = A.v0[h.tri], a1 = A.v1[h.tri], a2 = A.v2[h.tri];
         f3 n = unit_normal(mk3(a1.x - a0.x, a1.y - a0.y, a1.z - a0.z), mk3(a2.x - a0.x, a2.y - a0.y, a2.z - a0.z));
         if (dot3(n, d) > 0.0f) n = mk3(n.x * -1.0f, n.y * -1.0f, n.z * -1.0f);
-        d = cosine_dir(n, A.seed, path, b);
+        d = cosine_dir(n, A.seed, p, b);
         o = x;
         pr = pr * alb.x;
         pg = pg * alb.y;
         pb = pb * alb.z;
-        if (b < 4) tris[b] = (uint32_t)h.tri;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (b == k) tris[k] = (uint32_t)h.tri;
+        bounce = b + 1;
+        return true;
     }
+};
+
+__global__ __launch_bounds__(64) void k_photon_paths(PhotonArgs A, uint32_t width) {
+    __shared__ __align__(8) uint32_t s_wave[kTraceWords];
+    const RayDeal deal{blockIdx.x, gridDim.x, A.num_paths, width};
+    PathSource src{0u, deal.count(), deal, A};
+    trace_stream<false, kTraceStack>(A.nodes, A.recs, A.root, A.eps, 0.0f, width, s_wave, src);
 }
 
 // Stable compaction of the valid slots into the output, up to `limit` photons.
@@ -210,7 +230,8 @@ extern "C" int mnrt_photons_generate(const mnrt_tree* tree, const float* d_v0, c
         uint32_t* scr = tot + 4;
         A.path_begin = shot;
         A.num_paths = np;
-        hipLaunchKernelGGL(k_photon_paths, dim3((np + 255) / 256), dim3(256), trace_lds_bytes(kTraceLds, 256), st, A);
+        const uint32_t width = trace_width(np);
+        hipLaunchKernelGGL(k_photon_paths, dim3(trace_waves(np, width)), dim3(64), 0, st, A, width);
         if (scan_exclusive(A.valid, pos, (uint32_t)nslots, tot, scr, st) != hipSuccess) {
             rc = MNRT_ERR_HIP;
             break;

@@ -2,9 +2,9 @@
 //
 // Replaces kernel_SampleAreaLight, kernel_TraceShadowRaysDelta and
 // kernel_TraceShadowRaysArea (raytracing.cu:963-1114), which call the kd-tree traversal
-// with needClosest = false.  One lane per segment, 256-lane workgroups; the segment is
+// with needClosest = false.  One wave per run of segments (trace_dev.h); a segment is
 // built in registers (no intermediate ray arrays), the top of the traversal stack lives
-// in LDS and the search stops at the first occluder (trace_any in trace_dev.h).
+// in LDS and the search stops at the first occluder.
 // Differences from the reference, all deliberate:
 //   * the light is a kernel argument instead of __constant__ c_LightData, the tree an
 //     argument instead of the bound KDTreeData;
@@ -106,46 +106,59 @@ enum : int { kSegPoint = 0, kSegDirectional = 1, kSegArea = 2, kSegExplicit = 3 
 // out = 1 when unoccluded.  kSegExplicit: ray (pts[i], dirs[i]) limited by tmax[i],
 // out = 1 when something is hit.
 template <int kMode>
-__global__ __launch_bounds__(256) void k_any_hit(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
-                                                 RootBox root, LightArgs L, uint32_t n,
-                                                 const float4* __restrict__ pts, const float4* __restrict__ dirs,
-                                                 const float* __restrict__ tmax, float eps,
-                                                 uint32_t* __restrict__ out) {
-    extern __shared__ uint32_t s_stack[];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t* lane = s_stack + threadIdx.x;
-    const f3 p = xyz(pts[i]);
-    if (kMode == kSegExplicit) {
-        const float lim = tmax ? tmax[i] : kInf;
-        out[i] = trace_any<kTraceStack, kTraceLds>(nodes, recs, root, p, xyz(dirs[i]), eps, lim, 0.0f, lane,
-                                                   blockDim.x)
-                     ? 1u : 0u;
-        return;
-    }
-    f3 d;
-    float dist = kInf, slack = 0.0f;
-    if (kMode == kSegDirectional) {
-        d = mk3(-L.dir.x, -L.dir.y, -L.dir.z);
-    } else {
-        const f3 target = (kMode == kSegArea) ? xyz(dirs[i]) : L.pos;
-        const f3 v = sub3(target, p);
-        dist = sqrtf(dot3(v, v));
-        if (!(dist > 0.0f)) {
-            out[i] = (kMode == kSegPoint) ? 1u : 0u;
-            return;
-        }
-        d = mk3(v.x / dist, v.y / dist, v.z / dist);
-        if (kMode == kSegArea) {
-            slack = eps;
-            if (!(dot3(mk3(-d.x, -d.y, -d.z), L.dir) > 0.0f)) {
+struct SegSource {
+    uint32_t next, end;
+    RayDeal deal;
+    const LightArgs& L;
+    const float4* __restrict__ pts;
+    const float4* __restrict__ dirs;
+    const float* __restrict__ tmax;
+    uint32_t* __restrict__ out;
+    uint32_t seg = 0;
+
+    __device__ __forceinline__ bool start(uint32_t i, f3& o, f3& d, float& dist) {
+        const uint64_t at = deal.ray(i);
+        if (at >= deal.n) return false;
+        i = seg = (uint32_t)at;
+        o = xyz(pts[i]);
+        dist = kInf;
+        if (kMode == kSegExplicit) {
+            if (tmax) dist = tmax[i];
+            d = xyz(dirs[i]);
+        } else if (kMode == kSegDirectional) {
+            d = mk3(-L.dir.x, -L.dir.y, -L.dir.z);
+        } else {
+            const f3 target = (kMode == kSegArea) ? xyz(dirs[i]) : L.pos;
+            const f3 v = sub3(target, o);
+            dist = sqrtf(dot3(v, v));
+            if (!(dist > 0.0f)) {
+                out[i] = (kMode == kSegPoint) ? 1u : 0u;
+                return false;
+            }
+            d = mk3(v.x / dist, v.y / dist, v.z / dist);
+            if (kMode == kSegArea && !(dot3(mk3(-d.x, -d.y, -d.z), L.dir) > 0.0f)) {
                 out[i] = 0u;
-                return;
+                return false;
             }
         }
+        return true;
     }
-    out[i] = trace_any<kTraceStack, kTraceLds>(nodes, recs, root, p, d, eps, dist, slack, lane, blockDim.x) ? 0u
-                                                                                                             : 1u;
+    __device__ __forceinline__ bool finish(f3&, f3&, float, const Hit& h) {
+        out[seg] = (h.tri >= 0) == (kMode == kSegExplicit) ? 1u : 0u;
+        return false;
+    }
+};
+
+template <int kMode>
+__global__ __launch_bounds__(64) void k_any_hit(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
+                                                RootBox root, LightArgs L, uint32_t n, uint32_t width,
+                                                const float4* __restrict__ pts, const float4* __restrict__ dirs,
+                                                const float* __restrict__ tmax, float eps,
+                                                uint32_t* __restrict__ out) {
+    __shared__ __align__(8) uint32_t s_wave[kTraceWords];
+    const RayDeal deal{blockIdx.x, gridDim.x, n, width};
+    SegSource<kMode> src{0u, deal.count(), deal, L, pts, dirs, tmax, out};
+    trace_stream<true, kTraceStack>(nodes, recs, root, eps, kMode == kSegArea ? eps : 0.0f, width, s_wave, src);
 }
 
 static int launch_any_hit(int mode, const mnrt_tree* tree, const LightArgs& L, uint32_t n, const float* d_pts4,
@@ -159,27 +172,27 @@ static int launch_any_hit(int mode, const mnrt_tree* tree, const LightArgs& L, u
         rb.lo[a] = tree->root_min[a];
         rb.hi[a] = tree->root_max[a];
     }
-    const dim3 grid((n + 255) / 256), block(256);
-    const uint32_t lds = trace_lds_bytes(kTraceLds, 256);
+    const uint32_t width = trace_width(n);
+    const dim3 grid(trace_waves(n, width)), block(64);
     const uint2* nodes = (const uint2*)tree->d_nodes;
     const float4* recs = (const float4*)tree->d_recs;
     const float4* pts = (const float4*)d_pts4;
     const float4* dirs = (const float4*)d_dirs4;
     switch (mode) {
         case kSegPoint:
-            hipLaunchKernelGGL(k_any_hit<kSegPoint>, grid, block, lds, st, nodes, recs, rb, L, n, pts, dirs, d_tmax,
+            hipLaunchKernelGGL(k_any_hit<kSegPoint>, grid, block, 0, st, nodes, recs, rb, L, n, width, pts, dirs, d_tmax,
                                eps, d_out);
             break;
         case kSegDirectional:
-            hipLaunchKernelGGL(k_any_hit<kSegDirectional>, grid, block, lds, st, nodes, recs, rb, L, n, pts, dirs,
+            hipLaunchKernelGGL(k_any_hit<kSegDirectional>, grid, block, 0, st, nodes, recs, rb, L, n, width, pts, dirs,
                                d_tmax, eps, d_out);
             break;
         case kSegArea:
-            hipLaunchKernelGGL(k_any_hit<kSegArea>, grid, block, lds, st, nodes, recs, rb, L, n, pts, dirs, d_tmax,
+            hipLaunchKernelGGL(k_any_hit<kSegArea>, grid, block, 0, st, nodes, recs, rb, L, n, width, pts, dirs, d_tmax,
                                eps, d_out);
             break;
         default:
-            hipLaunchKernelGGL(k_any_hit<kSegExplicit>, grid, block, lds, st, nodes, recs, rb, L, n, pts, dirs,
+            hipLaunchKernelGGL(k_any_hit<kSegExplicit>, grid, block, 0, st, nodes, recs, rb, L, n, width, pts, dirs,
                                d_tmax, eps, d_out);
             break;
     }

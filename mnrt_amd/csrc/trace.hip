@@ -2,7 +2,7 @@
 //
 // Replaces kernel_FindIntersections + dev_FindNextIntersectionKDWhileWhile<true>
 // (raytracing.cu:503-645, 854-879) and its wrapper KernelRTTraceRays
-// (raytracing.cu:1617-1635).  One lane per ray, 256-lane workgroups.  Differences from
+// (raytracing.cu:1617-1635).  One wave per run of rays (trace_dev.h).  Differences from
 // the reference, all deliberate:
 //   * the tree and triangles are kernel arguments (no __constant__ / texture binding),
 //     so several trees can be traced at once;
@@ -18,22 +18,58 @@
 
 namespace mnrt {
 
-__global__ __launch_bounds__(256) void k_trace_closest(
-    const uint2* __restrict__ nodes, const float4* __restrict__ recs, RootBox root, uint32_t n,
+// Rays first..last of arrays; results as they are asked for.
+struct RaySource {
+    uint32_t next, end;
+    RayDeal deal;
+    uint32_t first;
+    const float4* __restrict__ orig;
+    const float4* __restrict__ dir;
+    const float4* __restrict__ recs;
+    int32_t* __restrict__ out_tri;
+    float* __restrict__ out_t;
+    float2* __restrict__ out_bary;
+    float4* __restrict__ out_pt;
+    uint32_t* __restrict__ out_valid;
+    uint32_t ray = 0;
+
+    __device__ __forceinline__ bool start(uint32_t i, f3& o, f3& d, float&) {
+        const uint64_t at = deal.ray(i);
+        if (at >= deal.n) return false;
+        i = ray = first + (uint32_t)at;
+        o = xyz(orig[i]);
+        d = xyz(dir[i]);
+        return true;
+    }
+    __device__ __forceinline__ bool finish(f3& o, f3& d, float, const Hit& h) {
+        const bool hit = h.tri >= 0;
+        const float t = hit ? h.t : 0.0f;
+        out_tri[ray] = h.tri;
+        if (out_t) out_t[ray] = t;
+        if (out_bary) {
+            float lam, u = 0.0f, v = 0.0f;
+            if (hit) {  // the hit's test again: the same operations, the same bits
+                const float4* r = recs + 3ull * h.rec;
+                ray_tri(xyz(r[0]), xyz(r[1]), xyz(r[2]), o, d, lam, u, v);
+            }
+            out_bary[ray] = make_float2(u, v);
+        }
+        if (out_pt) out_pt[ray] = make_float4(o.x + d.x * t, o.y + d.y * t, o.z + d.z * t, 0.0f);
+        if (out_valid) out_valid[ray] = hit ? 1u : 0u;
+        return false;
+    }
+};
+
+// One wave per workgroup: its LDS goes to the next when its own run is done.
+__global__ __launch_bounds__(64) void k_trace_closest(
+    const uint2* __restrict__ nodes, const float4* __restrict__ recs, RootBox root, uint32_t n, uint32_t width,
     const float4* __restrict__ orig, const float4* __restrict__ dir, float eps,
     int32_t* __restrict__ out_tri, float* __restrict__ out_t, float2* __restrict__ out_bary,
     float4* __restrict__ out_pt, uint32_t* __restrict__ out_valid) {
-    extern __shared__ uint32_t s_stack[];
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    f3 o = xyz(orig[i]);
-    f3 d = xyz(dir[i]);
-    Hit h = trace_ray<kTraceStack, kTraceLds>(nodes, recs, root, o, d, eps, s_stack + threadIdx.x, blockDim.x);
-    out_tri[i] = h.tri;
-    if (out_t) out_t[i] = h.t;
-    if (out_bary) out_bary[i] = make_float2(h.u, h.v);
-    if (out_pt) out_pt[i] = make_float4(o.x + d.x * h.t, o.y + d.y * h.t, o.z + d.z * h.t, 0.0f);
-    if (out_valid) out_valid[i] = h.tri >= 0 ? 1u : 0u;
+    __shared__ __align__(8) uint32_t s_wave[kTraceWords];
+    const RayDeal deal{blockIdx.x, gridDim.x, n, width};
+    RaySource src{0u, deal.count(), deal, 0u, orig, dir, recs, out_tri, out_t, out_bary, out_pt, out_valid};
+    trace_stream<false, kTraceStack>(nodes, recs, root, eps, 0.0f, width, s_wave, src);
 }
 
 }  // namespace mnrt
@@ -52,10 +88,10 @@ extern "C" int mnrt_trace_closest(const mnrt_tree* tree, uint32_t n, const float
         rb.lo[a] = tree->root_min[a];
         rb.hi[a] = tree->root_max[a];
     }
-    dim3 block(256), grid((n + 255) / 256);
-    hipLaunchKernelGGL(mnrt::k_trace_closest, grid, block, mnrt::trace_lds_bytes(mnrt::kTraceLds, 256),
+    const uint32_t width = mnrt::trace_width(n);
+    hipLaunchKernelGGL(mnrt::k_trace_closest, dim3(mnrt::trace_waves(n, width)), dim3(64), 0,
                        (hipStream_t)stream,
-                       (const uint2*)tree->d_nodes, (const float4*)tree->d_recs, rb, n,
+                       (const uint2*)tree->d_nodes, (const float4*)tree->d_recs, rb, n, width,
                        (const float4*)d_orig4, (const float4*)d_dir4, eps, d_out_tri, d_out_t,
                        (float2*)d_out_bary2, (float4*)d_out_pt4, d_out_valid);
     MNRT_HIP_CHECK(hipGetLastError());
@@ -71,11 +107,12 @@ namespace mnrt {
 // mod 8 on MI355X) has its own counter over a contiguous share of the tiles, so an
 // XCD's L2 holds the trees of the scenes it traces; a workgroup whose share is done
 // takes tiles from the next XCD's share.
+// Each wave of a workgroup traces its share of a tile as one run.
 template <int kStack>
 __global__ __launch_bounds__(256) void k_trace_batch(TraceBatchArgs B) {
     __shared__ uint32_t s_tile;
-    extern __shared__ uint32_t s_stack[];
-    const uint32_t xcd = blockIdx.x % B.num_parts;
+    extern __shared__ __align__(8) uint32_t s_waves[];
+    const uint32_t xcd = blockIdx.x % B.num_parts, wave = uniform(threadIdx.x >> 6), waves = blockDim.x >> 6;
     for (uint32_t part = 0; part < B.num_parts; ++part) {
         const uint32_t p = (xcd + part) % B.num_parts;
         const uint32_t end = B.part_end[p];
@@ -88,28 +125,22 @@ __global__ __launch_bounds__(256) void k_trace_batch(TraceBatchArgs B) {
             const uint32_t s = seg_of(B.tile_begin, B.num_scenes, t);
             const TraceScene& d = B.scenes[s];
             const uint32_t first = d.ray_begin + (t - B.tile_begin[s]) * B.tile_rays;
-            const uint32_t last = min(first + B.tile_rays, d.ray_end);
+            const RayDeal deal{wave, waves, min(B.tile_rays, d.ray_end - first), 64u};
             RootBox root;
             for (int a = 0; a < 3; ++a) {
                 root.lo[a] = d.lo[a];
                 root.hi[a] = d.hi[a];
             }
-            for (uint32_t i = first + threadIdx.x; i < last; i += blockDim.x) {
-                f3 o = xyz(B.orig[i]);
-                f3 dd = xyz(B.dir[i]);
-                Hit h = trace_ray<kStack, kTraceLds>(d.nodes, d.recs, root, o, dd, d.eps, s_stack + threadIdx.x,
-                                                     blockDim.x);
-                B.out_tri[i] = h.tri;
-                if (B.out_t) B.out_t[i] = h.t;
-                if (B.out_bary) B.out_bary[i] = make_float2(h.u, h.v);
-            }
+            RaySource src{0u, deal.count(), deal, first, B.orig, B.dir, d.recs, B.out_tri, B.out_t, B.out_bary, nullptr,
+                          nullptr};
+            trace_stream<false, kStack>(d.nodes, d.recs, root, d.eps, 0.0f, 64u, s_waves + wave * kTraceWords, src);
         }
     }
 }
 
 int launch_trace_batch(const TraceBatchArgs& B, int stack, uint32_t grid, uint32_t block, hipStream_t st) {
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, B.work, B.num_parts, 0u);
-    const uint32_t lds = trace_lds_bytes(kTraceLds, block);
+    const uint32_t lds = 4u * kTraceWords * (block / 64u);
     switch (stack) {
         case 16: hipLaunchKernelGGL(k_trace_batch<16>, dim3(grid), dim3(block), lds, st, B); break;
         case 24: hipLaunchKernelGGL(k_trace_batch<24>, dim3(grid), dim3(block), lds, st, B); break;

@@ -14,6 +14,19 @@
 //   * the stack is bounded by the build's level cap; its top kLds entries per lane live
 //     in LDS, deeper ones in the lane's private array (the reference keeps the whole
 //     stack in local memory).
+//
+// A wave traces a run of rays (trace_stream), not one ray per lane to its end.  With a lane per
+// ray the wave steps until its longest ray is done and tests as many triangles per leaf as the
+// fullest leaf among its lanes holds: for bounce rays 10 % of the lanes worked (47 k wave
+// instructions per 64 rays, 68 triangle tests a ray).  So
+//   * a lane whose ray is done takes the next ray of the wave's run, kRefill lanes at a time;
+//   * lanes walk to their next leaf until fewer than kWalkMin still walk, and wait there;
+//   * the waiting leaves' (ray, triangle) pairs are dealt to all lanes, 64 at a time, unless the lanes' own leaves are about as full as each other, as they are
+//     for camera rays, when each lane tests its own.
+// Bound by instruction issue: about 25 k vector instructions per 64 bounce rays of the 1.03M-triangle
+// scene (206 walk steps with 29 lanes, 85 dealt tests with 49 pairs, 37 own tests), 83 tests and 93
+// steps a ray.  2.07M bounce rays 2612 -> 1670 us, 785 k area-light shadow rays 962 -> 672 us, 6144
+// camera rays 65 -> 44 us.
 #pragma once
 
 #include "mnrt_common.h"
@@ -26,96 +39,96 @@ struct RootBox {
 
 struct Hit {
     int32_t tri;
-    float t, u, v;
+    float t;
+    uint32_t rec;  // the triangle's record
 };
 
 constexpr int kTraceStack = MNRT_MAX_LEVEL + 2;
 
-// LDS entries per lane of the traversal stack.  On the 1M-triangle workload about 0.5 %
-// of pushes land deeper than 8 entries and 5 % deeper than 6.
-#ifndef MNRT_TRACE_LDS
-#define MNRT_TRACE_LDS 6
-#endif
-constexpr int kTraceLds = MNRT_TRACE_LDS;
+// LDS entries per lane of the traversal stack: as many as leave room for 24 waves on a CU.  On
+// the 1M-triangle workload 5 % of pushes land deeper than 6 entries, so some lane of a wave often
+// goes to scratch memory there; 6 entries instead of 7: 1670 -> 1721 us.
+constexpr int kTraceLds = 7;
 
-// LDS bytes a workgroup of `block` lanes needs for kLds stack entries per lane.
-__host__ __device__ constexpr uint32_t trace_lds_bytes(int lds, uint32_t block) {
-    return (uint32_t)lds * 3u * 4u * block;
+// Waves of a launch: at most the 24 per CU that run at once (74 registers, 6.4 KB of LDS); tiles of
+// 64 rays are dealt to them in turn.  A few more and a second round of waves runs almost alone
+// (6400: 2190 us, 6144: 1670 us).
+constexpr uint32_t kTraceWaves = 6144;
+
+// Rays a wave traces at once: 64, or fewer where a launch would leave SIMDs without a wave: its
+// longest ray and fullest leaves are then shorter, and the spare lanes test triangles.
+// 6144 camera rays: 16 a wave 44 us, 64 a wave 69 us.
+constexpr uint64_t kTraceSimds = 1024;
+inline uint32_t trace_width(uint64_t n) { return n >= 64u * kTraceSimds ? 64u : n >= 32u * kTraceSimds ? 32u : 16u; }
+
+// Of 64 rays, the lanes that take new rays together and the least number that goes on walking while
+// others wait at leaves.  16..32 and 6..16 are within 4 % of each other on bounce rays, shadow rays
+// and photon paths; fewer walkers suit small launches.
+constexpr uint32_t kRefill = 24, kWalkMin = 10;
+
+// LDS words of a wave: pair owners and best records (64 each), best keys (64 x 2), stack.
+constexpr uint32_t kTraceWords = 256u + 3u * 64u * (uint32_t)kTraceLds;
+
+inline uint32_t trace_waves(uint64_t n, uint32_t width) {
+    const uint64_t tiles = (n + width - 1u) / width;
+    return (uint32_t)(tiles < kTraceWaves ? tiles : kTraceWaves);
 }
 
-// Per-lane traversal stack of kStack entries (node, tmin, tmax).  Entry e < kLds is in
-// LDS at words (3e + c) * stride + lane (c = node, tmin, tmax: lanes of a wave touch
-// consecutive banks); deeper entries in a private array.  kStack entries suffice for a
-// tree of max level <= kStack: the entries are far children of distinct levels of the
-// current path.
-template <int kStack, int kLds>
-struct LaneStack {
-    static constexpr int kPriv = kStack > kLds ? kStack - kLds : 1;
-    __attribute__((address_space(3))) uint32_t* lds;  // this lane's column: lds_base + lane
-    uint32_t stride;
-    uint32_t pnode[kPriv];
-    float pmin[kPriv], pmax[kPriv];
-
-    __device__ __forceinline__ void put(int e, uint32_t node, float a, float b) {
-        if (kLds > 0 && e < kLds) {
-            lds[(3 * e) * stride] = node;
-            lds[(3 * e + 1) * stride] = __float_as_uint(a);
-            lds[(3 * e + 2) * stride] = __float_as_uint(b);
-        } else {
-            pnode[e - kLds] = node;
-            pmin[e - kLds] = a;
-            pmax[e - kLds] = b;
-        }
+// The rays of wave w of waves, numbered 0..count: tiles w, w + waves, ... (width rays each) of n.
+struct RayDeal {
+    uint32_t w, waves, n, width;  // width: a power of two
+    __device__ __forceinline__ uint32_t count() const {
+        const uint32_t tiles = (uint32_t)(((uint64_t)n + width - 1u) / width);
+        return tiles > w ? width * ((tiles - w - 1u) / waves + 1u) : 0u;
     }
-    __device__ __forceinline__ float tmin_of(int e) const {
-        if (kLds > 0 && e < kLds) return __uint_as_float(lds[(3 * e + 1) * stride]);
-        return pmin[e - kLds];
-    }
-    __device__ __forceinline__ void get(int e, uint32_t& node, float& a, float& b) const {
-        if (kLds > 0 && e < kLds) {
-            node = lds[(3 * e) * stride];
-            a = __uint_as_float(lds[(3 * e + 1) * stride]);
-            b = __uint_as_float(lds[(3 * e + 2) * stride]);
-        } else {
-            node = pnode[e - kLds];
-            a = pmin[e - kLds];
-            b = pmax[e - kLds];
-        }
+    __device__ __forceinline__ uint64_t ray(uint32_t i) const {
+        return (uint64_t)width * ((uint64_t)(i / width) * waves + w) + (i & (width - 1u));
     }
 };
 
-// Descends from `node` over [tmin, tmax] to a leaf, pushing far children; returns the
-// leaf's node word.
-template <int kStack, int kLds>
-__device__ __forceinline__ uint2 descend(const uint2* __restrict__ nodes, LaneStack<kStack, kLds>& st, int& sp,
-                                         uint32_t& node, float& tmin, float& tmax, f3 o, f3 d, f3 inv) {
-    uint2 nd = nodes[node];
-    while (!is_leaf(nd.y)) {
-        uint32_t a = nd.y >> 30;
-        float s = __uint_as_float(nd.x);
-        uint32_t left = node + 1, right = nd.y & MNRT_INDEX_MASK;
-        float oa = comp(o, a), da = comp(d, a), ia = comp(inv, a);
-        float tsplit = (s - oa) * ia;
-        bool below = (oa < s) || (oa == s && da > 0.0f);
-        uint32_t first = below ? left : right, second = below ? right : left;
-        if (tsplit != tsplit) {
-            if (sp < kStack) st.put(sp++, second, tmin, tmax);
-            node = first;
-        } else if (tsplit < 0.0f || tsplit > tmax * kTravTolHi) {
-            node = first;
-        } else if (tsplit < tmin * kTravTolLo) {
-            node = second;
-        } else {
-            if (sp < kStack) st.put(sp++, second, fmaxf(tmin, tsplit * kTravTolLo), tmax);
-            tmax = fminf(tmax, tsplit * kTravTolHi);
-            node = first;
-        }
-        nd = nodes[node];
+// Per-lane traversal stack of kStack entries (node, tmin, tmax).  Entry e < kTraceLds is in
+// LDS, (node, tmin) at pair e * 64 + lane and tmax at word e * 64 + lane of an array of its own
+// (lanes of a wave touch consecutive banks); deeper entries in a private array.  kStack entries
+// suffice for a tree of max level <= kStack: the entries are far children of distinct levels of the
+// current path.
+// (Only the array is a struct in memory: a pointer beside it would be loaded from scratch too.)
+template <int kStack>
+struct DeepStack {
+    static constexpr int kPriv = kStack > kTraceLds ? kStack - kTraceLds : 1;
+    unsigned long long lo[kPriv];
+    float hi[kPriv];
+};
+struct LdsStack {
+    __attribute__((address_space(3))) unsigned long long* lo;
+    __attribute__((address_space(3))) float* hi;
+};
+template <int kStack>
+__device__ __forceinline__ void stack_put(const LdsStack& l, DeepStack<kStack>& m, int e, uint32_t node, float a, float b) {
+    const unsigned long long v = (unsigned long long)__float_as_uint(a) << 32 | node;
+    if (e < kTraceLds) {
+        l.lo[e * 64] = v;
+        l.hi[e * 64] = b;
+    } else {
+        m.lo[e - kTraceLds] = v;
+        m.hi[e - kTraceLds] = b;
     }
-    return nd;
+}
+template <int kStack>
+__device__ __forceinline__ void stack_get(const LdsStack& l, const DeepStack<kStack>& m, int e, uint32_t& node, float& a,
+                                          float& b) {
+    unsigned long long v;
+    if (e < kTraceLds) {
+        v = l.lo[e * 64];
+        b = l.hi[e * 64];
+    } else {
+        v = m.lo[e - kTraceLds];
+        b = m.hi[e - kTraceLds];
+    }
+    node = (uint32_t)v;
+    a = __uint_as_float((uint32_t)(v >> 32));
 }
 
-// Calls test(a, e1, e2) on the count triangle records from rec (3 float4 each) until it
+// Calls test(a, e1, e2, r) on the count triangle records from rec (3 float4 each) until it
 // returns true; returns whether it did.  Two record buffers alternate, so the next record
 // loads while the current one is tested and no registers are copied between tests; the
 // loads are unconditional (past the leaf's end they re-read its last record, which is
@@ -128,102 +141,226 @@ __device__ __forceinline__ bool for_leaf_tris(const float4* rec, uint32_t count,
     for (uint32_t r = 0;; r += 2) {
         const float4* p1 = rec + 3u * min(r + 1u, last);
         const float4 a1 = p1[0], b1 = p1[1], c1 = p1[2];
-        if (test(a0, b0, c0)) return true;
+        if (test(a0, b0, c0, r)) return true;
         if (r + 1 >= count) return false;
         const float4* p2 = rec + 3u * min(r + 2u, last);
         a0 = p2[0];
         b0 = p2[1];
         c0 = p2[2];
-        if (test(a1, b1, c1)) return true;
+        if (test(a1, b1, c1, r + 1u)) return true;
         if (r + 2 >= count) return false;
     }
 }
 
-// Closest hit.  lds_lane: this lane's column of the workgroup's stack area (kLds > 0),
-// stride = lanes in the workgroup.
-template <int kStack = kTraceStack, int kLds = 0>
-__device__ __forceinline__ Hit trace_ray(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
-                                         const RootBox& root, f3 o, f3 d, float eps,
-                                         uint32_t* lds_lane = nullptr, uint32_t stride = 0) {
-    f3 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    float t0, t1;
-    int32_t best_tri = -1;
-    float best_t = 0.0f, bu = 0.0f, bv = 0.0f;
-    if (ray_box(root.lo, root.hi, o, inv, eps, kInf, t0, t1)) {
-        t1 = t1 + eps;
-        best_t = t1;
-        LaneStack<kStack, kLds> st;
-        st.lds = (__attribute__((address_space(3))) uint32_t*)lds_lane;
-        st.stride = stride;
-        int sp = 0;
-        uint32_t node = 0;
-        float tmin = t0, tmax = t1;
-        for (;;) {
-            uint2 nd = descend(nodes, st, sp, node, tmin, tmax, o, d, inv);
-            const uint32_t count = nd.x, begin = nd.y & MNRT_INDEX_MASK;
-            for_leaf_tris(recs + 3ull * begin, count, [&](const float4& a4, const float4& e14, const float4& e24) {
-                float lam, u, v;
-                if (ray_tri(xyz(a4), xyz(e14), xyz(e24), o, d, lam, u, v) && lam > eps) {
-                    const int32_t tri = (int32_t)__float_as_uint(a4.w);
-                    if (lam < best_t || (lam == best_t && best_tri >= 0 && tri < best_tri)) {
-                        best_t = lam;
-                        best_tri = tri;
-                        bu = u;
-                        bv = v;
-                    }
-                }
-                return false;
-            });
-            while (sp > 0 && best_tri >= 0 && best_t < st.tmin_of(sp - 1)) --sp;
-            if (sp == 0) break;
-            --sp;
-            st.get(sp, node, tmin, tmax);
-        }
-    }
-    Hit h;
-    h.tri = best_tri;
-    h.t = (best_tri >= 0) ? best_t : 0.0f;
-    h.u = (best_tri >= 0) ? bu : 0.0f;
-    h.v = (best_tri >= 0) ? bv : 0.0f;
-    return h;
+// Order of floats as unsigned words (any sign).
+__device__ __forceinline__ uint32_t order_bits(float f) {
+    const uint32_t u = __float_as_uint(f);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float order_float(uint32_t u) {
+    return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
 }
 
-// Any-hit traversal (dev_FindNextIntersectionKDWhileWhile<false>, raytracing.cu:503-645,
-// as the shadow-ray kernels use it, raytracing.cu:1019-1114).  Returns true iff some
-// triangle is hit at lambda with
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, uint32_t lane) {
+    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(lane * 4u), (int)v);
+}
+__device__ __forceinline__ float from_lane(float v, uint32_t lane) {
+    return __uint_as_float(from_lane(__float_as_uint(v), lane));
+}
+
+// Traces the rays a source hands out to the wave's lanes, until it has no more.
+//   src.next, src.end: ray numbers not handed out yet (uniform);
+//   src.start(i, o, d, dist): ray i; false when there is nothing to trace;
+//   src.finish(o, d, dist, hit): result of the lane's ray; true when the lane goes on with
+//     another ray that it put in o, d.
+// Closest hit (kAny false): the brute-force closest hit, lambda > eps, up to where the ray leaves
+// the root box, + eps.
+// Any hit (dev_FindNextIntersectionKDWhileWhile<false>, raytracing.cu:503-645, as the
+// shadow-ray kernels use it, raytracing.cu:1019-1114): hit.tri >= 0 iff some triangle is hit at
+// lambda with
 //     lambda > eps,  lambda < min(t_exit, dist) + eps,  lambda + slack < dist
 // (t_exit: where the ray leaves the root box).  The reference tests only the first
 // hit it meets against the light distance (`lambda >= distance`, `lambda + eps >=
 // distance`), so which triangle decides depends on the order of a leaf's list; here
 // any occluding triangle decides, so the result equals the brute-force predicate
-// whatever the tree.  Same interval widening and stack as trace_ray; the search ends
-// at the first occluder.
-template <int kStack = kTraceStack, int kLds = 0>
-__device__ __forceinline__ bool trace_any(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
-                                          const RootBox& root, f3 o, f3 d, float eps, float dist, float slack,
-                                          uint32_t* lds_lane = nullptr, uint32_t stride = 0) {
-    f3 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    float t0, t1;
-    if (!ray_box(root.lo, root.hi, o, inv, eps, kInf, t0, t1)) return false;
-    const float tlim = fminf(t1, dist) + eps;
-    LaneStack<kStack, kLds> st;
-    st.lds = (__attribute__((address_space(3))) uint32_t*)lds_lane;
-    st.stride = stride;
+// whatever the tree.  The search ends at the first occluder.
+// width: rays at once (lanes 0..width).  lds: the wave's kTraceWords.  Whole wave, every lane active.
+template <bool kAny, int kStack, typename Src>
+__device__ __forceinline__ void trace_stream(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
+                                             const RootBox& root, float eps, float slack, uint32_t width, uint32_t* lds, Src& src) {
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    typedef __attribute__((address_space(3))) unsigned long long lds_u64;
+    enum : uint32_t { kIdle, kDone, kWalk, kLeaf };
+    const uint32_t lane = threadIdx.x & 63u;
+    lds_u32* own = (lds_u32*)lds;
+    lds_u32* brec = own + 64;
+    lds_u64* key = (lds_u64*)(own + 128);
+    DeepStack<kStack> deep;
+    const LdsStack top{(lds_u64*)(own + 256) + lane, (__attribute__((address_space(3))) float*)(own + 256 + 128 * kTraceLds) + lane};
+    const uint32_t refill = width * kRefill / 64u, walk_min = width * kWalkMin / 64u;
+    uint32_t state = kIdle, node = 0, best_rec = 0;
+    int32_t best_tri = -1;
+    f3 o = mk3(0.0f, 0.0f, 0.0f), d = o, inv = o;
+    float dist = 0.0f, best_t = 0.0f, tmin = 0.0f, tmax = 0.0f;  // best_t: any hit: the limit on lambda
     int sp = 0;
-    uint32_t node = 0;
-    float tmin = t0, tmax = tlim;
+    uint2 nd = make_uint2(0u, 0u);
+
+    auto pop = [&]() {
+        state = kDone;
+        while (sp > 0) {
+            stack_get(top, deep, --sp, node, tmin, tmax);
+            if (!kAny && best_tri >= 0 && best_t < tmin) continue;
+            nd = nodes[node];
+            state = kWalk;
+            break;
+        }
+    };
     for (;;) {
-        uint2 nd = descend(nodes, st, sp, node, tmin, tmax, o, d, inv);
-        const uint32_t count = nd.x, begin = nd.y & MNRT_INDEX_MASK;
-        if (for_leaf_tris(recs + 3ull * begin, count, [&](const float4& a4, const float4& e14, const float4& e24) {
-                float lam, u, v;
-                return ray_tri(xyz(a4), xyz(e14), xyz(e24), o, d, lam, u, v) && lam > eps && lam < tlim &&
-                       lam + slack < dist;
-            }))
-            return true;
-        if (sp == 0) return false;
-        --sp;
-        st.get(sp, node, tmin, tmax);
+        const uint32_t busy = (uint32_t)__popcll(ballot(state >= kWalk));
+        const uint32_t done = (uint32_t)__popcll(ballot(state == kDone));
+        if (busy == 0u || (src.next < src.end ? width - busy : done) >= refill) {
+            bool ray = false;
+            if (state == kDone) {
+                ray = src.finish(o, d, dist, Hit{best_tri, best_t, best_rec});
+                state = kIdle;
+            }
+            const bool want = state == kIdle && !ray && lane < width;
+            const uint64_t m = ballot(want);
+            const uint32_t rank = mask_prefix(m), left = src.end - src.next;
+            if (want && rank < left) ray = src.start(src.next + rank, o, d, dist);
+            src.next += min((uint32_t)__popcll(m), left);
+            if (ray) {
+                inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+                best_tri = -1;
+                sp = 0;
+                node = 0;
+                float t0, t1;
+                state = kDone;
+                if (ray_box(root.lo, root.hi, o, inv, eps, kInf, t0, t1)) {
+                    best_t = (kAny ? fminf(t1, dist) : t1) + eps;
+                    tmin = t0;
+                    tmax = best_t;
+                    nd = nodes[0];
+                    state = kWalk;
+                }
+            }
+            if (ballot(state != kIdle) == 0ull && left == 0u) break;
+        }
+        // to the next leaf
+        for (;;) {
+            const uint64_t m = ballot(state == kWalk);
+            if (m == 0ull || ((uint32_t)__popcll(m) < walk_min && ballot(state == kLeaf) != 0ull)) break;
+            if (state == kWalk) {
+                if (is_leaf(nd.y)) {
+                    if (nd.x != 0u) state = kLeaf;
+                    else pop();
+                } else {
+                    const uint32_t a = nd.y >> 30;
+                    const float s = __uint_as_float(nd.x);
+                    const uint32_t left = node + 1, right = nd.y & MNRT_INDEX_MASK;
+                    const float oa = comp(o, a), da = comp(d, a), ia = comp(inv, a);
+                    const float tsplit = (s - oa) * ia;
+                    const bool below = (oa < s) | ((oa == s) & (da > 0.0f));
+                    const uint32_t first = below ? left : right, second = below ? right : left;
+                    // (a NaN tsplit compares false throughout: both children over the whole interval)
+                    const bool near = (tsplit < 0.0f) | (tsplit > tmax * kTravTolHi);
+                    const bool far = !near & (tsplit < tmin * kTravTolLo);
+                    node = far ? second : first;
+                    nd = nodes[node];
+                    if (!(near | far)) {
+                        if (sp < kStack) stack_put(top, deep, sp++, second, fmaxf(tmin, tsplit * kTravTolLo), tmax);
+                        tmax = fminf(tmax, tsplit * kTravTolHi);
+                    }
+                }
+            }
+        }
+        const bool at_leaf = state == kLeaf;
+        if (ballot(at_leaf) == 0ull) continue;
+        const uint32_t cnt = at_leaf ? nd.x : 0u, begin = nd.y & MNRT_INDEX_MASK;
+        const uint32_t incl = wave_scan_u32(cnt), total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        const uint32_t most = wave_max_u32(cnt);
+        if (3u * ((total + 63u) >> 6) >= 2u * most) {
+            // about equally full leaves (a lane's own test costs two thirds of a dealt one)
+            if (at_leaf)
+                for_leaf_tris(recs + 3ull * begin, cnt, [&](const float4& a4, const float4& e14, const float4& e24, uint32_t r) {
+                    float lam, u, v;
+                    if (!(ray_tri(xyz(a4), xyz(e14), xyz(e24), o, d, lam, u, v) && lam > eps)) return false;
+                    if (kAny) {
+                        if (!(lam < best_t && lam + slack < dist)) return false;
+                        best_tri = 0;
+                        return true;
+                    }
+                    const int32_t tri = (int32_t)__float_as_uint(a4.w);
+                    if (lam < best_t || (lam == best_t && best_tri >= 0 && tri < best_tri)) {
+                        best_t = lam;
+                        best_tri = tri;
+                        best_rec = begin + r;
+                    }
+                    return false;
+                });
+        } else {
+            const uint32_t first = incl - cnt, shift = begin - first;
+            // a key is (lambda, triangle); before any hit (limit, 0), which no hit equals or
+            // exceeds and counts
+            const unsigned long long key0 =
+                (unsigned long long)order_bits(best_t) << 32 | (uint32_t)(best_tri < 0 ? 0 : best_tri);
+            key[lane] = kAny ? 1ull : key0;
+            uint32_t carry = 0;
+            for (uint32_t base = 0; base < total; base += 64u) {
+                // the lane whose leaf holds pair base + lane
+                own[lane] = 0u;
+                wave_sync();
+                if (cnt != 0u && first - base < 64u) own[first - base] = lane + 1u;
+                wave_sync();
+                uint32_t w = own[lane];
+                if (lane == 0u) w = max(w, carry);
+                w = wave_max_scan_u32(w);
+                carry = (uint32_t)__builtin_amdgcn_readlane((int)w, 63);
+                const uint32_t r = w - 1u, pair = base + lane;
+                const bool valid = pair < total;
+                const uint32_t rec = from_lane(shift, r) + pair;
+                const f3 ro = mk3(from_lane(o.x, r), from_lane(o.y, r), from_lane(o.z, r));
+                const f3 rd = mk3(from_lane(d.x, r), from_lane(d.y, r), from_lane(d.z, r));
+                const float rt = from_lane(best_t, r), rdist = kAny ? from_lane(dist, r) : 0.0f;
+                const float4* t = recs + 3ull * (valid ? rec : begin);
+                bool hit = false;
+                float lam = 0.0f;
+                uint32_t tri = 0;
+                if (valid) {
+                    const float4 a4 = t[0], e14 = t[1], e24 = t[2];
+                    float u, v;
+                    hit = ray_tri(xyz(a4), xyz(e14), xyz(e24), ro, rd, lam, u, v) && lam > eps;
+                    hit = hit && (kAny ? lam < rt && lam + slack < rdist : lam <= rt);
+                    tri = __float_as_uint(a4.w);
+                }
+                if (ballot(hit) != 0ull) {
+                    if (kAny) {
+                        if (hit) key[r] = 0ull;
+                    } else {
+                        const unsigned long long mine = (unsigned long long)order_bits(lam) << 32 | tri;
+                        if (hit) __hip_atomic_fetch_min(&key[r], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        wave_sync();
+                        if (hit && key[r] == mine) brec[r] = rec;
+                    }
+                }
+                wave_sync();
+            }
+            if (at_leaf) {
+                const unsigned long long k = key[lane];
+                if (kAny) {
+                    if (k == 0ull) best_tri = 0;
+                } else if (k != key0) {
+                    best_t = order_float((uint32_t)(k >> 32));
+                    best_tri = (int32_t)(uint32_t)k;
+                    best_rec = brec[lane];
+                }
+            }
+            wave_sync();
+        }
+        if (at_leaf) {
+            if (kAny && best_tri >= 0) state = kDone;
+            else pop();
+        }
     }
 }
 
