@@ -42,7 +42,7 @@ struct mnrt_batch {
     uint32_t* d_tri_begin = nullptr;   // ns
     uint32_t* d_tparts = nullptr;      // 2 * kMaxParts: trace part begin / end (tiles)
     uint32_t* d_kparts = nullptr;      // 2 * kMaxParts: kNN part begin / end (slots)
-    uint32_t* d_work = nullptr;        // 2 * kMaxParts
+    uint32_t* d_work = nullptr;        // 2 * kMaxParts * kWorkStride
     uint32_t* d_flags = nullptr;       // total_slots + 1
     uint32_t* d_pos = nullptr;         // total_slots + 1
     uint32_t* d_scan = nullptr;
@@ -133,6 +133,7 @@ int run_trace(mnrt_batch& b, const mnrt_batch_io& io, hipStream_t st) {
     A.tile_begin = b.d_tile_begin;
     A.num_scenes = b.ns;
     A.tile_rays = b.tun.trace_tile;
+    A.unit = trace_unit(b.total_slots);
     A.num_parts = b.tun.parts;
     A.part_begin = b.d_tparts;
     A.part_end = b.d_tparts + kMaxParts;
@@ -193,7 +194,7 @@ int run_knn(mnrt_batch& b, const mnrt_batch_io& io, hipStream_t st) {
     G.out_nbr = io.d_out_nbr;
     G.out_count = io.d_out_count;
     return launch_knn_batch(G, b.d_knn, b.d_slot_begin, b.ns, io.d_sp_count, b.tun.knn_chunk, b.tun.parts,
-                            b.d_tparts + 2 * kMaxParts, b.d_tparts + 3 * kMaxParts, b.d_work + kMaxParts,
+                            b.d_tparts + 2 * kMaxParts, b.d_tparts + 3 * kMaxParts, b.d_work + kMaxParts * kWorkStride,
                             b.tun.knn_cap, b.tun.knn_waves, b.tun.knn_grid, b.boxes, st);
 }
 
@@ -251,7 +252,7 @@ int run_knn_bwd(mnrt_batch& b, const mnrt_batch_io& io, hipStream_t st) {
     G.out_grad_clr = (float4*)io.d_grad_clr4;
     return launch_knn_bwd_batch(G, b.d_knn, b.d_slot_begin, b.ns, io.d_sp_count, b.d_poff, b.h_poff[b.ns],
                                 io.d_out_r2, io.d_out_count, b.d_wmax, b.d_scale, b.tun.parts,
-                                b.d_tparts + 2 * kMaxParts, b.d_tparts + 3 * kMaxParts, b.d_work + kMaxParts,
+                                b.d_tparts + 2 * kMaxParts, b.d_tparts + 3 * kMaxParts, b.d_work + kMaxParts * kWorkStride,
                                 b.tun.knn_grid, b.boxes, io.d_grad_pow4, st);
 }
 
@@ -385,7 +386,7 @@ extern "C" int mnrt_batch_create(const mnrt_batch_desc* d, mnrt_batch** out) {
         };
         size_t o_trace = carve(sizeof(TraceScene) * ns), o_knn = carve(sizeof(KnnScene) * ns);
         size_t o_tile = carve(4 * (ns + 1)), o_slot = carve(4 * (ns + 1)), o_tri = carve(4 * ns);
-        size_t o_parts = carve(4 * 4 * kMaxParts), o_work = carve(4 * 2 * kMaxParts);
+        size_t o_parts = carve(4 * 4 * kMaxParts), o_work = carve(4 * 2 * kMaxParts * kWorkStride);
         size_t o_flags = carve(4 * n1), o_pos = carve(4 * n1), o_scan = carve(4 * scan_scratch_words((uint32_t)n1));
         if (hipMalloc(&b->d_buf, bytes) != hipSuccess) rc = MNRT_ERR_NOMEM;
         if (rc == MNRT_OK) {
@@ -410,13 +411,11 @@ extern "C" int mnrt_batch_create(const mnrt_batch_desc* d, mnrt_batch** out) {
     if (rc == MNRT_OK) {
         mnrt_batch_tuning& t = b->tun;
         t.trace_block = 256;
-        // a wave's share of a tile is one set of rays until the tiles fill the chip (131072 rays of 32
-        // scenes are 512 workgroups, not 128), then a run that refills
-        t.trace_tile = b->total_slots >= (1u << 20) ? 1024 : 256;
+        t.trace_tile = 1024;
         t.trace_grid = 8 * b->cus;
         t.trace_stack = smallest_stack(b->max_level);
         t.knn_waves = 4;
-        t.knn_chunk = 16;
+        t.knn_chunk = std::min<uint32_t>(16u, std::max<uint32_t>(1u, b->total_slots / 24576u));
         t.knn_grid = 8 * b->cus;
         t.knn_cap = knn ? min_cap(b->k) : 128;
         t.parts = kMaxParts;

@@ -25,6 +25,21 @@ __device__ __forceinline__ uint32_t seg_of(const uint32_t* off, uint32_t n, uint
 }
 
 constexpr uint32_t kMaxParts = 8;  // work-counter shares (one per XCD)
+// Work counters lie a cache line apart: atomics on one line wait for each other.
+constexpr uint32_t kWorkStride = 32;
+
+// The next of share p's units, or a number >= units when there are none left (uniform).  The share
+// of another XCD is looked at first: with thousands of waves that run out together, the
+// atomics that find a share empty would take longer than its work.
+__device__ __forceinline__ uint32_t take_unit(uint32_t* work, uint32_t p, uint32_t units, bool look, uint32_t lane) {
+    uint32_t c = 0;
+    if (lane == 0) {
+        uint32_t* w = work + p * kWorkStride;
+        if (look) c = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (c < units) c = atomicAdd(w, 1u);
+    }
+    return uniform(c);
+}
 constexpr int kTraceStackAbi = MNRT_MAX_LEVEL + 2;  // the full-depth traversal stack
 
 struct TraceScene {
@@ -40,6 +55,7 @@ struct TraceBatchArgs {
     const uint32_t* tile_begin;  // num_scenes + 1
     uint32_t num_scenes;
     uint32_t tile_rays;
+    uint32_t unit;  // rays a wave takes and traces at once: a part of a tile
     uint32_t num_parts;
     const uint32_t* part_begin;  // first tile of each share
     const uint32_t* part_end;
@@ -119,6 +135,8 @@ struct ShadeBatchArgs {
     uint32_t* out_count;          // hits per scene
 };
 
+// Rays a wave takes at once when a batch has `rays`.
+uint32_t trace_unit(uint64_t rays);
 int launch_trace_batch(const TraceBatchArgs& B, int stack, uint32_t grid, uint32_t block, hipStream_t st);
 int launch_knn_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* slot_begin, uint32_t ns,
                      const uint32_t* count, uint32_t chunk, uint32_t num_parts, const uint32_t* part_begin,

@@ -948,12 +948,11 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(8, 
     for (uint32_t part = 0; part < num_parts; ++part) {
         const uint32_t p = (xcd + part) % num_parts;
         const uint32_t pb = part_begin[p], pe = part_end[p];
+        const uint32_t units = (uint32_t)(((uint64_t)(pe - pb) + chunk - 1u) / chunk);
         for (;;) {
-            uint32_t c = 0;
-            if (lane == 0) c = atomicAdd(&work[p], 1u);
-            c = uniform(__shfl(c, 0, 64));
+            const uint32_t c = take_unit(work, p, units, part > 0u, lane);
+            if (c >= units) break;
             const uint64_t c0 = (uint64_t)pb + (uint64_t)c * chunk;
-            if (c0 >= pe) break;
             const uint32_t c1 = (uint32_t)min<uint64_t>(c0 + chunk, pe);
             // the scene of the chunk's slots, refreshed only when a slot crosses into the next
             uint32_t s = uniform(seg_of(slot_begin, ns, (uint32_t)c0));
@@ -1222,12 +1221,11 @@ __global__ __launch_bounds__(256) void k_knn_bwd_batch(KnnArgs G, const KnnScene
     for (uint32_t part = 0; part < num_parts; ++part) {
         const uint32_t p = (xcd + part) % num_parts;
         const uint32_t pb = part_begin[p], pe = part_end[p];
+        const uint32_t units = (uint32_t)(((uint64_t)(pe - pb) + chunk - 1u) / chunk);
         for (;;) {
-            uint32_t c = 0;
-            if (lane == 0) c = atomicAdd(&work[p], 1u);
-            c = uniform(__shfl(c, 0, 64));
+            const uint32_t c = take_unit(work, p, units, part > 0u, lane);
+            if (c >= units) break;
             const uint64_t g0 = (uint64_t)pb + (uint64_t)c * chunk;
-            if (g0 >= pe) break;
             const uint32_t n = (uint32_t)min<uint64_t>(chunk, pe - g0);
             uint32_t s = uniform(seg_of(slot_begin, ns, (uint32_t)g0));
             uint32_t b = 0, e = 0, m = 0;
@@ -1339,7 +1337,7 @@ int launch_knn_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* s
                      const uint32_t* count, uint32_t chunk, uint32_t num_parts, const uint32_t* part_begin,
                      const uint32_t* part_end, uint32_t* work, uint32_t cap, uint32_t waves,
                      uint32_t grid, bool boxes, hipStream_t st) {
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, work, num_parts, 0u);
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, work, num_parts * kWorkStride, 0u);
 #define MNRT_KB(C, W, X)                                                                                   \
     hipLaunchKernelGGL((k_knn_batch<C, W, X>), dim3(grid), dim3(64 * W), 0, st, G, scenes, slot_begin, ns, \
                        count, chunk, num_parts, part_begin, part_end, work)
@@ -1369,7 +1367,7 @@ int launch_knn_bwd_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_
                          const float* fwd_r2, const uint32_t* fwd_count, uint32_t* wmax, double* scale, uint32_t num_parts, const uint32_t* part_begin,
                          const uint32_t* part_end, uint32_t* work, uint32_t grid, bool boxes, float* grad_pow4, hipStream_t st) {
     const uint32_t n = G.n;
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, work, num_parts, 0u);
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, work, num_parts * kWorkStride, 0u);
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, wmax, ns, 0u);
     const uint64_t words = 3ull * total_photons;
     if (words) {

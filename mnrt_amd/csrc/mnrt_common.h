@@ -243,6 +243,17 @@ __device__ __forceinline__ T ld_uniform(const T* p, uint32_t i) {
     return p[i];
 #endif
 }
+// A pointer to global memory that was read from memory itself: said to be one, or its loads and
+// stores would be flat ones, which wait for the LDS counter too.
+template <typename T>
+__device__ __forceinline__ T* global_ptr(T* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
+#else
+    return p;
+#endif
+}
+
 // ld_uniform of an 8-byte node word pair at a 32-bit byte offset: one scalar load with an
 // SGPR offset, no 64-bit address arithmetic.  Valid for i < kUniform8MaxIndex.
 constexpr uint32_t kUniform8MaxIndex = 1u << 29;

@@ -51,17 +51,15 @@ struct PhotonArgs {
 
 // Paths of a run; a lane's next ray is its path's next bounce, or the next path.
 struct PathSource {
-    uint32_t next, end;
-    RayDeal deal;
+    static constexpr uint32_t kTogether = 65;  // never: only a path's first ray has neighbours
+    RayWindow rays;
     const PhotonArgs& A;
     uint32_t path, light, bounce;
     float pr, pg, pb;
     uint32_t tris[4];
 
     __device__ __forceinline__ bool start(uint32_t i, f3& o, f3& d, float&) {
-        const uint64_t at = deal.ray(i);
-        if (at >= deal.n) return false;
-        i = path = (uint32_t)at;
+        path = i;
         const uint32_t p = A.path_begin + i, slots = A.max_bounces + 1;
         for (uint32_t b = 0; b < slots; ++b) A.valid[(size_t)i * slots + b] = 0u;
         light = p % A.num_lights;
@@ -116,11 +114,10 @@ struct PathSource {
     }
 };
 
-__global__ __launch_bounds__(64) void k_photon_paths(PhotonArgs A, uint32_t width) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_photon_paths(PhotonArgs A, uint32_t width) {
     __shared__ __align__(8) uint32_t s_wave[kTraceWords];
-    const RayDeal deal{blockIdx.x, gridDim.x, A.num_paths, width};
-    PathSource src{0u, deal.count(), deal, A};
-    trace_stream<false, kTraceStack>(A.nodes, A.recs, A.root, A.eps, 0.0f, width, s_wave, src);
+    PathSource src{RayWindow(blockIdx.x * width, A.num_paths, width, nullptr), A};
+    trace_stream<false, kTraceStack>(A.nodes, A.recs, A.root, A.eps, 0.0f, s_wave, src);
 }
 
 // Stable compaction of the valid slots into the output, up to `limit` photons.
@@ -231,7 +228,7 @@ extern "C" int mnrt_photons_generate(const mnrt_tree* tree, const float* d_v0, c
         A.path_begin = shot;
         A.num_paths = np;
         const uint32_t width = trace_width(np);
-        hipLaunchKernelGGL(k_photon_paths, dim3(trace_waves(np, width)), dim3(64), 0, st, A, width);
+        hipLaunchKernelGGL(k_photon_paths, dim3(trace_windows(np, width)), dim3(64), 0, st, A, width);
         if (scan_exclusive(A.valid, pos, (uint32_t)nslots, tot, scr, st) != hipSuccess) {
             rc = MNRT_ERR_HIP;
             break;

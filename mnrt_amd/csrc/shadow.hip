@@ -107,8 +107,8 @@ enum : int { kSegPoint = 0, kSegDirectional = 1, kSegArea = 2, kSegExplicit = 3 
 // out = 1 when something is hit.
 template <int kMode>
 struct SegSource {
-    uint32_t next, end;
-    RayDeal deal;
+    static constexpr uint32_t kTogether = 36;  // 24: area lights 6 % slower, point lights 1 % faster
+    RayWindow rays;
     const LightArgs& L;
     const float4* __restrict__ pts;
     const float4* __restrict__ dirs;
@@ -117,9 +117,7 @@ struct SegSource {
     uint32_t seg = 0;
 
     __device__ __forceinline__ bool start(uint32_t i, f3& o, f3& d, float& dist) {
-        const uint64_t at = deal.ray(i);
-        if (at >= deal.n) return false;
-        i = seg = (uint32_t)at;
+        seg = i;
         o = xyz(pts[i]);
         dist = kInf;
         if (kMode == kSegExplicit) {
@@ -150,15 +148,14 @@ struct SegSource {
 };
 
 template <int kMode>
-__global__ __launch_bounds__(64) void k_any_hit(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_any_hit(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
                                                 RootBox root, LightArgs L, uint32_t n, uint32_t width,
                                                 const float4* __restrict__ pts, const float4* __restrict__ dirs,
                                                 const float* __restrict__ tmax, float eps,
                                                 uint32_t* __restrict__ out) {
     __shared__ __align__(8) uint32_t s_wave[kTraceWords];
-    const RayDeal deal{blockIdx.x, gridDim.x, n, width};
-    SegSource<kMode> src{0u, deal.count(), deal, L, pts, dirs, tmax, out};
-    trace_stream<true, kTraceStack>(nodes, recs, root, eps, kMode == kSegArea ? eps : 0.0f, width, s_wave, src);
+    SegSource<kMode> src{RayWindow(blockIdx.x * width, n, width, nullptr), L, pts, dirs, tmax, out};
+    trace_stream<true, kTraceStack>(nodes, recs, root, eps, kMode == kSegArea ? eps : 0.0f, s_wave, src);
 }
 
 static int launch_any_hit(int mode, const mnrt_tree* tree, const LightArgs& L, uint32_t n, const float* d_pts4,
@@ -173,7 +170,7 @@ static int launch_any_hit(int mode, const mnrt_tree* tree, const LightArgs& L, u
         rb.hi[a] = tree->root_max[a];
     }
     const uint32_t width = trace_width(n);
-    const dim3 grid(trace_waves(n, width)), block(64);
+    const dim3 grid(trace_windows(n, width)), block(64);
     const uint2* nodes = (const uint2*)tree->d_nodes;
     const float4* recs = (const float4*)tree->d_recs;
     const float4* pts = (const float4*)d_pts4;

@@ -18,11 +18,27 @@
 
 namespace mnrt {
 
+RayCounter::RayCounter(uint64_t n, uint32_t width, hipStream_t st) : st_(st) {
+    waves = trace_windows(n, width);
+    if (waves <= kWindowWaves) return;
+    // (a captured launch keeps a wave per window: no allocation is recorded)
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
+    void* buf = nullptr;
+    if (n > 0xFFFFFFFFull - (uint64_t)width * kTraceWaves || pool_alloc(&buf, 4, st) != hipSuccess) return;
+    p = (uint32_t*)buf;
+    waves = kTraceWaves;
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, p, 1u, width * kTraceWaves);
+}
+RayCounter::~RayCounter() {
+    if (p) (void)pool_free(p, st_);
+}
+
 // Rays first..last of arrays; results as they are asked for.
 struct RaySource {
-    uint32_t next, end;
-    RayDeal deal;
-    uint32_t first;
+    static constexpr uint32_t kTogether = kRaysTogether;
+    RayWindow rays;
+    uint32_t first;  // of the scene's rays
     const float4* __restrict__ orig;
     const float4* __restrict__ dir;
     const float4* __restrict__ recs;
@@ -34,9 +50,7 @@ struct RaySource {
     uint32_t ray = 0;
 
     __device__ __forceinline__ bool start(uint32_t i, f3& o, f3& d, float&) {
-        const uint64_t at = deal.ray(i);
-        if (at >= deal.n) return false;
-        i = ray = first + (uint32_t)at;
+        i = ray = first + i;
         o = xyz(orig[i]);
         d = xyz(dir[i]);
         return true;
@@ -61,15 +75,14 @@ struct RaySource {
 };
 
 // One wave per workgroup: its LDS goes to the next when its own run is done.
-__global__ __launch_bounds__(64) void k_trace_closest(
-    const uint2* __restrict__ nodes, const float4* __restrict__ recs, RootBox root, uint32_t n, uint32_t width,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_trace_closest(
+    const uint2* __restrict__ nodes, const float4* __restrict__ recs, RootBox root, uint32_t n, uint32_t width, uint32_t* __restrict__ counter,
     const float4* __restrict__ orig, const float4* __restrict__ dir, float eps,
     int32_t* __restrict__ out_tri, float* __restrict__ out_t, float2* __restrict__ out_bary,
     float4* __restrict__ out_pt, uint32_t* __restrict__ out_valid) {
     __shared__ __align__(8) uint32_t s_wave[kTraceWords];
-    const RayDeal deal{blockIdx.x, gridDim.x, n, width};
-    RaySource src{0u, deal.count(), deal, 0u, orig, dir, recs, out_tri, out_t, out_bary, out_pt, out_valid};
-    trace_stream<false, kTraceStack>(nodes, recs, root, eps, 0.0f, width, s_wave, src);
+    RaySource src{RayWindow(blockIdx.x * width, n, width, counter), 0u, orig, dir, recs, out_tri, out_t, out_bary, out_pt, out_valid};
+    trace_stream<false, kTraceStack>(nodes, recs, root, eps, 0.0f, s_wave, src);
 }
 
 }  // namespace mnrt
@@ -89,9 +102,10 @@ extern "C" int mnrt_trace_closest(const mnrt_tree* tree, uint32_t n, const float
         rb.hi[a] = tree->root_max[a];
     }
     const uint32_t width = mnrt::trace_width(n);
-    hipLaunchKernelGGL(mnrt::k_trace_closest, dim3(mnrt::trace_waves(n, width)), dim3(64), 0,
+    const mnrt::RayCounter counter(n, width, (hipStream_t)stream);
+    hipLaunchKernelGGL(mnrt::k_trace_closest, dim3(counter.waves), dim3(64), 0,
                        (hipStream_t)stream,
-                       (const uint2*)tree->d_nodes, (const float4*)tree->d_recs, rb, n, width,
+                       (const uint2*)tree->d_nodes, (const float4*)tree->d_recs, rb, n, width, counter.p,
                        (const float4*)d_orig4, (const float4*)d_dir4, eps, d_out_tri, d_out_t,
                        (float2*)d_out_bary2, (float4*)d_out_pt4, d_out_valid);
     MNRT_HIP_CHECK(hipGetLastError());
@@ -102,44 +116,45 @@ extern "C" int mnrt_trace_closest(const mnrt_tree* tree, uint32_t n, const float
 
 namespace mnrt {
 
-// Workgroups take tiles of consecutive rays from a work counter until every tile is
-// done; tile t belongs to the scene whose tile range holds it.  Each XCD (workgroup id
+// Waves take units of consecutive rays, parts of a tile, from a work counter until every tile
+// is done; tile t belongs to the scene whose tile range holds it.  Each XCD (workgroup id
 // mod 8 on MI355X) has its own counter over a contiguous share of the tiles, so an
-// XCD's L2 holds the trees of the scenes it traces; a workgroup whose share is done
-// takes tiles from the next XCD's share.
-// Each wave of a workgroup traces its share of a tile as one run.
+// XCD's L2 holds the trees of the scenes it traces; a wave whose share is done
+// takes units from the next XCD's share.
 template <int kStack>
-__global__ __launch_bounds__(256) void k_trace_batch(TraceBatchArgs B) {
-    __shared__ uint32_t s_tile;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_trace_batch(TraceBatchArgs B) {
     extern __shared__ __align__(8) uint32_t s_waves[];
-    const uint32_t xcd = blockIdx.x % B.num_parts, wave = uniform(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const uint32_t xcd = blockIdx.x % B.num_parts, wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t per_tile = B.tile_rays / B.unit;
     for (uint32_t part = 0; part < B.num_parts; ++part) {
         const uint32_t p = (xcd + part) % B.num_parts;
-        const uint32_t end = B.part_end[p];
+        const uint32_t begin = B.part_begin[p], units = (B.part_end[p] - begin) * per_tile;
         for (;;) {
-            if (threadIdx.x == 0) s_tile = B.part_begin[p] + atomicAdd(&B.work[p], 1u);
-            __syncthreads();
-            const uint32_t t = s_tile;
-            __syncthreads();
-            if (t >= end) break;
+            const uint32_t u = take_unit(B.work, p, units, part > 0u, lane);
+            if (u >= units) break;
+            const uint32_t t = begin + u / per_tile;
             const uint32_t s = seg_of(B.tile_begin, B.num_scenes, t);
             const TraceScene& d = B.scenes[s];
-            const uint32_t first = d.ray_begin + (t - B.tile_begin[s]) * B.tile_rays;
-            const RayDeal deal{wave, waves, min(B.tile_rays, d.ray_end - first), 64u};
+            const uint32_t first = d.ray_begin + (t - B.tile_begin[s]) * B.tile_rays + (u % per_tile) * B.unit;
+            if (first >= d.ray_end) continue;
             RootBox root;
             for (int a = 0; a < 3; ++a) {
                 root.lo[a] = d.lo[a];
                 root.hi[a] = d.hi[a];
             }
-            RaySource src{0u, deal.count(), deal, first, B.orig, B.dir, d.recs, B.out_tri, B.out_t, B.out_bary, nullptr,
+            const float4* recs = global_ptr(d.recs);
+            RaySource src{RayWindow(0u, min(B.unit, d.ray_end - first), B.unit, nullptr), first, B.orig, B.dir, recs, B.out_tri, B.out_t, B.out_bary, nullptr,
                           nullptr};
-            trace_stream<false, kStack>(d.nodes, d.recs, root, d.eps, 0.0f, 64u, s_waves + wave * kTraceWords, src);
+            trace_stream<false, kStack>(global_ptr(d.nodes), recs, root, d.eps, 0.0f, s_waves + wave * kTraceWords,
+                                        src);
         }
     }
 }
 
+uint32_t trace_unit(uint64_t rays) { return trace_width(rays); }
+
 int launch_trace_batch(const TraceBatchArgs& B, int stack, uint32_t grid, uint32_t block, hipStream_t st) {
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, B.work, B.num_parts, 0u);
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, B.work, B.num_parts * kWorkStride, 0u);
     const uint32_t lds = 4u * kTraceWords * (block / 64u);
     switch (stack) {
         case 16: hipLaunchKernelGGL(k_trace_batch<16>, dim3(grid), dim3(block), lds, st, B); break;

@@ -15,18 +15,18 @@
 //     in LDS, deeper ones in the lane's private array (the reference keeps the whole
 //     stack in local memory).
 //
-// A wave traces a run of rays (trace_stream), not one ray per lane to its end.  With a lane per
+// A wave traces windows of rays (trace_stream), not one ray per lane to its end.  With a lane per
 // ray the wave steps until its longest ray is done and tests as many triangles per leaf as the
 // fullest leaf among its lanes holds: for bounce rays 10 % of the lanes worked (47 k wave
-// instructions per 64 rays, 68 triangle tests a ray).  So
-//   * a lane whose ray is done takes the next ray of the wave's run, kRefill lanes at a time;
+// instructions per 64 rays, 68 triangle tests a ray).  So, unless the rays go together (kTogether),
+//   * a lane whose ray is done takes the next ray, kRefill lanes at a time;
 //   * lanes walk to their next leaf until fewer than kWalkMin still walk, and wait there;
-//   * the waiting leaves' (ray, triangle) pairs are dealt to all lanes, 64 at a time, unless the lanes' own leaves are about as full as each other, as they are
-//     for camera rays, when each lane tests its own.
+//   * the waiting leaves' (ray, triangle) pairs are dealt to all lanes, 64 at a time, unless
+//     the lanes' own leaves are about as full as each other, when each lane tests its own.
 // Bound by instruction issue: about 25 k vector instructions per 64 bounce rays of the 1.03M-triangle
 // scene (206 walk steps with 29 lanes, 85 dealt tests with 49 pairs, 37 own tests), 83 tests and 93
-// steps a ray.  2.07M bounce rays 2612 -> 1670 us, 785 k area-light shadow rays 962 -> 672 us, 6144
-// camera rays 65 -> 44 us.
+// steps a ray.  2.07M bounce rays 2248 -> 1466 us, 785 k area-light shadow rays 830 -> 573 us,
+// 6144 camera rays 67 -> 47 us, 1.69M camera rays (205001 triangles) 1048 -> 1010 us.
 #pragma once
 
 #include "mnrt_common.h"
@@ -50,40 +50,65 @@ constexpr int kTraceStack = MNRT_MAX_LEVEL + 2;
 // goes to scratch memory there; 6 entries instead of 7: 1670 -> 1721 us.
 constexpr int kTraceLds = 7;
 
-// Waves of a launch: at most the 24 per CU that run at once (74 registers, 6.4 KB of LDS); tiles of
-// 64 rays are dealt to them in turn.  A few more and a second round of waves runs almost alone
-// (6400: 2190 us, 6144: 1670 us).
-constexpr uint32_t kTraceWaves = 6144;
+// Waves that run at once: 24 per CU (80 registers, 6.4 KB of LDS).
+constexpr uint32_t kTraceWaves = 6144, kWindowWaves = kTraceWaves + kTraceWaves / 2u;
 
-// Rays a wave traces at once: 64, or fewer where a launch would leave SIMDs without a wave: its
-// longest ray and fullest leaves are then shorter, and the spare lanes test triangles.
-// 6144 camera rays: 16 a wave 44 us, 64 a wave 69 us.
-constexpr uint64_t kTraceSimds = 1024;
-inline uint32_t trace_width(uint64_t n) { return n >= 64u * kTraceSimds ? 64u : n >= 32u * kTraceSimds ? 32u : 16u; }
+// Rays a wave traces at once: 64, or fewer while all the waves run at once: a wave's longest ray
+// and fullest leaves are then shorter, and the spare lanes test triangles.  6144 camera rays: 16 a
+// wave 44 us, 64 a wave 69 us; 131044 bounce rays (205001 triangles): 32 a wave 421 us, 64 466 us.
+inline uint32_t trace_width(uint64_t n) { return n > 32u * kTraceWaves ? 64u : n > 16u * kTraceWaves ? 32u : 16u; }
+inline uint32_t trace_windows(uint64_t n, uint32_t width) { return (uint32_t)((n + width - 1u) / width); }
 
 // Of 64 rays, the lanes that take new rays together and the least number that goes on walking while
 // others wait at leaves.  16..32 and 6..16 are within 4 % of each other on bounce rays, shadow rays
 // and photon paths; fewer walkers suit small launches.
 constexpr uint32_t kRefill = 24, kWalkMin = 10;
+// A set of 64 rays of which on average at least kTogether lanes walk, while at least kEarly are
+// still traced, is traced to its end as it is: for camera rays every refill, wait and dealt test is
+// overhead.  Between 24 and 36, bounce rays gain 2 % and camera rays lose 10 %; at 18 bounce rays
+// lose 10 %.
+constexpr uint32_t kEarly = 48, kRaysTogether = 24;
 
 // LDS words of a wave: pair owners and best records (64 each), best keys (64 x 2), stack.
 constexpr uint32_t kTraceWords = 256u + 3u * 64u * (uint32_t)kTraceLds;
 
-inline uint32_t trace_waves(uint64_t n, uint32_t width) {
-    const uint64_t tiles = (n + width - 1u) / width;
-    return (uint32_t)(tiles < kTraceWaves ? tiles : kTraceWaves);
-}
+// Rays of a wave: a window of `width` consecutive ones at a time, the first by its number, the
+// next from a counter that the launch's waves share (null: none).  A launch of up to
+// kWindowWaves windows has a wave for each, which the hardware starts as others end: 524176 camera rays
+// (205001 triangles) 505 us, from a counter 550; from there on lanes that refill gain more: 1.69M bounce
+// rays 1483 us, a wave per window 2093.  (A fixed share of the rays for every wave that fits at
+// once: waves of slow rays end late, camera rays up to 40 % slower.)  Shadow rays always have a wave per window: 1.76M from a point
+// light (20000 triangles) 427 us, from a counter 592.
+struct RayWindow {
+    uint32_t next, end;  // rays of the window not handed out yet
+    uint32_t n, width;
+    uint32_t* counter;   // rays in windows taken so far
+    bool open;           // there may be more windows
 
-// The rays of wave w of waves, numbered 0..count: tiles w, w + waves, ... (width rays each) of n.
-struct RayDeal {
-    uint32_t w, waves, n, width;  // width: a power of two
-    __device__ __forceinline__ uint32_t count() const {
-        const uint32_t tiles = (uint32_t)(((uint64_t)n + width - 1u) / width);
-        return tiles > w ? width * ((tiles - w - 1u) / waves + 1u) : 0u;
+    __device__ __forceinline__ RayWindow(uint32_t first, uint32_t n_, uint32_t width_, uint32_t* counter_)
+        : next(min(first, n_)), end(next + min(width_, n_ - next)), n(n_), width(width_), counter(counter_), open(counter_ != nullptr) {}
+    // The next window, if there is one (uniform, whole wave).
+    __device__ __forceinline__ void take(uint32_t lane) {
+        uint32_t c = 0;
+        if (lane == 0u) c = atomicAdd(counter, width);
+        c = uniform(c);
+        open = c < n;  // (the counter passes n by a window per wave at most)
+        next = min(c, n);
+        end = next + min(width, n - next);
     }
-    __device__ __forceinline__ uint64_t ray(uint32_t i) const {
-        return (uint64_t)width * ((uint64_t)(i / width) * waves + w) + (i & (width - 1u));
-    }
+};
+
+// Counter of a launch of n rays on a stream, or null where none is needed or to be had (then a wave
+// per window).  It lives until the launch is done.
+class RayCounter {
+   public:
+    RayCounter(uint64_t n, uint32_t width, hipStream_t st);
+    ~RayCounter();
+    uint32_t* p = nullptr;
+    uint32_t waves = 0;
+
+   private:
+    hipStream_t st_;
 };
 
 // Per-lane traversal stack of kStack entries (node, tmin, tmax).  Entry e < kTraceLds is in
@@ -169,7 +194,7 @@ __device__ __forceinline__ float from_lane(float v, uint32_t lane) {
 }
 
 // Traces the rays a source hands out to the wave's lanes, until it has no more.
-//   src.next, src.end: ray numbers not handed out yet (uniform);
+//   src.rays: ray numbers to hand out (RayWindow);
 //   src.start(i, o, d, dist): ray i; false when there is nothing to trace;
 //   src.finish(o, d, dist, hit): result of the lane's ray; true when the lane goes on with
 //     another ray that it put in o, d.
@@ -184,10 +209,10 @@ __device__ __forceinline__ float from_lane(float v, uint32_t lane) {
 // distance`), so which triangle decides depends on the order of a leaf's list; here
 // any occluding triangle decides, so the result equals the brute-force predicate
 // whatever the tree.  The search ends at the first occluder.
-// width: rays at once (lanes 0..width).  lds: the wave's kTraceWords.  Whole wave, every lane active.
+// lds: the wave's kTraceWords.  Whole wave, every lane active.
 template <bool kAny, int kStack, typename Src>
 __device__ __forceinline__ void trace_stream(const uint2* __restrict__ nodes, const float4* __restrict__ recs,
-                                             const RootBox& root, float eps, float slack, uint32_t width, uint32_t* lds, Src& src) {
+                                             const RootBox& root, float eps, float slack, uint32_t* lds, Src& src) {
     typedef __attribute__((address_space(3))) uint32_t lds_u32;
     typedef __attribute__((address_space(3))) unsigned long long lds_u64;
     enum : uint32_t { kIdle, kDone, kWalk, kLeaf };
@@ -197,6 +222,8 @@ __device__ __forceinline__ void trace_stream(const uint2* __restrict__ nodes, co
     lds_u64* key = (lds_u64*)(own + 128);
     DeepStack<kStack> deep;
     const LdsStack top{(lds_u64*)(own + 256) + lane, (__attribute__((address_space(3))) float*)(own + 256 + 128 * kTraceLds) + lane};
+    const uint32_t width = src.rays.width;
+    uint32_t steps = 0, lanes = 0;
     const uint32_t refill = width * kRefill / 64u, walk_min = width * kWalkMin / 64u;
     uint32_t state = kIdle, node = 0, best_rec = 0;
     int32_t best_tri = -1;
@@ -215,20 +242,68 @@ __device__ __forceinline__ void trace_stream(const uint2* __restrict__ nodes, co
             break;
         }
     };
+    // One step of a walking lane.
+    auto step = [&]() {
+        if (is_leaf(nd.y)) {
+            if (nd.x != 0u) state = kLeaf;
+            else pop();
+        } else {
+            const uint32_t a = nd.y >> 30;
+            const float s = __uint_as_float(nd.x);
+            const uint32_t left = node + 1, right = nd.y & MNRT_INDEX_MASK;
+            const float oa = comp(o, a), da = comp(d, a), ia = comp(inv, a);
+            const float tsplit = (s - oa) * ia;
+            const bool below = (oa < s) | ((oa == s) & (da > 0.0f));
+            const uint32_t first = below ? left : right, second = below ? right : left;
+            // (a NaN tsplit compares false throughout: both children over the whole interval)
+            const bool near = (tsplit < 0.0f) | (tsplit > tmax * kTravTolHi);
+            const bool far = !near & (tsplit < tmin * kTravTolLo);
+            node = far ? second : first;
+            nd = nodes[node];
+            if (!(near | far)) {
+                if (sp < kStack) stack_put(top, deep, sp++, second, fmaxf(tmin, tsplit * kTravTolLo), tmax);
+                tmax = fminf(tmax, tsplit * kTravTolHi);
+            }
+        }
+    };
+    // The lane's own leaf.
+    auto own_tests = [&]() {
+        const uint32_t begin = nd.y & MNRT_INDEX_MASK;
+        for_leaf_tris(recs + 3ull * begin, nd.x, [&](const float4& a4, const float4& e14, const float4& e24, uint32_t r) {
+            float lam, u, v;
+            if (!(ray_tri(xyz(a4), xyz(e14), xyz(e24), o, d, lam, u, v) && lam > eps)) return false;
+            if (kAny) {
+                if (!(lam < best_t && lam + slack < dist)) return false;
+                best_tri = 0;
+                return true;
+            }
+            const int32_t tri = (int32_t)__float_as_uint(a4.w);
+            if (lam < best_t || (lam == best_t && best_tri >= 0 && tri < best_tri)) {
+                best_t = lam;
+                best_tri = tri;
+                best_rec = begin + r;
+            }
+            return false;
+        });
+    };
     for (;;) {
+        const bool together = width == 64u && lanes >= steps * Src::kTogether;
         const uint32_t busy = (uint32_t)__popcll(ballot(state >= kWalk));
         const uint32_t done = (uint32_t)__popcll(ballot(state == kDone));
-        if (busy == 0u || (src.next < src.end ? width - busy : done) >= refill) {
+        // rays that walk together (steps, lanes: of the set so far) end together: the wave waits for them
+        if (busy == 0u || ((src.rays.open || src.rays.next < src.rays.end ? width - busy : done) >= refill && !together)) {
+            if (busy == 0u) steps = lanes = 0u;
             bool ray = false;
             if (state == kDone) {
                 ray = src.finish(o, d, dist, Hit{best_tri, best_t, best_rec});
                 state = kIdle;
             }
             const bool want = state == kIdle && !ray && lane < width;
+            if (src.rays.next == src.rays.end && src.rays.open) src.rays.take(lane);
             const uint64_t m = ballot(want);
-            const uint32_t rank = mask_prefix(m), left = src.end - src.next;
-            if (want && rank < left) ray = src.start(src.next + rank, o, d, dist);
-            src.next += min((uint32_t)__popcll(m), left);
+            const uint32_t rank = mask_prefix(m), left = src.rays.end - src.rays.next;
+            if (want && rank < left) ray = src.start(src.rays.next + rank, o, d, dist);
+            src.rays.next += min((uint32_t)__popcll(m), left);
             if (ray) {
                 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
                 best_tri = -1;
@@ -244,35 +319,32 @@ __device__ __forceinline__ void trace_stream(const uint2* __restrict__ nodes, co
                     state = kWalk;
                 }
             }
-            if (ballot(state != kIdle) == 0ull && left == 0u) break;
+            if (ballot(state != kIdle) == 0ull && left == 0u && !src.rays.open) break;
+        }
+        if (together) {
+            // every lane to its leaf, and through it
+            for (;;) {
+                const uint32_t walking = (uint32_t)__popcll(ballot(state == kWalk));
+                if (walking == 0u) break;
+                if (busy >= kEarly) {
+                    ++steps;
+                    lanes += walking;
+                }
+                if (state == kWalk) step();
+            }
+            if (state == kLeaf) {
+                own_tests();
+                if (kAny && best_tri >= 0) state = kDone;
+                else pop();
+            }
+            continue;
         }
         // to the next leaf
         for (;;) {
             const uint64_t m = ballot(state == kWalk);
-            if (m == 0ull || ((uint32_t)__popcll(m) < walk_min && ballot(state == kLeaf) != 0ull)) break;
-            if (state == kWalk) {
-                if (is_leaf(nd.y)) {
-                    if (nd.x != 0u) state = kLeaf;
-                    else pop();
-                } else {
-                    const uint32_t a = nd.y >> 30;
-                    const float s = __uint_as_float(nd.x);
-                    const uint32_t left = node + 1, right = nd.y & MNRT_INDEX_MASK;
-                    const float oa = comp(o, a), da = comp(d, a), ia = comp(inv, a);
-                    const float tsplit = (s - oa) * ia;
-                    const bool below = (oa < s) | ((oa == s) & (da > 0.0f));
-                    const uint32_t first = below ? left : right, second = below ? right : left;
-                    // (a NaN tsplit compares false throughout: both children over the whole interval)
-                    const bool near = (tsplit < 0.0f) | (tsplit > tmax * kTravTolHi);
-                    const bool far = !near & (tsplit < tmin * kTravTolLo);
-                    node = far ? second : first;
-                    nd = nodes[node];
-                    if (!(near | far)) {
-                        if (sp < kStack) stack_put(top, deep, sp++, second, fmaxf(tmin, tsplit * kTravTolLo), tmax);
-                        tmax = fminf(tmax, tsplit * kTravTolHi);
-                    }
-                }
-            }
+            const uint32_t walking = (uint32_t)__popcll(m);
+            if (walking == 0u || (walking < walk_min && ballot(state == kLeaf) != 0ull)) break;
+            if (state == kWalk) step();
         }
         const bool at_leaf = state == kLeaf;
         if (ballot(at_leaf) == 0ull) continue;
@@ -282,22 +354,7 @@ __device__ __forceinline__ void trace_stream(const uint2* __restrict__ nodes, co
         if (3u * ((total + 63u) >> 6) >= 2u * most) {
             // about equally full leaves (a lane's own test costs two thirds of a dealt one)
             if (at_leaf)
-                for_leaf_tris(recs + 3ull * begin, cnt, [&](const float4& a4, const float4& e14, const float4& e24, uint32_t r) {
-                    float lam, u, v;
-                    if (!(ray_tri(xyz(a4), xyz(e14), xyz(e24), o, d, lam, u, v) && lam > eps)) return false;
-                    if (kAny) {
-                        if (!(lam < best_t && lam + slack < dist)) return false;
-                        best_tri = 0;
-                        return true;
-                    }
-                    const int32_t tri = (int32_t)__float_as_uint(a4.w);
-                    if (lam < best_t || (lam == best_t && best_tri >= 0 && tri < best_tri)) {
-                        best_t = lam;
-                        best_tri = tri;
-                        best_rec = begin + r;
-                    }
-                    return false;
-                });
+                own_tests();
         } else {
             const uint32_t first = incl - cnt, shift = begin - first;
             // a key is (lambda, triangle); before any hit (limit, 0), which no hit equals or

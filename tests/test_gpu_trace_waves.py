@@ -1,5 +1,5 @@
 """Ray launches at the sizes where a wave's share changes: fewer rays than lanes, the widths of 16,
-32 and 64 rays a wave, partial tiles, and runs that refill (more tiles than waves); with rays that
+32 and 64 rays a wave, partial windows, and waves that take further windows from a counter; with rays that
 miss, leaves of very different sizes and equal lambdas.  Closest hits (index, lambda, barycentrics)
 and occlusion equal the oracle's bit for bit."""
 
@@ -31,7 +31,7 @@ def trees(orc, cuda):
     return v, T, DT
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 1000, 32767, 32768, 32769, 65535, 65536, 65537, 393216, 393217, 500001])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 1000, 32767, 32768, 32769, 65535, 65536, 65537, 98305, 196609, 589824, 589825, 700001])
 def test_ray_counts(orc, cuda, trees, n):
     v, T, DT = trees
     rng = np.random.default_rng(n)
