@@ -1002,16 +1002,26 @@ struct SmallOut {
     const uint32_t* ref_base;
 };
 
-// Returns `old` with lane `lane` replaced by the wave-uniform `v` (v_writelane_b32, which
-// ignores exec; with an SGPR source the lane select has to be m0).
-__device__ __forceinline__ uint32_t write_lane(uint32_t v, int lane, uint32_t old) {
-    uint32_t r;
-    asm("v_writelane_b32 %0, %1, m0"
-        : "=v"(r)
-        : "s"(__builtin_amdgcn_readfirstlane(v)), "{m0}"(__builtin_amdgcn_readfirstlane(lane)), "0"(old));
-    return r;
+// m = 2 m + (u < v) and 2 m + (u > v), u wave-uniform: the comparison's result is the carry.
+__device__ __forceinline__ void shift_in_less(uint32_t& m, float u, float v) {
+    asm("v_cmp_lt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "s"(u), "v"(v) : "vcc");
+}
+__device__ __forceinline__ void shift_in_greater(uint32_t& m, float u, float v) {
+    asm("v_cmp_gt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "s"(u), "v"(v) : "vcc");
+}
+// The floats next to a finite one (+0 for either zero).
+__device__ __forceinline__ float next_down(float f) {
+    const uint32_t u = __float_as_uint(f);
+    return __uint_as_float(f > 0.0f ? u - 1u : (f < 0.0f ? u + 1u : 0x80000001u));
+}
+__device__ __forceinline__ float next_up(float f) {
+    const uint32_t u = __float_as_uint(f);
+    return __uint_as_float(f > 0.0f ? u + 1u : (f < 0.0f ? u - 1u : 1u));
 }
 
+// Bound by instruction issue: 7.0 k vector instructions per root of the 1.03M-triangle build (42 k
+// roots, 439 us; 586 us with the masks built candidate by candidate, both children through the stack and
+// every node's candidates evaluated).
 // kMode kSmallStage: subtree sizes, and the subtree written to its staging area while it
 // fits; kSmallEmit: written at its final address (only roots with st_ovf set
 // when st_ovf is given).
@@ -1047,67 +1057,51 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, const Sm
     const bool mleft = plane_goes_left(midx);
     // Candidates axis-major, minimums then maximums (kernel_CreateSplitCandidates,
     // kdtree.cu:1035-1082), c = isMax * 3n + axis * n + i; masks as kernel_InitSplitMasks
-    // (kdtree.cu:1110-1251).  One candidate per step: every lane compares its element with
-    // the plane, the comparisons' lane masks combine into the candidate's masks (element
-    // i itself, and elements lying in the plane, by the rules below), and lane i keeps
-    // them for its own candidate (writelane); each lane writes its candidates at the end
-    // of the axis.  Lane i keeps the masks of its element's candidates in registers (slot
-    // isMax * 3 + axis: candidate c = slot * n + i).
+    // (kdtree.cu:1110-1251).  Lane i holds its element's candidates and compares them with one element
+    // per step, whose bounds are broadcast; a comparison's result is shifted into the lane's mask
+    // by an add with carry, so a step is 10 instructions for four masks (one lane mask per
+    // candidate, combined and written to its lane, took about 50).  Lane i keeps the masks of its
+    // element's candidates in registers (slot isMax * 3 + axis: candidate c = slot * n + i).
     //   triangles: L = min < s, R = s < max; the candidate's own element goes right of
     //              its minimum and left of its maximum; a flat element in the plane goes
     //              left if plane_goes_left, else right;
     //   points:    L = p < s, R = s < p; a point in the plane goes left if
     //              plane_goes_left, else right.
+    // "In the plane as well" is a comparison with the next float below or above (no candidate of
+    // use is infinite).
     uint64_t cmL[kSlots], cmR[kSlots];
-    const uint64_t vmask = (n >= 64) ? ~0ull : ((1ull << n) - 1ull);
-    const uint64_t leftm = __builtin_amdgcn_ballot_w64(mleft) & vmask;
-    for (uint32_t ax = 0; ax < 3; ++ax) {
-        const float mn = ax == 0 ? mlo.x : (ax == 1 ? mlo.y : mlo.z);
-        const float mx = ax == 0 ? mhi.x : (ax == 1 ? mhi.y : mhi.z);
-        const uint64_t flat = (kind == MNRT_KIND_TRI) ? __builtin_amdgcn_ballot_w64(mn == mx) & vmask : vmask;
-        // this lane's minimum (0) and maximum (1) candidate: masks as 32-bit halves
-        uint32_t l0lo = 0, l0hi = 0, r0lo = 0, r0hi = 0, l1lo = 0, l1hi = 0, r1lo = 0, r1hi = 0;
-        for (uint32_t i = 0; i < n; ++i) {
-            const uint64_t self = 1ull << i;
+    const uint64_t self = 1ull << lane;
 #pragma unroll
-            for (int isMax = 0; isMax < (kind == MNRT_KIND_TRI ? 2 : 1); ++isMax) {
-                const float sp = __uint_as_float(
-                    __builtin_amdgcn_readlane(__float_as_uint(isMax ? mx : mn), (int)i));
-                const uint64_t lt = __builtin_amdgcn_ballot_w64(mn < sp);
-                const uint64_t gt = __builtin_amdgcn_ballot_w64(sp < mx);
-                const uint64_t eq = __builtin_amdgcn_ballot_w64(mn == sp) & flat;
-                uint64_t ml, mr;
+    for (int ax = 0; ax < 3; ++ax) {
+        const float mn = f4c(mlo, ax), mx = f4c(mhi, ax);
+        const bool in_plane = (kind == MNRT_KIND_POINT || mn == mx) && fabsf(mn) < kInf;
+        const float below = in_plane && mleft ? next_down(mn) : mn, above = in_plane && !mleft ? next_up(mx) : mx;
+        uint32_t w[2][4];  // halves of the masks: left and right of the minimum, of the maximum
+#pragma unroll
+        for (int half = 1; half >= 0; --half) {
+            uint32_t l0 = 0, r0 = 0, l1 = 0, r1 = 0;
+            for (int j = (int)min(n, half ? 64u : 32u) - 1; j >= 32 * half; --j) {
+                const float lo_j = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(below), j));
+                const float hi_j = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(above), j));
+                shift_in_less(l0, lo_j, mn);
+                shift_in_greater(r0, hi_j, mn);
                 if (kind == MNRT_KIND_TRI) {
-                    const uint64_t planar = eq & ~self;
-                    ml = (lt | (planar & leftm) | (isMax ? self : 0ull)) & vmask;
-                    mr = (gt | (planar & ~leftm) | (isMax ? 0ull : self)) & vmask;
-                } else {
-                    ml = (lt | (eq & leftm)) & vmask;
-                    mr = (gt | (eq & ~leftm)) & vmask;
-                }
-                if (isMax) {
-                    l1lo = write_lane((uint32_t)ml, (int)i, l1lo);
-                    l1hi = write_lane((uint32_t)(ml >> 32), (int)i, l1hi);
-                    r1lo = write_lane((uint32_t)mr, (int)i, r1lo);
-                    r1hi = write_lane((uint32_t)(mr >> 32), (int)i, r1hi);
-                } else {
-                    l0lo = write_lane((uint32_t)ml, (int)i, l0lo);
-                    l0hi = write_lane((uint32_t)(ml >> 32), (int)i, l0hi);
-                    r0lo = write_lane((uint32_t)mr, (int)i, r0lo);
-                    r0hi = write_lane((uint32_t)(mr >> 32), (int)i, r0hi);
+                    shift_in_less(l1, lo_j, mx);
+                    shift_in_greater(r1, hi_j, mx);
                 }
             }
+            w[half][0] = l0;
+            w[half][1] = r0;
+            w[half][2] = l1;
+            w[half][3] = r1;
         }
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {  // registers by constant index: the axis as selects
-            if (ax == (uint32_t)k) {
-                cmL[k] = ((uint64_t)l0hi << 32) | l0lo;
-                cmR[k] = ((uint64_t)r0hi << 32) | r0lo;
-                if (kind == MNRT_KIND_TRI) {
-                    cmL[3 + k] = ((uint64_t)l1hi << 32) | l1lo;
-                    cmR[3 + k] = ((uint64_t)r1hi << 32) | r1lo;
-                }
-            }
+        cmL[ax] = (uint64_t)w[1][0] << 32 | w[0][0];
+        cmR[ax] = (uint64_t)w[1][1] << 32 | w[0][1];
+        if (kind == MNRT_KIND_TRI) {
+            cmL[ax] &= ~self;
+            cmR[ax] |= self;
+            cmL[3 + ax] = ((uint64_t)w[1][2] << 32 | w[0][2]) | self;
+            cmR[3 + ax] = ((uint64_t)w[1][3] << 32 | w[0][3]) & ~self;
         }
     }
 
@@ -1132,25 +1126,18 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, const Sm
         refs = O.st_refs + off;
         lim_nodes = lim_refs = O.st_cap.of(n);
     }
+    // the node at hand; left children follow at once, right ones wait on the stack
     int sp = 0;
-    if (lane == 0) {
-        SmallStackEnt e;
-        e.mask = (n == 64) ? ~0ull : ((1ull << n) - 1ull);
-        for (int k = 0; k < 3; ++k) {
-            e.lo[k] = root.lo[k];
-            e.hi[k] = root.hi[k];
-        }
-        e.lvl_ax = root.level;
-        e.patch = kNone;
-        stack[0] = e;
+    SmallStackEnt e;
+    e.mask = (n == 64) ? ~0ull : ((1ull << n) - 1ull);
+    for (int k = 0; k < 3; ++k) {
+        e.lo[k] = root.lo[k];
+        e.hi[k] = root.hi[k];
     }
-    sp = 1;
-    wave_sync();
+    e.lvl_ax = root.level;
+    e.patch = kNone;
     const float qr2 = 2.0f * scene_qr[scene];
-    while (sp > 0) {
-        --sp;
-        SmallStackEnt e = stack[sp];
-        wave_sync();
+    for (;;) {
         if (writing && (addr >= lim_nodes || rbase > lim_refs)) {
             if (kMode == kSmallEmit) {
                 if (lane == 0) atomicOr(&O.W[W_ERR], 4u);
@@ -1163,8 +1150,13 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, const Sm
         const uint32_t cnt = (uint32_t)__popcll(e.mask);
         float best_cost = kInf;
         uint32_t best = kNone;
-        if (cnt > 0 && e.level() < MNRT_MAX_LEVEL) {
-            float ext[3] = {e.hi[0] - e.lo[0], e.hi[1] - e.lo[1], e.hi[2] - e.lo[2]};
+        const float ext[3] = {e.hi[0] - e.lo[0], e.hi[1] - e.lo[1], e.hi[2] - e.lo[2]};
+        // A split leaves elements on both sides, so it costs kCostTraverse and at least the node's own
+        // area or volume once: 4 and more, up to rounding, which three elements never exceed.  (In a box
+        // turned inside out, as a caller may give it, areas do not add up.)
+        const bool plain = ext[0] >= 0.0f && ext[1] >= 0.0f && ext[2] >= 0.0f && (kind == MNRT_KIND_TRI || qr2 >= 0.0f);
+        const bool never = plain && cnt <= 3u;
+        if (cnt > 0 && !never && e.level() < MNRT_MAX_LEVEL) {
             float denom;
             if (kind == MNRT_KIND_POINT) {
                 float vol = 1.0f;
@@ -1246,6 +1238,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, const Sm
             }
             ++addr;
             rbase += cnt;
+            if (sp == 0) break;
+            --sp;
+            wave_sync();
+            e = stack[sp];
             continue;
         }
         // the chosen candidate: slot and element lane from the key, its plane and masks
@@ -1273,23 +1269,19 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_small(DN dnsmall, const Sm
             nodes[2 * addr + 1] = a << 30;
         }
         if (lane == 0) {
-            SmallStackEnt R = e, L = e;
+            SmallStackEnt R = e;
             R.mask = selR & e.mask;
-            for (uint32_t k = 0; k < 3; ++k) {  // the plane bounds the split axis (selects, not indexing)
-                R.lo[k] = (a == k) ? s : e.lo[k];
-                L.hi[k] = (a == k) ? s : e.hi[k];
-            }
+            for (uint32_t k = 0; k < 3; ++k) R.lo[k] = (a == k) ? s : e.lo[k];  // (selects, not indexing)
             R.lvl_ax = (e.level() + 1) | (a << 30);
             R.patch = addr;
-            L.mask = selL & e.mask;
-            L.lvl_ax = e.level() + 1;
-            L.patch = kNone;
             stack[sp] = R;
-            stack[sp + 1] = L;
         }
-        sp += 2;
+        ++sp;
         ++addr;
-        wave_sync();
+        e.mask &= selL;
+        for (uint32_t k = 0; k < 3; ++k) e.hi[k] = (a == k) ? s : e.hi[k];
+        e.lvl_ax = e.level() + 1;
+        e.patch = kNone;
     }
     if (kMode == kSmallStage && lane == 0) {
         O.nsize[r] = addr;
