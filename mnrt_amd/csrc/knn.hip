@@ -1103,7 +1103,11 @@ __global__ __launch_bounds__(256) void k_scatter_runs(const float4* __restrict__
 
 // Bound on |weight| per query for the fixed-point scale of the backward pass, from the
 // forward's r2 and neighbour counts (same expressions as the backward kernel).
-__global__ __launch_bounds__(256) void k_bwd_wmax(uint32_t n, const float4* __restrict__ grad,
+// Workgroups of the passes that bound the weights: one atomic each (per scene), or the atomics of all
+// waves on one address would take longer than the pass (6.6 ns each).
+constexpr uint32_t kWmaxBlock = 1024;
+
+__global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax(uint32_t n, const float4* __restrict__ grad,
                                                   const float4* __restrict__ clr, const float4* __restrict__ infl,
                                                   const float* __restrict__ r2, const uint32_t* __restrict__ count,
                                                   uint32_t* __restrict__ wmax_bits) {
@@ -1123,8 +1127,15 @@ __global__ __launch_bounds__(256) void k_bwd_wmax(uint32_t n, const float4* __re
             if (!(m <= kInf)) m = kInf;  // NaN / inf gradients saturate the bound
         }
     }
-    for (uint32_t o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    if ((threadIdx.x & 63u) == 0 && m > 0.0f) atomicMax(wmax_bits, __float_as_uint(m));
+    __shared__ uint32_t s_max[kWmaxBlock / 64];
+    const uint32_t b = wave_max_u32(__float_as_uint(m));  // (m >= 0: order of the bits)
+    if ((threadIdx.x & 63u) == 0) s_max[threadIdx.x >> 6] = b;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (uint32_t w = 0; w < kWmaxBlock / 64; ++w) t = max(t, s_max[w]);
+        if (t) atomicMax(wmax_bits, t);
+    }
 }
 
 __global__ __launch_bounds__(256) void k_fix_to_float(uint32_t np, const unsigned long long* __restrict__ acc,
@@ -1140,7 +1151,7 @@ __global__ __launch_bounds__(256) void k_fix_to_float(uint32_t np, const unsigne
 
 // Per-scene weight bounds: slot g of scene s (g - slot_begin[s] < count[s]) adds its
 // bound to wmax[s]; a wave whose slots lie in one scene reduces first.
-__global__ __launch_bounds__(256) void k_bwd_wmax_batch(uint32_t n, const uint32_t* __restrict__ slot_begin,
+__global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax_batch(uint32_t n, const uint32_t* __restrict__ slot_begin,
                                                         uint32_t ns, const uint32_t* __restrict__ count,
                                                         const float4* __restrict__ grad,
                                                         const float4* __restrict__ clr,
@@ -1169,12 +1180,23 @@ __global__ __launch_bounds__(256) void k_bwd_wmax_batch(uint32_t n, const uint32
             }
         }
     }
-    const uint32_t s0 = uniform(s);
-    if (ballot(s != s0) == 0ull) {
-        for (uint32_t o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-        if ((threadIdx.x & 63u) == 0 && m > 0.0f) atomicMax(&wmax_bits[s0], __float_as_uint(m));
-    } else if (m > 0.0f) {
-        atomicMax(&wmax_bits[s], __float_as_uint(m));
+    __shared__ uint32_t s_max[kWmaxBlock / 64], s_scene[kWmaxBlock / 64];
+    const uint32_t s0 = uniform(s), wave = threadIdx.x >> 6;
+    const bool one = ballot(s != s0) == 0ull;  // the wave's slots are one scene's
+    const uint32_t b = wave_max_u32(one ? __float_as_uint(m) : 0u);  // (m >= 0: order of the bits)
+    if ((threadIdx.x & 63u) == 0) {
+        s_max[wave] = b;
+        s_scene[wave] = s0;
+    }
+    if (!one && m > 0.0f) atomicMax(&wmax_bits[s], __float_as_uint(m));
+    __syncthreads();
+    if (threadIdx.x < kWmaxBlock / 64) {  // one atomic per run of waves of one scene
+        const uint32_t i = threadIdx.x, sc = s_scene[i];
+        if (i == 0u || s_scene[i - 1u] != sc) {
+            uint32_t t = 0;
+            for (uint32_t w = i; w < kWmaxBlock / 64 && s_scene[w] == sc; ++w) t = max(t, s_max[w]);
+            if (t) atomicMax(&wmax_bits[sc], t);
+        }
     }
 }
 
@@ -1375,7 +1397,7 @@ int launch_knn_bwd_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_
         hipLaunchKernelGGL(k_zero_u64, dim3(zb), dim3(256), 0, st, G.acc, words);
     }
     if (n)
-        hipLaunchKernelGGL(k_bwd_wmax_batch, dim3((n + 255) / 256), dim3(256), 0, st, n, slot_begin, ns, count,
+        hipLaunchKernelGGL(k_bwd_wmax_batch, dim3((n + kWmaxBlock - 1) / kWmaxBlock), dim3(kWmaxBlock), 0, st, n, slot_begin, ns, count,
                            G.grad, G.clr, G.infl, fwd_r2, fwd_count, wmax);
     hipLaunchKernelGGL(k_bwd_scale_batch, dim3(1), dim3(64), 0, st, ns, slot_begin, count, wmax, scale);
     const uint32_t chunk = std::max<uint32_t>(1u, std::min<uint32_t>(kBwdChunk, (uint32_t)kPairCap / G.k));
@@ -1625,7 +1647,8 @@ extern "C" int mnrt_knn_gather_bwd(const mnrt_tree* pmap, uint32_t k, float r_ma
     uint32_t h_wmax = 0;
     if (hipMemsetAsync(buf, 0, (size_t)np * 24 + 4, st) != hipSuccess) rc = MNRT_ERR_HIP;
     if (rc == MNRT_OK) {
-        hipLaunchKernelGGL(mnrt::k_bwd_wmax, dim3((n + 255) / 256), dim3(256), 0, st, n, (const float4*)d_grad_rad4,
+        hipLaunchKernelGGL(mnrt::k_bwd_wmax, dim3((n + mnrt::kWmaxBlock - 1) / mnrt::kWmaxBlock), dim3(mnrt::kWmaxBlock), 0, st, n,
+                           (const float4*)d_grad_rad4,
                            (const float4*)d_clr4, (const float4*)d_infl4, d_r2, d_count, wmax);
         if (hipMemcpyAsync(&h_wmax, wmax, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
             hipStreamSynchronize(st) != hipSuccess)

@@ -173,8 +173,14 @@ __device__ __forceinline__ uint32_t bound_bits(float m) {
     return (m <= kInf) ? __float_as_uint(m) : 0x7F800000u;
 }
 
-// Pass 1: the largest |term| of each output array (emission, albedo), one atomic per wave.
-__global__ __launch_bounds__(256) void k_rw_bound(RwArgs A, uint32_t* __restrict__ bound) {
+// Workgroups of the two passes over the photons: many waves, since what a workgroup adds to
+// addresses that all of them share (bounds, emission sums) is reduced in LDS first.  Atomics of all
+// waves on one line took 94 us of the bound pass (524288 photons: 8192 waves).
+constexpr uint32_t kRwBlock = 1024;
+constexpr uint32_t kRwLights = 256;  // lights whose sums a workgroup keeps in LDS
+
+// Pass 1: the largest |term| of each output array (emission, albedo), one atomic per workgroup.
+__global__ __launch_bounds__(kRwBlock) void k_rw_bound(RwArgs A, uint32_t* __restrict__ bound) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     float me = 0.0f, ma = 0.0f;
     if (i < A.np) {
@@ -192,10 +198,17 @@ __global__ __launch_bounds__(256) void k_rw_bound(RwArgs A, uint32_t* __restrict
             ma = fmaxf(ma, abs_max3(v));
         }
     }
+    __shared__ uint32_t s_max[2][kRwBlock / 64];
     const uint32_t be = wave_max_u32(bound_bits(me)), ba = wave_max_u32(bound_bits(ma));
     if ((threadIdx.x & 63u) == 0) {
-        if (be) atomicMax(&bound[0], be);
-        if (ba) atomicMax(&bound[1], ba);
+        s_max[0][threadIdx.x >> 6] = be;
+        s_max[1][threadIdx.x >> 6] = ba;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2u) {
+        uint32_t m = 0;
+        for (uint32_t w = 0; w < kRwBlock / 64; ++w) m = max(m, s_max[threadIdx.x][w]);
+        if (m) atomicMax(&bound[threadIdx.x], m);
     }
 }
 
@@ -219,7 +232,7 @@ __device__ __forceinline__ long long to_fixed(float v, double unit) {
 // key are summed by a wave reduction first (up to kShareRounds distinct keys, taken in
 // lane order), the rest add on their own.  Called by every lane of the wave.
 __device__ __forceinline__ void add_shared(uint32_t key, long long x, long long y, long long z,
-                                           unsigned long long* __restrict__ acc, uint32_t lane) {
+                                           unsigned long long* acc, uint32_t lane) {
     bool pending = key != kNone && (x != 0 || y != 0 || z != 0);
     for (int round = 0; round < kShareRounds; ++round) {
         const uint64_t act = __ballot(pending);
@@ -246,7 +259,7 @@ __device__ __forceinline__ void add_shared(uint32_t key, long long x, long long 
 
 // Pass 2: every term in its array's unit, summed per output.  No lane leaves early (the
 // wave reductions need them all).
-__global__ __launch_bounds__(256) void k_rw_accumulate(RwArgs A, const uint32_t* __restrict__ bound,
+__global__ __launch_bounds__(kRwBlock) void k_rw_accumulate(RwArgs A, const uint32_t* __restrict__ bound,
                                                        double terms_e, double terms_a,
                                                        unsigned long long* __restrict__ acc_e,
                                                        unsigned long long* __restrict__ acc_a) {
@@ -254,6 +267,12 @@ __global__ __launch_bounds__(256) void k_rw_accumulate(RwArgs A, const uint32_t*
     const uint32_t lane = threadIdx.x & 63u;
     const double ue = fixed_unit(bound[0], terms_e), ua = fixed_unit(bound[1], terms_a);
     if (ue < 0.0 || ua < 0.0) return;  // non-finite gradients: the outputs become NaN (uniform)
+    __shared__ unsigned long long s_e[3 * kRwLights];
+    const bool few = A.num_lights <= kRwLights;
+    if (few) {
+        for (uint32_t j = threadIdx.x; j < 3u * A.num_lights; j += kRwBlock) s_e[j] = 0ull;
+        __syncthreads();
+    }
     Path P{};
     PhotonTerms T{};
     const bool ph = i < A.np;
@@ -262,7 +281,14 @@ __global__ __launch_bounds__(256) void k_rw_accumulate(RwArgs A, const uint32_t*
         T = photon_terms(A, i, P);
     }
     const bool pe = ph && P.ok;
-    add_shared(pe ? P.l : kNone, to_fixed(T.e[0], ue), to_fixed(T.e[1], ue), to_fixed(T.e[2], ue), acc_e, lane);
+    if (few) {
+        add_shared(pe ? P.l : kNone, to_fixed(T.e[0], ue), to_fixed(T.e[1], ue), to_fixed(T.e[2], ue), s_e, lane);
+        __syncthreads();
+        for (uint32_t j = threadIdx.x; j < 3u * A.num_lights; j += kRwBlock)
+            if (s_e[j]) atomicAdd(&acc_e[j], s_e[j]);
+    } else {
+        add_shared(pe ? P.l : kNone, to_fixed(T.e[0], ue), to_fixed(T.e[1], ue), to_fixed(T.e[2], ue), acc_e, lane);
+    }
 #pragma unroll
     for (int k = 0; k < kPathTris; ++k)
         add_shared(pe ? P.t[k] : kNone, to_fixed(T.a[k][0], ua), to_fixed(T.a[k][1], ua), to_fixed(T.a[k][2], ua),
@@ -357,8 +383,8 @@ extern "C" int mnrt_photons_reweight_bwd(uint32_t np, const float* d_base_pow4, 
     const double terms_e = (double)np, terms_a = (double)kPathTris * np + (double)nq;
     const uint32_t n = std::max(np, nq);
     if (n > 0) {
-        hipLaunchKernelGGL(k_rw_bound, dim3((n + 255) / 256), dim3(256), 0, st, A, bound);
-        hipLaunchKernelGGL(k_rw_accumulate, dim3((n + 255) / 256), dim3(256), 0, st, A, (const uint32_t*)bound,
+        hipLaunchKernelGGL(k_rw_bound, dim3((n + kRwBlock - 1) / kRwBlock), dim3(kRwBlock), 0, st, A, bound);
+        hipLaunchKernelGGL(k_rw_accumulate, dim3((n + kRwBlock - 1) / kRwBlock), dim3(kRwBlock), 0, st, A, (const uint32_t*)bound,
                            terms_e, terms_a, acc_e, acc_a);
     }
     const size_t outs = 3ull * std::max(num_lights, num_tris);
