@@ -96,7 +96,7 @@ struct KnnArgs {
     // backward
     const float4* grad;            // dLoss/dradiance per query
     unsigned long long* acc;       // 3 fixed-point accumulators per photon (original index)
-    double fix_scale;              // accumulator units per unit gradient (a power of two)
+    const double* fix_scale;       // accumulator units per unit gradient (a power of two; 0: no weight)
     float4* out_grad_clr;          // dLoss/d(diffuse colour) per query
     uint32_t chain;                // consecutive queries per wave (plain launches, set there)
     const uint32_t* order;         // processing order of the queries (null: 0..n-1)

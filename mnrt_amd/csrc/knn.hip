@@ -1052,6 +1052,8 @@ __global__ __launch_bounds__(256) void k_knn_bwd_chunks(KnnArgs A, uint32_t chun
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t j0 = ((uint64_t)blockIdx.x * kWavesPerBlock + wave) * A.chain;
     if (j0 >= A.n) return;  // uniform per wave
+    const double fix_scale = ld_uniform(A.fix_scale, 0u);
+    if (!(fix_scale > 0.0) && !A.out_grad_clr) return;  // no weight: no gradient of the powers
     const uint32_t n = (uint32_t)min<uint64_t>(A.chain, A.n - j0);
     const KnnTree Tr{A.nodes, A.recs, A.boxes, A.r2max, A.r_max};
     WarmHint hint{-1.0f, A.order_far && !order_coherent(A.n, A.order_far)};
@@ -1068,7 +1070,7 @@ __global__ __launch_bounds__(256) void k_knn_bwd_chunks(KnnArgs A, uint32_t chun
                                                   s_soff[kBoxes ? 0 : wave], hint, F, &sink);
         }
         const KnnArgs L = late_args();
-        knn_finish<kModeBackward>(L, Q, F, lane >= c0 && lane < c1, L.r_max, lane - c0, L.fix_scale, s_w[wave]);
+        knn_finish<kModeBackward>(L, Q, F, lane >= c0 && lane < c1, L.r_max, lane - c0, fix_scale, s_w[wave]);
         wave_sync();
         merge_pairs(s_pairs[wave], sink.n, s_w[wave], L.acc, lane);
         wave_sync();
@@ -1139,9 +1141,10 @@ __global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax(uint32_t n, const float
 }
 
 __global__ __launch_bounds__(256) void k_fix_to_float(uint32_t np, const unsigned long long* __restrict__ acc,
-                                                      double inv_scale, float4* __restrict__ out) {
+                                                      const double* __restrict__ scale, float4* __restrict__ out) {
     uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
+    const double inv_scale = *scale > 0.0 ? 1.0 / *scale : 0.0;
     out[p] = make_float4((float)((double)(long long)acc[3ull * p] * inv_scale),
                          (float)((double)(long long)acc[3ull * p + 1] * inv_scale),
                          (float)((double)(long long)acc[3ull * p + 2] * inv_scale), 0.0f);
@@ -1202,20 +1205,26 @@ __global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax_batch(uint32_t n, const
 
 // Fixed-point unit per scene from its bound and query count: the largest power of two
 // with count * wmax * unit < 2^62 (the same expression as the single-scene entry point).
+__device__ __forceinline__ double bwd_scale(uint32_t n, uint32_t wmax_bits) {
+    const float wm = __uint_as_float(wmax_bits);
+    if (!(n > 0 && wm > 0.0f && wm <= kInf)) return 0.0;
+    int e = 0;
+    (void)frexp(4.611686018427387904e18 / ((double)n * (double)wm), &e);
+    return ldexp(1.0, e - 1);
+}
+
+__global__ __launch_bounds__(64) void k_bwd_scale(uint32_t n, const uint32_t* __restrict__ wmax_bits,
+                                                  double* __restrict__ scale) {
+    if (threadIdx.x == 0) *scale = bwd_scale(n, *wmax_bits);
+}
+
 __global__ __launch_bounds__(64) void k_bwd_scale_batch(uint32_t ns, const uint32_t* __restrict__ slot_begin,
                                                         const uint32_t* __restrict__ count,
                                                         const uint32_t* __restrict__ wmax_bits,
                                                         double* __restrict__ scale) {
     for (uint32_t s = threadIdx.x; s < ns; s += blockDim.x) {
         const uint32_t n = count ? count[s] : slot_begin[s + 1] - slot_begin[s];
-        const float wm = __uint_as_float(wmax_bits[s]);
-        double sc = 0.0;
-        if (n > 0 && wm > 0.0f && wm <= kInf) {
-            int e = 0;
-            (void)frexp(4.611686018427387904e18 / ((double)n * (double)wm), &e);
-            sc = ldexp(1.0, e - 1);
-        }
-        scale[s] = sc;
+        scale[s] = bwd_scale(n, wmax_bits[s]);
     }
 }
 
@@ -1639,38 +1648,32 @@ extern "C" int mnrt_knn_gather_bwd(const mnrt_tree* pmap, uint32_t k, float r_ma
     }
     if (!d_pos4 || !d_nrm4 || !d_dir4 || !d_infl4 || !d_grad_rad4 || !d_r2 || !d_count || !(r_max > 0.0f))
         return MNRT_ERR_ARG;
+    // (not for a stream that is being captured: the workspace is given back on return)
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    MNRT_HIP_CHECK(hipStreamIsCapturing(st, &cs));
+    if (cs != hipStreamCaptureStatusNone) return MNRT_ERR_HIP;
     void* buf = nullptr;
     MNRT_HIP_CHECK(mnrt::pool_alloc(&buf, (size_t)np * 24 + 256, st));
+    // accumulators, the largest weight, the scale: all on the device, so the call waits for nothing
+    // (reading the weight back and scaling on the host left the GPU idle for a fifth of a 131072-photon,
+    // 77361-query call)
     unsigned long long* acc = (unsigned long long*)buf;
-    uint32_t* wmax = (uint32_t*)((char*)buf + (size_t)np * 24);
-    rc = MNRT_OK;
-    uint32_t h_wmax = 0;
-    if (hipMemsetAsync(buf, 0, (size_t)np * 24 + 4, st) != hipSuccess) rc = MNRT_ERR_HIP;
-    if (rc == MNRT_OK) {
-        hipLaunchKernelGGL(mnrt::k_bwd_wmax, dim3((n + mnrt::kWmaxBlock - 1) / mnrt::kWmaxBlock), dim3(mnrt::kWmaxBlock), 0, st, n,
-                           (const float4*)d_grad_rad4,
-                           (const float4*)d_clr4, (const float4*)d_infl4, d_r2, d_count, wmax);
-        if (hipMemcpyAsync(&h_wmax, wmax, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess)
-            rc = MNRT_ERR_HIP;
-    }
-    float wm = 0.0f;
-    std::memcpy(&wm, &h_wmax, 4);
-    double scale = 0.0;
-    if (rc == MNRT_OK && wm > 0.0f && wm <= mnrt::kInf) {
-        // |sum| <= n * wmax * scale < 2^62
-        int e = 0;
-        std::frexp(4.611686018427387904e18 / ((double)n * (double)wm), &e);
-        scale = std::ldexp(1.0, e - 1);
-    } else if (rc == MNRT_OK && wm > mnrt::kInf) {
-        rc = MNRT_ERR_ARG;  // non-finite upstream gradient
-    }
+    uint32_t* wmax = (uint32_t*)(acc + 3ull * np);
+    double* scale = (double*)(acc + 3ull * np + 1u);
+    const uint64_t words = 3ull * np + 1u;
+    hipLaunchKernelGGL(mnrt::k_zero_u64, dim3((uint32_t)std::min<uint64_t>((words + 255) / 256, 8192)), dim3(256), 0, st,
+                       acc, words);
+    hipLaunchKernelGGL(mnrt::k_bwd_wmax, dim3((n + mnrt::kWmaxBlock - 1) / mnrt::kWmaxBlock), dim3(mnrt::kWmaxBlock), 0,
+                       st, n, (const float4*)d_grad_rad4, (const float4*)d_clr4, (const float4*)d_infl4, d_r2, d_count,
+                       wmax);
+    hipLaunchKernelGGL(mnrt::k_bwd_scale, dim3(1), dim3(64), 0, st, n, (const uint32_t*)wmax, scale);
+    rc = hipGetLastError() == hipSuccess ? MNRT_OK : MNRT_ERR_HIP;
     const uint32_t* order = nullptr;
     const uint32_t* order_far = nullptr;
     void* obuf = nullptr;
     if (rc == MNRT_OK)
         rc = mnrt::spatial_order(pmap->root_min, pmap->root_max, n, d_pos4, st, &order, &obuf, &order_far);
-    if (rc == MNRT_OK && scale > 0.0) {
+    if (rc == MNRT_OK) {
         mnrt::KnnArgs A{};
         A.order = order;
         A.order_far = order_far;
@@ -1692,32 +1695,10 @@ extern "C" int mnrt_knn_gather_bwd(const mnrt_tree* pmap, uint32_t k, float r_ma
         A.fix_scale = scale;
         A.out_grad_clr = (float4*)d_grad_clr4;
         rc = mnrt::launch_knn_bwd(A, st);
-    } else if (rc == MNRT_OK && d_grad_clr4) {
-        // all weights zero: dLoss/drho still needs the recomputed irradiance
-        mnrt::KnnArgs A{};
-        A.order = order;
-        A.nodes = (const uint2*)(pmap->d_qnodes ? pmap->d_qnodes : pmap->d_nodes);
-        A.recs = (const float4*)pmap->d_recs;
-        A.boxes = mnrt::box_tree(*pmap);
-        A.k = k;
-        A.r2max = r_max * r_max;
-        A.r_max = r_max;
-        A.n = n;
-        A.pos = (const float4*)d_pos4;
-        A.nrm = (const float4*)d_nrm4;
-        A.dir = (const float4*)d_dir4;
-        A.infl = (const float4*)d_infl4;
-        A.clr = (const float4*)d_clr4;
-        A.r_query = d_query_radius;
-        A.grad = (const float4*)d_grad_rad4;
-        A.acc = acc;
-        A.fix_scale = 0.0;
-        A.out_grad_clr = (float4*)d_grad_clr4;
-        rc = mnrt::launch_knn_bwd(A, st);
     }
     if (rc == MNRT_OK) {
         hipLaunchKernelGGL(mnrt::k_fix_to_float, dim3((np + 255) / 256), dim3(256), 0, st, np, acc,
-                           scale > 0.0 ? 1.0 / scale : 0.0, (float4*)d_grad_pow4);
+                           (const double*)scale, (float4*)d_grad_pow4);
         if (hipGetLastError() != hipSuccess) rc = MNRT_ERR_HIP;
     }
     if (obuf) (void)mnrt::pool_free(obuf, st);
