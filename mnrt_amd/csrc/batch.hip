@@ -133,7 +133,7 @@ int run_trace(mnrt_batch& b, const mnrt_batch_io& io, hipStream_t st) {
     A.tile_begin = b.d_tile_begin;
     A.num_scenes = b.ns;
     A.tile_rays = b.tun.trace_tile;
-    A.unit = trace_unit(b.total_slots);
+    A.unit = trace_unit(b.total_slots, A.tile_rays);
     A.num_parts = b.tun.parts;
     A.part_begin = b.d_tparts;
     A.part_end = b.d_tparts + kMaxParts;

@@ -55,7 +55,7 @@ struct TraceBatchArgs {
     const uint32_t* tile_begin;  // num_scenes + 1
     uint32_t num_scenes;
     uint32_t tile_rays;
-    uint32_t unit;  // rays a wave takes and traces at once: a part of a tile
+    uint32_t unit;  // rays a wave takes: a part of a tile
     uint32_t num_parts;
     const uint32_t* part_begin;  // first tile of each share
     const uint32_t* part_end;
@@ -135,8 +135,8 @@ struct ShadeBatchArgs {
     uint32_t* out_count;          // hits per scene
 };
 
-// Rays a wave takes at once when a batch has `rays`.
-uint32_t trace_unit(uint64_t rays);
+// Rays a wave takes at once when a batch has `rays`, in tiles of `tile`.
+uint32_t trace_unit(uint64_t rays, uint32_t tile);
 int launch_trace_batch(const TraceBatchArgs& B, int stack, uint32_t grid, uint32_t block, hipStream_t st);
 int launch_knn_batch(const KnnArgs& G, const KnnScene* scenes, const uint32_t* slot_begin, uint32_t ns,
                      const uint32_t* count, uint32_t chunk, uint32_t num_parts, const uint32_t* part_begin,

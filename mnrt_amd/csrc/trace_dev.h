@@ -85,8 +85,9 @@ struct RayWindow {
     uint32_t* counter;   // rays in windows taken so far
     bool open;           // there may be more windows
 
-    __device__ __forceinline__ RayWindow(uint32_t first, uint32_t n_, uint32_t width_, uint32_t* counter_)
-        : next(min(first, n_)), end(next + min(width_, n_ - next)), n(n_), width(width_), counter(counter_), open(counter_ != nullptr) {}
+    // span: the first window's rays, if more than width.
+    __device__ __forceinline__ RayWindow(uint32_t first, uint32_t n_, uint32_t width_, uint32_t* counter_, uint32_t span = 0u)
+        : next(min(first, n_)), end(next + min(max(width_, span), n_ - next)), n(n_), width(width_), counter(counter_), open(counter_ != nullptr) {}
     // The next window, if there is one (uniform, whole wave).
     __device__ __forceinline__ void take(uint32_t lane) {
         uint32_t c = 0;
