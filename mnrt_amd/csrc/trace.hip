@@ -23,9 +23,14 @@ RayCounter::RayCounter(uint64_t n, uint32_t width, hipStream_t st) : st_(st) {
     if (waves <= kWindowWaves) return;
     // (a captured launch keeps a wave per window: no allocation is recorded)
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
+    hipError_t rc = hipStreamIsCapturing(st, &cs);
+    if (cs != hipStreamCaptureStatusNone || n > 0xFFFFFFFFull - (uint64_t)width * kTraceWaves) return;
     void* buf = nullptr;
-    if (n > 0xFFFFFFFFull - (uint64_t)width * kTraceWaves || pool_alloc(&buf, 4, st) != hipSuccess) return;
+    if (rc == hipSuccess) rc = pool_alloc(&buf, 4, st);
+    if (rc != hipSuccess) {  // a wave per window does without; the launch's own check is for the launch
+        (void)hipGetLastError();
+        return;
+    }
     p = (uint32_t*)buf;
     waves = kTraceWaves;
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, p, 1u, width * kTraceWaves);

@@ -65,3 +65,27 @@ def test_odd_rays_leave_the_others_alone(orc, cuda, trees):
     gtri, gt, _, _ = [x.cpu().numpy() if x is not None else None for x in api.trace_closest(DT, o, d, 1e-4)]
     assert np.array_equal(gtri[~odd], tri[~odd])
     assert np.array_equal(gt[~odd].view(np.uint32), t[~odd].view(np.uint32))
+
+
+def test_captured_launch_has_a_wave_per_window(cuda, trees):
+    # more rays than a counter's launch starts at: a captured call records no allocation
+    torch = cuda
+    DT, n = trees[2], 700001
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    rays = [(torch.rand((n, 4), device="cuda", generator=g) * 2 - 1, torch.randn((n, 4), device="cuda", generator=g))
+            for _ in range(3)]
+    o, d = rays[0][0].clone(), rays[0][1].clone()
+    api.trace_closest(DT, o, d, 1e-4)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tri, t, uv, _ = api.trace_closest(DT, o, d, 1e-4)
+    for a, b in rays:
+        print("replay", flush=True)
+        o.copy_(a)
+        d.copy_(b)
+        graph.replay()
+        torch.cuda.synchronize()
+        etri, et, euv, _ = api.trace_closest(DT, a, b, 1e-4)
+        assert torch.equal(tri, etri) and torch.equal(t, et) and torch.equal(uv, euv)
