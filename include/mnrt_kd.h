@@ -451,8 +451,7 @@ int mnrt_scan_u32(const uint32_t* d_in, uint32_t n, int inclusive, uint32_t* d_o
  * capacity), read by the kernels, so the call can be recorded into a graph and replayed
  * after the count changes; d_out[0..n) = the scan of d_in[0..n) (d_out may equal d_in),
  * *d_total (device word, may be null) = the sum, and d_out[n] = the sum too when end_total
- * is nonzero (d_out then holds capacity + 1 words).  The recorded builds scan their
- * per-level counts with it. */
+ * is nonzero (d_out then holds capacity + 1 words). */
 int mnrt_scan_u32_counted(const uint32_t* d_in, const uint32_t* d_count, uint32_t capacity,
                           uint32_t* d_out, uint32_t* d_total, int end_total, void* stream);
 
@@ -498,7 +497,7 @@ int mnrt_bounce_rays(uint32_t n, const float* d_pos4, const float* d_nrm4, const
  * global device state (RTCore.cpp:404-439, PhotonMap.cpp:195-232).  Scene s owns ray and
  * query slots ray_offsets[s] .. ray_offsets[s+1]-1 of every per-ray / per-query array
  * and triangles tri_offsets[s] .. of the concatenated vertex and albedo arrays.  Each
- * phase is one persistent launch (workgroups take tiles from device work counters) and
+ * phase is one persistent launch (waves take units of slots from device work counters) and
  * enqueues kernels only, with no allocation and no host synchronisation, so a phase can
  * be captured in a hipGraph (mnrt_batch_capture) and replayed.  Per scene, results are
  * identical to mnrt_trace_closest / mnrt_shading_points / mnrt_knn_gather on that scene. */
@@ -518,7 +517,7 @@ typedef struct mnrt_batch_desc {
 /* Launch shape of the phases; mnrt_batch_autotune picks it by timing candidates. */
 typedef struct mnrt_batch_tuning {
     uint32_t trace_block; /* lanes per workgroup: 64, 128, 256 */
-    uint32_t trace_tile;  /* rays per work item, a multiple of trace_block */
+    uint32_t trace_tile;  /* rays per tile, a multiple of trace_block; waves take units of it */
     uint32_t trace_grid;  /* persistent workgroups */
     uint32_t trace_stack; /* traversal stack entries: 16, 24, 32, 50; >= every tree's max_level */
     uint32_t knn_waves;   /* waves (one query each) per workgroup: 1, 2, 4 */

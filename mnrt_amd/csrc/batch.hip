@@ -4,7 +4,7 @@
 // state and launches KernelRTTraceRays / KernelPMPhotonGather per scene
 // (RTCore.cpp:404-439, PhotonMap.cpp:195-232).  Here the per-scene trees and parameters
 // live in device descriptor tables; each phase is one persistent launch whose
-// workgroups take tiles from device work counters (one counter per XCD share), so one
+// waves take units of slots from device work counters (one counter per XCD share), so one
 // launch covers every scene however uneven their sizes, and the phases enqueue
 // kernels only and can be captured in hipGraphs.
 //

@@ -289,9 +289,10 @@ __device__ __forceinline__ uint32_t mask_prefix_from(uint64_t m, uint32_t base) 
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
 }
 
-// Query-time leaves of photon trees: subtrees with at most this many references (the kNN
-// kernel tests a leaf 64 photons per step; measured on 1M photons, k = 100, with the
-// warm-start chains of eight queries: 256 -> 512 saves 5-9 %, 1024 is slower again).
+// Query-time leaves of photon trees: subtrees with at most this many references.  Only maps
+// without a box hierarchy are walked over them (a leaf is tested 64 photons per step; measured
+// there on 1M photons, k = 100, with the warm-start chains of eight queries: 256 -> 512 saves
+// 5-9 %, 1024 is slower again).
 constexpr uint32_t kQueryLeafRefs = 512;
 
 // Device memory of the library: a stream-ordered pool per device that keeps freed blocks
