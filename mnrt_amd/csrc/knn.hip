@@ -1002,8 +1002,8 @@ constexpr int kPairCap = 256;
 constexpr uint32_t kBwdChunk = 8;  // queries per chunk, at most
 
 // Sorts a wave's (photon << 8 | slot) pairs by photon in LDS and adds each photon's summed
-// fixed-point weights with one atomic per channel.
-__device__ __forceinline__ void merge_pairs(uint64_t* pairs, uint32_t np, const long long* w,
+// fixed-point weights with one atomic per channel.  heads: room for kPairCap words.
+__device__ __forceinline__ void merge_pairs(uint64_t* pairs, uint32_t np, const long long* w, uint32_t* heads,
                                             unsigned long long* acc, uint32_t lane) {
     if (np == 0) return;
     // sort the pairs by (photon, slot); pad to a power of two with keys above every pair
@@ -1024,20 +1024,28 @@ __device__ __forceinline__ void merge_pairs(uint64_t* pairs, uint32_t np, const 
             wave_sync();
         }
     }
-    // one lane per run of equal photons: sum its queries' weights, one atomic per channel
-    for (uint32_t i = lane; i < np; i += 64) {
+    // the first pair of every photon's run
+    uint32_t runs = 0;
+    for (uint32_t t = 0; t < np; t += 64) {
+        const uint32_t i = t + lane;
+        const bool head = i < np && (i == 0u || (pairs[i - 1] >> 8) != (pairs[i] >> 8));
+        const uint64_t m = ballot(head);
+        if (head) heads[mask_prefix_from(m, runs)] = i;
+        runs += (uint32_t)__popcll(m);
+    }
+    wave_sync();
+    // A lane per (run, channel): sum the run's weights, one atomic.  The three channels of a photon lie
+    // together, so an instruction's 64 atomics touch a third of the lines that a lane per run makes:
+    // forward and backward of 77361 queries (k = 50, 131072 photons) 565 -> 468 us, the inverse step of
+    // 8 scenes 1564 -> 1425 us.
+    for (uint32_t t = lane; t < 3u * runs; t += 64) {
+        const uint32_t r = t / 3u, ch = t - 3u * r;
+        uint32_t i = heads[r];
         const uint64_t p = pairs[i] >> 8;
-        if (i > 0 && (pairs[i - 1] >> 8) == p) continue;
-        long long sx = 0, sy = 0, sz = 0;
-        for (uint32_t j = i; j < np && (pairs[j] >> 8) == p; ++j) {
-            const uint32_t sl = (uint32_t)(pairs[j] & 0xFFu);
-            sx += w[3 * sl + 0];
-            sy += w[3 * sl + 1];
-            sz += w[3 * sl + 2];
-        }
-        if (sx) atomicAdd(&acc[3 * p + 0], (unsigned long long)sx);
-        if (sy) atomicAdd(&acc[3 * p + 1], (unsigned long long)sy);
-        if (sz) atomicAdd(&acc[3 * p + 2], (unsigned long long)sz);
+        const uint32_t e = r + 1u < runs ? heads[r + 1u] : np;
+        long long sum = 0;
+        for (; i < e; ++i) sum += w[3u * ((uint32_t)pairs[i] & 0xFFu) + ch];
+        if (sum) atomicAdd(&acc[3 * p + ch], (unsigned long long)sum);
     }
 }
 
@@ -1048,6 +1056,7 @@ __global__ __launch_bounds__(256) void k_knn_bwd_chunks(KnnArgs A, uint32_t chun
     __shared__ float4 s_soff[kBoxes ? 1 : kWavesPerBlock][kBoxes ? 1 : kKnnStack];
     __shared__ uint64_t s_pairs[kWavesPerBlock][kPairCap];
     __shared__ long long s_w[kWavesPerBlock][3 * kBwdChunk];
+    static_assert(2 * CAP >= kPairCap, "merge_pairs keeps its runs in the candidate buffer");
     const uint32_t wave = uniform(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t j0 = ((uint64_t)blockIdx.x * kWavesPerBlock + wave) * A.chain;
@@ -1072,7 +1081,7 @@ __global__ __launch_bounds__(256) void k_knn_bwd_chunks(KnnArgs A, uint32_t chun
         const KnnArgs L = late_args();
         knn_finish<kModeBackward>(L, Q, F, lane >= c0 && lane < c1, L.r_max, lane - c0, fix_scale, s_w[wave]);
         wave_sync();
-        merge_pairs(s_pairs[wave], sink.n, s_w[wave], L.acc, lane);
+        merge_pairs(s_pairs[wave], sink.n, s_w[wave], (uint32_t*)s_cand[wave], L.acc, lane);
         wave_sync();
     }
 }
@@ -1246,6 +1255,7 @@ __global__ __launch_bounds__(256) void k_knn_bwd_batch(KnnArgs G, const KnnScene
     __shared__ float4 s_soff[kBoxes ? 1 : kWavesPerBlock][kBoxes ? 1 : kKnnStack];
     __shared__ uint64_t s_pairs[kWavesPerBlock][kPairCap];
     __shared__ long long s_w[kWavesPerBlock][3 * kBwdChunk];
+    static_assert(2 * CAP >= kPairCap, "merge_pairs keeps its runs in the candidate buffer");
     const uint32_t wave = uniform(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t xcd = blockIdx.x % num_parts;
@@ -1297,7 +1307,7 @@ __global__ __launch_bounds__(256) void k_knn_bwd_batch(KnnArgs G, const KnnScene
             const KnnArgs L = late_args();
             knn_finish<kModeBackward>(L, Q, F, (done >> lane) & 1ull, 0.0f, lane, fs_lane, s_w[wave]);
             wave_sync();
-            merge_pairs(s_pairs[wave], sink.n, s_w[wave], L.acc, lane);
+            merge_pairs(s_pairs[wave], sink.n, s_w[wave], (uint32_t*)s_cand[wave], L.acc, lane);
             wave_sync();
         }
     }
