@@ -353,8 +353,9 @@ int mnrt_knn_gather_noalloc(const mnrt_tree* pmap, uint32_t k, float r_max, uint
  *   d_grad_pow4[p] = dLoss/dpower of photon p (original photon index, num_elems entries),
  *   d_grad_clr4[q] = dLoss/d(diffuse colour rgb) of query q (optional).
  * Per-photon sums use 64-bit fixed-point atomic adds (scale a power of two fixed from the
- * largest weight), so results do not depend on scheduling.  d_idx_sp slots are not
- * supported here (radiance per query). */
+ * largest weight), so results do not depend on scheduling.  When a query's weight is not
+ * finite (a NaN or infinite dLoss/dradiance, say), every photon's gradient is NaN.  d_idx_sp
+ * slots are not supported here (radiance per query). */
 int mnrt_knn_gather_bwd(const mnrt_tree* pmap, uint32_t k, float r_max, uint32_t n,
                         const float* d_pos4, const float* d_nrm4, const float* d_dir4,
                         const float* d_infl4, const float* d_clr4, const float* d_query_radius,

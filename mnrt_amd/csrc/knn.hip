@@ -875,9 +875,10 @@ __device__ __forceinline__ void knn_finish(const KnnArgs& A, const QueryLanes& Q
                                             g.z * (((c4.w * kInvPi) * iz) * in4.z), 0.0f);
         // fixed-point adds are associative, so the per-photon sums do not depend on the
         // order in which queries arrive
-        w[3 * lane + 0] = __double2ll_rn((double)wx * fix_scale);
-        w[3 * lane + 1] = __double2ll_rn((double)wy * fix_scale);
-        w[3 * lane + 2] = __double2ll_rn((double)wz * fix_scale);
+        const bool sum = fix_scale > 0.0;
+        w[3 * lane + 0] = sum ? __double2ll_rn((double)wx * fix_scale) : 0ll;
+        w[3 * lane + 1] = sum ? __double2ll_rn((double)wy * fix_scale) : 0ll;
+        w[3 * lane + 2] = sum ? __double2ll_rn((double)wz * fix_scale) : 0ll;
         return;
     }
     const float rx = (((c4.w * c4.x) * kInvPi) * ix) * in4.x;
@@ -1131,11 +1132,10 @@ __global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax(uint32_t n, const float
         bool gated = (clr && count[q] < 8) || !(rr > 0.0f);
         if (!gated) {
             float den = rr * kPi;
-            float wx = (g.x * (((c4.w * c4.x) * kInvPi) * in4.x)) / den;
-            float wy = (g.y * (((c4.w * c4.y) * kInvPi) * in4.y)) / den;
-            float wz = (g.z * (((c4.w * c4.z) * kInvPi) * in4.z)) / den;
-            m = fmaxf(fabsf(wx), fmaxf(fabsf(wy), fabsf(wz)));
-            if (!(m <= kInf)) m = kInf;  // NaN / inf gradients saturate the bound
+            const float w[3] = {(g.x * (((c4.w * c4.x) * kInvPi) * in4.x)) / den,
+                                (g.y * (((c4.w * c4.y) * kInvPi) * in4.y)) / den,
+                                (g.z * (((c4.w * c4.z) * kInvPi) * in4.z)) / den};
+            m = abs_max3(w);  // (+infinity when a weight is not finite)
         }
     }
     __shared__ uint32_t s_max[kWmaxBlock / 64];
@@ -1149,14 +1149,21 @@ __global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax(uint32_t n, const float
     }
 }
 
+// A photon's gradient from its fixed-point sums (scale: bwd_scale).
+__device__ __forceinline__ float4 photon_grad(const unsigned long long* __restrict__ acc, double scale) {
+    const double inv = scale > 0.0 ? 1.0 / scale : 0.0;
+    if (scale < 0.0) {
+        const float nan = __uint_as_float(0x7FC00000u);
+        return make_float4(nan, nan, nan, 0.0f);
+    }
+    return make_float4((float)((double)(long long)acc[0] * inv), (float)((double)(long long)acc[1] * inv),
+                       (float)((double)(long long)acc[2] * inv), 0.0f);
+}
+
 __global__ __launch_bounds__(256) void k_fix_to_float(uint32_t np, const unsigned long long* __restrict__ acc,
                                                       const double* __restrict__ scale, float4* __restrict__ out) {
     uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    const double inv_scale = *scale > 0.0 ? 1.0 / *scale : 0.0;
-    out[p] = make_float4((float)((double)(long long)acc[3ull * p] * inv_scale),
-                         (float)((double)(long long)acc[3ull * p + 1] * inv_scale),
-                         (float)((double)(long long)acc[3ull * p + 2] * inv_scale), 0.0f);
+    if (p < np) out[p] = photon_grad(acc + 3ull * p, *scale);
 }
 
 // --- batched backward (one launch sequence for every scene of a batch) ---------------
@@ -1184,11 +1191,10 @@ __global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax_batch(uint32_t n, const
             bool gated = (clr && nbr_count[g] < 8) || !(rr > 0.0f);
             if (!gated) {
                 float den = rr * kPi;
-                float wx = (gr.x * (((c4.w * c4.x) * kInvPi) * in4.x)) / den;
-                float wy = (gr.y * (((c4.w * c4.y) * kInvPi) * in4.y)) / den;
-                float wz = (gr.z * (((c4.w * c4.z) * kInvPi) * in4.z)) / den;
-                m = fmaxf(fabsf(wx), fmaxf(fabsf(wy), fabsf(wz)));
-                if (!(m <= kInf)) m = kInf;
+                const float w[3] = {(gr.x * (((c4.w * c4.x) * kInvPi) * in4.x)) / den,
+                                    (gr.y * (((c4.w * c4.y) * kInvPi) * in4.y)) / den,
+                                    (gr.z * (((c4.w * c4.z) * kInvPi) * in4.z)) / den};
+                m = abs_max3(w);
             }
         }
     }
@@ -1213,10 +1219,13 @@ __global__ __launch_bounds__(kWmaxBlock) void k_bwd_wmax_batch(uint32_t n, const
 }
 
 // Fixed-point unit per scene from its bound and query count: the largest power of two
-// with count * wmax * unit < 2^62 (the same expression as the single-scene entry point).
+// with count * wmax * unit < 2^62 (the same expression as the single-scene entry point); 0 when no
+// query has weight, negative when a weight is not finite: no sum is taken then and the photon
+// gradients become NaN.
 __device__ __forceinline__ double bwd_scale(uint32_t n, uint32_t wmax_bits) {
     const float wm = __uint_as_float(wmax_bits);
-    if (!(n > 0 && wm > 0.0f && wm <= kInf)) return 0.0;
+    if (!(wm <= kInf)) return -1.0;
+    if (!(n > 0 && wm > 0.0f)) return 0.0;
     int e = 0;
     (void)frexp(4.611686018427387904e18 / ((double)n * (double)wm), &e);
     return ldexp(1.0, e - 1);
@@ -1320,12 +1329,7 @@ __global__ __launch_bounds__(256) void k_fix_to_float_batch(uint32_t np, const u
                                                             const double* __restrict__ scale,
                                                             float4* __restrict__ out) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    const double sc = scale[seg_of(photon_begin, ns, p)];
-    const double inv = sc > 0.0 ? 1.0 / sc : 0.0;
-    out[p] = make_float4((float)((double)(long long)acc[3ull * p] * inv),
-                         (float)((double)(long long)acc[3ull * p + 1] * inv),
-                         (float)((double)(long long)acc[3ull * p + 2] * inv), 0.0f);
+    if (p < np) out[p] = photon_grad(acc + 3ull * p, scale[seg_of(photon_begin, ns, p)]);
 }
 
 __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long* __restrict__ p, uint64_t n) {

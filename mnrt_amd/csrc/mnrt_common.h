@@ -85,6 +85,18 @@ __device__ __forceinline__ bool ray_box(const float* bmin, const float* bmax, f3
     return hit;
 }
 
+// Largest |v| of three, +infinity if one of them is not finite (fmaxf alone would drop a NaN).
+__device__ __forceinline__ float abs_max3(const float* v) {
+    float m = 0.0f;
+    bool finite = true;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        finite = finite && fabsf(v[c]) <= kInf;
+        m = fmaxf(m, fabsf(v[c]));
+    }
+    return finite ? m : __uint_as_float(0x7F800000u);
+}
+
 __device__ __forceinline__ float sgn1(float x) { return x >= 0.0f ? 1.0f : -1.0f; }
 
 // Octahedral direction code: two 16-bit signed coordinates.  Decoding does not

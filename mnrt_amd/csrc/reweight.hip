@@ -156,18 +156,6 @@ __device__ __forceinline__ PhotonTerms photon_terms(const RwArgs& A, uint32_t p,
     return T;
 }
 
-// Largest |v| of three, +infinity if one of them is not finite (fmaxf alone would drop a NaN).
-__device__ __forceinline__ float abs_max3(const float* v) {
-    float m = 0.0f;
-    bool finite = true;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        finite = finite && fabsf(v[c]) <= kInf;
-        m = fmaxf(m, fabsf(v[c]));
-    }
-    return finite ? m : __uint_as_float(0x7F800000u);
-}
-
 // Bits of a bound m >= 0 (+infinity marks a non-finite term; bit order = value order).
 __device__ __forceinline__ uint32_t bound_bits(float m) {
     return (m <= kInf) ? __float_as_uint(m) : 0x7F800000u;
