@@ -490,6 +490,7 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, c
     // distances leave only the exact selection
     auto window_keep = [&]() {
         constexpr int R = CAP / 64;
+        wave_sync();  // the lanes' candidates of the batches before
         uint32_t h[R], pos[R];
         uint64_t keep[R];
         load_cands(h, pos);
@@ -589,7 +590,6 @@ __device__ __forceinline__ void knn_query(const KnnArgs& A, const KnnTree& Tr, c
                         const uint32_t g = take_box(nearest, m0, e0);
                         bool tight = test_batch(rr, g * 2048u, g == last, left & 63u, 4096u * i1 + 64u * g);
                         if (decltype(nearest)::value && !full && cnt >= k) {
-                            wave_sync();
                             window_keep();
                             tight = true;
                         }
