@@ -393,7 +393,11 @@ int batch_tables(const mnrt_tree* t, uint32_t ns, const uint32_t* h_offsets, uin
         cover[s] = std::max(t[s].num_elems, t[s].num_refs);
         B.boxes = B.boxes && t[s].num_refs <= t[s].num_elems;
     }
-    mnrt::photon_tables(cover.data(), ns, eb + ns + 1, eb + 2 * (ns + 1));
+    uint32_t* const box_begin = eb + 2 * (ns + 1);
+    mnrt::photon_tables(cover.data(), ns, eb + ns + 1, box_begin);
+    // without hierarchies the query-time node words start at the array's first word, which
+    // mnrt_tree_release hands back
+    if (!B.boxes) std::fill(box_begin, box_begin + ns + 1, 0u);
     return MNRT_OK;
 }
 
