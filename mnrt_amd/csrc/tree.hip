@@ -298,10 +298,13 @@ static int ensure_recs(mnrt_tree* t, size_t floats_per_ref, hipStream_t st) {
 
 // Room for the box hierarchy and the query-time node words behind it (boxes.h).  Node words
 // that the caller supplied stay as they are, and so do trees with more references than
-// elements (no tree of the builders is one): queries then walk the node words.
-static int ensure_boxes(mnrt_tree* t, hipStream_t st) {
-    if ((t->owns_qnodes & MNRT_QNODES_BOXES) || (t->d_qnodes && !(t->owns_qnodes & MNRT_QNODES_OWNED)) ||
-        t->num_refs > t->num_elems)
+// elements (no tree of the builders is one): queries then walk the node words.  Words that
+// mnrt_tree_collapse made are replaced only where no query can have read them (had_recs false: the
+// tree had no records): batches, captured graphs and trees that view the same array keep their
+// address.
+static int ensure_boxes(mnrt_tree* t, bool had_recs, hipStream_t st) {
+    if ((t->owns_qnodes & MNRT_QNODES_BOXES) ||
+        (t->d_qnodes && (had_recs || !(t->owns_qnodes & MNRT_QNODES_OWNED))) || t->num_refs > t->num_elems)
         return MNRT_OK;
     const uint64_t bw = mnrt::box_words(t->num_elems);
     if (bw > 0xFFFFFFFFull) return MNRT_OK;
@@ -338,10 +341,11 @@ extern "C" int mnrt_tree_attach_photon_records(mnrt_tree* tree, const float* d_p
         return MNRT_ERR_ARG;
     if (tree->kind != MNRT_KIND_POINT) return MNRT_ERR_STATE;
     hipStream_t st = (hipStream_t)stream;
+    const bool had_recs = tree->d_recs != nullptr;
     int rc = ensure_recs(tree, 8, st);
     if (rc != MNRT_OK) return rc;
     if (tree->num_refs == 0) return MNRT_OK;
-    rc = ensure_boxes(tree, st);
+    rc = ensure_boxes(tree, had_recs, st);
     if (rc != MNRT_OK) return rc;
     mnrt::PhotonRecArgs A{tree->d_refs, (const float4*)d_pos4, (const float4*)d_pow4, (const float4*)d_dir4,
                           (float4*)tree->d_recs, tree->num_refs, tree->num_elems, {}, 0u, nullptr, nullptr};

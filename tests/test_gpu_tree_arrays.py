@@ -61,3 +61,49 @@ def test_caller_batch_releases(cuda, refs):
     cuda.cuda.synchronize()
     _release(B.arr[0])
     assert not B.arr[0].d_recs and not B.arr[0].d_qnodes and B.arr[0].d_nodes
+
+
+def _collapse(T, most):
+    N.check(N.load().mnrt_tree_collapse(T.ref(), most, N.stream_handle()), "mnrt_tree_collapse")
+
+
+def _radii(T, k, q):
+    return api.knn_radii(T, k, 9.0, q).cpu().numpy()
+
+
+def test_words_that_queries_read_are_kept(cuda):
+    """Records in the caller's array, node words from mnrt_tree_collapse: queries can have read both
+    when the records are attached again, so both stay where they are."""
+    pos, power, pdir = (api.dev(a) for a in _photons(3000))
+    want = api.build_points(pos)
+    api.attach_photon_records(want, pos, power, pdir)
+    T = api.build_points(pos)
+    recs = cuda.empty(3000 * 8, dtype=cuda.float32, device="cuda")
+    T.t.d_recs = recs.data_ptr()
+    _collapse(T, 64)
+    before = T.t.d_qnodes
+    api.attach_photon_records(T, pos, power, pdir)
+    assert T.t.d_qnodes == before and T.t.owns_qnodes == N.QNODES_OWNED
+    assert np.array_equal(_radii(T, 20, pos[:500].contiguous()), _radii(want, 20, pos[:500].contiguous()))
+    # without records before, no query can have: the words give way to a hierarchy with words
+    U = api.build_points(pos)
+    _collapse(U, 64)
+    api.attach_photon_records(U, pos, power, pdir)
+    assert U.t.owns_qnodes == N.QNODES_OWNED | N.QNODES_BOXES
+    assert np.array_equal(_radii(U, 20, pos[:500].contiguous()), _radii(want, 20, pos[:500].contiguous()))
+    for tree in (T, U, want):
+        tree.release()
+
+
+def test_first_tree_of_a_batch_keeps_the_shared_array(cuda):
+    """Records attached again to the first tree of a batch without hierarchies, which owns the array
+    that the other trees' node words lie in."""
+    refs = [[0, 1, 2], [0, 1, 2, 2, 1]]
+    B, keep, n = _caller_batch(cuda, refs)
+    ph = [api.dev(a) for a in _photons(n)]
+    api.attach_photon_records_batch(B, *ph)
+    before = [B.arr[s].d_qnodes for s in range(2)]
+    api.attach_photon_records(B[0], *(a[:3].contiguous() for a in ph))
+    assert [B.arr[s].d_qnodes for s in range(2)] == before
+    cuda.cuda.synchronize()
+    _release(B.arr[0])
