@@ -217,7 +217,7 @@ int ensure_bwd(mnrt_batch& b) {
         const size_t o_scale = o_wmax + ((4 * (size_t)ns + 255) & ~(size_t)255);
         const size_t o_poff = o_scale + ((8 * (size_t)ns + 255) & ~(size_t)255);
         const size_t bytes = o_poff + 4 * ((size_t)ns + 1);
-        if (hipMalloc(&b.d_bwd, bytes) != hipSuccess) {
+        if (device_alloc(&b.d_bwd, bytes) != hipSuccess) {
             b.d_bwd = nullptr;
             b.bwd_cap = 0;
             return MNRT_ERR_NOMEM;
@@ -388,7 +388,7 @@ extern "C" int mnrt_batch_create(const mnrt_batch_desc* d, mnrt_batch** out) {
         size_t o_tile = carve(4 * (ns + 1)), o_slot = carve(4 * (ns + 1)), o_tri = carve(4 * ns);
         size_t o_parts = carve(4 * 4 * kMaxParts), o_work = carve(4 * 2 * kMaxParts * kWorkStride);
         size_t o_flags = carve(4 * n1), o_pos = carve(4 * n1), o_scan = carve(4 * scan_scratch_words((uint32_t)n1));
-        if (hipMalloc(&b->d_buf, bytes) != hipSuccess) rc = MNRT_ERR_NOMEM;
+        if (device_alloc(&b->d_buf, bytes) != hipSuccess) rc = MNRT_ERR_NOMEM;
         if (rc == MNRT_OK) {
             char* base = (char*)b->d_buf;
             b->d_trace = (TraceScene*)(base + o_trace);

@@ -1533,7 +1533,7 @@ class Pool {
             (void)hipStreamSynchronize(st_);
             void* nb = nullptr;
             const size_t ncap = peak_ + peak_ / 4 + (size_t(64) << 20);
-            if (hipMalloc(&nb, ncap) == hipSuccess) {
+            if (device_alloc(&nb, ncap) == hipSuccess) {
                 if (arena_->base) (void)hipFree(arena_->base);
                 arena_->base = (char*)nb;
                 arena_->cap = ncap;
@@ -2290,7 +2290,7 @@ extern "C" int mnrt_build_graph_create(const mnrt_build_graph_desc* d, mnrt_tree
     // 2. the fixed device block, and the per-scene tables in it
     int rc = graph_record(*g, nullptr, nullptr);
     if (rc != MNRT_OK) return fail(rc);
-    if (hipMalloc((void**)&g->dbuf, g->dbytes) != hipSuccess) {
+    if (device_alloc((void**)&g->dbuf, g->dbytes) != hipSuccess) {
         g->dbuf = nullptr;
         return fail(MNRT_ERR_NOMEM);
     }

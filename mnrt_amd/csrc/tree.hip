@@ -242,11 +242,18 @@ hipMemPool_t device_pool() {
 }
 }  // namespace
 
+// The caller reports a failed allocation: it is not left for a later call's launch check to find.
+static hipError_t reported(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 hipError_t pool_alloc(void** p, size_t bytes, hipStream_t st) {
     hipMemPool_t mp = device_pool();
-    if (!mp) return hipErrorOutOfMemory;
-    return hipMallocFromPoolAsync(p, std::max<size_t>(bytes, 16), mp, st);
+    return reported(mp ? hipMallocFromPoolAsync(p, std::max<size_t>(bytes, 16), mp, st) : hipErrorOutOfMemory);
 }
+
+hipError_t device_alloc(void** p, size_t bytes) { return reported(hipMalloc(p, bytes)); }
 
 hipError_t pool_free(void* p, hipStream_t st) { return p ? hipFreeAsync(p, st) : hipSuccess; }
 
@@ -259,7 +266,7 @@ void* host_staging(int slot, size_t bytes) {
     if (cap[slot] < bytes) {
         size_t want = std::max<size_t>(bytes, 4096);
         void* p = nullptr;
-        if (hipHostMalloc(&p, want, hipHostMallocDefault) != hipSuccess) return nullptr;
+        if (reported(hipHostMalloc(&p, want, hipHostMallocDefault)) != hipSuccess) return nullptr;
         if (buf[slot]) (void)hipHostFree(buf[slot]);
         buf[slot] = p;
         cap[slot] = want;
