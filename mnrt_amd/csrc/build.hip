@@ -25,6 +25,7 @@
 // lowest candidate index), so the tree is identical, word for word, to the one the host
 // oracle builds.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include <cstdio>
@@ -282,14 +283,17 @@ enum : uint32_t {
     W_ERR = 0,
     W_MAXLEVEL,    // deepest build node
     W_SMALL_OVF,   // small roots whose subtree outgrew its staging area
+    W_ERRLEVEL,    // with kErrRoom: the level that outgrew a buffer
     W_NBN = 4,     // build nodes, elements of large-stage leaves: one 64-bit word
     W_LL = 5,
     W_NSE = 6,     // small-root elements, small roots: one 64-bit word
     W_NSMALL = 7,
-    W_LEVELS = 8,  // per level: waves, nodes (one 64-bit word), clip jobs, 0 (another)
+    // per level: waves, nodes (one 64-bit word), clip jobs, 0 (another), W_NBN .. W_NSMALL before it
+    W_LEVELS = 8,
 };
+constexpr uint32_t kLevelWords = 8;
 constexpr uint32_t kLevels = MNRT_MAX_LEVEL + 2;  // every level's nodes are deeper than the last's
-constexpr uint32_t kWords = W_LEVELS + 4 * (kLevels + 1);
+constexpr uint32_t kWords = W_LEVELS + kLevelWords * (kLevels + 1);
 
 constexpr uint32_t kErrRoom = 64u;          // a buffer was outgrown
 constexpr uint32_t kErrLevels = 128u;       // active nodes left after the last recorded level
@@ -369,10 +373,10 @@ __device__ __forceinline__ uint32_t sum_part(unsigned long long v, uint32_t k) {
 }
 
 __device__ __forceinline__ uint32_t level_waves(const LevelArgs& L) {
-    return L.W[W_ERR] != 0u ? 0u : min(L.W[W_LEVELS + 4 * L.level], L.cap.nw);
+    return L.W[W_ERR] != 0u ? 0u : min(L.W[W_LEVELS + kLevelWords * L.level], L.cap.nw);
 }
 __device__ __forceinline__ uint32_t level_nodes(const LevelArgs& L) {
-    return L.W[W_ERR] != 0u ? 0u : min(L.W[W_LEVELS + 4 * L.level + 1], L.cap.na);
+    return L.W[W_ERR] != 0u ? 0u : min(L.W[W_LEVELS + kLevelWords * L.level + 1], L.cap.na);
 }
 
 // Empty-space cuts then the spatial median split (kernel_CanCutOffEmptySpace,
@@ -449,6 +453,21 @@ __global__ __launch_bounds__(256) void k_build_init(uint32_t* __restrict__ W, ui
     for (uint32_t j = i; j < 6 * nscenes; j += gridDim.x * blockDim.x) stb[j] = 0xFFFFFFFFu;
     for (uint32_t j = i; j < nscenes; j += gridDim.x * blockDim.x) maxlvl[j] = 0u;
     for (uint32_t j = i; j < chunks_for(nw, na); j += gridDim.x * blockDim.x) cs[j] = 0ull;
+}
+
+// Puts a build back to where it was before `level`, which outgrew a buffer: totals, the level's clip
+// jobs, the next level, and the level's chunk sums.
+__global__ __launch_bounds__(256) void k_level_again(uint32_t* __restrict__ W, uint32_t level, uint64_t nchunks,
+                                                     unsigned long long* __restrict__ cs) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t* const T = W + W_LEVELS + kLevelWords * level;
+    if (i < 4u) {
+        W[W_NBN + i] = T[4 + i];
+        T[kLevelWords + i] = 0u;
+    }
+    if (i < 2u) T[2 + i] = 0u;
+    if (i == 0u) W[W_ERR] = 0u;
+    for (uint64_t j = i; j < nchunks; j += (uint64_t)gridDim.x * blockDim.x) cs[j] = 0ull;
 }
 
 // Per-scene placement decided on the host: an active (large) root or a small root, its index in
@@ -605,6 +624,9 @@ __global__ __launch_bounds__(kCountBlock) __attribute__((amdgpu_waves_per_eu(8))
     __shared__ unsigned long long s_sum[2][kCountWaves];
     __shared__ uint32_t s_chunk[2][kCountWaves];
     const uint32_t nw = level_waves(L), lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
+    // the totals before the level, for a build that goes on from here in larger buffers
+    if (blockIdx.x == 0 && threadIdx.x < 4u && L.W[W_ERR] == 0u)
+        L.W[W_LEVELS + kLevelWords * L.level + 4 + threadIdx.x] = L.W[W_NBN + threadIdx.x];
     uint32_t set = 0;
     for (uint32_t w0 = blockIdx.x * kCountWaves; w0 < nw; w0 += gridDim.x * kCountWaves) {  // uniform per workgroup
         const uint32_t w = w0 + wave;
@@ -722,11 +744,12 @@ __global__ __launch_bounds__(kChildBlock) __attribute__((amdgpu_waves_per_eu(8))
             unsigned long long at = 0;
             if (i == 15u) {
                 const uint32_t word = k == 0u ? W_NBN : k == 1u ? W_NSE
-                                      : k == 2u ? W_LEVELS + 4u * (L.level + 1u) : W_LEVELS + 4u * L.level + 2u;
+                                      : k == 2u ? W_LEVELS + kLevelWords * (L.level + 1u) : W_LEVELS + kLevelWords * L.level + 2u;
                 if ((ia | ib) != 0u) at = atomicAdd((unsigned long long*)&L.W[word], (unsigned long long)ib << 32 | ia);
                 const uint32_t ca = k == 0u ? L.cap.bn : k == 1u ? L.cap.se : L.cap.nw;
                 const uint32_t cb = k == 0u ? L.cap.ll : k == 1u ? L.cap.small : L.cap.na;
                 if (k < 3u && ((at & 0xFFFFFFFFull) + ia > ca || (at >> 32) + ib > cb)) {
+                    L.W[W_ERRLEVEL] = L.level;
                     atomicOr(&L.W[W_ERR], kErrRoom);
                     at = ~0ull;
                 }
@@ -922,7 +945,7 @@ __global__ __launch_bounds__(kClipBlock) void k_clip(LevelArgs L, Geometry G) {
     __shared__ float s_lists[2 * kClipVerts * 3 * kClipBlock];
     __attribute__((address_space(3))) float* col = (__attribute__((address_space(3))) float*)(s_lists + threadIdx.x);
     if (L.W[W_ERR] != 0u) return;
-    const uint32_t nq = 2u * L.W[W_LEVELS + 4 * L.level + 2], lane = threadIdx.x;
+    const uint32_t nq = 2u * L.W[W_LEVELS + kLevelWords * L.level + 2], lane = threadIdx.x;
     for (uint32_t j0 = blockIdx.x * kClipBlock; j0 < nq; j0 += gridDim.x * kClipBlock) {
         const uint32_t j = j0 + lane;
         uint32_t to = kNone;
@@ -1508,7 +1531,9 @@ using namespace mnrt;
 
 // Build workspace: one device block per host thread and device, kept across builds and
 // grown to the largest build seen, so a build in steady state allocates nothing but its
-// output arrays (allocation calls that must grow device memory cost milliseconds each).
+// output arrays (allocation calls that must grow device memory cost milliseconds each; buffers that a
+// build replaces by larger ones, taken from the stream-ordered pool and given back at once, made
+// 205001 triangles with small roots of one take 250 ms, 25 from the block).
 // Buffers are carved bump-wise and not reused within a build; a build that outgrows the
 // block takes the rest from the stream-ordered pool, and the block grows to fit when that
 // build ends.  The blocks live until the process ends.
@@ -1531,13 +1556,13 @@ class Pool {
         for (void* p : ptrs_) (void)pool_free(p, st_);
         if (arena_ && peak_ > arena_->cap) {
             (void)hipStreamSynchronize(st_);
+            if (arena_->base) (void)hipFree(arena_->base);
+            *arena_ = Arena{};
             void* nb = nullptr;
-            const size_t ncap = peak_ + peak_ / 4 + (size_t(64) << 20);
-            if (device_alloc(&nb, ncap) == hipSuccess) {
-                if (arena_->base) (void)hipFree(arena_->base);
-                arena_->base = (char*)nb;
-                arena_->cap = ncap;
-            }
+            const size_t ncap = peak_ + std::min(peak_ / 4, size_t(1) << 30) + (size_t(64) << 20);
+            // (what this build had from the pool lies there unused: it goes back to the device if need be)
+            if (device_alloc(&nb, ncap) == hipSuccess || (pool_trim(), device_alloc(&nb, ncap) == hipSuccess))
+                *arena_ = Arena{(char*)nb, ncap};
         }
     }
     template <typename T>
@@ -1557,18 +1582,6 @@ class Pool {
         }
         ptrs_.push_back(p);
         return (T*)p;
-    }
-    // Takes back every buffer handed out since mark() (work enqueued on the stream before may
-    // still use them: buffers handed out next are used on the same stream).
-    struct Mark {
-        size_t top, total, ptrs;
-    };
-    Mark mark() const { return Mark{top_, total_, ptrs_.size()}; }
-    void rewind(const Mark& m) {
-        for (size_t i = m.ptrs; i < ptrs_.size(); ++i) (void)pool_free(ptrs_[i], st_);
-        ptrs_.resize(m.ptrs);
-        top_ = m.top;
-        total_ = m.total;
     }
     bool ok = true;
 
@@ -1813,7 +1826,8 @@ struct BuildStats {
 
 // Buffer sizes a host-driven build starts with.  Points never straddle, so a level holds at
 // most the input and small_max + 1 elements per node; triangles are duplicated, and the rest is
-// what ordinary trees stay below.  A build that outgrows one of them is run again (grow_caps).
+// what ordinary trees stay below.  A build that outgrows one of them moves to larger ones and goes on
+// from the level that did (grow_caps, grow_levels).
 BuildCaps first_caps(int kind, uint32_t S_, uint32_t ntot, uint32_t small_max, const RootCounts& c) {
     const uint64_t ne = (kind == MNRT_KIND_TRI ? 2ull : 1ull) * ntot, lim = MNRT_INDEX_MASK;
     const uint64_t per = ntot / small_max;
@@ -1827,27 +1841,74 @@ BuildCaps first_caps(int kind, uint32_t S_, uint32_t ntot, uint32_t small_max, c
     return C;
 }
 
-// The sizes that the words W of an outgrown build exceed, at least doubled.  An element of a
-// level or a small root ends in a leaf, a build node in the tree: beyond MNRT_INDEX_MASK of them
-// the tree itself has no room (false).
+// The sizes that level `level` of an outgrown build exceeds, at least doubled, and with them those
+// of the totals that are more than half full: deeper levels add to them, and each time a build goes on
+// costs a synchronisation and copies.  An element of a level or a small root ends in a leaf, a
+// build node in the tree: beyond MNRT_INDEX_MASK of them the tree itself has no room (false).
 bool grow_caps(BuildCaps& C, const uint32_t* W, uint32_t level) {
     bool room = true, grown = false;
-    auto grow = [&](uint32_t& cap, uint64_t need, uint64_t lim) {
-        if (need <= cap) return;
-        grown = true;
-        if (cap >= lim) room = false;
+    auto grow = [&](uint32_t& cap, uint64_t need, uint64_t lim, bool total) {
+        if (need <= cap && !(total && 2 * need > cap)) return;
+        if (need > cap) {
+            grown = true;
+            if (cap >= lim) room = false;
+        }
         cap = (uint32_t)std::min<uint64_t>(lim, std::max<uint64_t>(2ull * cap, need + need / 4));
     };
     const uint64_t lim = MNRT_INDEX_MASK;
-    for (uint32_t l = 0; l <= level; ++l) {
-        grow(C.nw, W[W_LEVELS + 4 * l], lim / 64);
-        grow(C.na, W[W_LEVELS + 4 * l + 1], lim);
-    }
-    grow(C.bn, W[W_NBN], lim);
-    grow(C.small, W[W_NSMALL], lim);
-    grow(C.se, W[W_NSE], lim);
-    grow(C.ll, W[W_LL], lim);
+    const uint32_t* next = W + W_LEVELS + kLevelWords * (level + 1);
+    grow(C.nw, next[0], lim / 64, false);
+    grow(C.na, next[1], lim, false);
+    grow(C.bn, W[W_NBN], lim, true);
+    grow(C.small, W[W_NSMALL], lim, true);
+    grow(C.se, W[W_NSE], lim, true);
+    grow(C.ll, W[W_LL], lim, true);
     return room && grown;
+}
+
+// Moves a build that outgrew the sizes C at level `level` (device words W) to buffers of the sizes D:
+// what the levels before it left, which the level reads or adds to; the rest is written before
+// it is read.  A build that started over each time it outgrew a size (up to 13 times): 3001 triangles, small
+// roots of at most 4: 8.6 ms, now 2.4; 205001, at most 4: 15.7, now 5.7, at most one: 57, now 25;
+// 1.03M, at most 16: 7.0, now 3.7; 500000 points in 4913 places 6.6, now 2.5.
+int grow_levels(Pool& pool, int kind, LevelBufs& b, const BuildCaps& C, const BuildCaps& D, const uint32_t* W,
+                uint32_t level, hipStream_t st) {
+    const uint32_t* T = W + W_LEVELS + kLevelWords * level;
+    const uint64_t nw = T[0], na = T[1], nbn = T[4], ll = T[5], nse = T[6], nsmall = T[7];
+    hipError_t err = hipSuccess;
+    auto move = [&](auto*& p, uint64_t from, uint64_t to, uint64_t used) {
+        using E = std::remove_reference_t<decltype(*p)>;
+        if (to == from || !pool.ok || err != hipSuccess) return;
+        E* n = pool.get<E>(to);
+        if (!pool.ok) return;
+        if (used != 0) err = hipMemcpyAsync(n, p, used * sizeof(E), hipMemcpyDeviceToDevice, st);
+        p = n;
+    };
+    auto move_elems = [&](ElemView& V, uint64_t from, uint64_t to, uint64_t used) {
+        move(V.lo, from, to, used);
+        if (kind == MNRT_KIND_TRI) move(V.hi, from, to, used);
+        else V.hi = V.lo;
+    };
+    const uint64_t chunks = chunks_for(C.nw, C.na), more_chunks = chunks_for(D.nw, D.na);
+    for (uint32_t i = 0; i < 2; ++i) {
+        const bool cur = i == (level & 1u);
+        move(b.N[i], C.na, D.na, cur ? na : 0u);
+        move_elems(b.X[i], 64ull * C.nw, 64ull * D.nw, cur ? 64u * nw : 0u);
+        move(b.X[i].wnode, C.nw, D.nw, cur ? nw : 0u);
+        move(b.cs[i], chunks, more_chunks, 0u);
+    }
+    move_elems(b.Sm, C.se, D.se, nse);
+    move(b.S, C.small, D.small, nsmall);
+    move(b.B, C.bn, D.bn, nbn);
+    move(b.wc, C.nw, D.nw, 0u);
+    move(b.coff, chunks, more_chunks, 0u);
+    move(b.P, C.na, D.na, 0u);
+    move(b.ll_idx, C.ll, D.ll, ll);
+    if (kind == MNRT_KIND_TRI) move(b.q, 64ull * C.nw, 64ull * D.nw, 0u);
+    if (!pool.ok) return MNRT_ERR_NOMEM;
+    const uint64_t n = chunks_for(nw, na);
+    hipLaunchKernelGGL(k_level_again, blocks_to(n, 256, 256), dim3(256), 0, st, b.W, level, n, b.cs[level & 1u]);
+    return err == hipSuccess && hipGetLastError() == hipSuccess ? MNRT_OK : MNRT_ERR_HIP;
 }
 
 // Builds the trees of S scenes together: one level loop over the active nodes of all
@@ -1910,35 +1971,37 @@ int build_batch_impl(int kind, const float* d_v0, const float* d_v1, const float
         first_levels = std::min<uint32_t>(lg + lg / 2 + 1, kLevels);
     }
     BuildCaps C = first_caps(kind, S_, ntot, prm->small_node_max, c);
-    LevelBufs b{};
+    LevelBufs b = take_levels(pool, kind, S_, C);
+    if (!pool.ok) return MNRT_ERR_NOMEM;
+    launch_roots(b, G, ntot, RP, c, h_roots ? (const float*)T.given : (const float*)nullptr, T.rootbox, T.smaxlvl, st);
     uint32_t levels = 0;
-    const Pool::Mark mark = pool.mark();
-    for (;;) {
-        b = take_levels(pool, kind, S_, C);
-        if (!pool.ok) return MNRT_ERR_NOMEM;
-        launch_roots(b, G, ntot, RP, c, h_roots ? (const float*)T.given : (const float*)nullptr, T.rootbox, T.smaxlvl, st);
-        levels = 0;
-        for (uint32_t until = first_levels;; until = std::min(levels + 4u, kLevels)) {
-            for (; levels < until; ++levels)
-                launch_level(b, G, *prm, C, levels, std::min<uint64_t>(C.na, (uint64_t)c.na << levels), C.nw, st);
-            MNRT_HIP_CHECK(hipGetLastError());
-            MNRT_HIP_CHECK(hipMemcpyAsync(h_W, b.W, kWords * 4, hipMemcpyDeviceToHost, st));
-            MNRT_HIP_CHECK(hipStreamSynchronize(st));
-            if (h_W[W_ERR] != 0u || h_W[W_LEVELS + 4 * levels + 1] == 0u) break;
+    for (uint32_t until = first_levels;;) {
+        for (; levels < until; ++levels)
+            launch_level(b, G, *prm, C, levels, std::min<uint64_t>(C.na, (uint64_t)c.na << levels), C.nw, st);
+        MNRT_HIP_CHECK(hipGetLastError());
+        MNRT_HIP_CHECK(hipMemcpyAsync(h_W, b.W, kWords * 4, hipMemcpyDeviceToHost, st));
+        MNRT_HIP_CHECK(hipStreamSynchronize(st));
+        if (h_W[W_ERR] == 0u) {
+            if (h_W[W_LEVELS + kLevelWords * levels + 1] == 0u) break;
             if (levels == kLevels) return MNRT_ERR_STATE;
+            until = std::min(levels + 4u, kLevels);
+            continue;
         }
-        if (h_W[W_ERR] == 0u) break;
-        if (h_W[W_ERR] != kErrRoom) return MNRT_ERR_STATE;
-        if (!grow_caps(C, h_W, levels)) return MNRT_ERR_CAPACITY;
-        pool.rewind(mark);
+        if (h_W[W_ERR] != kErrRoom || h_W[W_ERRLEVEL] >= levels) return MNRT_ERR_STATE;
+        levels = h_W[W_ERRLEVEL];
+        BuildCaps D = C;
+        if (!grow_caps(D, h_W, levels)) return MNRT_ERR_CAPACITY;
+        const int rc = grow_levels(pool, kind, b, C, D, h_W, levels, st);
+        if (rc != MNRT_OK) return rc;
+        C = D;
     }
     const uint32_t nbn = h_W[W_NBN], nsmall = h_W[W_NSMALL], nse = h_W[W_NSE];
     if (stats) {
         *stats = BuildStats{};
         stats->roots = c;
-        for (uint32_t l = 0; l < levels && h_W[W_LEVELS + 4 * l + 1] != 0u; ++l) {
-            stats->level_nw.push_back(h_W[W_LEVELS + 4 * l]);
-            stats->level_na.push_back(h_W[W_LEVELS + 4 * l + 1]);
+        for (uint32_t l = 0; l < levels && h_W[W_LEVELS + kLevelWords * l + 1] != 0u; ++l) {
+            stats->level_nw.push_back(h_W[W_LEVELS + kLevelWords * l]);
+            stats->level_na.push_back(h_W[W_LEVELS + kLevelWords * l + 1]);
             stats->max_nw = std::max(stats->max_nw, stats->level_nw.back());
             stats->max_na = std::max(stats->max_na, stats->level_na.back());
         }
@@ -2026,7 +2089,7 @@ constexpr uint32_t kLayoutSpareLevels = 6u;
 
 // Active nodes left after the last recorded level.
 __global__ __launch_bounds__(64) void k_levels_done(uint32_t* __restrict__ W, uint32_t level) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && W[W_ERR] == 0u && W[W_LEVELS + 4 * level + 1] != 0u) W[W_ERR] = kErrLevels;
+    if (threadIdx.x == 0 && blockIdx.x == 0 && W[W_ERR] == 0u && W[W_LEVELS + kLevelWords * level + 1] != 0u) W[W_ERR] = kErrLevels;
 }
 
 }  // namespace

@@ -313,6 +313,8 @@ constexpr uint32_t kQueryLeafRefs = 512;
 // null stream.
 hipError_t pool_alloc(void** p, size_t bytes, hipStream_t st);
 hipError_t pool_free(void* p, hipStream_t st);
+// Returns the pool's unused blocks to the device.
+void pool_trim();
 // hipMalloc for blocks that live long.  Neither leaves an error in the runtime when it fails.
 hipError_t device_alloc(void** p, size_t bytes);
 // Pinned host staging buffer of at least `bytes`, one per host thread and slot, kept for

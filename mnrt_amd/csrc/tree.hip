@@ -253,6 +253,10 @@ hipError_t pool_alloc(void** p, size_t bytes, hipStream_t st) {
     return reported(mp ? hipMallocFromPoolAsync(p, std::max<size_t>(bytes, 16), mp, st) : hipErrorOutOfMemory);
 }
 
+void pool_trim() {
+    if (hipMemPool_t mp = device_pool()) (void)hipMemPoolTrimTo(mp, 0);
+}
+
 hipError_t device_alloc(void** p, size_t bytes) { return reported(hipMalloc(p, bytes)); }
 
 hipError_t pool_free(void* p, hipStream_t st) { return p ? hipFreeAsync(p, st) : hipSuccess; }
