@@ -18,24 +18,27 @@
 
 namespace mnrt {
 
-RayCounter::RayCounter(uint64_t n, uint32_t width, hipStream_t st) : st_(st) {
-    waves = trace_windows(n, width);
-    if (waves <= kWindowWaves) return;
-    // (a captured launch keeps a wave per window: no allocation is recorded)
+__global__ __launch_bounds__(256) void k_clear_words(uint32_t* __restrict__ p, uint64_t n) {
+    for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += gridDim.x * 256ull) p[i] = 0u;
+}
+
+RayShared::RayShared(uint32_t windows, hipStream_t st) : st_(st) {
+    if (windows <= kWindowWaves) return;
+    // (a captured launch does without: no allocation is recorded)
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hipError_t rc = hipStreamIsCapturing(st, &cs);
-    if (cs != hipStreamCaptureStatusNone || n > 0xFFFFFFFFull - (uint64_t)width * kTraceWaves) return;
+    if (cs != hipStreamCaptureStatusNone) return;
+    const uint64_t words = RayWindow::shared_words(windows);
     void* buf = nullptr;
-    if (rc == hipSuccess) rc = pool_alloc(&buf, 4, st);
-    if (rc != hipSuccess) {  // a wave per window does without; the launch's own check is for the launch
+    if (rc == hipSuccess) rc = pool_alloc(&buf, 4u * words, st);
+    if (rc != hipSuccess) {  // the launch does without; its own check is for the launch
         (void)hipGetLastError();
         return;
     }
     p = (uint32_t*)buf;
-    waves = kTraceWaves;
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, p, 1u, width * kTraceWaves);
+    hipLaunchKernelGGL(k_clear_words, dim3((uint32_t)std::min<uint64_t>((words + 255u) / 256u, 1024u)), dim3(256), 0, st, p, words);
 }
-RayCounter::~RayCounter() {
+RayShared::~RayShared() {
     if (p) (void)pool_free(p, st_);
 }
 
@@ -81,12 +84,13 @@ struct RaySource {
 
 // One wave per workgroup: its LDS goes to the next when its own run is done.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_trace_closest(
-    const uint2* __restrict__ nodes, const float4* __restrict__ recs, RootBox root, uint32_t n, uint32_t width, uint32_t* __restrict__ counter,
+    const uint2* __restrict__ nodes, const float4* __restrict__ recs, RootBox root, uint32_t n, uint32_t width, uint32_t* shared,
     const float4* __restrict__ orig, const float4* __restrict__ dir, float eps,
     int32_t* __restrict__ out_tri, float* __restrict__ out_t, float2* __restrict__ out_bary,
     float4* __restrict__ out_pt, uint32_t* __restrict__ out_valid) {
     __shared__ __align__(8) uint32_t s_wave[kTraceWords];
-    RaySource src{RayWindow(blockIdx.x * width, n, width, counter), 0u, orig, dir, recs, out_tri, out_t, out_bary, out_pt, out_valid};
+    if (shared && !RayWindow::claim(shared, blockIdx.x, threadIdx.x)) return;
+    RaySource src{RayWindow(blockIdx.x * width, n, width, shared), 0u, orig, dir, recs, out_tri, out_t, out_bary, out_pt, out_valid};
     trace_stream<false, kTraceStack>(nodes, recs, root, eps, 0.0f, s_wave, src);
 }
 
@@ -106,11 +110,11 @@ extern "C" int mnrt_trace_closest(const mnrt_tree* tree, uint32_t n, const float
         rb.lo[a] = tree->root_min[a];
         rb.hi[a] = tree->root_max[a];
     }
-    const uint32_t width = mnrt::trace_width(n);
-    const mnrt::RayCounter counter(n, width, (hipStream_t)stream);
-    hipLaunchKernelGGL(mnrt::k_trace_closest, dim3(counter.waves), dim3(64), 0,
+    const uint32_t width = mnrt::trace_width(n), windows = mnrt::trace_windows(n, width);
+    const mnrt::RayShared shared(windows, (hipStream_t)stream);
+    hipLaunchKernelGGL(mnrt::k_trace_closest, dim3(windows), dim3(64), 0,
                        (hipStream_t)stream,
-                       (const uint2*)tree->d_nodes, (const float4*)tree->d_recs, rb, n, width, counter.p,
+                       (const uint2*)tree->d_nodes, (const float4*)tree->d_recs, rb, n, width, shared.p,
                        (const float4*)d_orig4, (const float4*)d_dir4, eps, d_out_tri, d_out_t,
                        (float2*)d_out_bary2, (float4*)d_out_pt4, d_out_valid);
     MNRT_HIP_CHECK(hipGetLastError());

@@ -72,41 +72,58 @@ constexpr uint32_t kEarly = 48, kRaysTogether = 24;
 // LDS words of a wave: pair owners and best records (64 each), best keys (64 x 2), stack.
 constexpr uint32_t kTraceWords = 256u + 3u * 64u * (uint32_t)kTraceLds;
 
-// Rays of a wave: a window of `width` consecutive ones at a time, the first by its number, the
-// next from a counter that the launch's waves share (null: none).  A launch of up to
-// kWindowWaves windows has a wave for each, which the hardware starts as others end: 524176 camera rays
-// (205001 triangles) 505 us, from a counter 550; from there on lanes that refill gain more: 1.69M bounce
-// rays 1483 us, a wave per window 2093.  (A fixed share of the rays for every wave that fits at
-// once: waves of slow rays end late, camera rays up to 40 % slower.)  Shadow rays always have a wave per window: 1.76M from a point
-// light (20000 triangles) 427 us, from a counter 592.
+// Rays of a wave: a window of `width` consecutive ones, a wave per window, which the hardware starts as
+// others end.  In launches of more than kWindowWaves windows a wave whose rays do not go together takes
+// further ones, from the launch's end, whose own waves then find them taken: lanes that refill gain more
+// than new waves do (1.69M bounce rays 1483 us with windows from a counter, a wave per window 2093).  Rays
+// that go together, or miss the root box, leave the rest to the hardware.  2.07M rays with a window from
+// a counter for every 64, whose atomics come 12 ns apart, and now: camera rays of 1294 triangles 420 and
+// 226 us, of which most miss the box 398 and 50, of 1.03M triangles 1002 and 977; bounce rays of 1.03M 1713 and
+// 1738 (two atomics a window, and waves that find theirs taken).  (From the end by a fixed stride
+// instead of a count: bounce rays 5 to 10 % slower, camera rays up to 9 % faster; 128 rays a window: bounce
+// rays 4 to 7 % slower; a fixed share of the rays for every wave that fits at once: waves of slow rays end
+// late, camera rays up to 40 % slower.)  Shadow rays always have a wave per window: 1.76M from a point
+// light (20000 triangles) 427 us, with windows from a counter 592.
 struct RayWindow {
     uint32_t next, end;  // rays of the window not handed out yet
     uint32_t n, width;
-    uint32_t* counter;   // rays in windows taken so far
+    uint32_t* shared;    // kShared*; null: the wave's own window is all
     bool open;           // there may be more windows
 
     // span: the first window's rays, if more than width.
-    __device__ __forceinline__ RayWindow(uint32_t first, uint32_t n_, uint32_t width_, uint32_t* counter_, uint32_t span = 0u)
-        : next(min(first, n_)), end(next + min(max(width_, span), n_ - next)), n(n_), width(width_), counter(counter_), open(counter_ != nullptr) {}
-    // The next window, if there is one (uniform, whole wave).
+    __device__ __forceinline__ RayWindow(uint32_t first, uint32_t n_, uint32_t width_, uint32_t* shared_, uint32_t span = 0u)
+        : next(min(first, n_)), end(next + min(max(width_, span), n_ - next)), n(n_), width(width_), shared(shared_), open(shared_ != nullptr) {}
+    // Words that the waves of a launch share: windows taken from the end, then, from kSharedTaken on, a
+    // word for every window but the first kTraceWaves, whose waves start at once: 1 when it is taken.
+    static constexpr uint32_t kSharedTaken = 32;
+    static constexpr uint64_t shared_words(uint32_t windows) { return kSharedTaken + (windows - kTraceWaves); }
+    // Takes window w for this wave; false if another has it (uniform, whole wave).
+    static __device__ __forceinline__ bool claim(uint32_t* shared, uint32_t w, uint32_t lane) {
+        if (w < kTraceWaves) return true;
+        uint32_t old = 0;
+        if (lane == 0u) old = atomicExch(shared + kSharedTaken + (w - kTraceWaves), 1u);
+        return uniform(old) == 0u;
+    }
+    // Another window, if there is one (uniform, whole wave).  A window that is taken already has been
+    // started by the hardware, and so have those before it.
     __device__ __forceinline__ void take(uint32_t lane) {
         uint32_t c = 0;
-        if (lane == 0u) c = atomicAdd(counter, width);
+        if (lane == 0u) c = atomicAdd(shared, 1u);
         c = uniform(c);
-        open = c < n;  // (the counter passes n by a window per wave at most)
-        next = min(c, n);
+        const uint32_t w = gridDim.x - 1u - c;
+        open = c < gridDim.x - kTraceWaves && claim(shared, w, lane);
+        next = open ? w * width : n;
         end = next + min(width, n - next);
     }
 };
 
-// Counter of a launch of n rays on a stream, or null where none is needed or to be had (then a wave
-// per window).  It lives until the launch is done.
-class RayCounter {
+// The shared words of a launch of `windows` on a stream, or null where none are needed or to be had (then
+// every wave has its own window).  They live until the launch is done.
+class RayShared {
    public:
-    RayCounter(uint64_t n, uint32_t width, hipStream_t st);
-    ~RayCounter();
+    RayShared(uint32_t windows, hipStream_t st);
+    ~RayShared();
     uint32_t* p = nullptr;
-    uint32_t waves = 0;
 
    private:
     hipStream_t st_;
@@ -293,7 +310,10 @@ __device__ __forceinline__ void trace_stream(const uint2* __restrict__ nodes, co
         const uint32_t done = (uint32_t)__popcll(ballot(state == kDone));
         // rays that walk together (steps, lanes: of the set so far) end together: the wave waits for them
         if (busy == 0u || ((src.rays.open || src.rays.next < src.rays.end ? width - busy : done) >= refill && !together)) {
-            if (busy == 0u) steps = lanes = 0u;
+            if (busy == 0u) {
+                if (src.rays.next == src.rays.end && lanes >= steps * Src::kTogether) src.rays.open = false;
+                steps = lanes = 0u;
+            }
             bool ray = false;
             if (state == kDone) {
                 ray = src.finish(o, d, dist, Hit{best_tri, best_t, best_rec});
