@@ -906,7 +906,14 @@ __device__ __forceinline__ void knn_finish(const KnnArgs& A, const QueryLanes& Q
 // for the chip (8192 at a time) when there are few queries, and then their steps add up to the
 // launch's time: k = 100, 1M photons, camera hits, chains of 1 / 8 / 16: 4096 queries 46 / 126 /
 // 239 us, 61,440: 235 / 189 / 287 us, 524,288: 1747 / 812 / 810 us, 2.07M: 6.60 / 2.87 / 2.73 ms.
-inline uint32_t knn_chain(uint32_t n) { return std::min(16u, std::max(1u, n / 24576u)); }
+// Neighbouring queries are slow together where the map is uneven, so the slowest chain, not the mean, ends the
+// launch: chains of 16 wait until it has a dozen rounds of waves (k = 50, 1M photons, chains of 8 / 16, 784,641
+// queries: bounce hits 1091 / 1199 us, points anywhere in the room 3164 / 4188; 2.07M: 2591 / 2506 and
+// 6701 / 7254), and node words, over which slow searches are slower still, keep to 8 (points anywhere in the
+// room: 784,641 queries 4914 / 7049 us, 2.07M 9129 / 11054; bounce hits 1281 / 1382 and 3070 / 3006).
+inline uint32_t knn_chain(uint32_t n, bool boxes) {
+    return std::min(boxes && n >= 12u * 8192u * 16u ? 16u : 8u, std::max(1u, n / 24576u));
+}
 
 template <int CAP, int kMode, bool kBoxes>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_knn(KnnArgs A) {
@@ -1337,11 +1344,11 @@ __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long* __restrict
         p[i] = 0ull;
 }
 
-// Backward launches: a wave's chain of queries (knn_chain) in chunks of floor(kPairCap / k).
+// Backward launches: a wave's chain of queries in chunks of floor(kPairCap / k).
 int launch_knn_bwd(const KnnArgs& A0, hipStream_t st) {
     KnnArgs A = A0;
     const uint32_t chunk = std::max<uint32_t>(1u, std::min<uint32_t>(kBwdChunk, (uint32_t)kPairCap / A.k));
-    A.chain = chunk * std::max(1u, knn_chain(A.n) / chunk);  // whole chunks, at most 16 queries
+    A.chain = chunk * std::max(1u, std::min(16u, A.n / 24576u) / chunk);  // whole chunks, at most 16 queries
     const uint64_t per_block = (uint64_t)kWavesPerBlock * A.chain;
     dim3 block(64 * kWavesPerBlock), grid((uint32_t)((A.n + per_block - 1) / per_block));
     const uint32_t need = A.k + 64;
@@ -1361,7 +1368,7 @@ int launch_knn_bwd(const KnnArgs& A0, hipStream_t st) {
 template <int kMode>
 int launch_knn(const KnnArgs& A0, hipStream_t st) {
     KnnArgs A = A0;
-    A.chain = knn_chain(A.n);
+    A.chain = knn_chain(A.n, A.boxes.p != nullptr);
     const uint64_t per_block = (uint64_t)kWavesPerBlock * A.chain;
     dim3 block(64 * kWavesPerBlock), grid((uint32_t)((A.n + per_block - 1) / per_block));
     uint32_t need = A.k + 64;
