@@ -60,22 +60,26 @@ def test_chains(orc, cuda, order, k, rmax):
         assert np.array_equal(got["boxes"][c], got["words"][c]), c
 
 
-@pytest.mark.parametrize("n", [12 * 8192 * 16 - 1, 12 * 8192 * 16, 8 * 24576 + 5])
-def test_long_chains(orc, cuda, n):
-    # chains of 8, and of 16 from a dozen rounds of waves on; over node words 8 at most
+@pytest.mark.parametrize("n,rmax", [(12 * 8192 * 16 - 1, 0.4), (12 * 8192 * 16, 0.4), (8 * 24576 + 5, 0.4),
+                                    (8 * 24576 + 5, 0.03), (12 * 8192 * 16, 0.03)])
+def test_long_chains(orc, cuda, n, rmax):
+    # chains of 8, and of 16 from a dozen rounds of waves on; over node words 8 at most.  Within the small
+    # radius most queries find fewer than k, one after the other, and some find more
     rng = np.random.default_rng(n)
     pos, power, pdir = _map(rng, 4000)
     qp = f4(_path(rng, n))
     q = [api.dev(a) for a in (qp, f4(np.ones((n, 3))), f4(-np.ones((n, 3))), f4(np.ones((n, 3))))]
-    P = api.build_points(pos, api.default_params(N.KIND_POINT, ROOT, 0.4))
+    P = api.build_points(pos, api.default_params(N.KIND_POINT, ROOT, rmax))
     api.attach_photon_records(P, pos, power, pdir)
     words = api.DeviceTree(N.KIND_POINT, N.Tree.from_buffer_copy(P.t), batch=P)
     words.t.owns_qnodes = 0
-    print(f"{n} queries", flush=True)
-    a, b = (api.knn_gather(t, 10, 0.4, *q, want_nbr=True, want_r2=True, want_count=True) for t in (P, words))
+    print(f"{n} queries, radius {rmax}", flush=True)
+    a, b = (api.knn_gather(t, 10, rmax, *q, want_nbr=True, want_r2=True, want_count=True) for t in (P, words))
     for c in ("rad", "nbr", "r2", "count"):
         assert cuda.equal(a[c].view(cuda.int32), b[c].view(cuda.int32)), c
     some = np.concatenate([np.arange(2000), rng.integers(0, n, 2000), np.arange(n - 2000, n)])
-    nbr, cnt = orc.knn_brute(pos, qp[some], 10, 0.4)
+    nbr, cnt = orc.knn_brute(pos, qp[some], 10, rmax)
     assert np.array_equal(a["count"].cpu().numpy().view(np.uint32)[some], cnt)
     assert np.array_equal(a["nbr"].cpu().numpy().view(np.uint32)[some], nbr)
+    found = a["count"].cpu().numpy()
+    assert (found >= 10).any() and ((found < 10).mean() > 0.2) == (rmax < 0.1)
