@@ -100,12 +100,8 @@ extern "C" int mnrt_scan_u32_counted(const uint32_t* d_in, const uint32_t* d_cou
     hipStream_t st = (hipStream_t)stream;
     void* buf = nullptr;
     MNRT_HIP_CHECK(pool_alloc(&buf, (size_t)dscan_tiles(capacity) * 4, st));
-    DScanSet S{};
-    S.in[0] = d_in;
-    S.out[0] = d_out;
-    S.total[0] = d_total;
-    S.end_total = end_total ? 1u : 0u;
-    int rc = dscan(S, 1, dn(d_count, capacity), (uint32_t*)buf, st) == hipSuccess ? MNRT_OK : MNRT_ERR_HIP;
+    const DScan S{d_in, d_out, d_total, (uint32_t*)buf, end_total ? 1u : 0u};
+    int rc = dscan(S, dn(d_count, capacity), st) == hipSuccess ? MNRT_OK : MNRT_ERR_HIP;
     if (pool_free(buf, st) != hipSuccess && rc == MNRT_OK) rc = MNRT_ERR_HIP;
     return rc;
 }

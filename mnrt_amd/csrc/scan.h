@@ -151,26 +151,23 @@ inline hipError_t scan_exclusive(const uint32_t* in, uint32_t* out, uint32_t n, 
 
 // ---- scans of a device count: n = DN::get(), read by every kernel of the scan, so the
 // launches below can be recorded once and replayed on other sizes (up to the capacity n.v).
-// A capacity of at most kScanBig is scanned by one workgroup per scan (one launch);
-// larger ones reduce each 2048-element tile to its total (tiles_cap words per scan), then
+// A capacity of at most kScanBig is scanned by one workgroup (one launch);
+// larger ones reduce each 2048-element tile to its total, then
 // scan each tile from the sum of the totals before it (two launches; blocks stride over the
 // tiles and carry that sum from one of their tiles to the next).
-constexpr int kScanSetMax = 4;
-struct DScanSet {
-    const uint32_t* in[kScanSetMax];
-    uint32_t* out[kScanSetMax];
-    uint32_t* total[kScanSetMax];  // may be null
-    uint32_t* sums;                // tiles_cap words per scan
-    uint32_t tiles_cap;
-    uint32_t end_total;            // 1: the total is also written to out[n]
+struct DScan {
+    const uint32_t* in;
+    uint32_t* out;
+    uint32_t* total;     // may be null
+    uint32_t* sums;      // a word per tile
+    uint32_t end_total;  // 1: the total is also written to out[n]
 };
 
-// blockIdx.x picks the scan of the set; n <= kScanBig.
-__global__ __launch_bounds__(kScanBigBlock) void k_dscan_one(DScanSet S, DN dn_) {
+// n <= kScanBig.
+__global__ __launch_bounds__(kScanBigBlock) void k_dscan_one(DScan S, DN dn_) {
     const uint32_t n = dn_.get();
-    const uint32_t y = blockIdx.x;
-    const uint32_t t = block_scan_runs(S.in[y], n, S.out[y], S.total[y]);
-    if (S.end_total && threadIdx.x == kScanBigBlock - 1) S.out[y][n] = t;
+    const uint32_t t = block_scan_runs(S.in, n, S.out, S.total);
+    if (S.end_total && threadIdx.x == kScanBigBlock - 1) S.out[n] = t;
 }
 
 // Sum of one value per thread over the block, returned to every thread.  s_red: at least
@@ -188,13 +185,12 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* s_red) {
     return r;
 }
 
-__global__ __launch_bounds__(kScanBlock) void k_dscan_reduce(DScanSet S, DN dn_) {
+__global__ __launch_bounds__(kScanBlock) void k_dscan_reduce(DScan S, DN dn_) {
     __shared__ uint32_t s_red[kScanBlock / 64];
     const uint32_t n = dn_.get();
     const uint32_t tiles = (n + kScanTile - 1) / kScanTile;
-    const uint32_t y = blockIdx.y;
-    const uint32_t* in = S.in[y];
-    uint32_t* sums = S.sums + (size_t)y * S.tiles_cap;
+    const uint32_t* in = S.in;
+    uint32_t* sums = S.sums;
     for (uint32_t t = blockIdx.x; t < tiles; t += gridDim.x) {  // uniform per block
         const size_t base = (size_t)t * kScanTile + (size_t)threadIdx.x * kScanPerThread;
         uint32_t local = 0;
@@ -209,15 +205,14 @@ __global__ __launch_bounds__(kScanBlock) void k_dscan_reduce(DScanSet S, DN dn_)
 }
 
 // in and out may alias: each thread reads its elements before writing them.
-__global__ __launch_bounds__(kScanBlock) void k_dscan_scan(DScanSet S, DN dn_) {
+__global__ __launch_bounds__(kScanBlock) void k_dscan_scan(DScan S, DN dn_) {
     __shared__ uint32_t s_wave[kScanBlock / 64];
     __shared__ uint32_t s_red[kScanBlock / 64];
     const uint32_t n = dn_.get();
     const uint32_t tiles = (n + kScanTile - 1) / kScanTile;
-    const uint32_t y = blockIdx.y;
-    const uint32_t* in = S.in[y];
-    uint32_t* out = S.out[y];
-    const uint32_t* sums = S.sums + (size_t)y * S.tiles_cap;
+    const uint32_t* in = S.in;
+    uint32_t* out = S.out;
+    const uint32_t* sums = S.sums;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     uint32_t prefix = 0, done = 0;  // prefix = sum of sums[0 .. done)
     for (uint32_t t = blockIdx.x; t < tiles; t += gridDim.x) {  // uniform per block
@@ -247,35 +242,31 @@ __global__ __launch_bounds__(kScanBlock) void k_dscan_scan(DScanSet S, DN dn_) {
             run += v[j];
         }
         if (t == tiles - 1 && tid == kScanBlock - 1) {
-            if (S.total[y]) *S.total[y] = run;
+            if (S.total) *S.total = run;
             if (S.end_total) out[n] = run;
         }
         __syncthreads();  // s_wave is rewritten by the next tile
     }
     if (tiles == 0 && blockIdx.x == 0 && tid == 0) {
-        if (S.total[y]) *S.total[y] = 0u;
+        if (S.total) *S.total = 0u;
         if (S.end_total) out[0] = 0u;
     }
 }
 
-// Tiles (scratch words per scan) for a device-count scan of capacity cap.
+// Tiles (scratch words) of a device-count scan of capacity cap.
 inline uint32_t dscan_tiles(uint32_t cap) { return std::max<uint32_t>(1u, (cap + kScanTile - 1) / kScanTile); }
 
-// m (<= kScanSetMax) exclusive scans of the device count n (capacity n.v): out[y][i] =
-// sum(in[y][0..i)), *total[y] (may be null) = the sum, and out[y][n] too when end_total.
-// scratch: m * dscan_tiles(n.v) words.  Kernels only: the sequence can be captured.
-inline hipError_t dscan(const DScanSet& S0, int m, DN n, uint32_t* scratch, hipStream_t st) {
-    if (m <= 0 || m > kScanSetMax) return hipErrorInvalidValue;
-    DScanSet S = S0;
-    S.sums = scratch;
-    S.tiles_cap = dscan_tiles(n.v);
+// Exclusive scan of the device count n (capacity n.v): S.out[i] = sum(S.in[0..i)), *S.total the sum, and
+// S.out[n] too when end_total.  S.sums: dscan_tiles(n.v) words.  Kernels only: the sequence can be
+// captured.
+inline hipError_t dscan(const DScan& S, DN n, hipStream_t st) {
     if (n.v <= kScanBig) {
-        hipLaunchKernelGGL(k_dscan_one, dim3(m), dim3(kScanBigBlock), 0, st, S, n);
+        hipLaunchKernelGGL(k_dscan_one, dim3(1), dim3(kScanBigBlock), 0, st, S, n);
         return hipGetLastError();
     }
-    const uint32_t grid = std::min<uint32_t>(S.tiles_cap, 1024u);
-    hipLaunchKernelGGL(k_dscan_reduce, dim3(grid, m), dim3(kScanBlock), 0, st, S, n);
-    hipLaunchKernelGGL(k_dscan_scan, dim3(grid, m), dim3(kScanBlock), 0, st, S, n);
+    const uint32_t grid = std::min<uint32_t>(dscan_tiles(n.v), 1024u);
+    hipLaunchKernelGGL(k_dscan_reduce, dim3(grid), dim3(kScanBlock), 0, st, S, n);
+    hipLaunchKernelGGL(k_dscan_scan, dim3(grid), dim3(kScanBlock), 0, st, S, n);
     return hipGetLastError();
 }
 
