@@ -76,21 +76,6 @@ inline BoxTree box_tree(const mnrt_tree& t) {
     return b;
 }
 
-// The hierarchy for the queries of one tree: none where the tree is kDeepLevels deeper than a balanced one
-// over its photons would be, as it is where their density differs so much from place to place that runs of
-// 64 and 4096 consecutive records reach across many cells: their boxes lie over each other, and the walk
-// over node words is the faster one.  (A batch walks what its trees have: its phases may be captured
-// before a tree is built again.)  Levels beyond the balanced ones: 9 for 1M photons of a room, 13 where half
-// of them lie in eight spots, 14 for 20,001 of those; with cubes of normal coordinates 28, 27 and 20 for 1M,
-// 200,000 and 20,001.  k = 50, us, boxes / node words, 1M of the last: 4096 queries 180 / 64, 784,641
-// 4780 / 3081, 2.07M 10400 / 6772; 200,000: 62 / 60, 2874 / 2525, 6917 / 6255; 20,001: 64 / 47, 2541 / 2313.  1M with the
-// eight spots, camera hits: 4096 40 / 32, 784,641 997 / 1109, 2.07M 2152 / 2699.
-constexpr uint32_t kDeepLevels = 17;
-inline BoxTree query_boxes(const mnrt_tree& t) {
-    const uint32_t balanced = 32u - (uint32_t)__builtin_clz(t.num_elems | 1u);
-    return t.max_level > balanced + kDeepLevels ? BoxTree{} : box_tree(t);
-}
-
 __device__ __forceinline__ float wave_min_f32(float v) {
     auto dpp = [](float x, auto ctrl) { return __uint_as_float(dpp_mov<decltype(ctrl)::value>(__float_as_uint(x))); };
     v = fminf(v, dpp(v, std::integral_constant<int, kDppPairSwap>{}));

@@ -1515,7 +1515,7 @@ extern "C" int mnrt_knn_gather(const mnrt_tree* pmap, uint32_t k, float r_max, u
     mnrt::KnnArgs A{};
     A.nodes = (const uint2*)(pmap->d_qnodes ? pmap->d_qnodes : pmap->d_nodes);
     A.recs = (const float4*)pmap->d_recs;
-    A.boxes = mnrt::query_boxes(*pmap);
+    A.boxes = mnrt::box_tree(*pmap);
     A.k = k;
     A.r2max = r_max * r_max;
     A.r_max = r_max;
@@ -1590,7 +1590,7 @@ extern "C" int mnrt_knn_gather_noalloc(const mnrt_tree* pmap, uint32_t k, float 
     mnrt::KnnArgs A{};
     A.nodes = (const uint2*)(pmap->d_qnodes ? pmap->d_qnodes : pmap->d_nodes);
     A.recs = (const float4*)pmap->d_recs;
-    A.boxes = mnrt::query_boxes(*pmap);
+    A.boxes = mnrt::box_tree(*pmap);
     A.k = k;
     A.r2max = r_max * r_max;
     A.r_max = r_max;
@@ -1642,7 +1642,7 @@ extern "C" int mnrt_knn_radii(const mnrt_tree* pmap, uint32_t k, float r_max, ui
     mnrt::KnnArgs A{};
     A.nodes = (const uint2*)(pmap->d_qnodes ? pmap->d_qnodes : pmap->d_nodes);
     A.recs = (const float4*)pmap->d_recs;
-    A.boxes = mnrt::query_boxes(*pmap);
+    A.boxes = mnrt::box_tree(*pmap);
     A.k = k;
     A.r2max = r_max * r_max;
     A.r_max = r_max;
@@ -1706,7 +1706,7 @@ extern "C" int mnrt_knn_gather_bwd(const mnrt_tree* pmap, uint32_t k, float r_ma
         A.order_far = order_far;
         A.nodes = (const uint2*)(pmap->d_qnodes ? pmap->d_qnodes : pmap->d_nodes);
         A.recs = (const float4*)pmap->d_recs;
-        A.boxes = mnrt::query_boxes(*pmap);
+        A.boxes = mnrt::box_tree(*pmap);
         A.k = k;
         A.r2max = r_max * r_max;
         A.r_max = r_max;
