@@ -108,7 +108,10 @@ typedef struct mnrt_tree {
 
 /* owns_qnodes bits: the library allocated d_qnodes; a box hierarchy over the photon records
  * precedes d_qnodes (mnrt_tree_attach_photon_records and the batched and recorded builds
- * make it; kNN queries then read it instead of the node words). */
+ * make it; kNN queries then read it instead of the node words).  Ownership is the first bit, not
+ * the word: the trees of a batch or a recorded build that own nothing have the second alone.
+ * A caller that puts node words of its own in d_qnodes sets owns_qnodes to 0, or queries read
+ * what lies in front of them as boxes. */
 #define MNRT_QNODES_OWNED 1u
 #define MNRT_QNODES_BOXES 2u
 
@@ -213,8 +216,10 @@ int mnrt_tree_attach_photon_records(mnrt_tree* tree, const float* d_pos4, const 
 /* Query-time node words: every inner node whose subtree holds at most max_refs leaf
  * references becomes a leaf over that contiguous reference range (a subtree's leaves are
  * consecutive in preorder).  A wave then tests such a subtree's elements in one step.
- * The build's node words (d_nodes) are unchanged; queries read d_qnodes.  Query results
- * do not depend on it.  mnrt_tree_attach_photon_records applies max_refs = 512. */
+ * The build's node words (d_nodes) are unchanged; queries read d_qnodes, or the box hierarchy
+ * where there is one.  Query results do not depend on it.  mnrt_tree_attach_photon_records
+ * applies max_refs = 512, with a hierarchy where the tree has no words yet or, before its first
+ * records, words of this call: words that queries may have read stay where they are. */
 int mnrt_tree_collapse(mnrt_tree* tree, uint32_t max_refs, void* stream);
 
 /* Reference KDTreeData layout of a tree (KDTreeData, KDKernelDefs.h:76-194, as

@@ -298,7 +298,7 @@ constexpr uint32_t kWords = W_LEVELS + kLevelWords * (kLevels + 1);
 constexpr uint32_t kErrRoom = 64u;          // a buffer was outgrown
 constexpr uint32_t kErrLevels = 128u;       // active nodes left after the last recorded level
 constexpr uint32_t kErrOutputRoom = 256u;   // the trees outgrew the output arrays
-constexpr uint32_t kErrLayoutDepth = 512u;  // a build node deeper than the recording covers
+constexpr uint32_t kErrLayoutDepth = 512u;  // a leaf deeper than a recording promises (kLayoutSpareLevels)
 
 struct BuildCaps {
     uint32_t na;     // active nodes of a level
@@ -2084,7 +2084,8 @@ int build_batch_impl(int kind, const float* d_v0, const float* d_v1, const float
 // a recorded number of levels.  Capacities come from a host-driven build of the same scenes (its
 // BuildStats) with a margin; whatever would outgrow them sets an error bit instead.
 
-// Levels a recorded build covers beyond the first build's deepest large-stage node.
+// Levels a recorded build covers beyond the first build's deepest large-stage node.  The layout climbs
+// parent links and could place deeper trees too: the limit is what mnrt_build_graph_status states.
 constexpr uint32_t kLayoutSpareLevels = 6u;
 
 // Active nodes left after the last recorded level.

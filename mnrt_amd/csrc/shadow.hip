@@ -169,8 +169,8 @@ static int launch_any_hit(int mode, const mnrt_tree* tree, const LightArgs& L, u
         rb.lo[a] = tree->root_min[a];
         rb.hi[a] = tree->root_max[a];
     }
-    // A wave per window: further windows from a counter, as closest hits take them, are slower for all
-    // but the longest searches (20000 triangles: 785 k point segments 332 -> 361 us, 1.76M 416 -> 592;
+    // A wave per window and no others' windows: with windows from a counter, which helps bounce rays, all but
+    // the longest searches are slower (20000 triangles: 785 k point segments 332 -> 361 us, 1.76M 416 -> 592;
     // 205001 triangles, 785 k area segments 790 -> 787, 1.76M 1446 -> 1239).
     const uint32_t width = trace_width(n);
     const dim3 grid(trace_windows(n, width)), block(64);

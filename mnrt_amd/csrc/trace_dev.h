@@ -25,8 +25,9 @@
 //     the lanes' own leaves are about as full as each other, when each lane tests its own.
 // Bound by instruction issue: about 25 k vector instructions per 64 bounce rays of the 1.03M-triangle
 // scene (206 walk steps with 29 lanes, 85 dealt tests with 49 pairs, 37 own tests), 83 tests and 93
-// steps a ray.  2.07M bounce rays 2248 -> 1466 us, 785 k area-light shadow rays 830 -> 573 us,
-// 6144 camera rays 67 -> 47 us, 1.69M camera rays (205001 triangles) 1048 -> 1010 us.
+// steps a ray.  A lane per ray and now, us: 2.07M bounce rays of 1.03M triangles 2698 and 1738, 785 k
+// area-light shadow rays of 205001 triangles 981 and 781, 6144 camera rays of 1294 triangles 63 and 46;
+// 2.07M camera rays of 1.03M triangles 1043 and 977, of 205001 1172 and 1264, of 1294 213 and 221.
 #pragma once
 
 #include "mnrt_common.h"
@@ -81,7 +82,7 @@ constexpr uint32_t kTraceWords = 256u + 3u * 64u * (uint32_t)kTraceLds;
 // than new waves do (1.69M bounce rays 1483 us with windows from a counter, a wave per window 2093).  Rays
 // that go together, or miss the root box, leave the rest to the hardware.  2.07M rays with a window from
 // a counter for every 64, whose atomics come 12 ns apart, and now: camera rays of 1294 triangles 420 and
-// 226 us, of which most miss the box 398 and 50, of 1.03M triangles 1002 and 977; bounce rays of 1.03M 1713 and
+// 221 us, of which most miss the box 398 and 50, of 1.03M triangles 1002 and 977; bounce rays of 1.03M 1713 and
 // 1738 (two atomics a window, and waves that find theirs taken).  (From the end by a fixed stride
 // instead of a count: bounce rays 5 to 10 % slower, camera rays up to 9 % faster; 128 rays a window: bounce
 // rays 4 to 7 % slower; a fixed share of the rays for every wave that fits at once: waves of slow rays end
